@@ -143,30 +143,20 @@ __device__ void lookahead_consts(const DevCell &C, CellDyn &d, double dt, bool f
     step_consts_f32(d.kf[slot], d.k[slot]);
 }
 
-__device__ void sum_block_partials(const Partial *parts, int64_t first, int n, Partial &tot)
-{
-    fx_zero(tot.jlcc); fx_zero(tot.jxfer); fx_zero(tot.jtr); fx_zero(tot.jrel);
-    tot.clch = 0; tot.open = 0; tot.iters = 0; tot.err = 0;
-    for (int b = 0; b < n; ++b) {
-        const Partial &q = parts[first + b];
-        fx_add(tot.jlcc, q.jlcc);
-        fx_add(tot.jxfer, q.jxfer);
-        fx_add(tot.jtr, q.jtr);
-        fx_add(tot.jrel, q.jrel);
-        tot.clch += q.clch;
-        tot.open += q.open;
-        tot.iters += q.iters;
-        tot.err |= q.err;
-    }
-}
+// Exact sums over a cell's CRUs.
+struct FluxTotals {
+    Fx jlcc, jxfer, jtr, jrel;
+    int64_t clch, open;
+    int32_t err;
+};
 
-__device__ __forceinline__ void partial_zero(Partial &m)
+__device__ __forceinline__ void totals_zero(FluxTotals &m)
 {
     fx_zero(m.jlcc); fx_zero(m.jxfer); fx_zero(m.jtr); fx_zero(m.jrel);
-    m.clch = 0; m.open = 0; m.iters = 0; m.err = 0;
+    m.clch = 0; m.open = 0; m.err = 0;
 }
 
-__device__ void partial_add(Partial &a, const Partial &b)
+__device__ void totals_add(FluxTotals &a, const FluxTotals &b)
 {
     fx_add(a.jlcc, b.jlcc);
     fx_add(a.jxfer, b.jxfer);
@@ -174,31 +164,18 @@ __device__ void partial_add(Partial &a, const Partial &b)
     fx_add(a.jrel, b.jrel);
     a.clch += b.clch;
     a.open += b.open;
-    a.iters += b.iters;
     a.err |= b.err;
 }
 
-__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
+// The 128-bit value of three limb sums.
+__device__ __forceinline__ Fx limbs_fx(uint64_t S0, uint64_t S1, uint64_t S2)
 {
-    return static_cast<uint64_t>(__shfl_xor(static_cast<unsigned long long>(v), m));
-}
-
-// Exact sum of a partial over the 64 lanes of the calling wave, left in every
-// lane (a butterfly of lane exchanges). Every lane of the wave must call it.
-__device__ void partial_wave_sum(Partial &p)
-{
-    for (int m = kWave / 2; m > 0; m >>= 1) {
-        Partial o;
-        o.jlcc.lo = shfl_xor_u64(p.jlcc.lo, m);   o.jlcc.hi = shfl_xor_u64(p.jlcc.hi, m);
-        o.jxfer.lo = shfl_xor_u64(p.jxfer.lo, m); o.jxfer.hi = shfl_xor_u64(p.jxfer.hi, m);
-        o.jtr.lo = shfl_xor_u64(p.jtr.lo, m);     o.jtr.hi = shfl_xor_u64(p.jtr.hi, m);
-        o.jrel.lo = shfl_xor_u64(p.jrel.lo, m);   o.jrel.hi = shfl_xor_u64(p.jrel.hi, m);
-        o.clch = static_cast<int64_t>(shfl_xor_u64(static_cast<uint64_t>(p.clch), m));
-        o.open = static_cast<int64_t>(shfl_xor_u64(static_cast<uint64_t>(p.open), m));
-        o.iters = shfl_xor_u64(p.iters, m);
-        o.err = __shfl_xor(p.err, m);
-        partial_add(p, o);
-    }
+    Fx f;
+    f.lo = S0;
+    f.hi = 0;
+    fx_add_raw(f, S1 << 43, S1 >> 21);
+    fx_add_raw(f, 0, S2 << 22);
+    return f;
 }
 
 // Exact per-block sums of the SSA outputs. Each output's 128-bit fixed-point
@@ -228,25 +205,25 @@ __device__ __forceinline__ void acc_add_fx(BlockAcc &A, int q, const Fx &f)
     atomicAdd(&A.limb[q][2], static_cast<unsigned long long>(static_cast<int64_t>(f.hi) >> 22));
 }
 
-__device__ __forceinline__ Fx acc_fx(const BlockAcc &A, int q)
+// The block's partial of one step: its accumulators, one word per thread.
+__device__ __forceinline__ void write_partial(const KArgs &a, const BlockAcc &A, int64_t index)
 {
-    const uint64_t S0 = A.limb[q][0], S1 = A.limb[q][1], S2 = A.limb[q][2];
-    Fx f;
-    f.lo = S0;
-    f.hi = 0;
-    fx_add_raw(f, S1 << 43, S1 >> 21);
-    fx_add_raw(f, 0, S2 << 22);
-    return f;
+    static_assert(sizeof(BlockAcc) == sizeof(Partial), "a partial is the block's accumulators");
+    const int t = threadIdx.x;
+    if (t < PW_N) {
+        const uint64_t v = (&A.limb[0][0])[t];
+        a.partials[index].w[t] = t == PW_ERR ? (v != 0) : v;
+    }
 }
 
 template <int NT>
-__device__ void block_reduce(Partial *red, Partial mine)
+__device__ void block_reduce(FluxTotals *red, FluxTotals mine)
 {
     const int tid = threadIdx.x;
     red[tid] = mine;
     __syncthreads();
     for (int s = NT / 2; s > 0; s >>= 1) {
-        if (tid < s) partial_add(red[tid], red[tid + s]);
+        if (tid < s) totals_add(red[tid], red[tid + s]);
         __syncthreads();
     }
 }
@@ -310,12 +287,12 @@ __global__ void k_sample_rest(KArgs a)
 // ClCh of the given state -- then derivatives and SSA constants.
 __global__ void k_init_cells(KArgs a)
 {
-    __shared__ Partial red[kBlock];
+    __shared__ FluxTotals red[kBlock];
     const int cell = blockIdx.x;
     const DevCell &C = a.cells[cell];
     CellDyn &D = a.dyn[cell];
-    Partial mine;
-    partial_zero(mine);
+    FluxTotals mine;
+    totals_zero(mine);
     const double X = C.p.rxfer * (1.45370e-4 - 1.45273e-4);
     const double X4 = X + X + X + X;
     const double Y = C.p.rtr * (0.908882 - 0.908408);
@@ -334,7 +311,7 @@ __global__ void k_init_cells(KArgs a)
     }
     block_reduce<kBlock>(red, mine);
     if (threadIdx.x == 0) {
-        const Partial &t = red[0];
+        const FluxTotals &t = red[0];
         FluxSums S{fx_to_double(t.jlcc), fx_to_double(t.jxfer), fx_to_double(t.jtr), static_cast<double>(t.clch)};
         D.sums[0] = S.JLCC; D.sums[1] = S.Jxfer; D.sums[2] = S.Jtr; D.sums[3] = S.ClCh;
         D.sums[4] = static_cast<double>(t.open); D.sums[5] = 0.0;
@@ -454,46 +431,56 @@ __device__ __forceinline__ void ssa_block(const KArgs &a, int b, int64_t step0, 
         atomicAdd(&acc.ints[j], static_cast<unsigned long long>(iv));
     }
     __syncthreads();
-    if (tid == 0) {
-        Partial p;
-        p.jxfer = acc_fx(acc, 0);
-        p.jtr = acc_fx(acc, 1);
-        p.jlcc = acc_fx(acc, 2);
-        p.jrel = acc_fx(acc, 3);
-        p.iters = acc.ints[0];
-        p.open = static_cast<int64_t>(acc.ints[1]);
-        p.clch = static_cast<int64_t>(acc.ints[2]);
-        p.err = acc.ints[3] ? 1 : 0;
-        p.tag = 0;
-        a.partials[ks * a.nblocks + b] = p;
-    }
+    write_partial(a, acc, ks * a.nblocks + b);
 }
 
-constexpr int kGd0 = 7;   // V, Nai, Ki, Cai, CaNSR, CaLTRPN, CaHTRPN: the globals gd_finish_main derives
+// ---------------------------------------------------------------------------
+// The close of one cell's step, a block's work. A step of a small batch lasts
+// as long as this chain of dependent FP64 arithmetic, so it is cut into four
+// roles that run on the block's waves side by side (in turn where the block
+// has fewer waves) between three barriers, and within a role one value per
+// lane wherever the same operations serve many values:
+//   1. load:    parameters, globals and block partials, all in flight at once;
+//   2. values:  role 0 the exponentials of the derivatives, one per lane;
+//               role 1 the logarithms, the powers and the IK1 exponential, one
+//               per lane; role 2 the stimulus; role 3 the sums of the partials;
+//   3. terms:   role 0 the K currents; role 1 the Na and Ca currents and
+//               the uptake; role 2 the Kv chains, one generator entry, then one
+//               derivative per lane; role 3 the gates, the IKr chain and
+//               the currents formed from the sums;
+//   4. joining: roles 0 and 1 the increments and the next step's constants
+//               (its exponentials, then the rows of its LCC table, one per
+//               lane); role 2 observables and trace; role 3 the stores.
+// Each value is formed by the operations of the serial gd_finish and
+// step_consts, in their order, so the results are the same bits. Timed in one
+// cell of 12,500 CRUs: 26,500 cycles for the form that ran the sums as a
+// butterfly of 128-bit adds and the terms on single lanes.
+// ---------------------------------------------------------------------------
+constexpr int kGd0 = 7;   // V, Nai, Ki, Cai, CaNSR, CaLTRPN, CaHTRPN: the globals gd_combine derives
+constexpr int kSumLanes = PW_N / 2;   // lanes that read one partial, two words each
 
-// LDS of a close block. The working set of the close reuses the slots of the
-// partial-sum reduction once its total has been read.
+template <int NT>
 struct CloseLds {
+    static constexpr int kWaves = NT / kWave;
+    static constexpr int kGroups = NT / kSumLanes;
+    uint64_t red[kGroups][PW_N];  // partial sums by group of lanes
     double g[36];            // the globals the derivatives start from (gw_globals_t order)
-    double x[GD_N];          // arguments, then values, of the batched transcendentals
-    double py[GD_N - GD_POW0];
-    double sx[SC_N];         // arguments, then values, of the next step's constants
-    double lookahead[3];     // V, Cai, CaNSR of the next step
+    double x[GD_X];          // the values of the transcendentals
     double ch[29];           // the derivatives of the gates m, h, j, xKs and of the IKr, Kv4.3 and
                              // Kv1.4 chains (the last 29 globals, gw_globals_t order)
-    double dg0[kGd0];        // the derivatives of V and the concentrations (the first 7 globals)
+    double q[2][kv::kEntries];   // the generator entries of the Kv1.4 and Kv4.3 chains
+    double beta_cyto, dLTRPN, dHTRPN;
     double Istim;            // the stimulus of the new time
-    double ICaL;             // I_CaL of the close, for the observables
-    gw_params_t p;           // the cell's parameters, derived constants and observables,
-    CellConsts c;            // staged for the serial part (which would otherwise wait on
-    gw_cell_obs_t obs;       // them load by load)
-};
-union CloseShared {
-    Partial red[kWave];
-    CloseLds L;
+    double S[4];             // JLCC, Jxfer, Jtr and ClCh of the step's SSA
+    double jrel;
+    int64_t open;
+    int32_t err;
+    Currents cur;
+    gw_params_t p;           // the cell's parameters, derived constants and observables, staged
+    CellConsts c;            // once (each would otherwise be waited on load by load)
+    gw_cell_obs_t obs;
 };
 static_assert(sizeof(gw_globals_t) == 36 * sizeof(double), "globals are 36 doubles");
-static_assert(sizeof(CloseLds) <= sizeof(Partial) * kWave, "the close's working set fits the reduction slots");
 static_assert(sizeof(gw_params_t) % 8 == 0 && sizeof(CellConsts) % 8 == 0, "staged as 8-byte words");
 static_assert(offsetof(gw_globals_t, h) == offsetof(gw_globals_t, m) + sizeof(double) &&
                   offsetof(gw_globals_t, xKs) == offsetof(gw_globals_t, m) + 3 * sizeof(double) &&
@@ -504,26 +491,48 @@ static_assert(offsetof(gw_globals_t, h) == offsetof(gw_globals_t, m) + sizeof(do
                   offsetof(gw_globals_t, m) == kGd0 * sizeof(double),
               "the gates and the three chains are the last 29 globals: m, h, j, xKs, Kr, Kv4.3, Kv1.4");
 
+// Two adjacent words of a partial; COH reads them past the caches (the
+// persistent kernel's SSA blocks write them that way within the launch).
+template <bool COH>
+__device__ __forceinline__ void partial_pair(const uint64_t *p, uint64_t &x, uint64_t &y)
+{
+    if constexpr (COH) {
+        const unsigned long long *q = reinterpret_cast<const unsigned long long *>(p);
+        x = __hip_atomic_load(q, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        y = __hip_atomic_load(q + 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    } else {
+        const ulonglong2 v = *reinterpret_cast<const ulonglong2 *>(p);
+        x = v.x;
+        y = v.y;
+    }
+}
+
+__device__ __forceinline__ uint64_t shfl_u64(uint64_t v, int lane)
+{
+    return static_cast<uint64_t>(__shfl(static_cast<unsigned long long>(v), lane));
+}
+__device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
+{
+    return static_cast<uint64_t>(__shfl_xor(static_cast<unsigned long long>(v), m));
+}
+
 // Close step n = D.step of one cell: the exact sum of the cell's block
 // partials of step n, globals += dGlobals (GW.tpp:252-271), t += dt, the
 // derivatives of step n+1, observables and trace, and the SSA constants of
 // step n+2 (those of step n+1 were formed one close earlier and are in use by
-// the SSA blocks running beside this one). The step's 42 exponentials,
-// logarithms and powers that depend on the state alone are evaluated one per
-// lane, and the 5 exponentials of the next step's constants likewise; the
-// rest is the serial arithmetic of prepare_step and lookahead_consts. Every
-// thread of the block takes part (the block synchronises).
-// D is the cell's dynamic state: a.dyn[cell], or in the persistent kernel a
-// copy the close block keeps in LDS for the whole launch. With COH the block
-// partials are read with device-coherent atomic loads (the persistent
-// kernel's SSA blocks write them that way within the launch).
-template <int NS, bool COH = false>
-__device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D, CloseShared &sh)
+// the SSA blocks running beside this one). Every thread of the block (NT)
+// takes part. D is the cell's dynamic state: a.dyn[cell], or in the persistent
+// kernel a copy the close block keeps in LDS for the whole launch.
+template <int NT, bool COH = false>
+__device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D, CloseLds<NT> &L)
 {
+    constexpr int kWaves = NT / kWave;
     const DevCell &C = a.cells[cell];
     const int tid = threadIdx.x;
-    const int nw = static_cast<int>(blockDim.x) / kWave;
-    // the cell's status, step, time and potential, read before the reduction's barriers
+    const int lane = tid & (kWave - 1);
+    const int wave = kWaves > 1 ? __builtin_amdgcn_readfirstlane(tid / kWave) : 0;
+    auto role = [&](int r) { return wave == (r & (kWaves - 1)); };
+    // ---- 1. load
     const int status = D.status;
     const bool clamp = D.clamp != 0;
     const int64_t step_new = D.step + 1;
@@ -531,102 +540,52 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
     const double t_old = D.t;
     const double V_old = D.g.V;
     const double t_new = t_old + a.dt;
-    // the stimulus of the new time, on the last wave (the first leads the
-    // serial part below): formed below while that wave's first block partial
-    // is loading, or here where the partials are read coherently
-    const int istim_tid = (nw - 1) * kWave;
-    double Istim = 0.0;
-    if constexpr (COH) {
-        if (tid == istim_tid && status == 0) Istim = protocol_istim(C, t_new, step_new);
-    }
-    // the parameters, derived constants and observables, loaded now and stored
-    // to LDS once the reduction slots are free
-    constexpr int kPW = sizeof(gw_params_t) / 8, kCW = sizeof(CellConsts) / 8, kOW = sizeof(gw_cell_obs_t) / 8;
-    constexpr int kStage = (kPW + kCW + kOW + NS - 1) / NS;
-    unsigned long long stage[kStage];
-#pragma unroll
-    for (int r = 0; r < kStage; ++r) {
-        const int w = tid + r * NS;
-        stage[r] = 0;
-        if (tid < NS) {
-            if (w < kPW) stage[r] = reinterpret_cast<const unsigned long long *>(&C.p)[w];
-            else if (w < kPW + kCW) stage[r] = reinterpret_cast<const unsigned long long *>(&C.c)[w - kPW];
-            else if (w < kPW + kCW + kOW)
-                stage[r] = reinterpret_cast<const unsigned long long *>(&D.obs)[w - kPW - kCW];
-        }
-    }
-    // this thread's global and its increment, read now for globals_apply below
     double g_in = 0.0, dg_in = 0.0;
     if (tid < 36) {
         g_in = reinterpret_cast<const double *>(&D.g)[tid];
         dg_in = reinterpret_cast<const double *>(&D.dg)[tid];
     }
-    // the block partials: read by every wave (by the first alone where they
-    // are read coherently, after its wait for them), summed within each wave,
-    // then across the waves; the sums are exact, so the order does not matter
-    Partial mine;
-    partial_zero(mine);
+    constexpr int kPW = sizeof(gw_params_t) / 8, kCW = sizeof(CellConsts) / 8, kOW = sizeof(gw_cell_obs_t) / 8;
+    constexpr int kStage = (kPW + kCW + kOW + NT - 1) / NT;
+    unsigned long long stage[kStage];
+#pragma unroll
+    for (int r = 0; r < kStage; ++r) {
+        const int w = tid + r * NT;
+        stage[r] = 0;
+        if (w < kPW) stage[r] = reinterpret_cast<const unsigned long long *>(&C.p)[w];
+        else if (w < kPW + kCW) stage[r] = reinterpret_cast<const unsigned long long *>(&C.c)[w - kPW];
+        else if (w < kPW + kCW + kOW) stage[r] = reinterpret_cast<const unsigned long long *>(&D.obs)[w - kPW - kCW];
+    }
+    const GdArg arg = gd_arg_row(role(0) && lane < GD_LOG0 ? lane : 0);
+    const uint32_t kv_entry = kv::entry(lane < 2 * kv::kEntries ? lane % kv::kEntries : 0);
+    const kv::Row kv_row = kv::row(lane < 20 ? lane % 10 : 0);
     {
         const Partial *src = a.partials + ks * a.nblocks + C.blk0[a.shape];
         const int nb = C.nblk[a.shape];
-        if constexpr (COH) {
-            if (tid < NS) {
-                for (int q = tid; q < nb; q += NS) {
-                    Partial p;
-                    unsigned long long *pw = reinterpret_cast<unsigned long long *>(&p);
-                    const unsigned long long *sw = reinterpret_cast<const unsigned long long *>(src + q);
-                    for (int t = 0; t < static_cast<int>(sizeof(Partial) / 8); ++t)
-                        pw[t] = __hip_atomic_load(sw + t, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-                    partial_add(mine, p);
-                }
-            }
-        } else {
-            // the thread's first partial (the only one where the cell has no
-            // more blocks than the close has threads) is in flight while the
-            // stimulus is formed; the rest two at a time
-            const int nt = static_cast<int>(blockDim.x);
-            int q = tid;
-            Partial first;
-            const bool has_first = q < nb;
-            if (has_first) first = src[q];
-            if (tid == istim_tid && status == 0) Istim = protocol_istim(C, t_new, step_new);
-            if (has_first) partial_add(mine, first);
-            for (q += nt; q + nt < nb; q += 2 * nt) {
-                const Partial p0 = src[q], p1 = src[q + nt];
-                partial_add(mine, p0);
-                partial_add(mine, p1);
-            }
-            if (q < nb) partial_add(mine, src[q]);
-        }
-    }
-    partial_wave_sum(mine);
-    if ((tid & (kWave - 1)) == 0) sh.red[tid / kWave] = mine;
-    __syncthreads();
-    Partial tot = sh.red[0];
-    for (int w = 1; w < nw; ++w) partial_add(tot, sh.red[w]);
-    __syncthreads();   // the reduction slots are reused below
-    if (tid == 0 && a.iters_total) atomicAdd(a.iters_total, static_cast<unsigned long long>(tot.iters));
-    if (status != 0) return;
-    if (tot.err) {
-        if (tid == 0) {
-            D.status = GW_E_RANGE;
-            D.stop_step = step_new + 1;   // SSA(step_new) runs beside this close; none after it
-        }
-        return;
-    }
-    CloseLds &L = sh.L;
+        constexpr int kG = CloseLds<NT>::kGroups;
+        const int w2 = 2 * (tid & (kSumLanes - 1)), grp = tid / kSumLanes;
+        uint64_t s0 = 0, s1 = 0;
+        constexpr int kAhead = COH ? 1 : 4;   // reads in flight per lane
+        int q = grp;
+        for (; q + (kAhead - 1) * kG < nb; q += kAhead * kG) {
+            uint64_t x[kAhead], y[kAhead];
 #pragma unroll
-    for (int r = 0; r < kStage; ++r) {
-        const int w = tid + r * NS;
-        if (tid < NS) {
-            if (w < kPW) reinterpret_cast<unsigned long long *>(&L.p)[w] = stage[r];
-            else if (w < kPW + kCW) reinterpret_cast<unsigned long long *>(&L.c)[w - kPW] = stage[r];
-            else if (w < kPW + kCW + kOW) reinterpret_cast<unsigned long long *>(&L.obs)[w - kPW - kCW] = stage[r];
+            for (int u = 0; u < kAhead; ++u) partial_pair<COH>(src[q + u * kG].w + w2, x[u], y[u]);
+#pragma unroll
+            for (int u = 0; u < kAhead; ++u) {
+                s0 += x[u];
+                s1 += y[u];
+            }
         }
+        for (; q < nb; q += kG) {
+            uint64_t x, y;
+            partial_pair<COH>(src[q].w + w2, x, y);
+            s0 += x;
+            s1 += y;
+        }
+        L.red[grp][w2] = s0;
+        L.red[grp][w2 + 1] = s1;
     }
-    if (nw > 1 && tid == istim_tid) L.Istim = Istim;
-    const FluxSums S{fx_to_double(tot.jlcc), fx_to_double(tot.jxfer), fx_to_double(tot.jtr), static_cast<double>(tot.clch)};
-    const double jrel = fx_to_double(tot.jrel);
     // globals_apply (GW.tpp:252-271), one global per thread; V is held under a
     // clamp and then set to the clamp potential of the new time (prepare_step)
     if (tid < 36) {
@@ -635,131 +594,186 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
         if (tid == 0 && clamp) v = protocol_vclamp(C, t_new);
         L.g[tid] = v;
     }
+#pragma unroll
+    for (int r = 0; r < kStage; ++r) {
+        const int w = tid + r * NT;
+        if (w < kPW) reinterpret_cast<unsigned long long *>(&L.p)[w] = stage[r];
+        else if (w < kPW + kCW) reinterpret_cast<unsigned long long *>(&L.c)[w - kPW] = stage[r];
+        else if (w < kPW + kCW + kOW) reinterpret_cast<unsigned long long *>(&L.obs)[w - kPW - kCW] = stage[r];
+    }
     __syncthreads();
+    // ---- 2. values
     const gw_globals_t &g = *reinterpret_cast<const gw_globals_t *>(L.g);
-    const double VF_RT = g.V * L.c.F_RT;
-    // the arguments of the state-dependent transcendentals: the two halves on
-    // two waves when the block has them
-    if (tid == 0) {
-        gd_args_lo(L.p, g, VF_RT, L.x);
-        if (blockDim.x < 2 * kWave) gd_args_hi(L.p, g, L.x, L.py);
-    } else if (tid == kWave) {
-        gd_args_hi(L.p, g, L.x, L.py);
+    const gw_params_t &p = L.p;
+    const CellConsts &c = L.c;
+    const double VF_RT = g.V * c.F_RT;
+    if (role(0) && lane < GD_LOG0) L.x[lane] = gw::exp(gd_arg_value(arg, p, g.V, VF_RT));
+    if (role(1) && lane < GD_N - GD_LOG0) {
+        const int slot = GD_LOG0 + lane;
+        double y;
+        const double arg1 = gd_log_arg(slot, p, g, y);
+        const double lg = gw::log(arg1);
+        // the powers, and on LK's lane the IK1 exponential, are an exponential of the logarithm
+        const double e = gw::exp(slot == GD_LK ? gd_ik1_arg(c, g.V, lg) : y * lg);
+        L.x[slot] = slot < GD_POW0 ? lg : pow_special(arg1, y, e);
+        if (slot == GD_LK) L.x[GD_IK1] = e;
+    }
+    if (role(2) && lane == 0) L.Istim = status == 0 ? protocol_istim(C, t_new, step_new) : 0.0;
+    if (role(3)) {
+        const int w = lane & (PW_N - 1);
+        uint64_t v = 0;
+        for (int k = lane / PW_N; k < CloseLds<NT>::kGroups; k += kWave / PW_N) v += L.red[k][w];
+        for (int m = PW_N; m < kWave; m <<= 1) v += shfl_xor_u64(v, m);
+        // lane q < 4 recombines flux q; JLCC, Jxfer, Jtr, ClCh into S[0..3]
+        const int q3 = 3 * (lane & 3);
+        const double f = fx_to_double(limbs_fx(shfl_u64(v, q3), shfl_u64(v, q3 + 1), shfl_u64(v, q3 + 2)));
+        if (lane < 3) L.S[lane == 2 ? 0 : lane + 1] = f;
+        else if (lane == 3) L.jrel = f;
+        else if (lane == PW_CLCH) L.S[3] = static_cast<double>(static_cast<int64_t>(v));
+        else if (lane == PW_OPEN) L.open = static_cast<int64_t>(v);
+        else if (lane == PW_ERR) L.err = static_cast<uint32_t>(v) != 0;
+        else if (lane == PW_ITERS && a.iters_total) atomicAdd(a.iters_total, static_cast<unsigned long long>(v));
     }
     __syncthreads();
-    if (tid < GD_N) {
-        const double v = gd_eval(tid, L.x[tid], tid >= GD_POW0 ? L.py[tid - GD_POW0] : 0.0);
-        L.x[tid] = v;   // each thread reads and then overwrites its own slot
-    }
-    __syncthreads();
-    // gd_finish: the currents, concentrations and V on lane 0 of wave 0; the
-    // gates and the three K-channel chains on the block's second and third
-    // waves when it has them (they read only the parameters, the globals and
-    // the evaluated exponentials), on lane 0 otherwise
-    if (tid == 0) {
-        Currents cur;
-        gw_globals_t dg;
-        if (nw > 1) Istim = L.Istim;
-        const int rc = gd_finish_main(L.p, L.c, g, VF_RT, L.x, a.dt, Istim, S, dg, cur);
-        if (rc != GW_OK) D.status = rc;
-        L.ICaL = cur.ICaL;
-        if (nw == 1) {
-            double gates[4];
-            gd_gates(L.x, g, a.dt, gates);
-            dg.m = gates[0];
-            dg.h = gates[1];
-            dg.j = gates[2];
-            dg.xKs = gates[3];
-            gd_chain_kr(L.p, L.x, g, a.dt, dg.Kr);
-            gd_chain_kv(L.p, L.x, g, a.dt, 0, dg.Kv14);
-            gd_chain_kv(L.p, L.x, g, a.dt, 1, dg.Kv43);
+    if (status != 0) return;
+    if (L.err) {
+        if (tid == 0) {
+            D.status = GW_E_RANGE;
+            D.stop_step = step_new + 1;   // SSA(step_new) runs beside this close; none after it
         }
-        D.Istim = Istim;
-        if (nw == 1) D.dg = dg;
-        else for (int k = 0; k < kGd0; ++k) L.dg0[k] = reinterpret_cast<const double *>(&dg)[k];
+        return;
+    }
+    // ---- 3. terms
+    const FluxSums S{L.S[0], L.S[1], L.S[2], L.S[3]};
+    if (role(0)) {
+        Currents k;
+        gd_k_currents(p, c, g, VF_RT, L.x, k);
+        if (lane == 0) {
+            L.cur.IKr = k.IKr; L.cur.IKs = k.IKs; L.cur.Ito1 = k.Ito1; L.cur.IK1 = k.IK1; L.cur.IKp = k.IKp;
+        }
+    }
+    if (role(1)) {
+        Currents k;
+        double beta_cyto, dLTRPN, dHTRPN;
+        gd_na_ca_currents(p, c, g, L.x, k);
+        gd_uptake(p, c, g, L.x, k, beta_cyto, dLTRPN, dHTRPN);
+        if (lane == 0) {
+            L.cur.INa = k.INa; L.cur.INab = k.INab; L.cur.INaCa = k.INaCa; L.cur.INaK = k.INaK;
+            L.cur.ICab = k.ICab; L.cur.IpCa = k.IpCa; L.cur.Jup = k.Jup;
+            L.beta_cyto = beta_cyto; L.dLTRPN = dLTRPN; L.dHTRPN = dHTRPN;
+        }
+    }
+    if (role(2)) {
+        if (lane < 2 * kv::kEntries) {
+            const int chain = lane / kv::kEntries;
+            L.q[chain][lane % kv::kEntries] = kv::entry_value(kv_entry, p, L.x, chain);
+        }
+        __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");   // the entries pass between lanes of this wave
+        __builtin_amdgcn_wave_barrier();
+        __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+        if (lane < 20) {
+            const int chain = lane / 10;
+            L.ch[(chain == 0 ? 19 : 9) + lane % 10] =
+                kv::derivative(kv_row, lane % 10, L.q[chain], chain == 0 ? g.Kv14 : g.Kv43, a.dt);
+        }
+    }
+    if (role(3)) {
+        Currents k;
+        double gates[4], dKr[5];
+        gd_gates(L.x, g, a.dt, gates);
+        gd_chain_kr(p, L.x, g, a.dt, dKr);
+        gd_cru_currents(p, c, VF_RT, L.x, S, k);
+        if (lane == 0) {
+#pragma unroll
+            for (int i = 0; i < 4; ++i) L.ch[i] = gates[i];
+#pragma unroll
+            for (int i = 0; i < 5; ++i) L.ch[4 + i] = dKr[i];
+            L.cur.Ito2 = k.Ito2; L.cur.ICaL = k.ICaL; L.cur.Jtr_tot = k.Jtr_tot; L.cur.Jxfer_tot = k.Jxfer_tot;
+        }
+    }
+    __syncthreads();
+    // ---- 4. joining
+    const int slot = static_cast<int>((step_new + 1) & 1);
+    if (role(0) || role(1)) {
+        double d[kGd0];
+        gd_combine(c, L.cur, L.beta_cyto, L.dLTRPN, L.dHTRPN, a.dt, L.Istim, d);
         // lookahead_consts: the potential and concentrations the step after starts from
         double V = g.V, Cai = g.Cai, CaNSR = g.CaNSR;
         if (!a.frozen) {
-            if (!clamp) V += dg.V;
-            Cai += dg.Cai;
-            CaNSR += dg.CaNSR;
+            if (!clamp) V += d[0];
+            Cai += d[3];
+            CaNSR += d[4];
         }
         if (clamp) V = protocol_vclamp(C, t_new + a.dt);
-        sc_args(V, L.c.F_RT, L.sx);
-        L.lookahead[0] = V;
-        L.lookahead[1] = Cai;
-        L.lookahead[2] = CaNSR;
-    } else if (tid == kWave) {
-        gd_chain_kv(L.p, L.x, g, a.dt, 0, L.ch + 19);   // Kv1.4
-        gd_gates(L.x, g, a.dt, L.ch);                   // m, h, j, xKs
-        if (nw == 2) {
-            gd_chain_kv(L.p, L.x, g, a.dt, 1, L.ch + 9);
-            gd_chain_kr(L.p, L.x, g, a.dt, L.ch + 4);
+        const double e = gw::exp(sc_arg(lane < SC_N ? lane : 0, V, c.F_RT));
+        double X[SC_N];
+#pragma unroll
+        for (int i = 0; i < SC_N; ++i) X[i] = double_of(shfl_u64(bits_of(e), i));
+        if (role(0)) {
+            if (lane < kGd0) {
+                double v = d[0];
+#pragma unroll
+                for (int i = 1; i < kGd0; ++i)
+                    if (lane == i) v = d[i];
+                reinterpret_cast<double *>(&D.dg)[lane] = v;
+            }
+            StepConsts k;
+            step_consts_scalars(k, c, V, X, Cai, CaNSR, static_cast<uint32_t>((step_new + 1) & 0xffff));
+            if (lane == 0) {
+                StepConsts &K = D.k[slot];
+                K.Cai = k.Cai;
+                K.CaNSR = k.CaNSR;
+                K.inact0 = k.inact0;
+                K.inact1 = k.inact1;
+                K.JLCC_mult = k.JLCC_mult;
+                K.JLCC_exp = k.JLCC_exp;
+                K.step_lo = k.step_lo;
+                K._pad = 0;
+                step_consts_f32_scalars(D.kf[slot], k);
+            }
         }
-    } else if (tid == 2 * kWave) {
-        gd_chain_kv(L.p, L.x, g, a.dt, 1, L.ch + 9);    // Kv4.3
-        gd_chain_kr(L.p, L.x, g, a.dt, L.ch + 4);       // IKr
+        if (role(1) && lane < 13) {
+            const LccRow w = lcc_row(lane, p, c, X);
+            lcc_row_store(D.k[slot].lcc, lane, w);
+            lcc_row_store(D.kf[slot].lcc, lane, w);
+        }
     }
-    __syncthreads();
-    if (nw > 1 && tid < 36) reinterpret_cast<double *>(&D.dg)[tid] = tid < kGd0 ? L.dg0[tid] : L.ch[tid - kGd0];
-    if (tid < SC_N) {
-        const double v = gw::exp(L.sx[tid]);
-        L.sx[tid] = v;
-    }
-    __syncthreads();
-    if (tid < 36) reinterpret_cast<double *>(&D.g)[tid] = L.g[tid];
-    // the SSA constants of step_new + 1: the LCC rate table one state per lane
-    const int slot = static_cast<int>((step_new + 1) & 1);
-    if (tid < 13) {
-        const LccRow w = lcc_row(tid, L.p, L.c, L.sx);
-        lcc_row_store(D.k[slot].lcc, tid, w);
-        lcc_row_store(D.kf[slot].lcc, tid, w);
-    }
-    // the rest of the constants of step_new + 1, formed in registers and
-    // stored in both precisions: on the third wave when the block has one
-    if (tid == (nw > 2 ? 2 * kWave : 0)) {
-        StepConsts k;
-        step_consts_scalars(k, L.c, L.lookahead[0], L.sx, L.lookahead[1], L.lookahead[2],
-                            static_cast<uint32_t>((step_new + 1) & 0xffff));
-        StepConsts &K = D.k[slot];
-        K.Cai = k.Cai;
-        K.CaNSR = k.CaNSR;
-        K.inact0 = k.inact0;
-        K.inact1 = k.inact1;
-        K.JLCC_mult = k.JLCC_mult;
-        K.JLCC_exp = k.JLCC_exp;
-        K.step_lo = k.step_lo;
-        K._pad = 0;
-        step_consts_f32_scalars(D.kf[slot], k);
-    }
-    // observables and trace, on the second wave when the block has one
-    if (tid == (nw > 1 ? kWave : 0)) {
-        const double open_frac = static_cast<double>(tot.open) / (20.0 * C.n_cru);
+    if (role(2) && lane == 0) {
+        const double open_frac = static_cast<double>(L.open) / (20.0 * C.n_cru);
         gw_cell_obs_t o = L.obs;
-        obs_update(o, V_old, g.V, t_old, a.dt, g.Cai, L.ICaL, open_frac, jrel * L.c.CRU_factor);
+        obs_update(o, V_old, g.V, t_old, a.dt, g.Cai, L.cur.ICaL, open_frac, L.jrel * c.CRU_factor);
         D.obs = o;
         if (a.trace_every > 0 && (step_new % a.trace_every) == 0 && D.trace_rows < a.trace_cap) {
             double *row = a.trace + (D.trace_rows * a.ncells + cell) * 4;
             row[0] = g.V;
             row[1] = g.Cai;
-            row[2] = L.ICaL;
+            row[2] = L.cur.ICaL;
             row[3] = open_frac;
             D.trace_rows += 1;
         }
     }
-    if (tid != 0) return;
-    D.sums[0] = S.JLCC; D.sums[1] = S.Jxfer; D.sums[2] = S.Jtr; D.sums[3] = S.ClCh;
-    D.sums[4] = static_cast<double>(tot.open); D.sums[5] = jrel;
-    D.t = t_new;
-    D.step = step_new;
-    if (!(g.V == g.V) || !(g.Cai == g.Cai)) {
-        if (D.status == 0) D.status = GW_E_NAN;
+    if (role(3)) {
+        if (lane < 36) reinterpret_cast<double *>(&D.g)[lane] = L.g[lane];
+        if (lane >= kGd0 && lane < 36) reinterpret_cast<double *>(&D.dg)[lane] = L.ch[lane - kGd0];
+        if (lane == 0) {
+            D.Istim = L.Istim;
+            D.sums[0] = S.JLCC; D.sums[1] = S.Jxfer; D.sums[2] = S.Jtr; D.sums[3] = S.ClCh;
+            D.sums[4] = static_cast<double>(L.open); D.sums[5] = L.jrel;
+            D.t = t_new;
+            D.step = step_new;
+            int st = 0;
+            if (!gd_concentrations_ok(p, g)) st = GW_E_NONPOSITIVE_CONC;
+            else if (!(g.V == g.V) || !(g.Cai == g.Cai)) st = GW_E_NAN;
+            // A cell that fails here stops after the SSA of step_new, which runs beside
+            // this close in the same launch: the SSA blocks read stop_step, which only
+            // changes from a value above step_new to step_new + 1, so every block of
+            // that launch runs the step and none runs a later one.
+            if (st != 0) {
+                D.status = st;
+                D.stop_step = step_new + 1;
+            }
+        }
     }
-    // A cell that fails here stops after the SSA of step_new, which runs beside
-    // this close in the same launch: the SSA blocks read stop_step, which only
-    // changes from a value above step_new to step_new + 1, so every block of
-    // that launch runs the step and none runs a later one.
-    if (D.status != 0) D.stop_step = step_new + 1;
 }
 
 // One launch per Euler step: the first `nclose` blocks close step ssa_step-1
@@ -778,11 +792,11 @@ __global__ __launch_bounds__(BLOCK, kWavesPerSimd<R>) void k_step(KArgs a, int64
                                                                    const int64_t *base)
 {
     __shared__ LccTableT<R> T;
-    __shared__ CloseShared csh;
+    __shared__ CloseLds<BLOCK> csh;
     __shared__ BlockAcc acc;
     const int bid = blockIdx.x;
     if (bid < nclose) {
-        close_cell<kWave>(a, bid, a.dyn[bid], csh);
+        close_cell<BLOCK>(a, bid, a.dyn[bid], csh);
         return;
     }
     ssa_block<PRNG, DIGEST, R, BLOCK>(a, bid - nclose, base ? *base + ssa_step : ssa_step, 1, T, acc);
@@ -876,19 +890,7 @@ __device__ __forceinline__ void ssa_block_refill(const KArgs &a, int b, int64_t 
         next += __popcll(m);
     }
     __syncthreads();
-    if (tid == 0) {
-        Partial p;
-        p.jxfer = acc_fx(acc, 0);
-        p.jtr = acc_fx(acc, 1);
-        p.jlcc = acc_fx(acc, 2);
-        p.jrel = acc_fx(acc, 3);
-        p.iters = acc.ints[0];
-        p.open = static_cast<int64_t>(acc.ints[1]);
-        p.clch = static_cast<int64_t>(acc.ints[2]);
-        p.err = acc.ints[3] ? 1 : 0;
-        p.tag = 0;
-        a.partials[ks * a.nblocks + b] = p;
-    }
+    write_partial(a, acc, ks * a.nblocks + b);
 }
 
 // The refill loop keeps a CRU's addresses and the next CRU's index live beside
@@ -899,11 +901,11 @@ __global__ __launch_bounds__(BLOCK, 3) void k_step_refill(KArgs a, int64_t ssa_s
                                                            const int64_t *base)
 {
     __shared__ LccTableT<R> T;
-    __shared__ CloseShared csh;
+    __shared__ CloseLds<BLOCK> csh;
     __shared__ BlockAcc acc;
     const int bid = blockIdx.x;
     if (bid < nclose) {
-        close_cell<kWave>(a, bid, a.dyn[bid], csh);
+        close_cell<BLOCK>(a, bid, a.dyn[bid], csh);
         return;
     }
     ssa_block_refill<PRNG, R, BLOCK, CPT>(a, bid - nclose, base ? *base + ssa_step : ssa_step, T, acc);
@@ -1082,19 +1084,7 @@ __device__ __forceinline__ void ssa_block_lane(const KArgs &a, int b, int64_t st
     }
     lane_accumulate(acc, Ls.get(tid));
     __syncthreads();
-    if (tid == 0) {
-        Partial p;
-        p.jxfer = acc_fx(acc, 0);
-        p.jtr = acc_fx(acc, 1);
-        p.jlcc = acc_fx(acc, 2);
-        p.jrel = acc_fx(acc, 3);
-        p.iters = acc.ints[0];
-        p.open = static_cast<int64_t>(acc.ints[1]);
-        p.clch = static_cast<int64_t>(acc.ints[2]);
-        p.err = acc.ints[3] ? 1 : 0;
-        p.tag = 0;
-        a.partials[ks * a.nblocks + b] = p;
-    }
+    write_partial(a, acc, ks * a.nblocks + b);
 }
 
 // One lane per CRU needs about 100-128 VGPRs; 4 waves per SIMD keep it free
@@ -1103,12 +1093,12 @@ template <int PRNG, int BLOCK, int CPT>
 __global__ __launch_bounds__(BLOCK, 4) void k_step_lane(KArgs a, int64_t ssa_step, int32_t nclose, const int64_t *base)
 {
     __shared__ LccTableF T;
-    __shared__ CloseShared csh;
+    __shared__ CloseLds<BLOCK> csh;
     __shared__ BlockAcc acc;
     __shared__ LaneSums<BLOCK> Ls;
     const int bid = blockIdx.x;
     if (bid < nclose) {
-        close_cell<kWave>(a, bid, a.dyn[bid], csh);
+        close_cell<BLOCK>(a, bid, a.dyn[bid], csh);
         return;
     }
     ssa_block_lane<PRNG, BLOCK, CPT>(a, bid - nclose, base ? *base + ssa_step : ssa_step, T, acc, Ls);
@@ -1190,7 +1180,7 @@ __global__ void k_sync_init(KArgs a, int64_t step0)
     const DevCell &C = a.cells[c];
     for (int q = threadIdx.x; q < 2 * C.nblk[kShapeDefault]; q += blockDim.x) {
         const int par = q & 1, blk = q >> 1;
-        a.partials[par * a.nblocks + C.blk0[kShapeDefault] + blk].tag = 0;
+        a.partials[par * a.nblocks + C.blk0[kShapeDefault] + blk].w[PW_ERR] = 0;
     }
 }
 
@@ -1262,23 +1252,12 @@ __device__ __forceinline__ void ssa_block_persist(const KArgs &a, int b, int64_t
             atomicAdd(&acc.ints[j], static_cast<unsigned long long>(iv));
         }
         __syncthreads();
-        if (tid == 0) {
-            Partial p;
-            p.jxfer = acc_fx(acc, 0);
-            p.jtr = acc_fx(acc, 1);
-            p.jlcc = acc_fx(acc, 2);
-            p.jrel = acc_fx(acc, 3);
-            p.iters = acc.ints[0];
-            p.open = static_cast<int64_t>(acc.ints[1]);
-            p.clch = static_cast<int64_t>(acc.ints[2]);
-            p.err = acc.ints[3] ? 1 : 0;
-            p.tag = static_cast<int32_t>(n + 1);
-            const unsigned long long *pw = reinterpret_cast<const unsigned long long *>(&p);
-            unsigned long long *dst = reinterpret_cast<unsigned long long *>(a.partials + ks * a.nblocks + b);
-            constexpr int kLast = static_cast<int>(sizeof(Partial) / 8) - 1;   // the word holding err and tag
-            for (int t = 0; t < kLast; ++t) st_coh(dst + t, pw[t]);
+        if (tid < PW_N) {   // the words of the partial, then the one that holds the tag
+            uint64_t v = (&acc.limb[0][0])[tid];
+            unsigned long long *dst = reinterpret_cast<unsigned long long *>(a.partials[ks * a.nblocks + b].w) + tid;
+            if (tid != PW_ERR) st_coh(dst, v);
             stores_done();
-            st_coh(dst + kLast, pw[kLast]);
+            if (tid == PW_ERR) st_coh(dst, (v ? 1u : 0u) | static_cast<uint64_t>(n + 1) << 32);
         }
     }
     if (mine) {
@@ -1327,7 +1306,6 @@ __device__ __forceinline__ void publish_consts(CellSync &X, const CellDyn &D, in
 // SSA(n + 2), which writes the same slots, waits for the close of step n.
 __device__ bool wait_partials(const KArgs &a, const DevCell &C, int64_t n, int32_t *timeout, int64_t limit)
 {
-    constexpr int kTagWord = static_cast<int>(sizeof(Partial) / 8) - 1;
     const int nblk = C.nblk[kShapeDefault];
     const unsigned long long *base =
         reinterpret_cast<const unsigned long long *>(a.partials + (n & 1) * a.nblocks + C.blk0[kShapeDefault]);
@@ -1335,7 +1313,7 @@ __device__ bool wait_partials(const KArgs &a, const DevCell &C, int64_t n, int32
     for (int64_t it = 0;; ++it) {
         bool ok = true;
         for (int q = threadIdx.x; q < nblk; q += kWave)
-            ok = ok && static_cast<int32_t>(ld_coh(base + q * (sizeof(Partial) / 8) + kTagWord) >> 32) == want;
+            ok = ok && static_cast<int32_t>(ld_coh(base + q * PW_N + PW_ERR) >> 32) == want;
         if (__all(ok)) return true;
         if (__hip_atomic_load(timeout, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) != 0) return false;
         if (it >= limit) {
@@ -1353,7 +1331,7 @@ __device__ bool wait_partials(const KArgs &a, const DevCell &C, int64_t n, int32
 // formed.
 template <class R>
 __device__ __forceinline__ void close_persist(const KArgs &a, int cell, int64_t step0, int64_t nsteps, CellDyn &Dl,
-                                              CloseShared &sh, int &leave)
+                                              CloseLds<kBlock> &sh, int &leave)
 {
     static_assert(sizeof(CellDyn) % 8 == 0, "the dynamic state is whole 8-byte words");
     constexpr int kDynWords = sizeof(CellDyn) / 8;
@@ -1371,7 +1349,7 @@ __device__ __forceinline__ void close_persist(const KArgs &a, int cell, int64_t 
         }
         __syncthreads();
         if (leave) break;
-        close_cell<kWave, true>(a, cell, Dl, sh);
+        close_cell<kBlock, true>(a, cell, Dl, sh);
         __syncthreads();
         publish_consts<R>(X, Dl, n);
     }
@@ -1386,7 +1364,7 @@ template <int PRNG, bool DIGEST, class R>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<R>) void k_persist(KArgs a, int64_t step0, int64_t nsteps)
 {
     __shared__ LccTableT<R> T;
-    __shared__ CloseShared csh;
+    __shared__ CloseLds<kBlock> csh;
     __shared__ BlockAcc acc;
     __shared__ typename LocalState<R>::Consts K;
     __shared__ CellDyn Dl;
@@ -1431,22 +1409,6 @@ struct PairLds {
     BlockAcc acc[2];
     LaneSums<BLOCK> Ls[2];
 };
-
-// The block's exact partial of one step, from its accumulators.
-__device__ __forceinline__ void write_partial(const KArgs &a, const BlockAcc &acc, int64_t index)
-{
-    Partial p;
-    p.jxfer = acc_fx(acc, 0);
-    p.jtr = acc_fx(acc, 1);
-    p.jlcc = acc_fx(acc, 2);
-    p.jrel = acc_fx(acc, 3);
-    p.iters = acc.ints[0];
-    p.open = static_cast<int64_t>(acc.ints[1]);
-    p.clch = static_cast<int64_t>(acc.ints[2]);
-    p.err = acc.ints[3] ? 1 : 0;
-    p.tag = 0;
-    a.partials[index] = p;
-}
 
 template <int PRNG, int BLOCK, int CPT>
 __global__ __launch_bounds__(BLOCK, 4) void k_step_lane2(KArgs a, int64_t m, int32_t nss)
@@ -1526,23 +1488,20 @@ __global__ __launch_bounds__(BLOCK, 4) void k_step_lane2(KArgs a, int64_t m, int
     }
     for (int s = 0; s < nss; ++s) lane_accumulate(P.acc[s], P.Ls[s].get(tid));
     __syncthreads();
-    if (tid < nss) write_partial(a, P.acc[tid], ((m + tid) & 1) * a.nblocks + b);
+    for (int s = 0; s < nss; ++s) write_partial(a, P.acc[s], ((m + s) & 1) * a.nblocks + b);
 }
 
-// ncl consecutive closes of every cell, one block of two waves per cell (the
-// two-steps-per-launch sequence): the second wave forms the K-channel chains
-// beside the first. No occupancy target, so the close's serial arithmetic
-// keeps its values in registers (up to 256 VGPRs: two waves per SIMD, so the
-// blocks of 1,024 cells are resident at once; a third wave per block would
-// not be).
-__global__ __launch_bounds__(2 * kWave, 1) void k_close_cells(KArgs a, int32_t ncl)
+// One or two (ncl) consecutive closes of every cell, one block of four waves per cell (the
+// two-steps-per-launch sequence), one wave for each of the close's roles. At
+// 4 waves per SIMD the blocks of 1,024 cells are resident at once.
+__global__ __launch_bounds__(kBlock, 4) void k_close_cells(KArgs a, int32_t ncl)
 {
-    __shared__ CloseShared sh;
+    __shared__ CloseLds<kBlock> sh;
     const int cell = blockIdx.x;
-    for (int c = 0; c < ncl; ++c) {
-        close_cell<kWave>(a, cell, a.dyn[cell], sh);
-        __syncthreads();
-    }
+    close_cell<kBlock>(a, cell, a.dyn[cell], sh);
+    if (ncl < 2) return;
+    __syncthreads();   // written out, not a loop: a loop keeps the close's constants in registers across its turns and spills
+    close_cell<kBlock>(a, cell, a.dyn[cell], sh);
 }
 
 // Graph bookkeeping: the step index a replayed chunk starts at.
@@ -1566,12 +1525,16 @@ __global__ void k_frozen_close(KArgs a, int64_t step0, int64_t nsteps)
     if (cell >= a.ncells) return;
     const DevCell &C = a.cells[cell];
     CellDyn &D = a.dyn[cell];
-    Partial tot;
-    sum_block_partials(a.partials + (step0 & 1) * a.nblocks, C.blk0[a.shape], C.nblk[a.shape], tot);
-    if (a.iters_total) atomicAdd(a.iters_total, static_cast<unsigned long long>(tot.iters));
-    if (tot.err && D.status == 0) D.status = GW_E_RANGE;
-    D.sums[0] = fx_to_double(tot.jlcc); D.sums[1] = fx_to_double(tot.jxfer); D.sums[2] = fx_to_double(tot.jtr);
-    D.sums[3] = static_cast<double>(tot.clch); D.sums[4] = static_cast<double>(tot.open); D.sums[5] = fx_to_double(tot.jrel);
+    const Partial *src = a.partials + (step0 & 1) * a.nblocks + C.blk0[a.shape];
+    uint64_t w[PW_N] = {};
+    for (int b = 0; b < C.nblk[a.shape]; ++b)
+        for (int k = 0; k < PW_N; ++k) w[k] += src[b].w[k];
+    auto flux = [&](int q) { return fx_to_double(limbs_fx(w[3 * q], w[3 * q + 1], w[3 * q + 2])); };
+    if (a.iters_total) atomicAdd(a.iters_total, static_cast<unsigned long long>(w[PW_ITERS]));
+    if (w[PW_ERR] && D.status == 0) D.status = GW_E_RANGE;
+    D.sums[0] = flux(2); D.sums[1] = flux(0); D.sums[2] = flux(1);
+    D.sums[3] = static_cast<double>(static_cast<int64_t>(w[PW_CLCH]));
+    D.sums[4] = static_cast<double>(static_cast<int64_t>(w[PW_OPEN])); D.sums[5] = flux(3);
     for (int64_t s = 0; s < nsteps; ++s) D.t += a.dt;
     D.step += nsteps;
     if (D.status != 0 && D.stop_step > D.step) D.stop_step = D.step;
@@ -1677,12 +1640,12 @@ __global__ void k_reset_obs(CellDyn *dyn, int ncells)
 // out[2c + 1] = Ito2 of cell c.
 __global__ void k_posthoc_currents(KArgs a, double *out)
 {
-    __shared__ Partial red[kBlock];
+    __shared__ FluxTotals red[kBlock];
     const int cell = blockIdx.x;
     const DevCell &C = a.cells[cell];
     const CellDyn &D = a.dyn[cell];
-    Partial mine;
-    partial_zero(mine);
+    FluxTotals mine;
+    totals_zero(mine);
     for (int64_t i = threadIdx.x; i < C.n_cru; i += kBlock) {
         const int64_t slot = C.slot0 + i;
         double s = 0.0;
@@ -1699,7 +1662,7 @@ __global__ void k_posthoc_currents(KArgs a, double *out)
     }
     block_reduce<kBlock>(red, mine);
     if (threadIdx.x != 0) return;
-    const Partial &t = red[0];
+    const FluxTotals &t = red[0];
     const gw_params_t &p = C.p;
     const double V = D.g.V;
     const double x = V * C.c.F_RT;
@@ -1741,12 +1704,12 @@ __global__ void k_zero_trace_rows(CellDyn *dyn, int ncells)
 // per-CRU arrays only the SSA writes (GW.tpp:47-62), not part of GWCRUState.
 __global__ void k_refresh_cell(KArgs a, int cell, int resum)
 {
-    __shared__ Partial red[kBlock];
+    __shared__ FluxTotals red[kBlock];
     const DevCell &C = a.cells[cell];
     CellDyn &D = a.dyn[cell];
     if (resum) {
-        Partial mine;
-        partial_zero(mine);
+        FluxTotals mine;
+        totals_zero(mine);
         for (int64_t i = threadIdx.x; i < C.n_cru; i += kBlock) {
             const int64_t slot = C.slot0 + i;
             double jl[4];
@@ -2291,7 +2254,7 @@ void launch_lane2(gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0 = nullptr, 
 
 void launch_closes(gw_batch *B, int32_t ncl)
 {
-    hipLaunchKernelGGL(k_close_cells, dim3(B->ncells), dim3(2 * kWave), 0, B->ctx->stream, B->a, ncl);
+    hipLaunchKernelGGL(k_close_cells, dim3(B->ncells), dim3(kBlock), 0, B->ctx->stream, B->a, ncl);
 }
 
 // Steps step0 .. step0+n-1 two per launch: the first launch runs SSA(step0)

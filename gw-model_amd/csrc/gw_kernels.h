@@ -57,13 +57,14 @@ struct CellDyn {
     gw_cell_obs_t obs;
 };
 
-// Block partial of the per-step reductions.
-struct Partial {
-    Fx jlcc, jxfer, jtr, jrel;
-    int64_t clch, open;
-    uint64_t iters;
-    int32_t err;
-    int32_t tag;   // the persistent kernel's step tag (step index + 1); 0 elsewhere
+// Block partial of the per-step reductions: the block's accumulators as they
+// stand, 16 words that add independently of one another (the 43-bit limbs of
+// a cell's 2^20 CRUs stay within 64 bits), so that a close sums them without
+// carries, eight lanes to a partial, and recombines them once per cell.
+// Words 3q .. 3q + 2 hold flux q (Jxfer, Jtr, JLCC, Jrel) in limbs.
+enum PartialWord : int { PW_ITERS = 12, PW_OPEN, PW_CLCH, PW_ERR, PW_N };
+struct alignas(16) Partial {
+    uint64_t w[PW_N];   // PW_ERR: error flag, and in the persistent kernel the step tag (step index + 1) in the high half
 };
 
 // Per-cell exchange of the persistent step kernel: a counter, then the SSA

@@ -96,14 +96,16 @@ GW_HD double log(double x)
     return __builtin_fma(ed, 0x1.62e42fefa39efp-1, __builtin_fma(ed, 0x1.abc9e3b39803fp-56, lm));
 }
 
-GW_HD double pow(double x, double y)
+// x^y from e = exp(y log x): the special cases.
+GW_HD double pow_special(double x, double y, double e)
 {
     if (y == 0.0) return 1.0;
     if (x != x || y != y) return __builtin_nan("");
     if (x < 0.0) return __builtin_nan("");
     if (x == 0.0) return (y > 0.0) ? 0.0 : __builtin_inf();
-    return gw::exp(y * gw::log(x));
+    return e;
 }
+GW_HD double pow(double x, double y) { return pow_special(x, y, gw::exp(y * gw::log(x))); }
 
 // ---------------------------------------------------------------------------
 // Exact flux accumulator: 128-bit two's-complement fixed point with 2^-80

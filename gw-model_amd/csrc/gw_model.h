@@ -85,17 +85,16 @@ struct StepConsts {
 // the LCC (GW_utils.hpp:365-375, as exp(arg)), then exp(-V F/RT).
 enum ScSlot : int { SC_AL, SC_BE, SC_YINF, SC_TAU, SC_EXPM, SC_N };
 
-GW_HD void sc_args(double V, double F_RT, double *arg)
+GW_HD double sc_arg(int slot, double V, double F_RT)
 {
-    arg[SC_AL] = 0.012 * (V - 35.0);
-    arg[SC_BE] = -0.05 * (V - 35.0);
-    arg[SC_YINF] = (V + 12.5) / 5.0;
-    arg[SC_TAU] = (V + 30.0) / 12.0;
-    arg[SC_EXPM] = -(V * F_RT);
+    if (slot == SC_EXPM) return -(V * F_RT);
+    const double t = V + (slot <= SC_BE ? -35.0 : slot == SC_YINF ? 12.5 : 30.0);
+    const double c = slot == SC_AL ? 0.012 : slot == SC_BE ? -0.05 : slot == SC_YINF ? 5.0 : 12.0;
+    return slot <= SC_BE ? c * t : t / c;
 }
 
 // Per-step constants of GW_model::SSA (GW.tpp:216-221) from the exponentials
-// X[SC_*] of sc_args, without the LCC rate table. At V == 0 the multiplier
+// X[SC_*] of sc_arg's arguments, without the LCC rate table. At V == 0 the multiplier
 // takes its analytic limit JLCC_const / 2 instead of 0/0.
 GW_HD void step_consts_scalars(StepConsts &k, const CellConsts &c, double V, const double *X, double Cai, double CaNSR,
                                uint32_t step_lo)
@@ -124,23 +123,21 @@ struct LccRow {
 // (r0 + r1) + r2 + 0.
 GW_HD LccRow lcc_row(int s, const gw_params_t &p, const CellConsts &c, const double *X)
 {
+    // without a switch: on the device thirteen lanes form a row each
     const double al = 2.0 * X[SC_AL];
     const double be = 0.0882 * X[SC_BE];
+    const double k = static_cast<double>(s);
     double r0 = 0, r1 = 0, r2 = 0, q = 0;
-    switch (s) {
-    case 1: r0 = 4 * al; q = p.gamma0; break;
-    case 2: r0 = be; r1 = 3 * al; q = c.gamma0a; break;
-    case 3: r0 = 2 * be; r1 = 2 * al; q = c.gamma0a2; break;
-    case 4: r0 = 3 * be; r1 = al; q = c.gamma0a3; break;
-    case 5: r0 = 4 * be; r1 = p.f; q = c.gamma0a4; break;
-    case 6: r0 = p.g; break;
-    case 7: r0 = p.omega; r1 = 4 * al * p.a; break;
-    case 8: r0 = c.omega_b; r1 = be * c.binv; r2 = 3 * al * p.a; break;
-    case 9: r0 = c.omega_b2; r1 = 2 * be * c.binv; r2 = 2 * al * p.a; break;
-    case 10: r0 = c.omega_b3; r1 = 3 * be * c.binv; r2 = al * p.a; break;
-    case 11: r0 = c.omega_b4; r1 = 4 * be * c.binv; r2 = p.f1; break;
-    case 12: r0 = p.g1; break;
-    default: break;
+    if (s >= 1 && s <= 5) {
+        r0 = s == 1 ? 4 * al : (k - 1) * be;                       // 4 al, be, 2 be, 3 be, 4 be
+        r1 = s == 1 ? 0.0 : s == 5 ? p.f : (5 - k) * al;           // -, 3 al, 2 al, al, f
+        q = s == 1 ? p.gamma0 : s == 2 ? c.gamma0a : s == 3 ? c.gamma0a2 : s == 4 ? c.gamma0a3 : c.gamma0a4;
+    } else if (s >= 7 && s <= 11) {
+        r0 = s == 7 ? p.omega : s == 8 ? c.omega_b : s == 9 ? c.omega_b2 : s == 10 ? c.omega_b3 : c.omega_b4;
+        r1 = s == 7 ? 4 * al * p.a : (k - 7) * be * c.binv;        // 4 al a, be/b, 2 be/b, 3 be/b, 4 be/b
+        r2 = s == 7 ? 0.0 : s == 11 ? p.f1 : (11 - k) * al * p.a;  // -, 3 al a, 2 al a, al a, f1
+    } else if (s > 0) {
+        r0 = s == 6 ? p.g : p.g1;
     }
     LccRow w;
     w.R0 = r0;
@@ -162,7 +159,7 @@ GW_HD void lcc_row_store(LccTableT<R> &t, int s, const LccRow &w)
 }
 
 // Per-step constants of GW_model::SSA and the LCC rate table, from the
-// exponentials X[SC_*] of sc_args.
+// exponentials X[SC_*] of sc_arg's arguments.
 GW_HD void step_consts_x(StepConsts &k, const gw_params_t &p, const CellConsts &c, double V, const double *X,
                          double Cai, double CaNSR, uint32_t step_lo)
 {
@@ -175,8 +172,7 @@ GW_HD void step_consts(StepConsts &k, const gw_params_t &p, const CellConsts &c,
                        double Cai, double CaNSR, uint32_t step_lo)
 {
     double X[SC_N];
-    sc_args(V, c.F_RT, X);
-    for (int i = 0; i < SC_EXPM; ++i) X[i] = gw::exp(X[i]);
+    for (int i = 0; i < SC_EXPM; ++i) X[i] = gw::exp(sc_arg(i, V, c.F_RT));
     X[SC_EXPM] = expmVF_RT;
     step_consts_x(k, p, c, V, X, Cai, CaNSR, step_lo);
 }
@@ -235,7 +231,9 @@ enum GdSlot : int {
     GD_LNA = GD_LOG0, GD_LK, GD_LKS,          // log(Nao/Nai), log(Ko/Ki), the IKs reversal
     GD_POW0,                                  // powers from here (exponent py[slot - GD_POW0])
     GD_PNAK = GD_POW0, GD_PF, GD_PR,          // INaK, Jup forward and reverse
-    GD_N
+    GD_N,
+    GD_IK1 = GD_N,                            // exp(1.5 (V - EK) F/RT), IK1: its argument needs X[GD_LK]
+    GD_X                                      // values in all
 };
 
 GW_HD double gd_eval(int slot, double arg, double y)
@@ -243,9 +241,7 @@ GW_HD double gd_eval(int slot, double arg, double y)
     return slot < GD_LOG0 ? gw::exp(arg) : slot < GD_POW0 ? gw::log(arg) : gw::pow(arg, y);
 }
 
-// The arguments of the slots before GD_KR0 (gd_args_lo) and from it on
-// (gd_args_hi); gd_args is both.
-GW_HD void gd_args_lo(const gw_params_t &p, const gw_globals_t &g, double VF_RT, double *arg)
+GW_HD void gd_args(const gw_params_t &p, const gw_globals_t &g, double VF_RT, double *arg, double *py)
 {
     const double V = g.V;
     arg[GD_EXPM] = -VF_RT;
@@ -269,11 +265,6 @@ GW_HD void gd_args_lo(const gw_params_t &p, const gw_globals_t &g, double VF_RT,
     arg[GD_XKS] = -(V - 24.7) / 13.6;
     arg[GD_TXKS1] = -0.148 * (V - 10.0);
     arg[GD_TXKS2] = 0.0687 * (V - 10.0);
-}
-
-GW_HD void gd_args_hi(const gw_params_t &p, const gw_globals_t &g, double *arg, double *py)
-{
-    const double V = g.V;
     arg[GD_KR0] = 0.0272 * V;
     arg[GD_KR1] = -0.0431 * V;
     arg[GD_KR2] = 0.0262 * V;
@@ -298,23 +289,6 @@ GW_HD void gd_args_hi(const gw_params_t &p, const gw_globals_t &g, double *arg, 
     py[1] = p.Hf;
     arg[GD_PR] = g.CaNSR / p.Kmr;
     py[2] = p.Hr;
-}
-
-GW_HD void gd_args(const gw_params_t &p, const gw_globals_t &g, double VF_RT, double *arg, double *py)
-{
-    gd_args_lo(p, g, VF_RT, arg);
-    gd_args_hi(p, g, arg, py);
-}
-
-// Nernst potential (common.hpp:70-75) from lg = log(Xo / Xi); the reference
-// exits on a non-positive concentration, this clears ok instead.
-GW_HD double nernst(double Xi, double Xo, double lg, double RT_F, double z, bool &ok)
-{
-    if (Xi <= 0.0 || Xo <= 0.0) {
-        ok = false;
-        return 0.0;
-    }
-    return lg * RT_F / z;
 }
 
 // Gate rates (common.hpp:175-218) from the exponentials of gd_args.
@@ -397,32 +371,126 @@ struct Currents {
     double INa, INab, INaCa, INaK, IKr, IKs, Ito1, Ito2, IK1, IKp, ICaL, ICab, IpCa, Jup, Jtr_tot, Jxfer_tot;
 };
 
-// The derivatives from the values X[slot] of gd_args' arguments, except the
-// gates and the IKr and Kv chains (gd_gates, gd_chain_kr and gd_chain_kv
-// below); the one exponential whose argument needs a logarithm (IK1) is
-// evaluated here.
-GW_HD int gd_finish_main(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, double VF_RT, const double *X,
-                    double dt, double Istim, const FluxSums &S, gw_globals_t &dg, Currents &cur)
+// The same arguments one slot per lane: slot s < GD_LOG0 is (x + d) * c or
+// (x + d) / c of x = V or VF_RT, with c a number or a parameter times one;
+// negated and reordered forms of gd_args round alike.
+enum GdArgSrc : int32_t { GA_VF = 1, GA_DIV = 2, GA_PARAM = 4 };
+struct GdArg {
+    double d, c;
+    int32_t src, off;   // off: the parameter's word in gw_params_t
+};
+#define GW_GA_PARAM_(field, c, src) {0.0, c, GA_PARAM | (src), static_cast<int32_t>(offsetof(gw_params_t, field) / 8)}
+__device__ __constant__ const GdArg kGdArg[GD_LOG0] = {
+    {0.0, -1.0, GA_VF, 0},                                                            // EXPM
+    GW_GA_PARAM_(eta, 1.0, GA_VF), {0.0, -0.1, GA_VF, 0},                             // NACA, NAK
+    {0.0, 0.0446, 0, 0}, {-7.488, -5.98, GA_DIV, 0},                                  // KR_R, KP
+    {47.13, -0.1, 0, 0}, {0.0, -11.0, GA_DIV, 0},                                     // AM, BM
+    {80.0, -6.8, GA_DIV, 0}, {10.66, -11.1, GA_DIV, 0}, {0.0, 0.079, 0, 0}, {0.0, 0.35, 0, 0},   // AH, BH1..3
+    {0.0, 0.2444, 0, 0}, {0.0, -0.04391, 0, 0}, {79.23, 0.311, 0, 0},                 // AJ1..3
+    {0.0, -2.535e-7, 0, 0}, {32.0, -0.1, 0, 0}, {0.0, -0.01052, 0, 0}, {40.14, -0.1378, 0, 0},   // BJ1..4
+    {-24.7, -13.6, GA_DIV, 0}, {-10.0, -0.148, 0, 0}, {-10.0, 0.0687, 0, 0},          // XKS, TXKS1..2
+    {0.0, 0.0272, 0, 0}, {0.0, -0.0431, 0, 0}, {0.0, 0.0262, 0, 0}, {0.0, 2.71e-6, 0, 0},        // KR0..3
+    {0.0, -0.0269, 0, 0}, {0.0, 0.0120, 0, 0}, {0.0, -0.0443, 0, 0},                  // KR4..6
+    GW_GA_PARAM_(aaKv14, 1.0, 0), GW_GA_PARAM_(aaKv43, 1.0, 0), GW_GA_PARAM_(aiKv14, -1.0, 0), GW_GA_PARAM_(aiKv43, -1.0, 0),
+    GW_GA_PARAM_(baKv14, -1.0, 0), GW_GA_PARAM_(baKv43, -1.0, 0), GW_GA_PARAM_(biKv14, 1.0, 0), GW_GA_PARAM_(biKv43, 1.0, 0)};
+#undef GW_GA_PARAM_
+
+__device__ __forceinline__ GdArg gd_arg_row(int slot) { return kGdArg[slot]; }
+__device__ __forceinline__ double gd_arg_value(const GdArg &r, const gw_params_t &p, double V, double VF_RT)
+{
+    const double c = (r.src & GA_PARAM) ? r.c * reinterpret_cast<const double *>(&p)[r.off] : r.c;
+    const double t = ((r.src & GA_VF) ? VF_RT : V) + r.d;
+    return (r.src & GA_DIV) ? t / c : t * c;
+}
+
+// The argument of slot s >= GD_LOG0 and, for a power, its exponent (else 0).
+GW_HD double gd_log_arg(int slot, const gw_params_t &p, const gw_globals_t &g, double &y)
+{
+    y = slot == GD_PNAK ? 1.5 : slot == GD_PF ? p.Hf : slot == GD_PR ? p.Hr : 0.0;
+    const double num = slot == GD_LNA ? p.Nao : slot == GD_LK ? p.Ko : slot == GD_LKS ? p.Ko + 0.01833 * p.Nao
+                     : slot == GD_PNAK ? p.KmNai : slot == GD_PF ? g.Cai : g.CaNSR;
+    const double den = slot == GD_LNA ? g.Nai : slot == GD_LK ? g.Ki : slot == GD_LKS ? g.Ki + 0.01833 * g.Nai
+                     : slot == GD_PNAK ? g.Nai : slot == GD_PF ? p.Kmf : p.Kmr;
+    return num / den;
+}
+
+// The Kv chains one value per lane: a generator entry is m r u / v of one of
+// the chain's four rates r and factors u, v (kv_chain's expressions: a factor
+// left out is 1, which changes no bit), a derivative is two or three inflows
+// and the diagonal, in kv_chain's order.
+namespace kv {
+constexpr int kEntries = 26;
+// parameters of a chain, as words from its alphaa0: the rates' scales, then f1..f4, b1..b4
+enum Off : uint32_t { AA = 0, BA = 2, AI = 4, BI = 6, F1 = 8, F2, F3, F4, B1, B2, B3, B4, ONE = 31 };
+static_assert(offsetof(gw_params_t, b4Kv14) - offsetof(gw_params_t, alphaa0Kv14) == 15 * sizeof(double) &&
+                  offsetof(gw_params_t, f1Kv14) - offsetof(gw_params_t, alphaa0Kv14) == F1 * sizeof(double) &&
+                  offsetof(gw_params_t, b4Kv43) - offsetof(gw_params_t, alphaa0Kv43) == 15 * sizeof(double) &&
+                  offsetof(gw_params_t, f1Kv43) - offsetof(gw_params_t, alphaa0Kv43) == F1 * sizeof(double) &&
+                  offsetof(gw_params_t, betai0Kv14) - offsetof(gw_params_t, alphaa0Kv14) == BI * sizeof(double),
+              "both chains' parameters lie in the same order");
+constexpr uint32_t ent(uint32_t m, uint32_t r, uint32_t u = ONE, uint32_t v = ONE) { return m | r << 3 | u << 6 | v << 11; }
+__device__ __constant__ const uint32_t kEntry[kEntries] = {
+    ent(4, AA), ent(1, BI),                                   // 0: q01 q05
+    ent(1, BA), ent(3, AA), ent(1, BI, F1),                   // 2: q10 q12 q16
+    ent(2, BA), ent(2, AA), ent(1, BI, F2),                   // 5: q21 q23 q27
+    ent(3, BA), ent(1, AA), ent(1, BI, F3),                   // 8: q32 q34 q38
+    ent(4, BA), ent(1, BI, F4),                               // 11: q43 q49
+    ent(4, AA, B1), ent(1, AI),                               // 13: q56 q50
+    ent(1, BA, ONE, F1), ent(3, AA, B2, B1), ent(1, AI, ONE, B1),   // 15: q65 q67 q61
+    ent(2, BA, F1, F2), ent(2, AA, B3, B2), ent(1, AI, ONE, B2),    // 18: q76 q78 q72
+    ent(3, BA, F2, F3), ent(1, AA, B4, B3), ent(1, AI, ONE, B3),    // 21: q87 q89 q83
+    ent(4, BA, F3, F4), ent(1, AI, ONE, B4)};                 // 24: q98 q94
+// Row i: inflow k as (entry, from state); the outgoing entries are consecutive from `out`.
+struct Row {
+    uint8_t e[3], s[3], nin, out, nout;
+};
+__device__ __constant__ const Row kRow[10] = {
+    {{2, 14, 0}, {1, 5, 0}, 2, 0, 2},   {{0, 5, 17}, {0, 2, 6}, 3, 2, 3},  {{3, 8, 20}, {1, 3, 7}, 3, 5, 3},
+    {{6, 11, 23}, {2, 4, 8}, 3, 8, 3},  {{9, 25, 0}, {3, 9, 0}, 2, 11, 2}, {{15, 1, 0}, {6, 0, 0}, 2, 13, 2},
+    {{13, 18, 4}, {5, 7, 1}, 3, 15, 3}, {{16, 21, 7}, {6, 8, 2}, 3, 18, 3}, {{19, 24, 10}, {7, 9, 3}, 3, 21, 3},
+    {{22, 12, 0}, {8, 4, 0}, 2, 24, 2}};
+
+__device__ __forceinline__ uint32_t entry(int k) { return kEntry[k]; }
+__device__ __forceinline__ Row row(int i) { return kRow[i]; }
+__device__ __forceinline__ double entry_value(uint32_t e, const gw_params_t &p, const double *X, int chain)
+{
+    const double *P = chain == 0 ? &p.alphaa0Kv14 : &p.alphaa0Kv43;
+    const uint32_t r = (e >> 3) & 7, u = (e >> 6) & 31, v = (e >> 11) & 31;
+    // X[GD_KV0 ..]: aa, ai, ba, bi of Kv1.4 and Kv4.3 in turn
+    const int slot = GD_KV0 + (r == AA ? 0 : r == AI ? 2 : r == BA ? 4 : 6) + chain;
+    const double rate = P[r] * X[slot];
+    const double fu = P[u & 15], fv = P[v & 15];
+    return static_cast<double>(e & 7) * rate * (u == ONE ? 1.0 : fu) / (v == ONE ? 1.0 : fv);
+}
+__device__ __forceinline__ double derivative(const Row &r, int i, const double *q, const double *y, double dt)
+{
+    double out = q[r.out] + q[r.out + 1];
+    if (r.nout > 2) out += q[r.out + 2];
+    double in = q[r.e[0]] * y[r.s[0]] + q[r.e[1]] * y[r.s[1]];
+    if (r.nin > 2) in += q[r.e[2]] * y[r.s[2]];
+    return dt * (in + -out * y[i]);
+}
+}  // namespace kv
+
+// Whether every Nernst argument is positive (the reference exits where one is not, common.hpp:72-75).
+GW_HD bool gd_concentrations_ok(const gw_params_t &p, const gw_globals_t &g)
+{
+    return !(g.Nai <= 0.0 || p.Nao <= 0.0 || g.Ki <= 0.0 || p.Ko <= 0.0);
+}
+
+// The potassium reversal potential (common.hpp:70-75) and the argument of X[GD_IK1], from lk = X[GD_LK].
+GW_HD double gd_EK(const CellConsts &c, double lk) { return lk * c.RT_F / 1.0; }
+GW_HD double gd_ik1_arg(const CellConsts &c, double V, double lk) { return 1.5 * (V - gd_EK(c, lk)) * c.F_RT; }
+
+// The derivatives from the values X[slot], except the gates and the IKr and Kv
+// chains (gd_gates, gd_chain_kr and gd_chain_kv below), in four parts that
+// share only their inputs and gd_combine, which joins them.
+GW_HD void gd_k_currents(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, double VF_RT,
+                         const double *X, Currents &cur)
 {
     const double V = g.V;
     const double expmVF_RT = X[GD_EXPM];
-    bool ok = true;
-    const double ENa = nernst(g.Nai, p.Nao, X[GD_LNA], c.RT_F, 1.0, ok);
-    const double EK = nernst(g.Ki, p.Ko, X[GD_LK], c.RT_F, 1.0, ok);
-    const double ECa = nernst(g.Ki, p.Ko, X[GD_LK], c.RT_F, 2.0, ok);  // K-based, as GW.tpp:176
-    if (!ok) return GW_E_NONPOSITIVE_CONC;
-
-    cur.INa = p.GNa * cube(g.m) * g.h * g.j * (V - ENa);                       // common.hpp:89-92
-    cur.INab = p.GNab * (V - ENa);                                             // common.hpp:100-101
-    {   // common.hpp:163-168
-        const double e1 = X[GD_NACA];
-        const double e2 = e1 * expmVF_RT;
-        cur.INaCa = c.INaCa_const * (e1 * cube(g.Nai) * p.Cao - e2 * c.Nao3 * g.Cai) / (1.0 + p.ksat * e2);
-    }
-    {   // common.hpp:121-124, 140-143
-        const double fNaK = 1.0 / (1.0 + 0.1245 * X[GD_NAK] + 0.0365 * c.sigma * expmVF_RT);
-        cur.INaK = c.INaK_const * fNaK / (1.0 + X[GD_PNAK]);
-    }
+    const double EK = gd_EK(c, X[GD_LK]);
     {   // GW_utils.hpp:273-279
         const double RKr = 1.0 / (1.0 + 1.4945 * X[GD_KR_R]);
         cur.IKr = p.GKr * c.sqrtKo * RKr * g.Kr[3] * (V - EK) * 0.5;
@@ -441,45 +509,82 @@ GW_HD int gd_finish_main(const gw_params_t &p, const CellConsts &c, const gw_glo
     }
     const double IKv43 = p.GKv43 * g.Kv43[4] * (V - EK);                       // GW_utils.hpp:294-297
     cur.Ito1 = IKv14 + IKv43;
-    if (VF_RT == 0.0) cur.Ito2 = S.ClCh * c.Ito2_const * (p.Clo - p.Clcyto);    // limit of GW_utils.hpp:330
-    else cur.Ito2 = S.ClCh * c.Ito2_const * VF_RT * (p.Clcyto * expmVF_RT - p.Clo) / (expmVF_RT - 1.0);
     {   // GW_utils.hpp:306-312
-        const double K1inf = 1.0 / (2.0 + gw::exp(1.5 * (V - EK) * c.F_RT));
+        const double K1inf = 1.0 / (2.0 + X[GD_IK1]);
         cur.IK1 = p.GK1 * K1inf * c.IK1_const * (V - EK);
     }
     {   // GW_utils.hpp:315-319
         const double Kp = 1. / (1. + X[GD_KP]);
         cur.IKp = p.GKp * Kp * (V - EK);
     }
-    cur.ICaL = S.JLCC * c.ICaL_const;                                           // GW_utils.hpp:322-325
+}
+
+GW_HD void gd_na_ca_currents(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, const double *X,
+                             Currents &cur)
+{
+    const double V = g.V;
+    const double expmVF_RT = X[GD_EXPM];
+    const double ENa = X[GD_LNA] * c.RT_F / 1.0;
+    const double ECa = X[GD_LK] * c.RT_F / 2.0;                                 // K-based, as GW.tpp:176
+    cur.INa = p.GNa * cube(g.m) * g.h * g.j * (V - ENa);                       // common.hpp:89-92
+    cur.INab = p.GNab * (V - ENa);                                             // common.hpp:100-101
+    {   // common.hpp:163-168
+        const double e1 = X[GD_NACA];
+        const double e2 = e1 * expmVF_RT;
+        cur.INaCa = c.INaCa_const * (e1 * cube(g.Nai) * p.Cao - e2 * c.Nao3 * g.Cai) / (1.0 + p.ksat * e2);
+    }
+    {   // common.hpp:121-124, 140-143
+        const double fNaK = 1.0 / (1.0 + 0.1245 * X[GD_NAK] + 0.0365 * c.sigma * expmVF_RT);
+        cur.INaK = c.INaK_const * fNaK / (1.0 + X[GD_PNAK]);
+    }
     cur.ICab = p.GCab * (V - ECa);
     cur.IpCa = p.IpCamax * (g.Cai / (p.KmpCa + g.Cai));                         // common.hpp:109-110
+}
+
+// SERCA uptake, the cytosolic buffering factor and the troponin derivatives before the factor dt (GW.tpp:201-202).
+GW_HD void gd_uptake(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, const double *X, Currents &cur,
+                     double &beta_cyto, double &dLTRPN, double &dHTRPN)
+{
     {   // GW_utils.hpp:339-344
         const double f = X[GD_PF];
         const double r = X[GD_PR];
         cur.Jup = (p.Vmaxf * f - p.Vmaxr * r) / (1.0 + f + r);
     }
-    cur.Jtr_tot = S.Jtr * c.CRU_factor;                                         // GW_utils.hpp:354-355
-    cur.Jxfer_tot = S.Jxfer * c.CRU_factor;
-    double beta_cyto;
     {   // GW_utils.hpp:347-351
         const double x = p.KCMDN + g.Cai;
         beta_cyto = 1.0 / (1.0 + c.CMDN_const / sq(x));
     }
-    // GW.tpp:201-211
-    dg.CaLTRPN = p.kLTRPNp * g.Cai * (p.LTRPNtot - g.CaLTRPN) - p.kLTRPNm * g.CaLTRPN;
-    dg.CaHTRPN = p.kHTRPNp * g.Cai * (p.HTRPNtot - g.CaHTRPN) - p.kHTRPNm * g.CaHTRPN;
-    dg.Nai = -dt * c.CSA_FVcyto * (cur.INa + cur.INab + 3 * cur.INaCa + 3 * cur.INaK);
-    dg.Ki = -dt * c.CSA_FVcyto * (cur.IKr + cur.IKs + cur.Ito1 + cur.IK1 + cur.IKp - 2 * cur.INaK);
-    dg.Cai = dt * beta_cyto *
-             (-0.5 * c.CSA_FVcyto * (cur.ICab + cur.IpCa - 2 * cur.INaCa) + c.VSS_Vcyto * cur.Jxfer_tot - cur.Jup -
-              (dg.CaLTRPN + dg.CaHTRPN));
-    dg.CaNSR = dt * (c.Vcyto_VNSR * cur.Jup - c.VJSR_VNSR * cur.Jtr_tot);
-    dg.CaLTRPN *= dt;
-    dg.CaHTRPN *= dt;
-    dg.V = dt * (Istim - (cur.INa + cur.ICaL + cur.IKr + cur.IKs + cur.Ito1 + cur.IK1 + cur.IKp + cur.Ito2 +
+    dLTRPN = p.kLTRPNp * g.Cai * (p.LTRPNtot - g.CaLTRPN) - p.kLTRPNm * g.CaLTRPN;
+    dHTRPN = p.kHTRPNp * g.Cai * (p.HTRPNtot - g.CaHTRPN) - p.kHTRPNm * g.CaHTRPN;
+}
+
+// The currents and fluxes formed from the CRU sums.
+GW_HD void gd_cru_currents(const gw_params_t &p, const CellConsts &c, double VF_RT, const double *X, const FluxSums &S,
+                           Currents &cur)
+{
+    const double expmVF_RT = X[GD_EXPM];
+    if (VF_RT == 0.0) cur.Ito2 = S.ClCh * c.Ito2_const * (p.Clo - p.Clcyto);    // limit of GW_utils.hpp:330
+    else cur.Ito2 = S.ClCh * c.Ito2_const * VF_RT * (p.Clcyto * expmVF_RT - p.Clo) / (expmVF_RT - 1.0);
+    cur.ICaL = S.JLCC * c.ICaL_const;                                           // GW_utils.hpp:322-325
+    cur.Jtr_tot = S.Jtr * c.CRU_factor;                                         // GW_utils.hpp:354-355
+    cur.Jxfer_tot = S.Jxfer * c.CRU_factor;
+}
+
+// GW.tpp:201-211: the increments of V and the concentrations, into d[0..6]
+// (gw_globals_t order: V, Nai, Ki, Cai, CaNSR, CaLTRPN, CaHTRPN).
+GW_HD void gd_combine(const CellConsts &c, const Currents &cur, double beta_cyto, double dLTRPN, double dHTRPN, double dt,
+                      double Istim, double d[7])
+{
+    d[1] = -dt * c.CSA_FVcyto * (cur.INa + cur.INab + 3 * cur.INaCa + 3 * cur.INaK);
+    d[2] = -dt * c.CSA_FVcyto * (cur.IKr + cur.IKs + cur.Ito1 + cur.IK1 + cur.IKp - 2 * cur.INaK);
+    d[3] = dt * beta_cyto *
+           (-0.5 * c.CSA_FVcyto * (cur.ICab + cur.IpCa - 2 * cur.INaCa) + c.VSS_Vcyto * cur.Jxfer_tot - cur.Jup -
+            (dLTRPN + dHTRPN));
+    d[4] = dt * (c.Vcyto_VNSR * cur.Jup - c.VJSR_VNSR * cur.Jtr_tot);
+    d[5] = dLTRPN * dt;
+    d[6] = dHTRPN * dt;
+    d[0] = dt * (Istim - (cur.INa + cur.ICaL + cur.IKr + cur.IKs + cur.Ito1 + cur.IK1 + cur.IKp + cur.Ito2 +
                           cur.INaK + cur.INaCa + cur.IpCa + cur.ICab + cur.INab));
-    return GW_OK;
 }
 
 // GW.tpp:162-168: the derivatives of the gates m, h, j and xKs, into
@@ -521,13 +626,24 @@ GW_HD void gd_chain_kv(const gw_params_t &p, const double *X, const gw_globals_t
     }
 }
 
-// All the derivatives from the values X[slot] of gd_args' arguments.
+// All the derivatives from the values X[slot].
 GW_HD int gd_finish(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, double VF_RT, const double *X,
                     double dt, double Istim, const FluxSums &S, gw_globals_t &dg, Currents &cur)
 {
-    const int rc = gd_finish_main(p, c, g, VF_RT, X, dt, Istim, S, dg, cur);
-    if (rc != GW_OK) return rc;
-    double gates[4];
+    if (!gd_concentrations_ok(p, g)) return GW_E_NONPOSITIVE_CONC;
+    double beta_cyto, dLTRPN, dHTRPN, d[7], gates[4];
+    gd_k_currents(p, c, g, VF_RT, X, cur);
+    gd_na_ca_currents(p, c, g, X, cur);
+    gd_uptake(p, c, g, X, cur, beta_cyto, dLTRPN, dHTRPN);
+    gd_cru_currents(p, c, VF_RT, X, S, cur);
+    gd_combine(c, cur, beta_cyto, dLTRPN, dHTRPN, dt, Istim, d);
+    dg.V = d[0];
+    dg.Nai = d[1];
+    dg.Ki = d[2];
+    dg.Cai = d[3];
+    dg.CaNSR = d[4];
+    dg.CaLTRPN = d[5];
+    dg.CaHTRPN = d[6];
     gd_gates(X, g, dt, gates);
     dg.m = gates[0];
     dg.h = gates[1];
@@ -543,9 +659,10 @@ GW_HD int gd_finish(const gw_params_t &p, const CellConsts &c, const gw_globals_
 GW_HD int global_derivatives(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, double VF_RT,
                              double dt, double Istim, const FluxSums &S, gw_globals_t &dg, Currents &cur)
 {
-    double X[GD_N], py[GD_N - GD_POW0];
+    double X[GD_X], py[GD_N - GD_POW0];
     gd_args(p, g, VF_RT, X, py);
     for (int i = 0; i < GD_N; ++i) X[i] = gd_eval(i, X[i], i >= GD_POW0 ? py[i - GD_POW0] : 0.0);
+    X[GD_IK1] = gw::exp(gd_ik1_arg(c, g.V, X[GD_LK]));
     return gd_finish(p, c, g, VF_RT, X, dt, Istim, S, dg, cur);
 }
 
