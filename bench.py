@@ -176,6 +176,8 @@ def gpu_bench(capi, cell_list, steps, warmup, precision=0, autotune=200, launch=
 def kernel_name(tune, f32):
     """The step kernel a launch shape runs (xoshiro256** instantiation)."""
     lanes, blk, cpl = (tune["lanes_per_cru"], tune["block"], tune["crus_per_lane"]) if tune else (4, 256, 1)
+    if not f32 and tune and tune.get("steps_per_launch", 1) == 2:   # large FP64 batches: one lane per CRU
+        return "k_step2_lane64"
     if lanes == 1:
         if tune and tune.get("steps_per_launch", 1) == 2:
             return f"k_step_lane2<0, {blk}, {cpl}>"
@@ -185,7 +187,7 @@ def kernel_name(tune, f32):
 
 def measured_traffic(total_crus, form):
     """HBM bytes per SSA launch from the committed PMC summary, scaled to this batch
-    (form: fp64, fp32, or fp32_pair for two steps per launch)."""
+    (form: fp64 or fp32, with _pair for two steps per launch)."""
     path = os.path.join(ROOT, "profiles", "k_ssa_traffic.txt")
     if not os.path.exists(path):
         return None
@@ -195,7 +197,7 @@ def measured_traffic(total_crus, form):
             k, v = line.split("=", 1)
             vals[k.strip()] = v.strip()
     try:
-        key = "hbm_bytes_per_cru_launch_fp32_pair" if form == "fp32_pair" else f"hbm_bytes_per_cru_step_{form}"
+        key = f"hbm_bytes_per_cru_launch_{form}" if form.endswith("_pair") else f"hbm_bytes_per_cru_step_{form}"
         return float(vals[key]) * total_crus
     except (KeyError, ValueError):
         return None
@@ -341,7 +343,7 @@ def ensemble_run(capi, args):
         b = capi.Batch(ctx, cell_list, precision=prec)
         b.set_mode(frozen=False, digest=False)
         b.set_launch(*shapes[form])
-        b.set_steps_per_launch(args.steps_per_launch if form == "fp32" else 1)
+        b.set_steps_per_launch(args.steps_per_launch)
         t0 = time.perf_counter()
         for beat in range(args.ensemble_beats):
             if beat == args.ensemble_beats - 1:
@@ -397,7 +399,7 @@ def measure(capi, precision, args, total_crus):
     launch = tuple(int(x) for x in (fixed + "x1").split("x")[:3]) if fixed and args.autotune <= 0 else None
     ms, ssa_ms, launches, iters, g, obs, tune = gpu_bench(capi, cell_list, args.steps, advance_steps(args),
                                                           precision=precision, autotune=args.autotune, launch=launch,
-                                                          steps_per_launch=args.steps_per_launch if f32 else 1)
+                                                          steps_per_launch=args.steps_per_launch)
     pair = bool(tune and tune.get("steps_per_launch", 1) == 2)
     sim_ms = args.steps * 1e-3
     sec = ms / 1e3
@@ -423,7 +425,7 @@ def measure(capi, precision, args, total_crus):
             "peak": peak_f if valu else PEAK_HBM_GBS,
             "unit": "TFLOP/s" if valu else "GB/s",
             "frac": max(frac_f, frac_b),
-            "traffic": measured_traffic(total_crus, ("fp32_pair" if pair else "fp32") if f32 else "fp64"),
+            "traffic": measured_traffic(total_crus, ("fp32" if f32 else "fp64") + ("_pair" if pair else "")),
             "kernel": kernel_name(tune, f32),
             "avg_launch_us": per_launch_s * 1e6,
             "valu": {"achieved_tflops": achieved_tflops, "peak": peak_f, "frac": frac_f,
@@ -497,8 +499,8 @@ def main(argv=None):
     ap.add_argument("--launch-fp64", default="4x64", metavar="LxB",
                     help="FP64 launch shape; the default is the autotuner's choice on the seeds64 batch")
     ap.add_argument("--steps-per-launch", type=int, choices=[0, 1, 2], default=0,
-                    help="SSA steps per launch of the FP32-local form (2: each CRU advances two steps per launch "
-                         "with its state in registers, one-lane shapes of 64 threads; 0, the default: the "
+                    help="SSA steps per launch (2: each CRU advances two steps per launch with its state in registers, "
+                         "FP32-local one-lane shapes of 64 threads and large FP64 batches; 0, the default: the "
                          "library's choice, two when a launch's blocks are more than the GPU holds at once)")
     ap.add_argument("--precision", choices=["both", "fp32", "fp64"], default="both",
                     help="forms to time; with both, value is the batched FP32-local form and fp64 sits beside it")

@@ -167,13 +167,13 @@ __device__ void totals_add(FluxTotals &a, const FluxTotals &b)
     a.err |= b.err;
 }
 
-// The 128-bit value of three limb sums.
+// The 128-bit value of three (signed) limb sums.
 __device__ __forceinline__ Fx limbs_fx(uint64_t S0, uint64_t S1, uint64_t S2)
 {
     Fx f;
     f.lo = S0;
-    f.hi = 0;
-    fx_add_raw(f, S1 << 43, S1 >> 21);
+    f.hi = static_cast<uint64_t>(static_cast<int64_t>(S0) >> 63);
+    fx_add_raw(f, S1 << 43, static_cast<uint64_t>(static_cast<int64_t>(S1) >> 21));
     fx_add_raw(f, 0, S2 << 22);
     return f;
 }
@@ -1504,6 +1504,252 @@ __global__ __launch_bounds__(kBlock, 4) void k_close_cells(KArgs a, int32_t ncl)
     close_cell<kBlock>(a, cell, a.dyn[cell], sh);
 }
 
+// ---------------------------------------------------------------------------
+// FP64 with one lane per CRU (gw_ssa.h, lane64_*), one or two Euler steps per
+// launch, refilled from CPT CRUs per lane as in the FP32-local kernels. It
+// replaces the quads where a launch has more CRUs than the GPU can hold in
+// quads several times over (run_config): there a wave's instructions count,
+// and this form needs about half as many per CRU and step.
+//
+// Events wait: about 3% of the iterations end in an event, so in nearly every
+// trip of a wave of 64 CRUs one or two lanes would take the event path, a
+// third as long as the rest of the trip. A lane whose iteration ends in an event
+// leaves its CRU as it was and runs the same iteration again (it would idle
+// otherwise), until kEventBatch lanes of the wave hold an event, or no other
+// lane made progress, or no fresh CRU is left to keep the others busy; then
+// all of them commit at once. 12.8 M CRUs, 4 per lane: 552, 551, 542 and 543
+// us per step with batches of 1, 4, 8 and 16 events.
+//
+// Flux sums: a CRU's four outputs are split into three 43-bit limbs in FP64
+// arithmetic, truncated at 2^-80 like fx_add, and added as whole numbers into
+// sixteen copies of the block accumulators in LDS (below 2^53, so exact in
+// FP64, whatever the order).
+// ---------------------------------------------------------------------------
+constexpr int kEventBatch = 8;
+constexpr int kAccCopies = 16;
+
+struct Lane64Acc {
+    double limb[12][kAccCopies];
+    unsigned long long ints[kAccCopies];   // iterations in the low 40 bits, open ClCh above
+    int open[kAccCopies];
+    int err;
+};
+
+template <int NSS>
+struct Lane64Lds {
+    StepConsts K[NSS];
+    Lane64Acc acc[NSS];
+};
+
+// Adds v in limbs; false if it is not below 2^24 in magnitude (then it adds nothing).
+__device__ __forceinline__ bool lane64_add(Lane64Acc &A, int q, int copy, double v)
+{
+    const bool ok = __builtin_fabs(v) < 0x1p24;
+    v = ok ? v : 0.0;
+    const double hi = __builtin_trunc(v * 0x1p-6);
+    const double r = __builtin_fma(hi, -0x1p6, v);
+    const double mid = __builtin_trunc(r * 0x1p37);
+    const double r2 = __builtin_fma(mid, -0x1p-37, r);
+    const double lo = __builtin_trunc(r2 * 0x1p80);
+    unsafeAtomicAdd(&A.limb[3 * q][copy], lo);
+    unsafeAtomicAdd(&A.limb[3 * q + 1][copy], mid);
+    unsafeAtomicAdd(&A.limb[3 * q + 2][copy], hi);
+    return ok;
+}
+
+__device__ __forceinline__ void lane64_output(Lane64Acc &A, const Lane64State &S, double Jxfer, double Jtr, bool ok)
+{
+    const int copy = threadIdx.x & (kAccCopies - 1);
+    ok &= lane64_add(A, 0, copy, Jxfer);
+    ok &= lane64_add(A, 1, copy, Jtr);
+    ok &= lane64_add(A, 2, copy, S.jl[0] + S.jl[1] + S.jl[2] + S.jl[3]);
+    lane64_add(A, 3, copy, S.Jrel[0] + S.Jrel[1] + S.Jrel[2] + S.Jrel[3]);   // the range of Jrel is not checked
+    int open = 0, clch = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        open += ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
+        clch += sub_cl(S.w[j]);
+    }
+    atomicAdd(&A.ints[copy], static_cast<unsigned long long>(clch) << 40 | S.iters);
+    atomicAdd(&A.open[copy], open);
+    if (!ok) A.err = 1;
+}
+
+__device__ __forceinline__ void lane64_load(const KArgs &a, int64_t slot, Lane64State &S)
+{
+    const double2 *pc = reinterpret_cast<const double2 *>(a.CaSS + slot * 4);
+    const double2 c01 = pc[0], c23 = pc[1];
+    const double2 *pj = reinterpret_cast<const double2 *>(a.JLCC + slot * 4);
+    const double2 j01 = pj[0], j23 = pj[1];
+    const ulonglong2 *pw = reinterpret_cast<const ulonglong2 *>(a.sub + slot * 4);
+    const ulonglong2 w01 = pw[0], w23 = pw[1];
+    const ulonglong2 *pr = reinterpret_cast<const ulonglong2 *>(a.rng + slot * 4);
+    const ulonglong2 r01 = pr[0], r23 = pr[1];
+    S.q.jsr = a.CaJSR[slot];
+    S.ca[0] = c01.x; S.ca[1] = c01.y; S.ca[2] = c23.x; S.ca[3] = c23.y;
+    S.jl[0] = j01.x; S.jl[1] = j01.y; S.jl[2] = j23.x; S.jl[3] = j23.y;
+    S.w[0] = w01.x; S.w[1] = w01.y; S.w[2] = w23.x; S.w[3] = w23.y;
+    S.q.r0 = r01.x; S.q.r1 = r01.y; S.q.r2 = r23.x; S.q.r3 = r23.y;
+    S.changed = 0;
+}
+
+__device__ __forceinline__ void lane64_store(const KArgs &a, int64_t slot, const Lane64State &S)
+{
+    double2 *qc = reinterpret_cast<double2 *>(a.CaSS + slot * 4);
+    qc[0] = make_double2(S.ca[0], S.ca[1]);
+    qc[1] = make_double2(S.ca[2], S.ca[3]);
+    if (S.changed) {   // the channel words and JLCC change only at events and re-splits
+        double2 *qj = reinterpret_cast<double2 *>(a.JLCC + slot * 4);
+        qj[0] = make_double2(S.jl[0], S.jl[1]);
+        qj[1] = make_double2(S.jl[2], S.jl[3]);
+        ulonglong2 *qw = reinterpret_cast<ulonglong2 *>(a.sub + slot * 4);
+        qw[0] = make_ulonglong2(S.w[0], S.w[1]);
+        qw[1] = make_ulonglong2(S.w[2], S.w[3]);
+    }
+    ulonglong2 *qr = reinterpret_cast<ulonglong2 *>(a.rng + slot * 4);
+    qr[0] = make_ulonglong2(S.q.r0, S.q.r1);
+    qr[1] = make_ulonglong2(S.q.r2, S.q.r3);
+    a.CaJSR[slot] = S.q.jsr;
+}
+
+// SSA(m .. m + nss - 1) of block b (one wave, 64 * CPT CRUs of one cell), nss <= NSS.
+template <int PRNG, int CPT, int NSS>
+__device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t m, int nss, Lane64Lds<NSS> &P)
+{
+    constexpr int kMap = shape_of_crus(kWave * CPT);
+    static_assert(crus_per_block(kMap) == kWave * CPT, "CRUs per block must be 16 << map");
+    constexpr int kWords = sizeof(StepConsts) / 4;
+    const int lane = threadIdx.x;
+    const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
+    const DevCell &C = a.cells[cell];
+    const CellDyn &D = a.dyn[cell];
+#pragma unroll
+    for (int s = 0; s < NSS; ++s) {
+        if (s < nss)
+            for (int t = lane; t < kWords; t += kWave)
+                reinterpret_cast<uint32_t *>(&P.K[s])[t] = reinterpret_cast<const uint32_t *>(&D.k[(m + s) & 1])[t];
+        for (int t = lane; t < static_cast<int>(sizeof(Lane64Acc) / 4); t += kWave) reinterpret_cast<uint32_t *>(&P.acc[s])[t] = 0;
+    }
+    __syncthreads();
+    const double dt = a.dt;
+    const double rRyR = C.sp.rRyR;
+    const int64_t stop = D.stop_step;
+    const bool run1 = nss > 1 && m + 1 < stop;
+    const int64_t w0 = static_cast<int64_t>(b - C.blk0[kMap]) * (kWave * CPT);
+    const int w1 = static_cast<int>(min(static_cast<int64_t>(kWave * CPT), C.n_cru - w0));   // CRUs of the range
+    const int64_t slot0 = C.slot0 + w0;
+    int i = lane;
+    int next = kWave;   // first CRU of the range not yet taken (wave-uniform)
+    bool have = i < w1 && m < stop;
+    int sidx = 0;       // the step (0: m, 1: m + 1) this lane's CRU is in
+    Lane64State S;
+    if (have) {
+        lane64_load(a, slot0 + i, S);
+        lane64_begin(S, rRyR);
+    }
+    while (__ballot(have)) {
+        const SsaParams *spp = &C.sp;
+        asm volatile("" : "+s"(spp));   // read again in each trip: held over the loop they would not fit
+        const SsaParams sp = load_scalar(spp);
+        Lane64Try X;
+        bool ev = false;
+        if (have) {
+            lane64_try<PRNG>(S, X, sp, P.K[sidx], P.K[sidx].lcc, dt);
+            ev = !X.last;
+        }
+        const uint64_t m_ev = __ballot(ev);
+        const uint64_t m_last = __ballot(have && !ev);
+        const bool go = __popcll(m_ev) >= kEventBatch || m_last == 0 || next >= w1;   // wave-uniform
+        bool fin = have && !ev;
+        bool ok = true;
+        if (have && (go || !ev)) {
+            double old[4];
+            uint64_t w_pre[4];
+            lane64_commit<PRNG>(S, X, sp, old, w_pre);
+            if (ev && go) {
+                if (S.iters >= kMaxItersPerStep) {   // no physical state gets here; stop instead of spinning
+                    ok = false;
+                    fin = true;
+                } else if (!lane64_event<PRNG>(S, X, sp, P.K[sidx], P.K[sidx].lcc, old, w_pre)) {
+                    P.acc[sidx].err = 1;
+                }
+            }
+        }
+        if (fin) {
+            lane64_output(P.acc[sidx], S, X.Jxfer, X.Jtr, ok);
+            if (NSS > 1 && sidx == 0 && run1) {   // the same CRU, next step
+                sidx = 1;
+                lane64_begin(S, rRyR);
+                fin = false;
+            } else {
+                sidx = 0;
+                lane64_store(a, slot0 + i, S);
+            }
+        }
+        const uint64_t msk = __ballot(fin);
+        if (fin) {
+            if constexpr (CPT > 1) {
+                i = next + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(msk >> 32),
+                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(msk), 0u)));
+                have = i < w1;
+                if (have) {
+                    lane64_load(a, slot0 + i, S);
+                    lane64_begin(S, rRyR);
+                }
+            } else {
+                have = false;
+            }
+        }
+        next += __popcll(msk);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int s = 0; s < NSS; ++s) {
+        if (s >= nss || lane >= PW_N) continue;
+        const Lane64Acc &A = P.acc[s];
+        uint64_t v = 0;
+        if (lane < PW_ITERS) {
+            double d = 0.0;
+            for (int k = 0; k < kAccCopies; ++k) d += A.limb[lane][k];   // whole numbers below 2^53
+            v = static_cast<uint64_t>(static_cast<int64_t>(d));
+        } else if (lane == PW_ERR) {
+            v = A.err != 0;
+        } else {
+            for (int k = 0; k < kAccCopies; ++k)
+                v += lane == PW_OPEN ? static_cast<uint64_t>(static_cast<int64_t>(A.open[k]))
+                   : lane == PW_CLCH ? A.ints[k] >> 40 : A.ints[k] & ((1ULL << 40) - 1);
+        }
+        a.partials[((m + s) & 1) * a.nblocks + b].w[lane] = v;
+    }
+}
+
+// One step, the closes of the step before in the first blocks (as k_step).
+// 155 VGPRs: three waves per SIMD (at four, 23 spill and 12.8 M CRUs take 649
+// us per step against 542). Issue of vector instructions bounds them: 18.2 per
+// CRU and step, 80% of the time (the quads: 50.7, 87%).
+template <int PRNG, int CPT>
+__global__ __launch_bounds__(kWave, 3) void k_step_lane64(KArgs a, int64_t ssa_step, int32_t nclose, const int64_t *base)
+{
+    __shared__ union {
+        Lane64Lds<1> ssa;
+        CloseLds<kWave> close;
+    } sh;
+    const int bid = blockIdx.x;
+    if (bid < nclose) {
+        close_cell<kWave>(a, bid, a.dyn[bid], sh.close);
+        return;
+    }
+    ssa_block_lane64<PRNG, CPT, 1>(a, bid - nclose, base ? *base + ssa_step : ssa_step, 1, sh.ssa);
+}
+
+// One or two (nss) steps, their closes before them in k_close_cells.
+template <int PRNG, int CPT>
+__global__ __launch_bounds__(kWave, 3) void k_step2_lane64(KArgs a, int64_t m, int32_t nss)
+{
+    __shared__ Lane64Lds<2> sh;
+    ssa_block_lane64<PRNG, CPT, 2>(a, blockIdx.x, m, nss, sh);
+}
+
 // Graph bookkeeping: the step index a replayed chunk starts at.
 __global__ void k_set_base(int64_t *base, int64_t v) { *base = v; }
 __global__ void k_advance_base(int64_t *base, int64_t k) { *base += k; }
@@ -1816,13 +2062,15 @@ struct gw_batch {
     int32_t persist_mode = 0;        // persistent step kernel: 0 off (default), 1 on, 2 when every block fits at once
     int32_t persist_fit = -1;        // whether every block of the persistent kernel fits at once (-1: not known)
     int32_t steps_per_launch = 0;    // SSA steps per plain launch (FP32-local one-lane shapes of 64 threads): 1, 2, 0 automatic
-    int64_t pair_capacity[GW_LAUNCH_CONFIGS] = {};   // blocks of k_step_lane2 resident at once, per configuration (0: not known)
-    int32_t cfg = 2;                 // launch configuration (kConfigs), 4 x 256 by default
+    int64_t pair_capacity[GW_LAUNCH_CONFIGS + 2] = {};   // blocks of k_step_lane2 resident at once, per configuration (0: not known)
+    int32_t cfg = 2;                 // launch configuration (kConfigs) asked for, 4 x 256 by default
+    int32_t run_cfg = 2;             // the one the batch's shape arrays are set for (apply_shape)
+    int64_t ncrus = 0;               // CRUs of all cells
     // replayed graphs of step chunks (0 = plain launches)
     int32_t graph_steps = 0;
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
-    int32_t graph_steps_built = 0, graph_cfg = -1;
+    int32_t graph_steps_built = 0, graph_cfg = -1;   // graph_cfg: the configuration that ran (run_cfg)
     bool graph_digest = false;
     KArgs graph_args{};
     int64_t *d_step_base = nullptr;
@@ -1920,13 +2168,15 @@ struct LaunchCfg {
 };
 constexpr int kNumConfigs = GW_LAUNCH_CONFIGS;
 constexpr int kConfigDefault = 2;
-constexpr LaunchCfg kConfigs[kNumConfigs] = {
+constexpr int kLane64 = kNumConfigs;   // the FP64 one-lane kernels of 4 and 8 CRUs per lane, which run_config chooses
+constexpr LaunchCfg kConfigs[kNumConfigs + 2] = {
     {4, 64, 1},  {4, 128, 1}, {4, 256, 1}, {4, 512, 1},                 // quads: 16..128 CRUs per block
     {1, 64, 1},  {1, 128, 1}, {1, 256, 1},                               // one lane per CRU
     {1, 64, 2},  {1, 128, 2}, {1, 256, 2},                               // two CRUs per lane, refilled
     {1, 64, 4},  {1, 128, 4}, {1, 256, 4},                               // four
     {1, 64, 8},  {1, 128, 8}, {1, 256, 8},                               // eight (up to 2048 CRUs per block)
-    {4, 64, 2},  {4, 64, 4},  {4, 128, 4}, {4, 256, 4}};                 // quads refilled from 2 or 4 CRUs each
+    {4, 64, 2},  {4, 64, 4},  {4, 128, 4}, {4, 256, 4},                  // quads refilled from 2 or 4 CRUs each
+    {1, 64, 4},  {1, 64, 8}};                                            // FP64, one lane per CRU
 constexpr int config_shape(int c)
 {
     return shape_of_crus(kConfigs[c].threads / kConfigs[c].lanes * kConfigs[c].cpl);
@@ -1934,9 +2184,12 @@ constexpr int config_shape(int c)
 static_assert(config_shape(kConfigDefault) == kShapeDefault, "the default configuration uses the setup map");
 static_assert(config_shape(kNumConfigs - 1) < kNumShapes, "block -> cell maps cover every configuration");
 
-void set_shape(gw_batch *B, int c)
+// The launch configuration asked for; run_config chooses the one that runs.
+void set_shape(gw_batch *B, int c) { B->cfg = c; }
+
+void apply_shape(gw_batch *B, int c)
 {
-    B->cfg = c;
+    B->run_cfg = c;
     B->shape = config_shape(c);
     B->nblocks = B->nblocks_shape[B->shape];
     B->a.shape = B->shape;
@@ -1984,6 +2237,7 @@ void launch_frozen(gw_batch *B, int64_t step0, int64_t n)
 
 void launch_frozen_steps(gw_batch *B, int64_t step0, int64_t n)
 {
+    apply_shape(B, kConfigDefault);
     switch (B->prng) {
     case 0: launch_frozen<0>(B, step0, n); break;
     case 1: launch_frozen<1>(B, step0, n); break;
@@ -2038,9 +2292,11 @@ template <int PRNG>
 void launch_k_step(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent_t e0, hipEvent_t e1, const int64_t *base)
 {
     if constexpr (PRNG == GW_PRNG_XOSHIRO256SS) {
-        if (kConfigs[B->cfg].lanes == 1) {
+        if (kConfigs[B->run_cfg].lanes == 1) {
             const unsigned grid = step_grid(B, ssa_step, nclose);
-            switch (B->cfg) {
+            switch (B->run_cfg) {
+            case kLane64: dispatch(k_step_lane64<PRNG, 4>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
+            case kLane64 + 1: dispatch(k_step_lane64<PRNG, 8>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 4: dispatch(k_step_lane<PRNG, 64, 1>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 5: dispatch(k_step_lane<PRNG, 128, 1>, grid, 128, B, e0, e1, ssa_step, nclose, base); break;
             case 6: dispatch(k_step_lane<PRNG, 256, 1>, grid, 256, B, e0, e1, ssa_step, nclose, base); break;
@@ -2056,9 +2312,9 @@ void launch_k_step(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent_t e0,
             }
             return;
         }
-        if (kConfigs[B->cfg].cpl > 1) {
+        if (kConfigs[B->run_cfg].cpl > 1) {
             const unsigned grid = step_grid(B, ssa_step, nclose);
-            switch (B->cfg) {   // FP64 only (shape_allowed)
+            switch (B->run_cfg) {   // FP64 only (shape_allowed)
             case 16: dispatch(k_step_refill<PRNG, double, 64, 2>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 17: dispatch(k_step_refill<PRNG, double, 64, 4>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 18: dispatch(k_step_refill<PRNG, double, 128, 4>, grid, 128, B, e0, e1, ssa_step, nclose, base); break;
@@ -2094,7 +2350,7 @@ void launch_one(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent_t e0, hi
 // captured again whenever the launch arguments or shape change.
 bool graph_current(const gw_batch *B)
 {
-    return B->graph_exec && B->graph_steps_built == B->graph_steps && B->graph_cfg == B->cfg &&
+    return B->graph_exec && B->graph_steps_built == B->graph_steps && B->graph_cfg == B->run_cfg &&
            B->graph_digest == B->digest &&
            std::memcmp(&B->graph_args, &B->a, sizeof(KArgs)) == 0;
 }
@@ -2125,7 +2381,7 @@ hipError_t graph_build(gw_batch *B)
         return e;
     }
     B->graph_steps_built = B->graph_steps;
-    B->graph_cfg = B->cfg;
+    B->graph_cfg = B->run_cfg;
     B->graph_digest = B->digest;
     B->graph_args = B->a;
     return hipSuccess;
@@ -2172,6 +2428,23 @@ bool use_persist(gw_batch *B)
     return B->persist_mode != 0 && !B->frozen && B->cfg == kConfigDefault && persist_fits(B);
 }
 
+// The launch configuration the next steps run in: the one asked for, or for a
+// large FP64 batch a one-lane kernel, whose results are the same bits. Where
+// the lines lie, in us per step early in an action potential (4 x 64 quads;
+// one lane, 4 and 8 CRUs per lane): 300,000 CRUs 29.9, 38.7, 41.5; 600,000
+// 51.1, 50.0, 55.4; 800,000 65.3, 55.3, 57.6; 2.0 M 173, 97.9, 97.9; 5.0 M
+// 457, 218, 206; 12.8 M 1,182, 526, 479. Below, a batch is a few rounds of
+// quads and one round of lanes, whose trips are longer.
+constexpr int64_t kLane64Crus = 640000, kLane64Crus8 = 2500000;
+
+int run_config(gw_batch *B)
+{
+    if (B->precision != GW_PREC_FP64 || B->prng != GW_PRNG_XOSHIRO256SS || B->digest || B->frozen || use_persist(B) ||
+        B->ncrus < kLane64Crus)
+        return B->cfg;
+    return B->ncrus < kLane64Crus8 ? kLane64 : kLane64 + 1;
+}
+
 // Steps step0 .. step0+n-1 in one cooperative launch of the persistent kernel
 // (which closes every step itself), after its counters are set for step0.
 hipError_t launch_persist(gw_batch *B, int64_t step0, int64_t n)
@@ -2189,31 +2462,44 @@ hipError_t launch_persist(gw_batch *B, int64_t step0, int64_t n)
     return e;
 }
 
-// Whether the batch's plain launches run two SSA steps each (k_step_lane2):
-// asked for, FP32-local free-running steps on a one-lane shape of 64 threads
-// (xoshiro256**, no digests, as every one-lane shape), not persistent, no
-// replayed graphs.
+// Whether the batch's plain launches can run two SSA steps each: FP32-local
+// free-running steps on a one-lane shape of 64 threads (k_step_lane2;
+// xoshiro256**, no digests, as every one-lane shape), or FP64 steps that
+// run_config gives to the one-lane kernels (k_step2_lane64); not persistent,
+// no replayed graphs.
 bool pair_capable(gw_batch *B)
 {
     if (B->frozen || B->graph_steps > 0 || use_persist(B)) return false;
-    const LaunchCfg &L = kConfigs[B->cfg];
+    const int c = run_config(B);
+    const LaunchCfg &L = kConfigs[c];
+    if (c >= kLane64) return true;
     return B->precision == GW_PREC_FP32_LOCAL && L.lanes == 1 && L.threads == 64 && B->prng == GW_PRNG_XOSHIRO256SS;
 }
 
-// How many blocks of the batch's two-step kernel the GPU holds at once.
-int64_t pair_capacity(gw_batch *B)
+// The batch's two-step kernel.
+const void *pair_fn(int c)
 {
-    int64_t &cap = B->pair_capacity[B->cfg];
-    if (cap > 0) return cap;
-    const void *fn = nullptr;
-    switch (kConfigs[B->cfg].cpl) {
-    case 1: fn = reinterpret_cast<const void *>(&k_step_lane2<GW_PRNG_XOSHIRO256SS, 64, 1>); break;
-    case 2: fn = reinterpret_cast<const void *>(&k_step_lane2<GW_PRNG_XOSHIRO256SS, 64, 2>); break;
-    case 4: fn = reinterpret_cast<const void *>(&k_step_lane2<GW_PRNG_XOSHIRO256SS, 64, 4>); break;
-    default: fn = reinterpret_cast<const void *>(&k_step_lane2<GW_PRNG_XOSHIRO256SS, 64, 8>); break;
+    constexpr int P = GW_PRNG_XOSHIRO256SS;
+    switch (c) {
+    case kLane64: return reinterpret_cast<const void *>(&k_step2_lane64<P, 4>);
+    case kLane64 + 1: return reinterpret_cast<const void *>(&k_step2_lane64<P, 8>);
+    default: break;
     }
+    switch (kConfigs[c].cpl) {
+    case 1: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 1>);
+    case 2: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 2>);
+    case 4: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 4>);
+    default: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 8>);
+    }
+}
+
+// How many blocks of the batch's two-step kernel the GPU holds at once.
+int64_t pair_capacity(gw_batch *B, int c)
+{
+    int64_t &cap = B->pair_capacity[c];
+    if (cap > 0) return cap;
     int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, fn, 64, 0) == hipSuccess &&
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pair_fn(c), 64, 0) == hipSuccess &&
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, B->ctx->device) == hipSuccess)
         cap = static_cast<int64_t>(per_cu) * cus;
     return cap > 0 ? cap : INT64_MAX;
@@ -2226,13 +2512,15 @@ int64_t pair_capacity(gw_batch *B)
 bool use_pair(gw_batch *B)
 {
     if (B->steps_per_launch == 1 || !pair_capable(B)) return false;
-    return B->steps_per_launch == 2 || B->nblocks > pair_capacity(B);
+    const int c = run_config(B);
+    if (B->steps_per_launch == 2 || c >= kLane64) return true;
+    return B->nblocks_shape[config_shape(c)] > pair_capacity(B, c);
 }
 
-// One launch of k_step_lane2: SSA(m .. m + nss - 1); with e0/e1 the dispatch
-// records its own start and end.
+// One launch of the two-step kernel: SSA(m .. m + nss - 1); with e0/e1 the
+// dispatch records its own start and end.
 template <class K>
-void dispatch_lane2(K kernel, gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0, hipEvent_t e1)
+void dispatch_pair(K kernel, gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0, hipEvent_t e1)
 {
     const dim3 grid(static_cast<unsigned>(B->nblocks)), block(64);
     if (e0)
@@ -2241,14 +2529,19 @@ void dispatch_lane2(K kernel, gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0
         hipLaunchKernelGGL(kernel, grid, block, 0, B->ctx->stream, B->a, m, nss);
 }
 
-void launch_lane2(gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr)
+void launch_pair(gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr)
 {
     constexpr int P = GW_PRNG_XOSHIRO256SS;
-    switch (kConfigs[B->cfg].cpl) {
-    case 1: dispatch_lane2(k_step_lane2<P, 64, 1>, B, m, nss, e0, e1); break;
-    case 2: dispatch_lane2(k_step_lane2<P, 64, 2>, B, m, nss, e0, e1); break;
-    case 4: dispatch_lane2(k_step_lane2<P, 64, 4>, B, m, nss, e0, e1); break;
-    default: dispatch_lane2(k_step_lane2<P, 64, 8>, B, m, nss, e0, e1); break;
+    switch (B->run_cfg) {
+    case kLane64: dispatch_pair(k_step2_lane64<P, 4>, B, m, nss, e0, e1); return;
+    case kLane64 + 1: dispatch_pair(k_step2_lane64<P, 8>, B, m, nss, e0, e1); return;
+    default: break;
+    }
+    switch (kConfigs[B->run_cfg].cpl) {
+    case 1: dispatch_pair(k_step_lane2<P, 64, 1>, B, m, nss, e0, e1); break;
+    case 2: dispatch_pair(k_step_lane2<P, 64, 2>, B, m, nss, e0, e1); break;
+    case 4: dispatch_pair(k_step_lane2<P, 64, 4>, B, m, nss, e0, e1); break;
+    default: dispatch_pair(k_step_lane2<P, 64, 8>, B, m, nss, e0, e1); break;
     }
 }
 
@@ -2290,9 +2583,9 @@ hipError_t launch_steps_pair(gw_batch *B, int64_t step0, int64_t n, int64_t *lau
         if (ssa_ms) {
             const int r = static_cast<int>(count % kRing);
             if (count >= kRing && (e = harvest(r)) != hipSuccess) break;
-            launch_lane2(B, m, nss, ev[2 * r], ev[2 * r + 1]);
+            launch_pair(B, m, nss, ev[2 * r], ev[2 * r + 1]);
         } else {
-            launch_lane2(B, m, nss);
+            launch_pair(B, m, nss);
         }
         c += ncl;
         m += nss;
@@ -2317,6 +2610,7 @@ hipError_t launch_steps(gw_batch *B, int64_t step0, int64_t n, int64_t *launches
 {
     if (launches) *launches = 0;
     if (n <= 0) return hipSuccess;
+    apply_shape(B, run_config(B));
     if (use_persist(B)) {
         if (launches) *launches = 1;
         return launch_persist(B, step0, n);
@@ -2724,6 +3018,7 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
         B->max_nblocks = std::max(B->max_nblocks, blk);
     }
     B->ntot = slot;
+    for (int c = 0; c < ncells; ++c) B->ncrus += cells[c].n_cru;
     B->nblocks = B->nblocks_shape[kShapeDefault];
     const int64_t N = B->ntot;
     KArgs &a = B->a;
@@ -3347,6 +3642,7 @@ int gw_batch_time_steps(gw_batch *B, int64_t nsteps, double *ms, double *ssa_ms,
     HIP_TRY(hipEventCreate(&e0));
     HIP_TRY(hipEventCreate(&e1));
     HIP_TRY(hipEventRecord(e0, B->ctx->stream));
+    apply_shape(B, run_config(B));
     const bool persist = use_persist(B);
     int64_t nlaunch = nsteps;   // SSA launches
     if (ssa_ms && use_pair(B)) {   // two steps per launch, each SSA dispatch timed

@@ -56,24 +56,13 @@ GW_HD double exp(double x)
 // log: x = 2^e m with m in [sqrt(2)/2, sqrt(2)); log m = 2 atanh(s),
 // s = (m - 1)/(m + 1), atanh series through s^25 (Horner, fused).
 // ---------------------------------------------------------------------------
-GW_HD double log(double x)
+// log of 2^e m, m the fraction bits over [1, 2).
+GW_HD double log_em(int e, uint64_t frac)
 {
-    if (x != x) return x;
-    if (x < 0.0) return __builtin_nan("");
-    if (x == 0.0) return -__builtin_inf();
-    if (x == __builtin_inf()) return x;
-    uint64_t u = bits_of(x);
-    int e = static_cast<int>((u >> 52) & 0x7ff);
-    if (e == 0) {
-        u = bits_of(x * 0x1p54);
-        e = static_cast<int>((u >> 52) & 0x7ff) - 54;
-    }
-    e -= 1023;
-    double m = double_of((u & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
-    if (m > 0x1.6a09e667f3bcdp+0) {
-        m = m * 0.5;
-        e += 1;
-    }
+    double m = double_of((frac & 0x000fffffffffffffULL) | 0x3ff0000000000000ULL);
+    const bool up = m > 0x1.6a09e667f3bcdp+0;
+    m = up ? m * 0.5 : m;
+    e += up ? 1 : 0;
     const double f = m - 1.0;
     const double s = f / (2.0 + f);
     const double z = s * s;
@@ -94,6 +83,29 @@ GW_HD double log(double x)
     const double lm = __builtin_fma(s2, R, s2);
     const double ed = static_cast<double>(e);
     return __builtin_fma(ed, 0x1.62e42fefa39efp-1, __builtin_fma(ed, 0x1.abc9e3b39803fp-56, lm));
+}
+
+GW_HD double log(double x)
+{
+    if (x != x) return x;
+    if (x < 0.0) return __builtin_nan("");
+    if (x == 0.0) return -__builtin_inf();
+    if (x == __builtin_inf()) return x;
+    uint64_t u = bits_of(x);
+    int e = static_cast<int>((u >> 52) & 0x7ff);
+    if (e == 0) {
+        u = bits_of(x * 0x1p54);
+        e = static_cast<int>((u >> 52) & 0x7ff) - 54;
+    }
+    return log_em(e - 1023, u);
+}
+
+// log of a draw of u01: zero, or a normal number below 1.
+GW_HD double log_u01(double u)
+{
+    const uint64_t b = bits_of(u);
+    const double r = log_em(static_cast<int>(b >> 52) - 1023, b);
+    return u == 0.0 ? -__builtin_inf() : r;
 }
 
 // x^y from e = exp(y log x): the special cases.

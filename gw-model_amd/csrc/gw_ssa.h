@@ -100,12 +100,28 @@ GW_HD void ssa_params_f32(SsaParamsF &f, const SsaParams &s)
     for (int i = 0; i < static_cast<int>(sizeof(SsaParams) / sizeof(double)); ++i) dst[i] = static_cast<float>(src[i]);
 }
 
+// The parameters of a cell's SSA through the scalar cache, into scalar
+// registers (they are the same for every lane). The compiler does this by
+// itself only where no store of the kernel can come before the load; where the
+// kernel stores a CRU and goes on, it keeps them in vector registers, 72 in
+// FP64 and 36 in FP32, which are what limits the waves in flight.
+template <class T>
+__device__ __forceinline__ T load_scalar(const T *p)
+{
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    struct Words { uint32_t w[sizeof(T) / 4]; } v;
+    const auto *q = (const __attribute__((address_space(4))) uint32_t *)(reinterpret_cast<uintptr_t>(p));
+#pragma unroll
+    for (unsigned i = 0; i < sizeof(T) / 4; ++i) v.w[i] = q[i];
+    return __builtin_bit_cast(T, v);
+}
+
 // Local arithmetic of the SSA. FP64: IEEE division and the shared log, bit-exact
 // with the oracle. FP32 (the FP32-local variant): one hardware reciprocal
 // (v_rcp_f32, 1 ulp) times the numerator, and the hardware log2 (v_log_f32).
 __device__ __forceinline__ double ldiv(double a, double b) { return a / b; }
 __device__ __forceinline__ float ldiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
-__device__ __forceinline__ double lneglog(double u) { return -gw::log(u); }
+__device__ __forceinline__ double lneglog(double u) { return -gw::log_u01(u); }
 __device__ __forceinline__ float lneglog(float u) { return -(__builtin_amdgcn_logf(u) * 0.693147182f); }
 __device__ __forceinline__ float sq(float x) { return x * x; }
 
@@ -145,21 +161,42 @@ __device__ __forceinline__ void ryr_rates(const SsaParamsT<R> &P, uint64_t w, R 
     const int n4 = ryr_get(w, 3), n5 = ryr_get(w, 4), n6 = ryr_get(w, 5);
     const bool hi34 = ca > R(3.685e-2);
     const bool hi56 = ca > R(1.15e-4);
-    R tau34 = R(0), eq56 = R(0);
-    if (hi34) tau34 = ldiv(R(1), P.k34 * C2 + P.k43);
-    if (hi56) eq56 = ldiv(P.k65, P.k56 * C2 + P.k65);
+    const R a3 = static_cast<R>(n3), a4 = static_cast<R>(n4), a5 = static_cast<R>(n5);
+    R r3 = a3 * P.k34 * C2, r4 = a4 * P.k45, r7 = a3 * P.k32, r8 = a4 * P.k43;
+    if (hi34) {
+        const R tau34 = ldiv(R(1), P.k34 * C2 + P.k43);
+        const R a = static_cast<R>(n3 + n4);
+        r3 = R(0);
+        r4 = a * P.k45 * P.k34 * C2 * tau34;
+        r7 = a * P.k32 * P.k43 * tau34;
+        r8 = R(0);
+    }
+    R r5, r9, r10, r11;
+    if (hi56) {
+        const R eq56 = ldiv(P.k65, P.k56 * C2 + P.k65);
+        const R a = static_cast<R>(n5 + n6);
+        r5 = R(0);
+        r9 = a * P.k52 * eq56;
+        r10 = a * P.k54 * C2 * eq56;
+        r11 = R(0);
+    } else {
+        r5 = a5 * P.k56 * C2;
+        r9 = a5 * P.k52;
+        r10 = a5 * P.k54 * C2;
+        r11 = static_cast<R>(n6) * P.k65;
+    }
     f(0, static_cast<R>(n1) * P.k12 * C2);
     f(1, static_cast<R>(n2) * P.k23 * C2);
     f(2, static_cast<R>(n2) * P.k25 * C2);
-    f(3, hi34 ? R(0) : static_cast<R>(n3) * P.k34 * C2);
-    f(4, hi34 ? static_cast<R>(n3 + n4) * P.k45 * P.k34 * C2 * tau34 : static_cast<R>(n4) * P.k45);
-    f(5, hi56 ? R(0) : static_cast<R>(n5) * P.k56 * C2);
+    f(3, r3);
+    f(4, r4);
+    f(5, r5);
     f(6, static_cast<R>(n2) * P.k21);
-    f(7, hi34 ? static_cast<R>(n3 + n4) * P.k32 * P.k43 * tau34 : static_cast<R>(n3) * P.k32);
-    f(8, hi34 ? R(0) : static_cast<R>(n4) * P.k43);
-    f(9, hi56 ? static_cast<R>(n5 + n6) * P.k52 * eq56 : static_cast<R>(n5) * P.k52);
-    f(10, hi56 ? static_cast<R>(n5 + n6) * P.k54 * C2 * eq56 : static_cast<R>(n5) * P.k54 * C2);
-    f(11, hi56 ? R(0) : static_cast<R>(n6) * P.k65);
+    f(7, r7);
+    f(8, r8);
+    f(9, r9);
+    f(10, r10);
+    f(11, r11);
 }
 
 // Subunit total. FP64: in the reference accumulation order (SSA.tpp:48-56),
@@ -327,14 +364,17 @@ __device__ __forceinline__ int ryr_pick(const SsaParamsT<R> &P, uint64_t w, R ca
 {
     int tr = sizeof(R) == 8 ? 0 : -1;
     R cum = R(0);
-    bool done = false;
-    ryr_rates(P, w, ca, [&](int k, R r) {
-        if (done) return;
-        if (sizeof(R) == 8) {
-            if (k == 0) cum = r;
-            else if (cum < uu) { tr = k; cum += r; }
-            else done = true;
-        } else {
+    if constexpr (sizeof(R) == 8) {   // without branches: `live` falls once a cumulative rate has reached uu
+        bool live = true;
+        ryr_rates(P, w, ca, [&](int k, R r) {
+            if (k > 0) live = live & (cum < uu);
+            tr = live ? k : tr;
+            cum += live ? r : R(0);
+        });
+    } else {
+        bool done = false;
+        ryr_rates(P, w, ca, [&](int k, R r) {
+            if (done) return;
             if (k == 0) {
                 cum = r;
                 if (r > R(0)) tr = 0;
@@ -344,8 +384,8 @@ __device__ __forceinline__ int ryr_pick(const SsaParamsT<R> &P, uint64_t w, R ca
             } else {
                 done = true;
             }
-        }
-    });
+        });
+    }
     return tr;
 }
 
@@ -893,6 +933,192 @@ __device__ __forceinline__ LaneOut lane_outputs(const LaneState &S)
     out.iters = S.iters;
     out.err = S.err;
     return out;
+}
+
+// ---------------------------------------------------------------------------
+// One lane per CRU in FP64: the operations of quad_iterate, in its order and
+// with its draws, so the results are the same bits. The quad spends a wave
+// instruction on 16 CRUs for everything that belongs to a CRU and not to a
+// subunit (the draws, the waiting time's logarithm, CaJSR) and moves the rest
+// between its lanes; one lane per CRU spends it on 64.
+// An iteration comes in three parts, so that a wave can let its events wait:
+//   lane64_try     rates, waiting time and the updated concentrations, none of
+//                  them stored: a lane whose event has to wait runs the same
+//                  iteration again;
+//   lane64_commit  stores them, with the re-splits of the update;
+//   lane64_event   chooses and applies the event that ends the iteration.
+// ---------------------------------------------------------------------------
+struct Lane64State {
+    double ca[4];
+    double jl[4];
+    double Jrel[4];
+    uint64_t w[4];
+    CruQ q;
+    double t;
+    uint32_t open;    // open RyRs of the four subunits, a signed byte each
+    uint32_t iters;
+    int changed;      // the subunit words or JLCC changed since the CRU was loaded
+};
+
+struct Lane64Consts {
+    double Cai, CaNSR, inact0, inact1;
+};
+
+struct Lane64Try {
+    double ca[4];     // CaSS after the update
+    double s[4];      // subunit totals
+    double total, h, jump, jsr, Jxfer, Jtr;
+    uint64_t r0, r1, r2, r3;   // the engine after the waiting time's draw
+    int split;        // split_mask of subunit j at bits 2j, 2j + 1
+    bool last;
+};
+
+__device__ __forceinline__ int open_get(uint32_t o, int j) { return static_cast<int8_t>(o >> (8 * j)); }
+
+__device__ __forceinline__ void lane64_begin(Lane64State &S, double rRyR)
+{
+    S.open = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int open = ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
+        S.open |= static_cast<uint32_t>(static_cast<uint8_t>(open)) << (8 * j);
+        S.Jrel[j] = rRyR * static_cast<double>(open) * (S.q.jsr - S.ca[j]);
+    }
+    S.t = 0.0;
+    S.iters = 0;
+}
+
+template <int PRNG>
+__device__ __forceinline__ void lane64_try(const Lane64State &S, Lane64Try &X, const SsaParams &P, const StepConsts &K,
+                                           const LccTable &T, double dt)
+{
+    const Lane64Consts k{K.Cai, K.CaNSR, K.inact0, K.inact1};   // read once: chosen where they lie, each choice is a branch
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        X.s[j] = subunit_total(P, k, T, S.w[j], S.ca[j]);
+        asm volatile("" : "+v"(X.s[j]));   // one subunit after another: interleaved, they need twice the registers
+    }
+    X.total = X.s[0] + X.s[1] + X.s[2] + X.s[3];
+    X.r0 = S.q.r0; X.r1 = S.q.r1; X.r2 = S.q.r2; X.r3 = S.q.r3;
+    X.jump = lneglog(u01(rng_next<PRNG>(X.r0, X.r1, X.r2, X.r3))) / X.total;
+    X.last = !(S.t + X.jump < dt);
+    X.h = X.last ? dt - S.t : X.jump;
+    X.split = 0;
+    double Jx[4];
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {   // update_CaSS (SSA.tpp:87-99)
+        const double old = S.ca[j];
+        const double Jiss = P.riss * (S.ca[(j + 1) & 3] + S.ca[(j + 3) & 3] - 2 * old);
+        Jx[j] = P.rxfer * (old - k.Cai);
+        const double d = X.h * (S.jl[j] + S.Jrel[j] - Jx[j] + Jiss) * beta_ss(P, old);
+        X.ca[j] = old + d;
+        asm volatile("" : "+v"(X.ca[j]));
+        X.split |= split_mask<double>(old, X.ca[j]) << (2 * j);
+    }
+    X.Jxfer = Jx[0] + Jx[1] + Jx[2] + Jx[3];
+    // update_CaJSR (SSA.hpp:67-71)
+    X.Jtr = P.rtr * (k.CaNSR - S.q.jsr);
+    const double Jsum = S.Jrel[0] + S.Jrel[1] + S.Jrel[2] + S.Jrel[3];
+    X.jsr = S.q.jsr + X.h * beta_jsr(P, S.q.jsr) * (X.Jtr - P.VSS_VJSR * Jsum);
+}
+
+// old: the concentrations the iteration started from; w_pre: the words before the re-splits.
+template <int PRNG>
+__device__ __forceinline__ void lane64_commit(Lane64State &S, const Lane64Try &X, const SsaParams &P, double (&old)[4],
+                                              uint64_t (&w_pre)[4])
+{
+    S.q.r0 = X.r0; S.q.r1 = X.r1; S.q.r2 = X.r2; S.q.r3 = X.r3;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        old[j] = S.ca[j];
+        w_pre[j] = S.w[j];
+    }
+    // sample_RyR56 / sample_RyR34 (SSA.tpp:59-84), in subunit order
+#pragma unroll 1
+    for (int m = X.split; m != 0; m &= m - 1) {
+        const int bit = __builtin_ctz(m), j = bit >> 1;
+        const int sh = (bit & 1) ? 16 : 32;   // the (3,4) or the (5,6) pair's bytes
+        uint64_t w = sel4(S.w, j);
+        const double C2 = sq(sel4(old, j));
+        const double kb = (bit & 1) ? P.k43 : P.k65, kf = (bit & 1) ? P.k34 : P.k56;
+        const double pr = kb / (kb + kf * C2);
+        const int n = static_cast<int8_t>(w >> sh) + static_cast<int8_t>(w >> (sh + 8));
+        int c = 0;
+        for (int i = 0; i < n; ++i)
+            if (u01(rng_next<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3)) < pr) c++;
+        const uint64_t pair = n > 0 ? static_cast<uint64_t>(c & 0xff) | static_cast<uint64_t>((n - c) & 0xff) << 8 : 0;
+        w = (w & ~(0xffffULL << sh)) | pair << sh;
+        put4(S.w, j, w);
+        S.changed = 1;
+    }
+#pragma unroll
+    for (int j = 0; j < 4; ++j) S.ca[j] = X.ca[j];
+    S.q.jsr = X.jsr;
+    S.iters++;
+}
+
+// sample_weights over the subunits (common.hpp:49-59) and sample_new_state
+// (SSA.tpp:262-283) on the chosen one; false if a count left the range its
+// byte holds.
+template <int PRNG>
+__device__ __forceinline__ bool lane64_event(Lane64State &S, const Lane64Try &X, const SsaParams &P, const StepConsts &K,
+                                             const LccTable &T, const double (&old)[4], const uint64_t (&w_pre)[4])
+{
+    S.t += X.jump;
+    S.changed = 1;
+    int js = 0;
+    {
+        const double u = u01(rng_next<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3)) * X.total;
+        double cum = X.s[0];
+        if (cum < u) { js = 1; cum += X.s[1];
+            if (cum < u) { js = 2; cum += X.s[2];
+                if (cum < u) { js = 3; } } }
+    }
+    const double u3 = u01(rng_next<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3));
+    uint64_t w = sel4(S.w, js);
+    const double o = sel4(old, js), s_me = sel4(X.s, js), ca = sel4(S.ca, js);
+    double jl = sel4(S.jl, js);
+    const int L = sub_lcc(w), y = sub_y(w), cl = sub_cl(w);
+    const double Q = T.Q[L], r0 = T.R0[L], R1 = T.R1[L], i0 = K.inact0, i1 = K.inact1;
+    const double J = K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * ca);   // the flux of a channel that opens now
+    const double sum_LCC = T.P[L] + Q * o;
+    const double inact = y ? i1 : i0;
+    const double clr = cl ? P.kbClCh : P.kfClCh * o;
+    const double sum_RyR = s_me - (sum_LCC + inact + clr);
+    const double u = u3 * s_me;
+    const int cls = (u < sum_LCC) ? 0 : (u < (sum_LCC + inact)) ? 1 : (u < (sum_LCC + inact + sum_RyR)) ? 2 : 3;
+    const double u4 = (cls == 0 || cls == 2) ? u01(rng_next<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3)) : 0.0;
+    bool ok = true;
+    if (cls == 0) {
+        // sample_LCC (SSA.tpp:103-197); the scan never compares after adding r2
+        const double uu = u4 * sum_LCC;
+        const double r01 = r0 + ((L == 1) ? Q * o : R1);
+        const int tr = r0 < uu ? (r01 < uu ? 2 : 1) : 0;
+        const int Ln = lcc_next(L, tr);
+        if ((L == 5 && Ln == 6) || (L == 11 && Ln == 12))
+            jl = (y == 1) ? J : 0.0;
+        else if (L == 6 || L == 12)
+            jl = 0.0;
+        w = sub_set_lcc(w, Ln);
+    } else if (cls == 1) {
+        w = sub_flip_y(w);
+        if (y == 1) jl = 0.0;
+        else if (L == 6 || L == 12) jl = J;
+    } else if (cls == 2) {
+        // sample_RyR (SSA.tpp:200-259) over the propensities before this iteration's update
+        const int tr = ryr_pick(P, sel4(w_pre, js), o, u4 * sum_RyR);
+        ok = ryr_in_range(w, tr);
+        w = ryr_apply(w, tr);
+        int open = open_get(S.open, js);
+        open += (tr == 1 || tr == 10) ? 1 : (tr == 4 || tr == 7) ? -1 : 0;
+        S.open = (S.open & ~(0xffu << (8 * js))) | (static_cast<uint32_t>(static_cast<uint8_t>(open)) << (8 * js));
+        put4(S.Jrel, js, P.rRyR * static_cast<double>(open) * (S.q.jsr - ca));
+    } else {
+        w = sub_flip_cl(w);
+    }
+    put4(S.w, js, w);
+    put4(S.jl, js, jl);
+    return ok;
 }
 
 }  // namespace gw

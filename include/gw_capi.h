@@ -376,7 +376,8 @@ int gw_batch_get_persistent(gw_batch *b, int32_t *active);
  * CRU two steps with its state held in registers, so the CRU state crosses HBM once per
  * two steps; the two closes the launch's SSA steps need run just before it, in a kernel
  * of their own. Other shapes, FP64, frozen globals, replayed graphs and the persistent
- * kernel keep one step per launch. With one CRU per lane the results are bit-identical
+ * kernel keep one step per launch; FP64 batches of 640,000 CRUs and more (xoshiro256**,
+ * no digests) run two with a request of 0 or 2, whatever their shape. With one CRU per lane the results are bit-identical
  * to one step per launch; with refilled lanes they are deterministic, and the rounding
  * of the FP64 flux sums can differ (their order follows which CRUs each lane ran).
  * Automatic: two steps per launch when a launch's SSA blocks are more than the GPU
@@ -427,7 +428,7 @@ int gw_batch_get_iterations(gw_batch *b, uint64_t *iters);
  * or 256 threads); each wave then owns 64 x crus_per_lane consecutive CRUs (16 x
  * with quads) and a lane or quad whose CRU has finished its step takes the next
  * one, so waves wait less on their slowest CRU; 0 = 1. FP64 results do not depend on the shape (exact flux
- * sums). Shapes other than 4 x 256 exist for xoshiro256** batches without
+ * sums), and large FP64 batches run kernels of one lane per CRU instead of the quads asked for. Shapes other than 4 x 256 exist for xoshiro256** batches without
  * replay digests or frozen globals. No reference counterpart (the reference
  * has one OpenMP loop over CRUs, src/includes/GW.tpp:223-233).
  */
