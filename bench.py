@@ -501,7 +501,7 @@ def main(argv=None):
     ap.add_argument("--steps-per-launch", type=int, choices=[0, 1, 2], default=0,
                     help="SSA steps per launch (2: each CRU advances two steps per launch with its state in registers, "
                          "FP32-local one-lane shapes of 64 threads and large FP64 batches; 0, the default: the "
-                         "library's choice, two when a launch's blocks are more than the GPU holds at once)")
+                         "library's choice, two for batches of 450,000 CRUs and more)")
     ap.add_argument("--precision", choices=["both", "fp32", "fp64"], default="both",
                     help="forms to time; with both, value is the batched FP32-local form and fp64 sits beside it")
     ap.add_argument("--ensemble-beats", type=int, default=0, metavar="N",

@@ -940,6 +940,7 @@ __device__ __forceinline__ void lane_load(const KArgs &a, int64_t slot, LaneStat
     const ulonglong2 r01 = pr[0], r23 = pr[1];
     S.q.r0 = r01.x; S.q.r1 = r01.y; S.q.r2 = r23.x; S.q.r3 = r23.y;
     S.q.jsr = a.CaJSR[slot];
+    S.changed = 0;
 }
 
 __device__ __forceinline__ void lane_store(const KArgs &a, int64_t slot, const LaneState &S)
@@ -959,56 +960,56 @@ __device__ __forceinline__ void lane_store(const KArgs &a, int64_t slot, const L
     a.CaJSR[slot] = S.q.jsr;
 }
 
-// Running sums of the outputs of the CRUs each lane finishes, in finishing
-// order, one LDS slot per thread (kept out of the registers the SSA needs).
+// Running FP64 sums of the outputs of the CRUs each lane finishes, in
+// finishing order, one LDS slot per thread (kept out of the registers the SSA
+// needs), added by LDS atomics that no one waits for.
 template <int BLOCK>
 struct LaneSums {
     double Jxfer[BLOCK], Jtr[BLOCK], JLCC[BLOCK], Jrel[BLOCK];
-    int open[BLOCK], clch[BLOCK], iters[BLOCK], err[BLOCK];
+    unsigned long long ints[BLOCK];   // iterations, open RyRs from bit 32, open ClCh from bit 48
+    int err;
     __device__ __forceinline__ void zero(int t)
     {
         Jxfer[t] = Jtr[t] = JLCC[t] = Jrel[t] = 0.0;
-        open[t] = clch[t] = iters[t] = err[t] = 0;
+        ints[t] = 0;
+        if (t == 0) err = 0;
     }
-    __device__ __forceinline__ void add(int t, const LaneOut &o)
+    // outputs of update_CRUstate_from_temp (GW.tpp:47-62), summed in subunit order in FP64
+    __device__ __forceinline__ void add(int t, const LaneState &S, const LaneTry &X)
     {
-        Jxfer[t] += o.Jxfer;
-        Jtr[t] += o.Jtr;
-        JLCC[t] += o.JLCC;
-        Jrel[t] += o.Jrel;
-        open[t] += o.open;
-        clch[t] += o.clch;
-        iters[t] += static_cast<int>(o.iters);
-        err[t] |= o.err;
-    }
-    __device__ __forceinline__ LaneOut get(int t) const
-    {
-        LaneOut o;
-        o.Jxfer = Jxfer[t];
-        o.Jtr = Jtr[t];
-        o.JLCC = JLCC[t];
-        o.Jrel = Jrel[t];
-        o.open = open[t];
-        o.clch = clch[t];
-        o.iters = static_cast<uint32_t>(iters[t]);
-        o.err = err[t];
-        return o;
+        unsafeAtomicAdd(&Jxfer[t], X.Jxfer);
+        unsafeAtomicAdd(&Jtr[t], static_cast<double>(X.Jtr));
+        unsafeAtomicAdd(&JLCC[t], ((static_cast<double>(S.jl[0]) + S.jl[1]) + S.jl[2]) + S.jl[3]);
+        unsafeAtomicAdd(&Jrel[t], ((static_cast<double>(S.Jrel[0]) + S.Jrel[1]) + S.Jrel[2]) + S.Jrel[3]);
+        int open = 0, clch = 0;
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            open += ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
+            clch += sub_cl(S.w[j]);
+        }
+        const int64_t v = (static_cast<int64_t>(clch) << 48) + (static_cast<int64_t>(open) << 32) + S.iters;
+        atomicAdd(&ints[t], static_cast<unsigned long long>(v));
     }
 };
 
 // Per-wave sums of the lanes' output sums (a fixed FP64 xor butterfly, the
 // same in every lane), added exactly into the block accumulators by lanes 0..3.
-__device__ __forceinline__ void lane_accumulate(BlockAcc &acc, const LaneOut &o)
+template <int BLOCK>
+__device__ __forceinline__ void lane_accumulate(BlockAcc &acc, const LaneSums<BLOCK> &Ls, int t)
 {
-    const int lane = threadIdx.x & (kWave - 1);
-    const double sx = wave_sum(o.Jxfer), st = wave_sum(o.Jtr), sl = wave_sum(o.JLCC), sr = wave_sum(o.Jrel);
-    const int n_it = wave_sum(static_cast<int>(o.iters)), n_open = wave_sum(o.open), n_cl = wave_sum(o.clch);
+    const int lane = t & (kWave - 1);
+    const double sx = wave_sum(Ls.Jxfer[t]), st = wave_sum(Ls.Jtr[t]), sl = wave_sum(Ls.JLCC[t]), sr = wave_sum(Ls.Jrel[t]);
+    const int64_t v64 = static_cast<int64_t>(Ls.ints[t]);
+    const int iters = static_cast<int>(v64 & 0xffffffff);
+    const int open = static_cast<int16_t>((v64 >> 32) & 0xffff);
+    const int clch = static_cast<int>((v64 - (static_cast<int64_t>(open) << 32)) >> 48);
+    const int n_it = wave_sum(iters), n_open = wave_sum(open), n_cl = wave_sum(clch);
     const int k = lane & 3;
     const double v = k == 0 ? sx : k == 1 ? st : k == 2 ? sl : sr;
     Fx f;
     fx_zero(f);
     const int fl = fx_add(f, v);
-    const bool bad = (__ballot(o.err != 0) | __ballot(lane < 3 && fl != 0)) != 0;
+    const bool bad = __ballot(lane < 3 && fl != 0) != 0 || Ls.err != 0;
     if (lane < 4) {
         acc_add_fx(acc, lane, f);
         const int64_t iv = lane == 0 ? n_it : lane == 1 ? n_open : lane == 2 ? n_cl : (bad ? 1 : 0);
@@ -1016,92 +1017,140 @@ __device__ __forceinline__ void lane_accumulate(BlockAcc &acc, const LaneOut &o)
     }
 }
 
-// The SSA of block b with one lane per CRU (FP32-local variant). Wave w of the
-// block owns kWave * CPT consecutive CRUs of the block's cell. Its lanes start
-// on the first kWave of them; a lane whose CRU has finished the step takes the
-// next CRU of the range not yet taken (the finishing lanes in lane order, by
-// a ballot), so the wave makes about (iterations of its range) / kWave trips
-// rather than CPT times the most iterations of any one CRU. Which lane runs
-// which CRU depends only on the CRUs' own iteration counts, the same on every
-// run. Each lane sums the outputs of its CRUs in FP64 as it finishes them; the
-// per-wave sums are a fixed xor butterfly, added exactly across waves and
-// blocks.
-template <int PRNG, int BLOCK, int CPT>
-__device__ __forceinline__ void ssa_block_lane(const KArgs &a, int b, int64_t step0, LccTableF &T, BlockAcc &acc,
-                                               LaneSums<BLOCK> &Ls)
+// The SSA of block b with one lane per CRU (FP32-local variant), steps m ..
+// m + nss - 1 (nss <= NSS). Wave w of the block owns kWave * CPT consecutive
+// CRUs of the block's cell. Its lanes start on the first kWave of them; a lane
+// whose CRU has finished its steps takes the next CRU of the range not yet
+// taken (the finishing lanes in lane order, by a ballot), so the wave makes
+// about (iterations of its range) / kWave trips rather than CPT times the most
+// iterations of any one CRU. Which lane runs which CRU depends only on the
+// CRUs' own iterations, the same on every run. Each lane sums the outputs of
+// its CRUs in FP64 as it finishes them; the per-wave sums are a fixed xor
+// butterfly, added exactly across waves and blocks.
+//
+// Events wait: in nearly every trip a lane or two of the 64 end their
+// iteration in an event, whose code is nearly as long as the rest of the
+// trip. Such a lane leaves its CRU as it was and runs the same iteration again
+// (it would idle otherwise), until event_batch lanes of the wave hold an
+// event, or no other lane made progress, or no fresh CRU is left. Early in an
+// action potential (1.9% of the iterations end in an event), two steps per
+// launch, batches of 1 and 8: 256 x 7,000 CRUs, 4 per lane, 51.1 and 49.2 us
+// per step, 64 x 12,500 32.6 and 31.3; 2 per lane 49.2 and 52.5: too few
+// iterations per lane to wait for, so there an event is applied at once.
+template <int BLOCK, int NSS>
+struct LaneLds {
+    StepConstsF K[NSS];
+    BlockAcc acc[NSS];
+    LaneSums<BLOCK> Ls[NSS];
+};
+
+constexpr int event_batch(int cpt) { return cpt >= 4 ? 8 : 1; }
+
+template <int PRNG, int BLOCK, int CPT, int NSS>
+__device__ __forceinline__ void ssa_block_lane(const KArgs &a, int b, int64_t m, int nss, LaneLds<BLOCK, NSS> &L)
 {
     constexpr int kMap = shape_of_crus(BLOCK * CPT);
     static_assert(crus_per_block(kMap) == BLOCK * CPT, "CRUs per block must be 16 << map");
+    constexpr int kWords = sizeof(StepConstsF) / 4;
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
     const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
-    const int ks = static_cast<int>(step0 & 1);
     const DevCell &C = a.cells[cell];
     const CellDyn &D = a.dyn[cell];
-    const SsaParamsF &sp = C.spf;
-    const StepConstsF &kk = D.kf[ks];
+    const float rRyR = C.spf.rRyR;
     const float dt = static_cast<float>(a.dt);
-    load_lcc_table(kk, T);
-    acc_zero(acc);
-    Ls.zero(tid);
+#pragma unroll
+    for (int s = 0; s < NSS; ++s) {
+        if (s < nss)
+            for (int t = tid; t < kWords; t += BLOCK)
+                reinterpret_cast<uint32_t *>(&L.K[s])[t] = reinterpret_cast<const uint32_t *>(&D.kf[(m + s) & 1])[t];
+        acc_zero(L.acc[s]);
+        L.Ls[s].zero(tid);
+    }
     __syncthreads();
+    const int64_t stop = D.stop_step;
+    const bool run1 = nss > 1 && m + 1 < stop;
     const int64_t w0 = static_cast<int64_t>(b - C.blk0[kMap]) * (BLOCK * CPT) + wave * (kWave * CPT);
-    const int64_t w1 = min(w0 + kWave * CPT, static_cast<int64_t>(C.n_cru));
-    int64_t i = w0 + lane;
-    int64_t next = w0 + kWave;   // first CRU of the range not yet taken (wave-uniform)
-    bool have = (i < w1) && (step0 < D.stop_step);
+    const int w1 = static_cast<int>(min(static_cast<int64_t>(kWave * CPT), C.n_cru - w0));   // CRUs of the wave's range
+    const int64_t slot0 = C.slot0 + w0;
+    int i = lane;
+    int next = kWave;   // first CRU of the range not yet taken (wave-uniform)
+    bool have = i < w1 && m < stop;
+    int sidx = 0;       // the step (0: m, 1: m + 1) this lane's CRU is in
     LaneState S;
     if (have) {
-        lane_load(a, C.slot0 + i, S);
-        lane_begin(S, sp);
+        lane_load(a, slot0 + i, S);
+        lane_begin(S, rRyR);
     }
     while (__ballot(have)) {
-        bool fin = false;
+        const SsaParamsF *spp = &C.spf;
+        asm volatile("" : "+s"(spp));   // read again in each trip: held over the loop they push others out
+        const SsaParamsF sp = load_scalar(spp);
+        LaneTry X;
+        bool ev = false;
+        const StepConstsF &K = L.K[NSS > 1 ? sidx : 0];
         if (have) {
-            fin = lane_iterate<PRNG>(S, sp, kk, T, dt);
-            if (fin) {
-                lane_store(a, C.slot0 + i, S);
-                Ls.add(tid, lane_outputs(S));
+            lane_try<PRNG>(S, X, sp, LaneConsts{K.Cai_d, K.CaNSR_d, K.inact0, K.inact1}, K.lcc, dt);
+            ev = !X.last;
+        }
+        const uint64_t m_ev = __ballot(ev);
+        const uint64_t m_last = __ballot(have && !ev);
+        const bool go = __popcll(m_ev) >= event_batch(CPT) || m_last == 0 || next >= w1;   // wave-uniform
+        bool fin = have && !ev;
+        if (have && (go || !ev)) {
+            if (!lane_commit<PRNG>(S, X, sp, K, ev && go)) {
+                L.Ls[sidx].err = 1;
+                fin = fin || S.iters >= kMaxItersPerStep;
             }
         }
-        if constexpr (CPT > 1) {
-            const uint64_t m = __ballot(fin);
-            if (fin) {
-                const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(m >> 32),
-                                                  __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(m), 0u)));
-                i = next + rank;
+        if (fin) {
+            L.Ls[NSS > 1 ? sidx : 0].add(tid, S, X);
+            if (NSS > 1 && sidx == 0 && run1) {   // the same CRU, next step
+                sidx = 1;
+                lane_begin(S, rRyR);
+                fin = false;
+            } else {
+                sidx = 0;
+                lane_store(a, slot0 + i, S);
+            }
+        }
+        const uint64_t msk = __ballot(fin);
+        if (fin) {
+            if constexpr (CPT > 1) {
+                i = next + static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(msk >> 32),
+                                            __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(msk), 0u)));
                 have = i < w1;
                 if (have) {
-                    lane_load(a, C.slot0 + i, S);
-                    lane_begin(S, sp);
+                    lane_load(a, slot0 + i, S);
+                    lane_begin(S, rRyR);
                 }
+            } else {
+                have = false;
             }
-            next += __popcll(m);
-        } else {
-            if (fin) have = false;
         }
+        next += __popcll(msk);
     }
-    lane_accumulate(acc, Ls.get(tid));
+    for (int s = 0; s < nss; ++s) lane_accumulate(L.acc[s], L.Ls[s], tid);
     __syncthreads();
-    write_partial(a, acc, ks * a.nblocks + b);
+    for (int s = 0; s < nss; ++s) write_partial(a, L.acc[s], ((m + s) & 1) * a.nblocks + b);
 }
 
-// One lane per CRU needs about 100-128 VGPRs; 4 waves per SIMD keep it free
-// of spills and still hold 256 lanes per SIMD.
+// One lane per CRU needs about 100 VGPRs; 4 waves per SIMD keep it, and the
+// close in its first blocks, free of spills.
 template <int PRNG, int BLOCK, int CPT>
 __global__ __launch_bounds__(BLOCK, 4) void k_step_lane(KArgs a, int64_t ssa_step, int32_t nclose, const int64_t *base)
 {
-    __shared__ LccTableF T;
-    __shared__ CloseLds<BLOCK> csh;
-    __shared__ BlockAcc acc;
-    __shared__ LaneSums<BLOCK> Ls;
+    __shared__ union {
+        LaneLds<BLOCK, 1> ssa;
+        CloseLds<BLOCK> close;
+    } sh;
     const int bid = blockIdx.x;
     if (bid < nclose) {
-        close_cell<BLOCK>(a, bid, a.dyn[bid], csh);
+        close_cell<BLOCK>(a, bid, a.dyn[bid], sh.close);
         return;
     }
-    ssa_block_lane<PRNG, BLOCK, CPT>(a, bid - nclose, base ? *base + ssa_step : ssa_step, T, acc, Ls);
+    ssa_block_lane<PRNG, BLOCK, CPT, 1>(a, bid - nclose, base ? *base + ssa_step : ssa_step, 1, sh.ssa);
 }
 
 // ---------------------------------------------------------------------------
@@ -1402,93 +1451,18 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<R>) void k_persist(KArgs a, i
 // to one step per launch; with refilled lanes the order of a lane's FP64 sums
 // depends on which CRUs it ran, which can change their rounding.
 // ---------------------------------------------------------------------------
-template <int BLOCK>
-struct PairLds {
-    StepConstsF K[2];       // constants of steps m and m + 1
-    LccTableF T[2];
-    BlockAcc acc[2];
-    LaneSums<BLOCK> Ls[2];
-};
-
+// What bounds it on 12.8 M CRUs is HBM: the state in and out, 207 B per CRU
+// measured, at 4.4 TB/s (a copy of this size reaches 4.9), 318 us per step.
+// Before its parameters lay in scalar registers and the step's constants were
+// read at the top of a trip (chosen in LDS, each choice was a branch) it took
+// 418. 98 VGPRs with four or more CRUs per lane, where a fifth wave per SIMD
+// changes nothing (321); with one or two it does (1 per lane 372 and 327, 2
+// per lane 335 and 311 us).
 template <int PRNG, int BLOCK, int CPT>
-__global__ __launch_bounds__(BLOCK, 4) void k_step_lane2(KArgs a, int64_t m, int32_t nss)
+__global__ __launch_bounds__(BLOCK, CPT <= 2 ? 5 : 4) void k_step_lane2(KArgs a, int64_t m, int32_t nss)
 {
-    constexpr int kMap = shape_of_crus(BLOCK * CPT);
-    static_assert(crus_per_block(kMap) == BLOCK * CPT, "CRUs per block must be 16 << map");
-    constexpr int kWords = sizeof(StepConstsF) / 4;
-    __shared__ PairLds<BLOCK> P;
-    const int b = blockIdx.x;
-    const int tid = threadIdx.x;
-    const int lane = tid & (kWave - 1);
-    const int wave = tid / kWave;
-    const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
-    const DevCell &C = a.cells[cell];
-    const CellDyn &D = a.dyn[cell];
-    const SsaParamsF &sp = C.spf;
-    for (int t = tid; t < 2 * kWords; t += BLOCK) {
-        const int s = t / kWords, w = t % kWords;
-        if (s < nss) reinterpret_cast<uint32_t *>(&P.K[s])[w] = reinterpret_cast<const uint32_t *>(&D.kf[(m + s) & 1])[w];
-    }
-    acc_zero(P.acc[0]);
-    acc_zero(P.acc[1]);
-    P.Ls[0].zero(tid);
-    P.Ls[1].zero(tid);
-    __syncthreads();
-    for (int s = 0; s < nss; ++s) load_lcc_table(P.K[s], P.T[s]);
-    __syncthreads();
-    const float dt = static_cast<float>(a.dt);
-    const int64_t stop = D.stop_step;   // set by the closes before this launch
-    const bool run0 = m < stop;
-    const bool run1 = nss > 1 && m + 1 < stop;
-    const int64_t w0 = static_cast<int64_t>(b - C.blk0[kMap]) * (BLOCK * CPT) + wave * (kWave * CPT);
-    const int64_t w1 = min(w0 + kWave * CPT, static_cast<int64_t>(C.n_cru));
-    int64_t i = w0 + lane;
-    int64_t next = w0 + kWave;   // first CRU of the range not yet taken (wave-uniform)
-    bool have = (i < w1) && run0;
-    int sidx = 0;                // the step (0: m, 1: m + 1) this lane's CRU is in
-    LaneState S;
-    if (have) {
-        lane_load(a, C.slot0 + i, S);
-        lane_begin(S, sp);
-    }
-    while (__ballot(have)) {
-        bool fin = false;
-        if (have) {
-            fin = lane_iterate<PRNG>(S, sp, P.K[sidx], P.T[sidx], dt);
-            if (fin) {
-                P.Ls[sidx].add(tid, lane_outputs(S));
-                if (sidx == 0 && run1) {   // the same CRU, next step
-                    const int changed = S.changed;   // the store after step m + 1 keeps step m's changes
-                    sidx = 1;
-                    lane_begin(S, sp);
-                    S.changed = changed;
-                    fin = false;
-                } else {
-                    sidx = 0;
-                    lane_store(a, C.slot0 + i, S);
-                }
-            }
-        }
-        if constexpr (CPT > 1) {
-            const uint64_t msk = __ballot(fin);
-            if (fin) {
-                const int rank = static_cast<int>(__builtin_amdgcn_mbcnt_hi(static_cast<uint32_t>(msk >> 32),
-                                                  __builtin_amdgcn_mbcnt_lo(static_cast<uint32_t>(msk), 0u)));
-                i = next + rank;
-                have = i < w1;
-                if (have) {
-                    lane_load(a, C.slot0 + i, S);
-                    lane_begin(S, sp);
-                }
-            }
-            next += __popcll(msk);
-        } else {
-            if (fin) have = false;
-        }
-    }
-    for (int s = 0; s < nss; ++s) lane_accumulate(P.acc[s], P.Ls[s].get(tid));
-    __syncthreads();
-    for (int s = 0; s < nss; ++s) write_partial(a, P.acc[s], ((m + s) & 1) * a.nblocks + b);
+    __shared__ LaneLds<BLOCK, 2> sh;
+    ssa_block_lane<PRNG, BLOCK, CPT, 2>(a, blockIdx.x, m, nss, sh);
 }
 
 // One or two (ncl) consecutive closes of every cell, one block of four waves per cell (the
@@ -1515,7 +1489,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_close_cells(KArgs a, int32_t ncl)
 // trip of a wave of 64 CRUs one or two lanes would take the event path, a
 // third as long as the rest of the trip. A lane whose iteration ends in an event
 // leaves its CRU as it was and runs the same iteration again (it would idle
-// otherwise), until kEventBatch lanes of the wave hold an event, or no other
+// otherwise), until event_batch lanes of the wave hold an event, or no other
 // lane made progress, or no fresh CRU is left to keep the others busy; then
 // all of them commit at once. 12.8 M CRUs, 4 per lane: 552, 551, 542 and 543
 // us per step with batches of 1, 4, 8 and 16 events.
@@ -1525,7 +1499,6 @@ __global__ __launch_bounds__(kBlock, 4) void k_close_cells(KArgs a, int32_t ncl)
 // sixteen copies of the block accumulators in LDS (below 2^53, so exact in
 // FP64, whatever the order).
 // ---------------------------------------------------------------------------
-constexpr int kEventBatch = 8;
 constexpr int kAccCopies = 16;
 
 struct Lane64Acc {
@@ -1659,7 +1632,7 @@ __device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t 
         }
         const uint64_t m_ev = __ballot(ev);
         const uint64_t m_last = __ballot(have && !ev);
-        const bool go = __popcll(m_ev) >= kEventBatch || m_last == 0 || next >= w1;   // wave-uniform
+        const bool go = __popcll(m_ev) >= event_batch(CPT) || m_last == 0 || next >= w1;   // wave-uniform
         bool fin = have && !ev;
         bool ok = true;
         if (have && (go || !ev)) {
@@ -2061,8 +2034,7 @@ struct gw_batch {
     int32_t shape = kShapeDefault;   // block -> cell map in use (16 << shape CRUs per block)
     int32_t persist_mode = 0;        // persistent step kernel: 0 off (default), 1 on, 2 when every block fits at once
     int32_t persist_fit = -1;        // whether every block of the persistent kernel fits at once (-1: not known)
-    int32_t steps_per_launch = 0;    // SSA steps per plain launch (FP32-local one-lane shapes of 64 threads): 1, 2, 0 automatic
-    int64_t pair_capacity[GW_LAUNCH_CONFIGS + 2] = {};   // blocks of k_step_lane2 resident at once, per configuration (0: not known)
+    int32_t steps_per_launch = 0;    // SSA steps per plain launch where the kernel can run two: 1, 2, 0 automatic
     int32_t cfg = 2;                 // launch configuration (kConfigs) asked for, 4 x 256 by default
     int32_t run_cfg = 2;             // the one the batch's shape arrays are set for (apply_shape)
     int64_t ncrus = 0;               // CRUs of all cells
@@ -2476,45 +2448,18 @@ bool pair_capable(gw_batch *B)
     return B->precision == GW_PREC_FP32_LOCAL && L.lanes == 1 && L.threads == 64 && B->prng == GW_PRNG_XOSHIRO256SS;
 }
 
-// The batch's two-step kernel.
-const void *pair_fn(int c)
-{
-    constexpr int P = GW_PRNG_XOSHIRO256SS;
-    switch (c) {
-    case kLane64: return reinterpret_cast<const void *>(&k_step2_lane64<P, 4>);
-    case kLane64 + 1: return reinterpret_cast<const void *>(&k_step2_lane64<P, 8>);
-    default: break;
-    }
-    switch (kConfigs[c].cpl) {
-    case 1: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 1>);
-    case 2: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 2>);
-    case 4: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 4>);
-    default: return reinterpret_cast<const void *>(&k_step_lane2<P, 64, 8>);
-    }
-}
+// Two steps per launch when asked for (2), or automatically (0) for batches of
+// 450,000 CRUs and more: there the state's HBM traffic is worth more than the
+// separate close kernel costs, about 17 us per two steps. FP32-local, one and two steps
+// per launch, in us per step: 400,000 CRUs 25.2 and 25.0 (four CRUs per lane), 24.7 and 24.0 (one);
+// 600,000 31.5 and 27.9, 30.8 and 28.5; 200,000 20.7 and 21.6, 15.1 and 17.3.
+// FP64 batches on the one-lane kernels are all larger (650,000: 50.2 and 46.7).
+constexpr int64_t kPairCrus = 450000;
 
-// How many blocks of the batch's two-step kernel the GPU holds at once.
-int64_t pair_capacity(gw_batch *B, int c)
-{
-    int64_t &cap = B->pair_capacity[c];
-    if (cap > 0) return cap;
-    int per_cu = 0, cus = 0;
-    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, pair_fn(c), 64, 0) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, B->ctx->device) == hipSuccess)
-        cap = static_cast<int64_t>(per_cu) * cus;
-    return cap > 0 ? cap : INT64_MAX;
-}
-
-// Two steps per launch when asked for (2), or automatically (0) when the SSA
-// blocks of a launch are more than the GPU holds at once: then the state's
-// HBM traffic binds and halving it pays for the separate close kernel; a batch
-// whose blocks all fit at once is bound by latency, which that kernel adds to.
 bool use_pair(gw_batch *B)
 {
     if (B->steps_per_launch == 1 || !pair_capable(B)) return false;
-    const int c = run_config(B);
-    if (B->steps_per_launch == 2 || c >= kLane64) return true;
-    return B->nblocks_shape[config_shape(c)] > pair_capacity(B, c);
+    return B->steps_per_launch == 2 || B->ncrus >= kPairCrus;
 }
 
 // One launch of the two-step kernel: SSA(m .. m + nss - 1); with e0/e1 the

@@ -262,14 +262,22 @@ GW_HD void rng_seed(int prng, uint64_t s[4], uint64_t seed)
     }
 }
 
+// The engine's next output, and its step to the state after it.
 template <int PRNG>
-GW_HD uint64_t rng_next(uint64_t &s0, uint64_t &s1, uint64_t &s2, uint64_t &s3)
+GW_HD uint64_t rng_output(uint64_t s0, uint64_t s1, uint64_t, uint64_t s3)
 {
-    uint64_t result;
+    if constexpr (PRNG == 0) return rotl64(s1 * 5, 7) * 9;
+    else if constexpr (PRNG == 1) return rotl64(s0 + s3, 23) + s0;
+    else if constexpr (PRNG == 2) return s0 + s3;
+    else if constexpr (PRNG == 3) return rotl64(s0 * 5, 7) * 9;
+    else if constexpr (PRNG == 4) return rotl64(s0 + s1, 17) + s0;
+    else return s0 + s1;
+}
+
+template <int PRNG>
+GW_HD void rng_advance(uint64_t &s0, uint64_t &s1, uint64_t &s2, uint64_t &s3)
+{
     if constexpr (PRNG <= 2) {
-        if constexpr (PRNG == 0) result = rotl64(s1 * 5, 7) * 9;
-        else if constexpr (PRNG == 1) result = rotl64(s0 + s3, 23) + s0;
-        else result = s0 + s3;
         const uint64_t t = s1 << 17;
         s2 ^= s0;
         s3 ^= s1;
@@ -278,12 +286,7 @@ GW_HD uint64_t rng_next(uint64_t &s0, uint64_t &s1, uint64_t &s2, uint64_t &s3)
         s2 ^= t;
         s3 = rotl64(s3, 45);
     } else {
-        const uint64_t a = s0;
-        uint64_t b = s1;
-        if constexpr (PRNG == 3) result = rotl64(a * 5, 7) * 9;
-        else if constexpr (PRNG == 4) result = rotl64(a + b, 17) + a;
-        else result = a + b;
-        b ^= a;
+        const uint64_t a = s0, b = s1 ^ s0;
         if constexpr (PRNG == 4) {
             s0 = rotl64(a, 49) ^ b ^ (b << 21);
             s1 = rotl64(b, 28);
@@ -292,7 +295,14 @@ GW_HD uint64_t rng_next(uint64_t &s0, uint64_t &s1, uint64_t &s2, uint64_t &s3)
             s1 = rotl64(b, 37);
         }
     }
-    return result;
+}
+
+template <int PRNG>
+GW_HD uint64_t rng_next(uint64_t &s0, uint64_t &s1, uint64_t &s2, uint64_t &s3)
+{
+    const uint64_t r = rng_output<PRNG>(s0, s1, s2, s3);
+    rng_advance<PRNG>(s0, s1, s2, s3);
+    return r;
 }
 
 // Stream key of CRU i of a cell seeded with `seed` (the SSA stream); the

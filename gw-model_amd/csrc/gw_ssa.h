@@ -487,12 +487,15 @@ __device__ __forceinline__ R qdraw(CruQ &q)
 // FP32-local layout, built for xoshiro256** only, whose scrambled output has
 // no weak bit): an event iteration then advances the engine twice, not four
 // times.
+__device__ __forceinline__ void split2(uint64_t x, float &hi, float &mid)
+{
+    hi = static_cast<float>(static_cast<uint32_t>(x >> 40)) * 0x1p-24f;
+    mid = static_cast<float>(static_cast<uint32_t>(x >> 16) & 0xffffffu) * 0x1p-24f;
+}
 template <int PRNG>
 __device__ __forceinline__ void draw2(CruQ &q, float &hi, float &mid)
 {
-    const uint64_t x = rng_next<PRNG>(q.r0, q.r1, q.r2, q.r3);
-    hi = static_cast<float>(static_cast<uint32_t>(x >> 40)) * 0x1p-24f;
-    mid = static_cast<float>(static_cast<uint32_t>(x >> 16) & 0xffffffu) * 0x1p-24f;
+    split2(rng_next<PRNG>(q.r0, q.r1, q.r2, q.r3), hi, mid);
 }
 
 // One global step of SSA_single_CRU (SSA.tpp:286-310); lane j holds subunit j.
@@ -720,13 +723,6 @@ __device__ __forceinline__ void put4(T (&v)[4], int k, T x)
         if (k == j) v[j] = x;
 }
 
-struct LaneOut {
-    double Jxfer, Jtr, JLCC, Jrel;   // per-CRU sums in subunit order
-    int open, clch;
-    uint32_t iters;
-    int err;
-};
-
 // The working state of one CRU during one global step.
 struct LaneState {
     double ca[4];
@@ -734,205 +730,207 @@ struct LaneState {
     CruQ q;
     float jl[4];
     float Jrel[4];
-    float Jxfer[4];
-    int open[4];
-    float t, Jtr;
+    uint32_t open;   // open RyRs of the four subunits, a signed byte each
+    float t;
     uint32_t iters;
-    int err;
-    int changed;   // the subunit words or JLCC changed this step (an event or a re-split)
+    int changed;     // the subunit words or JLCC changed since the CRU was loaded (an event or a re-split)
 };
 
-// copy_from_CRUState (SSA.tpp:10-33): the step's starting fluxes.
-__device__ __forceinline__ void lane_begin(LaneState &S, const SsaParamsF &P)
+__device__ __forceinline__ int open_get(uint32_t o, int j) { return static_cast<int8_t>(o >> (8 * j)); }
+__device__ __forceinline__ void open_put(uint32_t &o, int j, int v)
 {
-#pragma clang fp contract(fast)   // FP32-local only: fused multiply-adds allowed
-    using R = float;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        S.open[j] = ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
-        S.Jrel[j] = P.rRyR * static_cast<R>(S.open[j]) * static_cast<R>(S.q.jsr - S.ca[j]);
-        S.Jxfer[j] = R(0);
-    }
-    S.t = R(0);
-    S.Jtr = R(0);
-    S.iters = 0;
-    S.err = 0;
-    S.changed = 0;
+    o = (o & ~(0xffu << (8 * j))) | (static_cast<uint32_t>(static_cast<uint8_t>(v)) << (8 * j));
 }
 
-// One iteration of SSA_single_CRU's loop (SSA.tpp:290-309); true when the
-// step is finished. The event (subunit, class, transition) is chosen from the
+// copy_from_CRUState (SSA.tpp:10-33): the step's starting fluxes.
+__device__ __forceinline__ void lane_begin(LaneState &S, float rRyR)
+{
+    S.open = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+        const int open = ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
+        S.open |= static_cast<uint32_t>(static_cast<uint8_t>(open)) << (8 * j);
+        S.Jrel[j] = rRyR * static_cast<float>(open) * static_cast<float>(S.q.jsr - S.ca[j]);
+    }
+    S.t = 0.0f;
+    S.iters = 0;
+}
+
+// An iteration of SSA_single_CRU's loop (SSA.tpp:290-309) comes in two parts,
+// so that a wave can let its events wait: lane_try forms the rates, the
+// waiting time and the increments without storing any of them (a lane whose
+// event has to wait runs the same iteration again), lane_commit stores them
+// with the re-splits of the update and, where the iteration ends in one,
+// chooses and applies the event. The event (subunit, class, transition) is chosen from the
 // propensities before this iteration's Ca update, as in the reference, but
 // its uniforms are drawn before the re-split Bernoulli draws of that update
 // rather than after them: the draws are independent, so the joint law of the
 // choice and the re-splits is the same, and only the choice (not the
 // pre-update channel words and totals) has to be kept across the update.
 // The four uniforms of an event iteration (waiting time, subunit, class,
-// transition) and the Bernoulli trials of a re-split come two per engine draw
-// (draw2).
+// transition) and the Bernoulli trials of a re-split come two per engine draw.
+struct LaneTry {
+    float s[4];        // subunit totals
+    float d[4], dj;    // the increments of CaSS and CaJSR
+    float total, jump, u_sub, Jtr;
+    double Jxfer;      // summed over the subunits in order
+    int split;         // split_mask of subunit j at bits 2j, 2j + 1
+    bool last;
+};
+
+// The step's constants an iteration reads, out of LDS once: chosen where they lie, each choice is a branch.
+struct LaneConsts {
+    double Cai, CaNSR;
+    float inact0, inact1;
+};
+
 template <int PRNG>
-__device__ __forceinline__ bool lane_iterate(LaneState &S, const SsaParamsF &P, const StepConstsF &K,
-                                             const LccTableF &T, float dt)
+__device__ __forceinline__ void lane_try(const LaneState &S, LaneTry &X, const SsaParamsF &P, const LaneConsts &K,
+                                         const LccTableF &T, float dt)
 {
 #pragma clang fp contract(fast)   // FP32-local only: fused multiply-adds allowed
-    using R = float;
-    const double Cai = K.Cai_d, CaNSR = K.CaNSR_d;
-    S.iters++;
     // update_fluxes + update_rates (SSA.tpp:37-56)
-    double oldA[4];
-    R old[4];
+    X.Jtr = P.rtr * static_cast<float>(K.CaNSR - S.q.jsr);
+    asm volatile("" : "+v"(X.Jtr));   // rounded here, not inside a fused operation below
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        oldA[j] = S.ca[j];
-        old[j] = static_cast<R>(oldA[j]);
+        X.s[j] = subunit_total(P, K, T, S.w[j], static_cast<float>(S.ca[j]));
+        asm volatile("" : "+v"(X.s[j]));   // one subunit after another: interleaved, they need twice the registers
     }
-    S.Jtr = P.rtr * static_cast<R>(CaNSR - S.q.jsr);
-    int js = 0, cls = 0, tr = 0;
-    R jump, h;
-    bool last;
-    {
-        R s[4];
-#pragma unroll
-        for (int j = 0; j < 4; ++j) s[j] = subunit_total(P, K, T, S.w[j], old[j]);
-        const R total = s[0] + s[1] + s[2] + s[3];
-        R u_jump, u_sub;
-        draw2<PRNG>(S.q, u_jump, u_sub);
-        jump = ldiv(lneglog(u_jump), total);
-        last = !(S.t + jump < dt);
-        h = last ? dt - S.t : jump;
-        if (!last) {
-            // sample_weights over the subunits (common.hpp:49-59)
-            const R u = u_sub * total;
-            R cum = s[0];
-            if (cum < u) { js = 1; cum += s[1];
-                if (cum < u) { js = 2; cum += s[2];
-                    if (cum < u) { js = 3; } } }
-            // the class and transition of sample_new_state (SSA.tpp:262-283) on subunit js
-            const uint64_t wj = sel4(S.w, js);
-            const R oldj = sel4(old, js);
-            const R sj = sel4(s, js);
-            const int L = sub_lcc(wj);
-            const R sum_LCC = T.P[L] + T.Q[L] * oldj;
-            const R inact = sub_y(wj) ? K.inact1 : K.inact0;
-            const R clr = sub_cl(wj) ? P.kbClCh : P.kfClCh * oldj;
-            const R sum_RyR = sj - (sum_LCC + inact + clr);
-            R u_cls, u_tr;
-            draw2<PRNG>(S.q, u_cls, u_tr);
-            const R u3 = u_cls * sj;
-            cls = (u3 < sum_LCC) ? 0 : (u3 < (sum_LCC + inact)) ? 1 : (u3 < (sum_LCC + inact + sum_RyR)) ? 2 : 3;
-            if (cls == 0) {
-                // sample_LCC (SSA.tpp:103-197)
-                const R r0 = T.R0[L];
-                const R r1 = (L == 1) ? T.Q[L] * oldj : T.R1[L];
-                const R uu = u_tr * sum_LCC;
-                R c = r0;
-                if (c < uu) { tr = 1; c += r1;
-                    if (c < uu) { tr = 2; } }
-            } else if (cls == 2) {
-                tr = ryr_pick(P, wj, oldj, u_tr * sum_RyR);
-            }
-        }
-    }
-    // update_CaSS (SSA.tpp:87-99): subunits in order, re-splits drawn as they come
+    X.total = X.s[0] + X.s[1] + X.s[2] + X.s[3];
+    float u_jump;
+    split2(rng_output<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3), u_jump, X.u_sub);
+    X.jump = ldiv(lneglog(u_jump), X.total);
+    X.last = !(S.t + X.jump < dt);
+    const float h = X.last ? dt - S.t : X.jump;
+    // update_CaSS (SSA.tpp:87-99)
+    X.split = 0;
+    X.Jxfer = 0.0;
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        const R Jiss = P.riss * static_cast<R>(oldA[(j + 1) & 3] + oldA[(j + 3) & 3] - 2 * oldA[j]);
-        S.Jxfer[j] = P.rxfer * static_cast<R>(oldA[j] - Cai);
-        const R betaSS = beta_ss(P, old[j]);
-        const R dCaSS = h * (S.jl[j] + S.Jrel[j] - S.Jxfer[j] + Jiss) * betaSS;
-        const double tmp = oldA[j] + static_cast<double>(dCaSS);
-        int split = split_mask<R>(oldA[j], tmp);
-        while (split) {
-            // sample_RyR56 / sample_RyR34 (SSA.tpp:59-84), the (5,6) pair first
-            const int bit = split & -split;
-            split ^= bit;
-            const int a_ = (bit == 1) ? 4 : 2;
-            const R pr = (bit == 1) ? ldiv(P.k65, P.k65 + P.k56 * sq(old[j])) : ldiv(P.k43, P.k43 + P.k34 * sq(old[j]));
-            const int n = ryr_get(S.w[j], a_) + ryr_get(S.w[j], a_ + 1);
-            int X = 0;
-            for (int i = 0; i < n; i += 2) {   // two Bernoulli trials per engine draw
-                R b0, b1;
-                draw2<PRNG>(S.q, b0, b1);
-                X += (b0 < pr) ? 1 : 0;
-                X += (i + 1 < n && b1 < pr) ? 1 : 0;
-            }
-            S.w[j] = ryr_set(ryr_set(S.w[j], a_, (n > 0) ? X : 0), a_ + 1, (n > 0) ? n - X : 0);
-            S.changed = 1;
-        }
-        S.ca[j] = tmp;
+        const double oldA = S.ca[j];
+        const float Jiss = P.riss * static_cast<float>(S.ca[(j + 1) & 3] + S.ca[(j + 3) & 3] - 2 * oldA);
+        const float Jxfer = P.rxfer * static_cast<float>(oldA - K.Cai);
+        const float betaSS = beta_ss(P, static_cast<float>(oldA));
+        X.d[j] = h * (S.jl[j] + S.Jrel[j] - Jxfer + Jiss) * betaSS;
+        asm volatile("" : "+v"(X.d[j]));
+        X.split |= split_mask<float>(oldA, oldA + static_cast<double>(X.d[j])) << (2 * j);
+        X.Jxfer = j == 0 ? static_cast<double>(Jxfer) : X.Jxfer + Jxfer;
     }
     // update_CaJSR (SSA.hpp:67-71)
-    {
-        const R Jsum = S.Jrel[0] + S.Jrel[1] + S.Jrel[2] + S.Jrel[3];
-        const R betaJSR = beta_jsr(P, static_cast<R>(S.q.jsr));
-        S.q.jsr += static_cast<double>(h * betaJSR * (S.Jtr - P.VSS_VJSR * Jsum));
+    const float Jsum = S.Jrel[0] + S.Jrel[1] + S.Jrel[2] + S.Jrel[3];
+    const float betaJSR = beta_jsr(P, static_cast<float>(S.q.jsr));
+    X.dj = h * betaJSR * (X.Jtr - P.VSS_VJSR * Jsum);
+}
+
+// ev: the iteration ends in an event; false if the iteration cap was hit or a
+// count left the range its byte holds. K: the step's constants in LDS.
+template <int PRNG>
+__device__ __forceinline__ bool lane_commit(LaneState &S, const LaneTry &X, const SsaParamsF &P, const StepConstsF &K, bool ev)
+{
+#pragma clang fp contract(fast)   // FP32-local only: fused multiply-adds allowed
+    const LccTableF &T = K.lcc;
+    rng_advance<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3);   // past the waiting time's draw
+    int js = 0, cls = 0, tr = 0;
+    if (ev) {
+        // sample_weights over the subunits (common.hpp:49-59)
+        const float u = X.u_sub * X.total;
+        float cum = X.s[0];
+        if (cum < u) { js = 1; cum += X.s[1];
+            if (cum < u) { js = 2; cum += X.s[2];
+                if (cum < u) { js = 3; } } }
+        // the class and transition of sample_new_state (SSA.tpp:262-283) on subunit js
+        const uint64_t wj = sel4(S.w, js);
+        const float oldj = static_cast<float>(sel4(S.ca, js));
+        const float sj = sel4(X.s, js);
+        const int L = sub_lcc(wj);
+        const float Q = T.Q[L], r0 = T.R0[L], R1 = T.R1[L], i0 = K.inact0, i1 = K.inact1;
+        const float sum_LCC = T.P[L] + Q * oldj;
+        const float inact = sub_y(wj) ? i1 : i0;
+        const float clr = sub_cl(wj) ? P.kbClCh : P.kfClCh * oldj;
+        const float sum_RyR = sj - (sum_LCC + inact + clr);
+        float u_cls, u_tr;
+        draw2<PRNG>(S.q, u_cls, u_tr);
+        const float u3 = u_cls * sj;
+        cls = (u3 < sum_LCC) ? 0 : (u3 < (sum_LCC + inact)) ? 1 : (u3 < (sum_LCC + inact + sum_RyR)) ? 2 : 3;
+        if (cls == 0) {
+            // sample_LCC (SSA.tpp:103-197)
+            float r1 = Q * oldj;
+            asm volatile("" : "+v"(r1));   // rounded before it is added
+            const float uu = u_tr * sum_LCC;
+            const float r01 = r0 + ((L == 1) ? r1 : R1);
+            tr = r0 < uu ? (r01 < uu ? 2 : 1) : 0;
+        } else if (cls == 2) {
+            tr = ryr_pick(P, wj, oldj, u_tr * sum_RyR);
+        }
     }
-    if (last) return true;
-    if (S.iters >= kMaxItersPerStep) {   // no physical state gets here; stop instead of spinning
-        S.err = 1;
-        return true;
+    // sample_RyR56 / sample_RyR34 (SSA.tpp:59-84), in subunit order, a subunit's (5,6) pair first
+#pragma unroll 1
+    for (int m = X.split; m != 0; m &= m - 1) {
+        const int bit = __builtin_ctz(m), j = bit >> 1;
+        const int sh = (bit & 1) ? 16 : 32;   // the (3,4) or the (5,6) pair's bytes
+        uint64_t w = sel4(S.w, j);
+        const float C2 = sq(static_cast<float>(sel4(S.ca, j)));
+        const float kb = (bit & 1) ? P.k43 : P.k65, kf = (bit & 1) ? P.k34 : P.k56;
+        const float pr = ldiv(kb, kb + kf * C2);
+        const int n = static_cast<int8_t>(w >> sh) + static_cast<int8_t>(w >> (sh + 8));
+        int c = 0;
+        for (int i = 0; i < n; i += 2) {   // two Bernoulli trials per engine draw
+            float b0, b1;
+            draw2<PRNG>(S.q, b0, b1);
+            c += (b0 < pr) ? 1 : 0;
+            c += (i + 1 < n && b1 < pr) ? 1 : 0;
+        }
+        const uint64_t pair = n > 0 ? static_cast<uint64_t>(c & 0xff) | static_cast<uint64_t>((n - c) & 0xff) << 8 : 0;
+        w = (w & ~(0xffffULL << sh)) | pair << sh;
+        put4(S.w, j, w);
+        S.changed = 1;
     }
-    S.t += jump;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) S.ca[j] += static_cast<double>(X.d[j]);
+    S.q.jsr += static_cast<double>(X.dj);
+    S.iters++;
+    if (!ev) return true;
+    if (S.iters >= kMaxItersPerStep) return false;   // no physical state gets here; stop instead of spinning
+    S.t += X.jump;
     S.changed = 1;
+    bool ok = true;
     // apply the chosen event to subunit js after the update (SSA.tpp:262-283)
     uint64_t wj = sel4(S.w, js);
     const double caj_d = sel4(S.ca, js);
-    const R caj = static_cast<R>(caj_d);
-    R jlj = sel4(S.jl, js);
-    R Jrelj = sel4(S.Jrel, js);
-    int openj = sel4(S.open, js);
+    const float caj = static_cast<float>(caj_d);
+    float jlj = sel4(S.jl, js);
     const int L = sub_lcc(wj);
     const int y = sub_y(wj);
+    const float J = K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * caj);   // the flux of a channel that opens now
     if (cls == 0) {
         const int Ln = lcc_next(L, tr);
         if ((L == 5 && Ln == 6) || (L == 11 && Ln == 12))
-            jlj = (y == 1) ? K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * caj) : R(0);
+            jlj = (y == 1) ? J : 0.0f;
         else if (L == 6 || L == 12)
-            jlj = R(0);
+            jlj = 0.0f;
         wj = sub_set_lcc(wj, Ln);
     } else if (cls == 1) {
-        const int yn = 1 - y;
         wj = sub_flip_y(wj);
-        if (yn == 0) jlj = R(0);
-        else if (L == 6 || L == 12) jlj = K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * caj);
+        if (y == 1) jlj = 0.0f;
+        else if (L == 6 || L == 12) jlj = J;
     } else if (cls == 2) {
         // sample_RyR (SSA.tpp:200-259): the transition chosen above, unless it
         // would take a RyR out of an empty state (ryr_allowed)
+        int open = open_get(S.open, js);
         if (tr >= 0 && ryr_allowed(wj, tr, caj_d)) {
-            if (!ryr_in_range(wj, tr)) S.err = 1;
+            ok = ryr_in_range(wj, tr);
             wj = ryr_apply(wj, tr);
-            if (tr == 1 || tr == 10) openj += 1;
-            else if (tr == 4 || tr == 7) openj -= 1;
+            open += (tr == 1 || tr == 10) ? 1 : (tr == 4 || tr == 7) ? -1 : 0;
+            open_put(S.open, js, open);
         }
-        Jrelj = P.rRyR * static_cast<R>(openj) * static_cast<R>(S.q.jsr - caj_d);
+        put4(S.Jrel, js, P.rRyR * static_cast<float>(open) * static_cast<float>(S.q.jsr - caj_d));
     } else {
         wj = sub_flip_cl(wj);
     }
     put4(S.w, js, wj);
     put4(S.jl, js, jlj);
-    put4(S.Jrel, js, Jrelj);
-    put4(S.open, js, openj);
-    return false;
-}
-
-// outputs of update_CRUstate_from_temp (GW.tpp:47-62), summed in subunit order in FP64
-__device__ __forceinline__ LaneOut lane_outputs(const LaneState &S)
-{
-    LaneOut out;
-    out.Jxfer = ((static_cast<double>(S.Jxfer[0]) + S.Jxfer[1]) + S.Jxfer[2]) + S.Jxfer[3];
-    out.Jtr = static_cast<double>(S.Jtr);
-    out.JLCC = ((static_cast<double>(S.jl[0]) + S.jl[1]) + S.jl[2]) + S.jl[3];
-    out.Jrel = ((static_cast<double>(S.Jrel[0]) + S.Jrel[1]) + S.Jrel[2]) + S.Jrel[3];
-    out.open = 0;
-    out.clch = 0;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) {
-        out.open += ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
-        out.clch += sub_cl(S.w[j]);
-    }
-    out.iters = S.iters;
-    out.err = S.err;
-    return out;
+    return ok;
 }
 
 // ---------------------------------------------------------------------------
@@ -968,12 +966,9 @@ struct Lane64Try {
     double ca[4];     // CaSS after the update
     double s[4];      // subunit totals
     double total, h, jump, jsr, Jxfer, Jtr;
-    uint64_t r0, r1, r2, r3;   // the engine after the waiting time's draw
     int split;        // split_mask of subunit j at bits 2j, 2j + 1
     bool last;
 };
-
-__device__ __forceinline__ int open_get(uint32_t o, int j) { return static_cast<int8_t>(o >> (8 * j)); }
 
 __device__ __forceinline__ void lane64_begin(Lane64State &S, double rRyR)
 {
@@ -999,8 +994,7 @@ __device__ __forceinline__ void lane64_try(const Lane64State &S, Lane64Try &X, c
         asm volatile("" : "+v"(X.s[j]));   // one subunit after another: interleaved, they need twice the registers
     }
     X.total = X.s[0] + X.s[1] + X.s[2] + X.s[3];
-    X.r0 = S.q.r0; X.r1 = S.q.r1; X.r2 = S.q.r2; X.r3 = S.q.r3;
-    X.jump = lneglog(u01(rng_next<PRNG>(X.r0, X.r1, X.r2, X.r3))) / X.total;
+    X.jump = lneglog(u01(rng_output<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3))) / X.total;
     X.last = !(S.t + X.jump < dt);
     X.h = X.last ? dt - S.t : X.jump;
     X.split = 0;
@@ -1027,7 +1021,7 @@ template <int PRNG>
 __device__ __forceinline__ void lane64_commit(Lane64State &S, const Lane64Try &X, const SsaParams &P, double (&old)[4],
                                               uint64_t (&w_pre)[4])
 {
-    S.q.r0 = X.r0; S.q.r1 = X.r1; S.q.r2 = X.r2; S.q.r3 = X.r3;
+    rng_advance<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3);
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         old[j] = S.ca[j];
@@ -1111,7 +1105,7 @@ __device__ __forceinline__ bool lane64_event(Lane64State &S, const Lane64Try &X,
         w = ryr_apply(w, tr);
         int open = open_get(S.open, js);
         open += (tr == 1 || tr == 10) ? 1 : (tr == 4 || tr == 7) ? -1 : 0;
-        S.open = (S.open & ~(0xffu << (8 * js))) | (static_cast<uint32_t>(static_cast<uint8_t>(open)) << (8 * js));
+        open_put(S.open, js, open);
         put4(S.Jrel, js, P.rRyR * static_cast<double>(open) * (S.q.jsr - ca));
     } else {
         w = sub_flip_cl(w);

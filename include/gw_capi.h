@@ -380,8 +380,8 @@ int gw_batch_get_persistent(gw_batch *b, int32_t *active);
  * no digests) run two with a request of 0 or 2, whatever their shape. With one CRU per lane the results are bit-identical
  * to one step per launch; with refilled lanes they are deterministic, and the rounding
  * of the FP64 flux sums can differ (their order follows which CRUs each lane ran).
- * Automatic: two steps per launch when a launch's SSA blocks are more than the GPU
- * holds at once (the state's HBM traffic binds), one otherwise (latency binds, and the
+ * Automatic: two steps per launch for batches of 450,000 CRUs and more (the state's
+ * HBM traffic binds), one otherwise (latency binds, and the
  * separate close kernel would add to it). gw_batch_get_steps_per_launch reports what
  * the next plain steps use.
  */
