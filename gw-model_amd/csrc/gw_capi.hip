@@ -2294,11 +2294,9 @@ void launch_k_step(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent_t e0,
             }
             return;
         }
-        switch (B->shape) {
-        case 0: launch_k_step_shape<PRNG, 64>(B, ssa_step, nclose, e0, e1, base); return;
-        case 1: launch_k_step_shape<PRNG, 128>(B, ssa_step, nclose, e0, e1, base); return;
-        case 3: launch_k_step_shape<PRNG, 512>(B, ssa_step, nclose, e0, e1, base); return;
-        default: break;
+        if (B->shape == 0) {   // plain quads run with 64 threads or the default's 256 (run_config)
+            launch_k_step_shape<PRNG, 64>(B, ssa_step, nclose, e0, e1, base);
+            return;
         }
     }
     launch_k_step_shape<PRNG, kBlock>(B, ssa_step, nclose, e0, e1, base);
@@ -2400,22 +2398,37 @@ bool use_persist(gw_batch *B)
     return B->persist_mode != 0 && !B->frozen && B->cfg == kConfigDefault && persist_fits(B);
 }
 
-// The launch configuration the next steps run in: the one asked for, or for a
-// large FP64 batch a one-lane kernel, whose results are the same bits. Where
-// the lines lie, in us per step early in an action potential (4 x 64 quads;
-// one lane, 4 and 8 CRUs per lane): 300,000 CRUs 29.9, 38.7, 41.5; 600,000
-// 51.1, 50.0, 55.4; 800,000 65.3, 55.3, 57.6; 2.0 M 173, 97.9, 97.9; 5.0 M
-// 457, 218, 206; 12.8 M 1,182, 526, 479. Below, a batch is a few rounds of
-// quads and one round of lanes, whose trips are longer.
+// The launch configuration the next steps run in: the one asked for, except
+// where another gives the same bits faster.
+//
+// Plain quads (FP64 or FP32-local) run with 256 threads per block, whose close
+// has four waves, while the close is the longer half of a step, and with 64,
+// whose blocks wait on fewer waves, where the SSA is. In us per step with 256
+// and 64 threads: FP64, 12,500 CRUs 7.4 and 16.8; 150,000 18.5 and 19.1;
+// 200,000 22.2 and 21.6; 450,000 44 and 40; 300 cells of 200 CRUs 14.5 and
+// 13.6; FP32-local, 300,000 CRUs 19.9 and 20.7; 400,000 24.8 and 23.1; 300
+// cells of 200 CRUs 11.3 and 13.5. (128 and 512 lie between or behind.)
+//
+// Large FP64 batches run one lane per CRU. In us per step early in an action
+// potential (4 x 64 quads; one lane, 4 and 8 CRUs per lane): 300,000 CRUs
+// 29.9, 38.7, 41.5; 600,000 51.1, 50.0, 55.4; 800,000 65.3, 55.3, 57.6; 2.0 M
+// 173, 97.9, 97.9; 5.0 M 457, 218, 206; 12.8 M 1,182, 526, 479. Below, a batch
+// is a few rounds of quads and one round of lanes, whose trips are longer.
 constexpr int64_t kLane64Crus = 640000, kLane64Crus8 = 2500000;
+constexpr int64_t kQuad64Crus = 180000, kQuad64CrusF32 = 350000;
+constexpr int kQuad64Cells = 256;
 
 int run_config(gw_batch *B)
 {
-    if (B->precision != GW_PREC_FP64 || B->prng != GW_PRNG_XOSHIRO256SS || B->digest || B->frozen || use_persist(B) ||
-        B->ncrus < kLane64Crus)
-        return B->cfg;
-    return B->ncrus < kLane64Crus8 ? kLane64 : kLane64 + 1;
+    const bool f32 = B->precision == GW_PREC_FP32_LOCAL;
+    if (B->prng != GW_PRNG_XOSHIRO256SS || B->frozen || (!f32 && B->digest) || use_persist(B)) return B->cfg;
+    if (!f32 && B->ncrus >= kLane64Crus) return B->ncrus < kLane64Crus8 ? kLane64 : kLane64 + 1;
+    const LaunchCfg &L = kConfigs[B->cfg];
+    if (L.lanes != 4 || L.cpl != 1) return B->cfg;
+    const bool narrow = f32 ? B->ncrus >= kQuad64CrusF32 : B->ncrus >= kQuad64Crus || B->ncells >= kQuad64Cells;
+    return narrow ? 0 : kConfigDefault;
 }
+static_assert(kConfigs[0].lanes == 4 && kConfigs[0].threads == 64 && kConfigs[kConfigDefault].threads == kBlock, "the two quad shapes");
 
 // Steps step0 .. step0+n-1 in one cooperative launch of the persistent kernel
 // (which closes every step itself), after its counters are set for step0.
