@@ -233,14 +233,25 @@ __device__ void block_reduce(FluxTotals *red, FluxTotals mine)
 // ===========================================================================
 // Thread t of an SSA-shaped block handles subunit (t & 3) of CRU (t >> 2).
 
+// The blocks of every cell in every shape (grid: cells, shapes).
+__global__ void k_block_info(const DevCell *cells, BlockInfo *out)
+{
+    const DevCell &C = cells[blockIdx.x];
+    const int sh = blockIdx.y;
+    const int per = crus_per_block(sh);
+    for (int b = threadIdx.x; b < C.nblk[sh]; b += blockDim.x)
+        out[C.blk_all[sh] + b] = BlockInfo{static_cast<int32_t>(blockIdx.x), min(per, C.n_cru - b * per),
+                                           C.slot0 + static_cast<int64_t>(b) * per};
+}
+
 // Seed the per-CRU engines and replay digests; give padding slots an inert state.
 __global__ void k_seed(KArgs a)
 {
     const int b = blockIdx.x;
-    const int cell = a.block_cell[b];
-    const DevCell &C = a.cells[cell];
+    const BlockInfo bi = a.blocks[b];
+    const DevCell &C = a.cells[bi.cell];
     const int j = threadIdx.x & 3;
-    const int64_t i = (b - C.blk0[kShapeDefault]) * kCruPerBlock + (threadIdx.x >> 2);
+    const int64_t i = bi.slot - C.slot0 + (threadIdx.x >> 2);
     const int64_t slot = C.slot0 + i;
     if (j == 0) {
         uint64_t s[4];
@@ -264,10 +275,10 @@ template <int PRNG>
 __global__ void k_sample_rest(KArgs a)
 {
     const int b = blockIdx.x;
-    const int cell = a.block_cell[b];
-    const DevCell &C = a.cells[cell];
+    const BlockInfo bi = a.blocks[b];
+    const DevCell &C = a.cells[bi.cell];
     if ((threadIdx.x & 3) != 0) return;
-    const int64_t i = (b - C.blk0[kShapeDefault]) * kCruPerBlock + (threadIdx.x >> 2);
+    const int64_t i = bi.slot - C.slot0 + (threadIdx.x >> 2);
     if (i >= C.n_cru) return;
     const int64_t slot = C.slot0 + i;
     double ca[4], jsr;
@@ -361,33 +372,33 @@ template <> struct LocalState<float> {
 template <int PRNG, bool DIGEST, class R, int BLOCK>
 __device__ __forceinline__ void ssa_block(const KArgs &a, int b, int64_t step0, int64_t nsteps, LccTableT<R> &T, BlockAcc &acc)
 {
-    constexpr int kShape = shape_of_block(BLOCK);
     using LS = LocalState<R>;
     const int tid = threadIdx.x;
     const int j = tid & 3;
-    const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
+    const BlockInfo bi = load_scalar(&a.blocks[b]);
     const int ks = static_cast<int>(step0 & 1);
-    const DevCell &C = a.cells[cell];
-    const CellDyn &D = a.dyn[cell];
-    const auto &sp = LS::params(C);
-    const auto &kk = LS::consts(D, ks);
-    load_lcc_table(kk, T);
+    const DevCell &C = a.cells[bi.cell];
+    const CellDyn &D = a.dyn[bi.cell];
+    // the CRU's state, in flight with the cell's parameters and constants and with the LCC table on its way into LDS
+    const int i = tid >> 2;
+    R *const JLCC = LS::jlcc(a);
+    const int64_t slot = bi.slot + min(i, bi.n - 1);
+    double ca = a.CaSS[slot * 4 + j];
+    R jl = JLCC[slot * 4 + j];
+    uint64_t w = a.sub[slot * 4 + j];
+    CruQ q;
+    q.jsr = a.CaJSR[slot];
+    q.r0 = a.rng[slot * 4];
+    q.r1 = a.rng[slot * 4 + 1];
+    q.r2 = a.rng[slot * 4 + 2];
+    q.r3 = a.rng[slot * 4 + 3];
+    const auto sp = load_scalar(&LS::params(C));
+    const QuadConsts<R> kk = quad_consts_scalar(LS::consts(D, ks));
+    load_lcc_table(LS::consts(D, ks), T);
     acc_zero(acc);
     __syncthreads();
-    const int64_t i = (b - C.blk0[kShape]) * (BLOCK / 4) + (tid >> 2);
-    const bool active = (i < C.n_cru) && (step0 < D.stop_step);
+    const bool active = i < bi.n && step0 < D.stop_step;
     if (active) {
-        R *const JLCC = LS::jlcc(a);
-        const int64_t slot = C.slot0 + i;
-        double ca = a.CaSS[slot * 4 + j];
-        R jl = JLCC[slot * 4 + j];
-        uint64_t w = a.sub[slot * 4 + j];
-        CruQ q;
-        q.jsr = a.CaJSR[slot];
-        q.r0 = a.rng[slot * 4];
-        q.r1 = a.rng[slot * 4 + 1];
-        q.r2 = a.rng[slot * 4 + 2];
-        q.r3 = a.rng[slot * 4 + 3];
         Digest dg{0, 0};
         if (DIGEST) {
             dg.count = a.dig[slot * 2];
@@ -820,19 +831,20 @@ __device__ __forceinline__ void ssa_block_refill(const KArgs &a, int b, int64_t 
     const int wave = tid / kWave;
     const int j = tid & 3;
     const int qd = lane >> 2;
-    const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
+    const BlockInfo bi = load_scalar(&a.blocks[b]);
     const int ks = static_cast<int>(step0 & 1);
-    const DevCell &C = a.cells[cell];
-    const CellDyn &D = a.dyn[cell];
-    const auto &sp = LS::params(C);
-    const auto &kk = LS::consts(D, ks);
-    load_lcc_table(kk, T);
+    const DevCell &C = a.cells[bi.cell];
+    const CellDyn &D = a.dyn[bi.cell];
+    const auto sp = load_scalar(&LS::params(C));
+    const QuadConsts<R> kk = quad_consts_scalar(LS::consts(D, ks));
+    load_lcc_table(LS::consts(D, ks), T);
     acc_zero(acc);
     __syncthreads();
-    const int64_t w0 = static_cast<int64_t>(b - C.blk0[kMap]) * (BLOCK / 4 * CPT) + wave * (kQuads * CPT);
-    const int64_t w1 = min(w0 + kQuads * CPT, static_cast<int64_t>(C.n_cru));
-    int64_t i = w0 + qd;
-    int64_t next = w0 + kQuads;   // first CRU of the range not yet taken (wave-uniform)
+    const int start = wave * (kQuads * CPT);
+    const int64_t slot0 = bi.slot + start;
+    const int w1 = min(kQuads * CPT, bi.n - start);   // CRUs of the wave's range
+    int i = qd;
+    int next = kQuads;   // first CRU of the range not yet taken (wave-uniform)
     bool have = (i < w1) && (step0 < D.stop_step);
     R *const JLCC = LS::jlcc(a);
     const R dt = static_cast<R>(a.dt);
@@ -850,13 +862,13 @@ __device__ __forceinline__ void ssa_block_refill(const KArgs &a, int b, int64_t 
         S.dig = Digest{0, 0};
         quad_begin(S, sp);
     };
-    if (have) load(C.slot0 + i);
+    if (have) load(slot0 + i);
     while (__ballot(have)) {
         bool fin = false;
         if (have) {
             fin = quad_iterate<PRNG, false>(S, sp, kk, T, dt, step_lo, j);
             if (fin) {
-                const int64_t slot = C.slot0 + i;
+                const int64_t slot = slot0 + i;
                 a.CaSS[slot * 4 + j] = S.ca;
                 if (S.changed) {   // the channel word and JLCC change only at events and re-splits
                     JLCC[slot * 4 + j] = S.jl;
@@ -883,9 +895,9 @@ __device__ __forceinline__ void ssa_block_refill(const KArgs &a, int b, int64_t 
         }
         const uint64_t m = __ballot(fin && j == 0);
         if (fin) {
-            i = next + static_cast<int64_t>(__popcll(m & ((1ULL << (4 * qd)) - 1)));
+            i = next + static_cast<int>(__popcll(m & ((1ULL << (4 * qd)) - 1)));
             have = i < w1;
-            if (have) load(C.slot0 + i);
+            if (have) load(slot0 + i);
         }
         next += __popcll(m);
     }
@@ -1055,9 +1067,9 @@ __device__ __forceinline__ void ssa_block_lane(const KArgs &a, int b, int64_t m,
     const int tid = threadIdx.x;
     const int lane = tid & (kWave - 1);
     const int wave = tid / kWave;
-    const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
-    const DevCell &C = a.cells[cell];
-    const CellDyn &D = a.dyn[cell];
+    const BlockInfo bi = load_scalar(&a.blocks[b]);
+    const DevCell &C = a.cells[bi.cell];
+    const CellDyn &D = a.dyn[bi.cell];
     const float rRyR = C.spf.rRyR;
     const float dt = static_cast<float>(a.dt);
 #pragma unroll
@@ -1071,9 +1083,9 @@ __device__ __forceinline__ void ssa_block_lane(const KArgs &a, int b, int64_t m,
     __syncthreads();
     const int64_t stop = D.stop_step;
     const bool run1 = nss > 1 && m + 1 < stop;
-    const int64_t w0 = static_cast<int64_t>(b - C.blk0[kMap]) * (BLOCK * CPT) + wave * (kWave * CPT);
-    const int w1 = static_cast<int>(min(static_cast<int64_t>(kWave * CPT), C.n_cru - w0));   // CRUs of the wave's range
-    const int64_t slot0 = C.slot0 + w0;
+    const int start = wave * (kWave * CPT);
+    const int w1 = min(kWave * CPT, bi.n - start);   // CRUs of the wave's range
+    const int64_t slot0 = bi.slot + start;
     int i = lane;
     int next = kWave;   // first CRU of the range not yet taken (wave-uniform)
     bool have = i < w1 && m < stop;
@@ -1244,13 +1256,12 @@ __device__ __forceinline__ void ssa_block_persist(const KArgs &a, int b, int64_t
     static_assert(sizeof(KT) % 8 == 0 && kWords < kXchgWords, "step constants fit the exchange slot");
     const int tid = threadIdx.x;
     const int j = tid & 3;
-    const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
-    const DevCell &C = a.cells[cell];
-    CellSync &X = a.sync[cell];
-    const auto &sp = LS::params(C);
-    const int64_t i = (b - C.blk0[kShapeDefault]) * (kBlock / 4) + (tid >> 2);
-    const bool mine = i < C.n_cru;
-    const int64_t slot = C.slot0 + (mine ? i : 0);
+    const BlockInfo bi = load_scalar(&a.blocks[b]);
+    const DevCell &C = a.cells[bi.cell];
+    CellSync &X = a.sync[bi.cell];
+    const auto sp = load_scalar(&LS::params(C));
+    const bool mine = (tid >> 2) < bi.n;
+    const int64_t slot = bi.slot + (mine ? tid >> 2 : 0);
     R *const JLCC = LS::jlcc(a);
     double ca = 0.0;
     R jl = R(0);
@@ -1288,7 +1299,7 @@ __device__ __forceinline__ void ssa_block_persist(const KArgs &a, int b, int64_t
         load_lcc_table(K, T);
         __syncthreads();
         if (mine && n < stop) {
-            const QuadOut o = ssa_step_quad<PRNG, DIGEST>(ca, jl, w, q, sp, K, T, dt, dg, static_cast<uint32_t>(n & 0xffff), j);
+            const QuadOut o = ssa_step_quad<PRNG, DIGEST>(ca, jl, w, q, sp, quad_consts(K), T, dt, dg, static_cast<uint32_t>(n & 0xffff), j);
             changed |= o.changed;
             // lane j adds output j of its CRU (update_CRUstate_from_temp, GW.tpp:47-62)
             const double v = j == 0 ? o.Jxfer : j == 1 ? o.Jtr : j == 2 ? o.JLCC : o.Jrel;
@@ -1593,9 +1604,9 @@ __device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t 
     static_assert(crus_per_block(kMap) == kWave * CPT, "CRUs per block must be 16 << map");
     constexpr int kWords = sizeof(StepConsts) / 4;
     const int lane = threadIdx.x;
-    const int cell = __builtin_amdgcn_readfirstlane(a.block_cell[b]);
-    const DevCell &C = a.cells[cell];
-    const CellDyn &D = a.dyn[cell];
+    const BlockInfo bi = load_scalar(&a.blocks[b]);
+    const DevCell &C = a.cells[bi.cell];
+    const CellDyn &D = a.dyn[bi.cell];
 #pragma unroll
     for (int s = 0; s < NSS; ++s) {
         if (s < nss)
@@ -1608,9 +1619,8 @@ __device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t 
     const double rRyR = C.sp.rRyR;
     const int64_t stop = D.stop_step;
     const bool run1 = nss > 1 && m + 1 < stop;
-    const int64_t w0 = static_cast<int64_t>(b - C.blk0[kMap]) * (kWave * CPT);
-    const int w1 = static_cast<int>(min(static_cast<int64_t>(kWave * CPT), C.n_cru - w0));   // CRUs of the range
-    const int64_t slot0 = C.slot0 + w0;
+    const int w1 = bi.n;   // CRUs of the range
+    const int64_t slot0 = bi.slot;
     int i = lane;
     int next = kWave;   // first CRU of the range not yet taken (wave-uniform)
     bool have = i < w1 && m < stop;
@@ -2050,13 +2060,12 @@ struct gw_batch {
     int64_t bc_off[kNumShapes] = {};   // offset of each map's block -> cell table
     int64_t max_nblocks = 0;
     std::vector<DevCell> cells_h;
-    std::vector<int32_t> block_cell_h;
     std::vector<gw_globals_t> g0;
     std::vector<double *> istim_dev;
     KArgs a{};
     DevCell *d_cells = nullptr;
     CellDyn *d_dyn = nullptr;
-    int32_t *d_block_cell = nullptr;
+    BlockInfo *d_blocks = nullptr;
     void *d_staging = nullptr;
     size_t staging_bytes = 0;
     int64_t *d_gather = nullptr;   // [2][ncells]: status, trace rows (k_gather_dyn)
@@ -2166,7 +2175,7 @@ void apply_shape(gw_batch *B, int c)
     B->nblocks = B->nblocks_shape[B->shape];
     B->a.shape = B->shape;
     B->a.nblocks = B->nblocks;
-    B->a.block_cell = B->d_block_cell + B->bc_off[B->shape];
+    B->a.blocks = B->d_blocks + B->bc_off[B->shape];
 }
 
 // Configurations other than the default are built for the fast path only:
@@ -2874,7 +2883,7 @@ int gw_batch_destroy(gw_batch *B)
         return GW_OK;
     }
     void *ptrs[] = {B->a.CaSS, B->a.CaJSR, B->a.JLCC, B->a.JLCCf, B->a.sub, B->a.rng, B->a.dig, B->a.partials,
-                    B->a.trace, B->a.iters_total, B->d_step_base, B->d_cells, B->d_dyn, B->d_block_cell, B->d_staging,
+                    B->a.trace, B->a.iters_total, B->d_step_base, B->d_cells, B->d_dyn, B->d_blocks, B->d_staging,
                     B->d_gather, B->a.sync, B->a.timeout};
     for (void *p : ptrs)
         if (p) (void)hipFree(p);
@@ -2963,16 +2972,18 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
         }
         slot += static_cast<int64_t>((d.n_cru + kSlotAlign - 1) / kSlotAlign) * kSlotAlign;
     }
+    int64_t nblocks_all = 0;
     for (int sh = 0; sh < kNumShapes; ++sh) {
-        B->bc_off[sh] = static_cast<int64_t>(B->block_cell_h.size());
+        B->bc_off[sh] = nblocks_all;
         int64_t blk = 0;
         for (int c = 0; c < ncells; ++c) {
             DevCell &C = B->cells_h[c];
             C.blk0[sh] = blk;
+            C.blk_all[sh] = nblocks_all + blk;
             blk += C.nblk[sh];
-            for (int b = 0; b < C.nblk[sh]; ++b) B->block_cell_h.push_back(c);
         }
         B->nblocks_shape[sh] = blk;
+        nblocks_all += blk;
         B->max_nblocks = std::max(B->max_nblocks, blk);
     }
     B->ntot = slot;
@@ -2994,7 +3005,7 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
         (rc = dmalloc(B, &B->d_gather, 2 * static_cast<size_t>(ncells) + 1, err, errlen)) ||
         (rc = dmalloc(B, &a.sync, static_cast<size_t>(ncells), err, errlen)) ||
         (rc = dmalloc(B, &a.timeout, 1, err, errlen)) ||
-        (rc = dmalloc(B, &B->d_block_cell, B->block_cell_h.size(), err, errlen))) {
+        (rc = dmalloc(B, &B->d_blocks, static_cast<size_t>(nblocks_all), err, errlen))) {
         gw_batch_destroy(B);
         return rc;
     }
@@ -3013,7 +3024,7 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
     }
     a.cells = B->d_cells;
     a.dyn = B->d_dyn;
-    a.block_cell = B->d_block_cell + B->bc_off[kShapeDefault];
+    a.blocks = B->d_blocks + B->bc_off[kShapeDefault];
     a.shape = kShapeDefault;
     a.ntot = N;
     a.nblocks = B->nblocks;
@@ -3043,7 +3054,8 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
     hipError_t e;
     if ((e = hipMemcpyAsync(B->d_cells, B->cells_h.data(), ncells * sizeof(DevCell), hipMemcpyHostToDevice, ctx->stream)) != hipSuccess) return fail(e);
     if ((e = hipMemcpyAsync(B->d_dyn, dyn.data(), ncells * sizeof(CellDyn), hipMemcpyHostToDevice, ctx->stream)) != hipSuccess) return fail(e);
-    if ((e = hipMemcpyAsync(B->d_block_cell, B->block_cell_h.data(), B->block_cell_h.size() * sizeof(int32_t), hipMemcpyHostToDevice, ctx->stream)) != hipSuccess) return fail(e);
+    hipLaunchKernelGGL(k_block_info, dim3(ncells, kNumShapes), dim3(kBlock), 0, ctx->stream, B->d_cells, B->d_blocks);
+    if ((e = hipGetLastError()) != hipSuccess) return fail(e);
     hipLaunchKernelGGL(k_fill_u64, dim3(1), dim3(64), 0, ctx->stream, a.iters_total, int64_t(1), 0ull);
     if ((e = hipGetLastError()) != hipSuccess) return fail(e);
     hipLaunchKernelGGL(k_fill_u64, dim3((ncells * (sizeof(CellSync) / 8) + 255) / 256), dim3(256), 0, ctx->stream,

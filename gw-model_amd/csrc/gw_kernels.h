@@ -24,6 +24,13 @@ __host__ __device__ constexpr int shape_threads(int s) { return 64 << s; }   // 
 __host__ __device__ constexpr int shape_of_block(int threads) { return threads == 64 ? 0 : threads == 128 ? 1 : threads == 256 ? 2 : 3; }
 __host__ __device__ constexpr int shape_of_crus(int crus) { return crus <= 16 ? 0 : 1 + shape_of_crus(crus / 2); }
 
+// What an SSA block works on: one read, from which the addresses of its CRUs follow.
+struct alignas(16) BlockInfo {
+    int32_t cell;
+    int32_t n;       // CRUs of the block (fewer than its shape holds at the end of a cell)
+    int64_t slot;    // its first CRU's slot
+};
+
 // Static description of one cell on the device.
 struct DevCell {
     gw_params_t p;
@@ -35,6 +42,7 @@ struct DevCell {
     int64_t istim_len;
     int64_t slot0;         // first CRU slot of this cell in the state arrays
     int64_t blk0[kNumShapes];  // first SSA block of this cell, per launch shape
+    int64_t blk_all[kNumShapes];  // the same in the table of all shapes' blocks
     uint64_t seed;
     int32_t n_cru;
     int32_t nblk[kNumShapes];  // SSA blocks of this cell, per launch shape
@@ -82,7 +90,7 @@ struct CellSync {
 struct KArgs {
     const DevCell *cells;
     CellDyn *dyn;
-    const int32_t *block_cell;   // cell of each SSA block of the current shape
+    const BlockInfo *blocks;     // the SSA blocks of the current shape
     double *CaSS;      // [ntot][4]   (both forms: Ca accumulates in FP64)
     double *CaJSR;     // [ntot]
     double *JLCC;      // [ntot][4]   (FP64 batches)

@@ -453,11 +453,36 @@ struct CruQ {
     uint64_t r0, r1, r2, r3;
 };
 
-// Cai and CaNSR of a step at the accumulator precision.
-GW_HD double kcai(const StepConsts &k) { return k.Cai; }
-GW_HD double kcansr(const StepConsts &k) { return k.CaNSR; }
-GW_HD double kcai(const StepConstsF &k) { return k.Cai_d; }
-GW_HD double kcansr(const StepConstsF &k) { return k.CaNSR_d; }
+// The step's constants a quad reads beside the LCC table, in registers (in
+// scalar ones where they come through load_scalar): chosen where they lie in
+// memory, each choice is a load with the whole latency in every iteration.
+// Cai and CaNSR at the accumulator precision.
+template <class R>
+struct QuadConsts {
+    double Cai, CaNSR;
+    R inact0, inact1, JLCC_mult, JLCC_exp;
+};
+GW_HD QuadConsts<double> quad_consts(const StepConsts &k)
+{
+    return {k.Cai, k.CaNSR, k.inact0, k.inact1, k.JLCC_mult, k.JLCC_exp};
+}
+GW_HD QuadConsts<float> quad_consts(const StepConstsF &k)
+{
+    return {k.Cai_d, k.CaNSR_d, k.inact0, k.inact1, k.JLCC_mult, k.JLCC_exp};
+}
+// The same from memory that no block of the launch writes.
+__device__ __forceinline__ QuadConsts<double> quad_consts_scalar(const StepConsts &k)
+{
+    struct Head { double v[6]; };
+    const Head h = load_scalar(reinterpret_cast<const Head *>(&k));
+    return {h.v[0], h.v[1], h.v[2], h.v[3], h.v[4], h.v[5]};
+}
+__device__ __forceinline__ QuadConsts<float> quad_consts_scalar(const StepConstsF &k)
+{
+    struct Head { double Cai_d, CaNSR_d; float Cai, CaNSR, inact0, inact1, JLCC_mult, JLCC_exp; };
+    const Head h = load_scalar(reinterpret_cast<const Head *>(&k));
+    return {h.Cai_d, h.CaNSR_d, h.inact0, h.inact1, h.JLCC_mult, h.JLCC_exp};
+}
 
 // Per-CRU outputs of one step for the reductions (identical in the 4 lanes).
 struct QuadOut {
@@ -532,11 +557,11 @@ __device__ __forceinline__ void quad_begin(QuadState<R> &S, const SsaParamsT<R> 
 
 // One iteration of SSA_single_CRU's loop (SSA.tpp:290-309) for a quad; true
 // when the step is finished (the same in the four lanes).
-template <int PRNG, bool DIGEST, class R, class KT>
-__device__ __forceinline__ bool quad_iterate(QuadState<R> &S, const SsaParamsT<R> &P, const KT &K,
+template <int PRNG, bool DIGEST, class R>
+__device__ __forceinline__ bool quad_iterate(QuadState<R> &S, const SsaParamsT<R> &P, const QuadConsts<R> &K,
                                              const LccTableT<R> &T, R dt, uint32_t step_lo, int j)
 {
-    const double Cai = kcai(K), CaNSR = kcansr(K);
+    const double Cai = K.Cai, CaNSR = K.CaNSR;
     S.iters++;
     // update_fluxes + update_rates (SSA.tpp:37-56)
     const double oldA = S.ca;
@@ -613,7 +638,8 @@ __device__ __forceinline__ bool quad_iterate(QuadState<R> &S, const SsaParamsT<R
     const int L = sub_lcc(S.w);
     const int y = sub_y(S.w);
     const int cl = sub_cl(S.w);
-    const R sum_LCC = T.P[L] + T.Q[L] * old;
+    const R Q = T.Q[L], r0 = T.R0[L], R1 = T.R1[L];
+    const R sum_LCC = T.P[L] + Q * old;
     const R inact = y ? K.inact1 : K.inact0;
     const R clr = cl ? P.kbClCh : P.kfClCh * old;
     const R sum_RyR = s_me - (sum_LCC + inact + clr);
@@ -624,19 +650,15 @@ __device__ __forceinline__ bool quad_iterate(QuadState<R> &S, const SsaParamsT<R
     int detail = 0;
     if (j == js) {
         S.changed = 1;
-        const R caR = static_cast<R>(S.ca);
+        const R J = K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * static_cast<R>(S.ca));   // the flux of a channel that opens now
         if (cls == 0) {
             // sample_LCC (SSA.tpp:103-197); the scan never compares after adding r2
-            const R r0 = T.R0[L];
-            const R r1 = (L == 1) ? T.Q[L] * old : T.R1[L];
             const R uu = u4 * sum_LCC;
-            R cum = r0;
-            int tr = 0;
-            if (cum < uu) { tr = 1; cum += r1;
-                if (cum < uu) { tr = 2; } }
+            const R r01 = r0 + ((L == 1) ? Q * old : R1);
+            const int tr = r0 < uu ? (r01 < uu ? 2 : 1) : 0;
             const int Ln = lcc_next(L, tr);
             if ((L == 5 && Ln == 6) || (L == 11 && Ln == 12))
-                S.jl = (y == 1) ? K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * caR) : R(0);
+                S.jl = (y == 1) ? J : R(0);
             else if (L == 6 || L == 12)
                 S.jl = R(0);
             S.w = sub_set_lcc(S.w, Ln);
@@ -645,7 +667,7 @@ __device__ __forceinline__ bool quad_iterate(QuadState<R> &S, const SsaParamsT<R
             const int yn = 1 - y;
             S.w = sub_flip_y(S.w);
             if (yn == 0) S.jl = R(0);
-            else if (L == 6 || L == 12) S.jl = K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * caR);
+            else if (L == 6 || L == 12) S.jl = J;
             detail = yn;
         } else if (cls == 2) {
             // sample_RyR (SSA.tpp:200-259) over the propensities before this iteration's update
@@ -686,9 +708,9 @@ __device__ __forceinline__ QuadOut quad_outputs(const QuadState<R> &S)
     return out;
 }
 
-template <int PRNG, bool DIGEST, class R, class KT>
+template <int PRNG, bool DIGEST, class R>
 __device__ QuadOut ssa_step_quad(double &ca, R &jl, uint64_t &w, CruQ &q, const SsaParamsT<R> &P,
-                                 const KT &K, const LccTableT<R> &T, R dt, Digest &dig, uint32_t step_lo, int j)
+                                 const QuadConsts<R> &K, const LccTableT<R> &T, R dt, Digest &dig, uint32_t step_lo, int j)
 {
     QuadState<R> S;
     S.ca = ca;
