@@ -178,42 +178,81 @@ __device__ __forceinline__ Fx limbs_fx(uint64_t S0, uint64_t S1, uint64_t S2)
     return f;
 }
 
-// Exact per-block sums of the SSA outputs. Each output's 128-bit fixed-point
-// value is split into three 43-bit limbs (the top one signed) that are added
-// into LDS with 64-bit atomics; 64 CRUs per block cannot overflow a limb sum,
-// and the limbs are recombined with carries into the same 128-bit total.
-// The integer outputs (iterations, open RyRs, open ClCh, error flags) are
-// added the same way, lane j of each quad adding output j, so that no atomic
-// address is shared by the whole wave (which would make the compiler scan
-// the active lanes one by one).
+// The three 43-bit limbs of v, whole numbers in FP64 (all of v's sign): the
+// 128-bit value fx_add forms, truncated at 2^-80, without its shifts. Where v
+// is not below 2^24 in magnitude they are zero and the answer is false.
+__device__ __forceinline__ bool limb_split(double v, double &lo, double &mid, double &hi)
+{
+    const bool ok = __builtin_fabs(v) < 0x1p24;
+    v = ok ? v : 0.0;
+    hi = __builtin_trunc(v * 0x1p-6);
+    const double r = __builtin_fma(hi, -0x1p6, v);
+    mid = __builtin_trunc(r * 0x1p37);
+    const double r2 = __builtin_fma(mid, -0x1p-37, r);
+    lo = __builtin_trunc(r2 * 0x1p80);
+    return ok;
+}
+
+// Exact per-block sums of the SSA outputs. Each flux is added in its three
+// limbs, whole numbers in FP64, into LDS; no block's CRUs reach 2^53 in a limb
+// sum, so the order does not matter. The integer outputs (iterations, open
+// RyRs, open ClCh, error flags) are added the same way, lane j of each quad
+// adding output j, so that no atomic address is shared by the whole wave
+// (which would make the compiler scan the active lanes one by one); four copies,
+// by quad, leave four lanes of a wave to an address.
+constexpr int kCopies = 4;
 struct BlockAcc {
-    unsigned long long limb[4][3];   // Jxfer, Jtr, JLCC, Jrel
-    unsigned long long ints[4];      // iterations, open RyRs, open ClCh, error flags
+    double limb[PW_ITERS][kCopies];   // Jxfer, Jtr, JLCC, Jrel, three limbs each
+    unsigned long long ints[PW_N - PW_ITERS][kCopies];   // iterations, open RyRs, open ClCh, error flags
 };
 
 __device__ __forceinline__ void acc_zero(BlockAcc &A)
 {
     const int t = threadIdx.x;
-    if (t < 16) (&A.limb[0][0])[t] = 0;
+    static_assert(sizeof(BlockAcc) == 64 * 8, "one word per thread of the smallest block");
+    if (t < 64) reinterpret_cast<unsigned long long *>(&A)[t] = 0;
 }
 
-__device__ __forceinline__ void acc_add_fx(BlockAcc &A, int q, const Fx &f)
+// Adds v to flux q's sum; false if it left the range (limb_split).
+__device__ __forceinline__ bool acc_add(BlockAcc &A, int q, int copy, double v)
 {
-    const uint64_t m43 = (1ULL << 43) - 1;
-    atomicAdd(&A.limb[q][0], static_cast<unsigned long long>(f.lo & m43));
-    atomicAdd(&A.limb[q][1], static_cast<unsigned long long>((f.lo >> 43) | ((f.hi & ((1ULL << 22) - 1)) << 21)));
-    atomicAdd(&A.limb[q][2], static_cast<unsigned long long>(static_cast<int64_t>(f.hi) >> 22));
+    double lo, mid, hi;
+    const bool ok = limb_split(v, lo, mid, hi);
+    unsafeAtomicAdd(&A.limb[3 * q][copy], lo);
+    unsafeAtomicAdd(&A.limb[3 * q + 1][copy], mid);
+    unsafeAtomicAdd(&A.limb[3 * q + 2][copy], hi);
+    return ok;
 }
 
-// The block's partial of one step: its accumulators, one word per thread.
+// The outputs of a quad's CRU: lane j adds output j (update_CRUstate_from_temp, GW.tpp:47-62).
+__device__ __forceinline__ void quad_add(BlockAcc &A, int j, const QuadOut &o, uint64_t iters)
+{
+    const int copy = (threadIdx.x >> 2) & (kCopies - 1);
+    const int fl = acc_add(A, j, copy, j == 0 ? o.Jxfer : j == 1 ? o.Jtr : j == 2 ? o.JLCC : o.Jrel) ? 0 : 1;
+    // error flags of the three summed fluxes (the range of Jrel is not checked)
+    const int e = (qgeti<0>(fl) | qgeti<1>(fl) | qgeti<2>(fl)) | (o.err ? 4 : 0);
+    const int64_t iv = j == 0 ? static_cast<int64_t>(iters) : j == 1 ? o.open : j == 2 ? o.clch : e;
+    atomicAdd(&A.ints[j][copy], static_cast<unsigned long long>(iv));
+}
+
+// Word t of the block's partial.
+__device__ __forceinline__ uint64_t acc_word(const BlockAcc &A, int t)
+{
+    if (t < PW_ITERS) {
+        double d = A.limb[t][0];
+        for (int k = 1; k < kCopies; ++k) d += A.limb[t][k];
+        return static_cast<uint64_t>(static_cast<int64_t>(d));
+    }
+    uint64_t v = A.ints[t - PW_ITERS][0];
+    for (int k = 1; k < kCopies; ++k) v += A.ints[t - PW_ITERS][k];
+    return t == PW_ERR ? (v != 0) : v;
+}
+
+// The block's partial of one step, one word per thread.
 __device__ __forceinline__ void write_partial(const KArgs &a, const BlockAcc &A, int64_t index)
 {
-    static_assert(sizeof(BlockAcc) == sizeof(Partial), "a partial is the block's accumulators");
     const int t = threadIdx.x;
-    if (t < PW_N) {
-        const uint64_t v = (&A.limb[0][0])[t];
-        a.partials[index].w[t] = t == PW_ERR ? (v != 0) : v;
-    }
+    if (t < PW_N) a.partials[index].w[t] = acc_word(A, t);
 }
 
 template <int NT>
@@ -430,16 +469,7 @@ __device__ __forceinline__ void ssa_block(const KArgs &a, int b, int64_t step0, 
                 a.dig[slot * 2 + 1] = dg.hash;
             }
         }
-        // lane j adds output j of its CRU (update_CRUstate_from_temp, GW.tpp:47-62)
-        const double v = j == 0 ? o.Jxfer : j == 1 ? o.Jtr : j == 2 ? o.JLCC : o.Jrel;
-        Fx f;
-        fx_zero(f);
-        const int fl = fx_add(f, v);
-        acc_add_fx(acc, j, f);
-        // error flags of the three summed fluxes (the range of Jrel is not checked)
-        const int e = (qgeti<0>(fl) | qgeti<1>(fl) | qgeti<2>(fl)) | (o.err ? 4 : 0);
-        const int64_t iv = j == 0 ? static_cast<int64_t>(iters) : j == 1 ? o.open : j == 2 ? o.clch : e;
-        atomicAdd(&acc.ints[j], static_cast<unsigned long long>(iv));
+        quad_add(acc, j, o, iters);
     }
     __syncthreads();
     write_partial(a, acc, ks * a.nblocks + b);
@@ -527,6 +557,33 @@ __device__ __forceinline__ uint64_t shfl_xor_u64(uint64_t v, int m)
     return static_cast<uint64_t>(__shfl_xor(static_cast<unsigned long long>(v), m));
 }
 
+__device__ __forceinline__ double read_lane(double v, int lane)
+{
+    const uint64_t u = bits_of(v);
+    const uint32_t lo = __builtin_amdgcn_readlane(static_cast<uint32_t>(u), lane);
+    const uint32_t hi = __builtin_amdgcn_readlane(static_cast<uint32_t>(u >> 32), lane);
+    return double_of(static_cast<uint64_t>(hi) << 32 | lo);
+}
+
+// The quotients of a wave-uniform part, one per lane: a correctly rounded FP64
+// division is eleven instructions, spent once for all of them.
+struct LaneQuot {
+    int lane;
+    template <int N>
+    __device__ __forceinline__ void operator()(const double (&num)[N], const double (&den)[N], double (&q)[N]) const
+    {
+        double n = num[0], d = den[0];
+#pragma unroll
+        for (int i = 1; i < N; ++i) {
+            n = lane == i ? num[i] : n;
+            d = lane == i ? den[i] : d;
+        }
+        const double r = n / d;
+#pragma unroll
+        for (int i = 0; i < N; ++i) q[i] = read_lane(r, i);
+    }
+};
+
 // Close step n = D.step of one cell: the exact sum of the cell's block
 // partials of step n, globals += dGlobals (GW.tpp:252-271), t += dt, the
 // derivatives of step n+1, observables and trace, and the SSA constants of
@@ -576,23 +633,17 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
         constexpr int kG = CloseLds<NT>::kGroups;
         const int w2 = 2 * (tid & (kSumLanes - 1)), grp = tid / kSumLanes;
         uint64_t s0 = 0, s1 = 0;
-        constexpr int kAhead = COH ? 1 : 4;   // reads in flight per lane
-        int q = grp;
-        for (; q + (kAhead - 1) * kG < nb; q += kAhead * kG) {
+        constexpr int kAhead = COH ? 1 : 8;   // reads in flight per lane
+        for (int q = grp; q < nb; q += kAhead * kG) {
             uint64_t x[kAhead], y[kAhead];
 #pragma unroll
-            for (int u = 0; u < kAhead; ++u) partial_pair<COH>(src[q + u * kG].w + w2, x[u], y[u]);
+            for (int u = 0; u < kAhead; ++u) partial_pair<COH>(src[min(q + u * kG, nb - 1)].w + w2, x[u], y[u]);
 #pragma unroll
             for (int u = 0; u < kAhead; ++u) {
-                s0 += x[u];
-                s1 += y[u];
+                const bool in = q + u * kG < nb;
+                s0 += in ? x[u] : 0;
+                s1 += in ? y[u] : 0;
             }
-        }
-        for (; q < nb; q += kG) {
-            uint64_t x, y;
-            partial_pair<COH>(src[q].w + w2, x, y);
-            s0 += x;
-            s1 += y;
         }
         L.red[grp][w2] = s0;
         L.red[grp][w2 + 1] = s1;
@@ -658,7 +709,7 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
     const FluxSums S{L.S[0], L.S[1], L.S[2], L.S[3]};
     if (role(0)) {
         Currents k;
-        gd_k_currents(p, c, g, VF_RT, L.x, k);
+        gd_k_currents(p, c, g, VF_RT, L.x, k, LaneQuot{lane});
         if (lane == 0) {
             L.cur.IKr = k.IKr; L.cur.IKs = k.IKs; L.cur.Ito1 = k.Ito1; L.cur.IK1 = k.IK1; L.cur.IKp = k.IKp;
         }
@@ -666,8 +717,7 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
     if (role(1)) {
         Currents k;
         double beta_cyto, dLTRPN, dHTRPN;
-        gd_na_ca_currents(p, c, g, L.x, k);
-        gd_uptake(p, c, g, L.x, k, beta_cyto, dLTRPN, dHTRPN);
+        gd_na_ca_currents(p, c, g, L.x, k, beta_cyto, dLTRPN, dHTRPN, LaneQuot{lane});
         if (lane == 0) {
             L.cur.INa = k.INa; L.cur.INab = k.INab; L.cur.INaCa = k.INaCa; L.cur.INaK = k.INaK;
             L.cur.ICab = k.ICab; L.cur.IpCa = k.IpCa; L.cur.Jup = k.Jup;
@@ -690,15 +740,11 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
     }
     if (role(3)) {
         Currents k;
-        double gates[4], dKr[5];
-        gd_gates(L.x, g, a.dt, gates);
-        gd_chain_kr(p, L.x, g, a.dt, dKr);
-        gd_cru_currents(p, c, VF_RT, L.x, S, k);
+        double d[9];
+        gd_gates_kr_cru(p, c, g, VF_RT, L.x, S, a.dt, d, k, LaneQuot{lane});
         if (lane == 0) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i) L.ch[i] = gates[i];
-#pragma unroll
-            for (int i = 0; i < 5; ++i) L.ch[4 + i] = dKr[i];
+            for (int i = 0; i < 9; ++i) L.ch[i] = d[i];
             L.cur.Ito2 = k.Ito2; L.cur.ICaL = k.ICaL; L.cur.Jtr_tot = k.Jtr_tot; L.cur.Jxfer_tot = k.Jxfer_tot;
         }
     }
@@ -719,7 +765,7 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
         const double e = gw::exp(sc_arg(lane < SC_N ? lane : 0, V, c.F_RT));
         double X[SC_N];
 #pragma unroll
-        for (int i = 0; i < SC_N; ++i) X[i] = double_of(shfl_u64(bits_of(e), i));
+        for (int i = 0; i < SC_N; ++i) X[i] = read_lane(e, i);
         if (role(0)) {
             if (lane < kGd0) {
                 double v = d[0];
@@ -729,7 +775,7 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
                 reinterpret_cast<double *>(&D.dg)[lane] = v;
             }
             StepConsts k;
-            step_consts_scalars(k, c, V, X, Cai, CaNSR, static_cast<uint32_t>((step_new + 1) & 0xffff));
+            step_consts_scalars(k, c, V, X, Cai, CaNSR, static_cast<uint32_t>((step_new + 1) & 0xffff), LaneQuot{lane});
             if (lane == 0) {
                 StepConsts &K = D.k[slot];
                 K.Cai = k.Cai;
@@ -882,15 +928,7 @@ __device__ __forceinline__ void ssa_block_refill(const KArgs &a, int b, int64_t 
                     a.rng[slot * 4 + 3] = S.q.r3;
                 }
                 const QuadOut o = quad_outputs(S);
-                // lane j adds output j of its CRU (update_CRUstate_from_temp, GW.tpp:47-62)
-                const double v = j == 0 ? o.Jxfer : j == 1 ? o.Jtr : j == 2 ? o.JLCC : o.Jrel;
-                Fx f;
-                fx_zero(f);
-                const int fl = fx_add(f, v);
-                acc_add_fx(acc, j, f);
-                const int e = (qgeti<0>(fl) | qgeti<1>(fl) | qgeti<2>(fl)) | (o.err ? 4 : 0);
-                const int64_t iv = j == 0 ? static_cast<int64_t>(o.iters) : j == 1 ? o.open : j == 2 ? o.clch : e;
-                atomicAdd(&acc.ints[j], static_cast<unsigned long long>(iv));
+                quad_add(acc, j, o, o.iters);
             }
         }
         const uint64_t m = __ballot(fin && j == 0);
@@ -1018,14 +1056,11 @@ __device__ __forceinline__ void lane_accumulate(BlockAcc &acc, const LaneSums<BL
     const int n_it = wave_sum(iters), n_open = wave_sum(open), n_cl = wave_sum(clch);
     const int k = lane & 3;
     const double v = k == 0 ? sx : k == 1 ? st : k == 2 ? sl : sr;
-    Fx f;
-    fx_zero(f);
-    const int fl = fx_add(f, v);
-    const bool bad = __ballot(lane < 3 && fl != 0) != 0 || Ls.err != 0;
+    const bool bad = __ballot(lane < 3 && !(__builtin_fabs(v) < 0x1p24)) != 0 || Ls.err != 0;
     if (lane < 4) {
-        acc_add_fx(acc, lane, f);
+        acc_add(acc, lane, 0, v);
         const int64_t iv = lane == 0 ? n_it : lane == 1 ? n_open : lane == 2 ? n_cl : (bad ? 1 : 0);
-        atomicAdd(&acc.ints[lane], static_cast<unsigned long long>(iv));
+        atomicAdd(&acc.ints[lane][0], static_cast<unsigned long long>(iv));
     }
 }
 
@@ -1301,19 +1336,11 @@ __device__ __forceinline__ void ssa_block_persist(const KArgs &a, int b, int64_t
         if (mine && n < stop) {
             const QuadOut o = ssa_step_quad<PRNG, DIGEST>(ca, jl, w, q, sp, quad_consts(K), T, dt, dg, static_cast<uint32_t>(n & 0xffff), j);
             changed |= o.changed;
-            // lane j adds output j of its CRU (update_CRUstate_from_temp, GW.tpp:47-62)
-            const double v = j == 0 ? o.Jxfer : j == 1 ? o.Jtr : j == 2 ? o.JLCC : o.Jrel;
-            Fx f;
-            fx_zero(f);
-            const int fl = fx_add(f, v);
-            acc_add_fx(acc, j, f);
-            const int e = (qgeti<0>(fl) | qgeti<1>(fl) | qgeti<2>(fl)) | (o.err ? 4 : 0);
-            const int64_t iv = j == 0 ? static_cast<int64_t>(o.iters) : j == 1 ? o.open : j == 2 ? o.clch : e;
-            atomicAdd(&acc.ints[j], static_cast<unsigned long long>(iv));
+            quad_add(acc, j, o, o.iters);
         }
         __syncthreads();
         if (tid < PW_N) {   // the words of the partial, then the one that holds the tag
-            uint64_t v = (&acc.limb[0][0])[tid];
+            const uint64_t v = acc_word(acc, tid);
             unsigned long long *dst = reinterpret_cast<unsigned long long *>(a.partials[ks * a.nblocks + b].w) + tid;
             if (tid != PW_ERR) st_coh(dst, v);
             stores_done();
@@ -1528,13 +1555,8 @@ struct Lane64Lds {
 // Adds v in limbs; false if it is not below 2^24 in magnitude (then it adds nothing).
 __device__ __forceinline__ bool lane64_add(Lane64Acc &A, int q, int copy, double v)
 {
-    const bool ok = __builtin_fabs(v) < 0x1p24;
-    v = ok ? v : 0.0;
-    const double hi = __builtin_trunc(v * 0x1p-6);
-    const double r = __builtin_fma(hi, -0x1p6, v);
-    const double mid = __builtin_trunc(r * 0x1p37);
-    const double r2 = __builtin_fma(mid, -0x1p-37, r);
-    const double lo = __builtin_trunc(r2 * 0x1p80);
+    double lo, mid, hi;
+    const bool ok = limb_split(v, lo, mid, hi);
     unsafeAtomicAdd(&A.limb[3 * q][copy], lo);
     unsafeAtomicAdd(&A.limb[3 * q + 1][copy], mid);
     unsafeAtomicAdd(&A.limb[3 * q + 2][copy], hi);

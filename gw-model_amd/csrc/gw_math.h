@@ -26,9 +26,6 @@ GW_HD double pow2i(int k) { return double_of(static_cast<uint64_t>(k + 1023) << 
 
 GW_HD double exp(double x)
 {
-    if (x != x) return x;
-    if (x > 709.79) return __builtin_inf();
-    if (x < -745.2) return 0.0;
     const double kd = __builtin_rint(x * 0x1.71547652b82fep+0);
     double r = __builtin_fma(-kd, 0x1.62e42fefa39efp-1, x);
     r = __builtin_fma(-kd, 0x1.abc9e3b39803fp-56, r);
@@ -46,10 +43,15 @@ GW_HD double exp(double x)
     p = __builtin_fma(p, r, 0.5);
     p = __builtin_fma(p, r, 1.0);
     p = __builtin_fma(p, r, 1.0);
-    const int k = static_cast<int>(kd);
-    if (k > 1023) return (p * pow2i(1023)) * pow2i(k - 1023);
-    if (k < -1021) return (p * pow2i(k + 1000)) * pow2i(-1000);
-    return p * pow2i(k);
+    // scaled in two factors at the ends of the range (in one elsewhere: the
+    // second is 1), the special cases chosen last: without branches, which the
+    // lanes of a wave would take in turn
+    const bool big = x > 709.79, tiny = x < -745.2, nan = x != x;
+    const int k = (big || tiny || nan) ? 0 : static_cast<int>(kd);
+    const int k1 = k > 1023 ? 1023 : k < -1021 ? k + 1000 : k;
+    const int k2 = k > 1023 ? k - 1023 : k < -1021 ? -1000 : 0;
+    const double e = (p * pow2i(k1)) * pow2i(k2);
+    return nan ? x : big ? __builtin_inf() : tiny ? 0.0 : e;
 }
 
 // ---------------------------------------------------------------------------

@@ -59,6 +59,16 @@ GW_HD void cell_consts_init(CellConsts &c, const gw_params_t &p, int nCRU)
     c.CMDN_const = p.KCMDN * p.CMDNT;
 }
 
+// Independent quotients, one after another. The close forms them one per lane
+// of a wave instead.
+struct Serial {
+    template <int N>
+    GW_HD void operator()(const double (&num)[N], const double (&den)[N], double (&q)[N]) const
+    {
+        for (int i = 0; i < N; ++i) q[i] = num[i] / den[i];
+    }
+};
+
 // Constants the SSA reads during one step (frozen inside GW_model::SSA,
 // src/includes/GW.tpp:214-233). The LCC propensities of a subunit in state s
 // are tabulated so that (r0 + r1) + r2 = lccP[s] + lccQ[s] * CaSS bit for bit;
@@ -96,18 +106,23 @@ GW_HD double sc_arg(int slot, double V, double F_RT)
 // Per-step constants of GW_model::SSA (GW.tpp:216-221) from the exponentials
 // X[SC_*] of sc_arg's arguments, without the LCC rate table. At V == 0 the multiplier
 // takes its analytic limit JLCC_const / 2 instead of 0/0.
+template <class Quot>
 GW_HD void step_consts_scalars(StepConsts &k, const CellConsts &c, double V, const double *X, double Cai, double CaNSR,
-                               uint32_t step_lo)
+                               uint32_t step_lo, Quot &&quot)
 {
-    const double expmVF_RT = X[SC_EXPM];
-    const double yinf = 0.4 / (1.0 + X[SC_YINF]) + 0.6;
-    const double tau = 340.0 / (1.0 + X[SC_TAU]) + 60.0;
+    const double num[3] = {0.4, 340.0, 1.0}, den[3] = {1.0 + X[SC_YINF], 1.0 + X[SC_TAU], X[SC_EXPM]};
+    double q[3], q2[3];
+    quot(num, den, q);
+    const double yinf = q[0] + 0.6;
+    const double tau = q[1] + 60.0;
     k.Cai = Cai;
     k.CaNSR = CaNSR;
-    k.inact0 = yinf / tau;
-    k.inact1 = (1.0 - yinf) / tau;
-    k.JLCC_exp = sq(1.0 / expmVF_RT);
-    k.JLCC_mult = (V == 0.0) ? c.JLCC_const / 2.0 : c.JLCC_const * V * c.F_RT / (k.JLCC_exp - 1);
+    k.JLCC_exp = sq(q[2]);
+    const double num2[3] = {yinf, 1.0 - yinf, c.JLCC_const * V * c.F_RT}, den2[3] = {tau, tau, k.JLCC_exp - 1};
+    quot(num2, den2, q2);
+    k.inact0 = q2[0];
+    k.inact1 = q2[1];
+    k.JLCC_mult = (V == 0.0) ? c.JLCC_const / 2.0 : q2[2];
     k.step_lo = step_lo;
     k._pad = 0;
 }
@@ -163,7 +178,7 @@ GW_HD void lcc_row_store(LccTableT<R> &t, int s, const LccRow &w)
 GW_HD void step_consts_x(StepConsts &k, const gw_params_t &p, const CellConsts &c, double V, const double *X,
                          double Cai, double CaNSR, uint32_t step_lo)
 {
-    step_consts_scalars(k, c, V, X, Cai, CaNSR, step_lo);
+    step_consts_scalars(k, c, V, X, Cai, CaNSR, step_lo, Serial());
     for (int s = 0; s < 13; ++s) lcc_row_store(k.lcc, s, lcc_row(s, p, c, X));
 }
 
@@ -291,54 +306,6 @@ GW_HD void gd_args(const gw_params_t &p, const gw_globals_t &g, double VF_RT, do
     py[2] = p.Hr;
 }
 
-// Gate rates (common.hpp:175-218) from the exponentials of gd_args.
-GW_HD double alpha_m(double V, const double *X) { return (V == -47.13) ? 3.2 : 0.32 * (V + 47.13) / (1.0 - X[GD_AM]); }
-GW_HD double beta_m(const double *X) { return 0.08 * X[GD_BM]; }
-GW_HD double alpha_h(double V, const double *X) { return (V >= -40.0) ? 0.0 : 0.135 * X[GD_AH]; }
-GW_HD double beta_h(double V, const double *X)
-{
-    return (V >= -40.0) ? 1.0 / (0.13 * (1.0 + X[GD_BH1])) : 3.56 * X[GD_BH2] + 3.1e5 * X[GD_BH3];
-}
-GW_HD double alpha_j(double V, const double *X)
-{
-    return (V >= -40.0) ? 0.0 : (-127140.0 * X[GD_AJ1] - 3.474e-5 * X[GD_AJ2]) * (V + 37.78) / (1.0 + X[GD_AJ3]);
-}
-GW_HD double beta_j(double V, const double *X)
-{
-    return (V >= -40.0) ? 0.3 * X[GD_BJ1] / (1.0 + X[GD_BJ2]) : 0.1212 * X[GD_BJ3] / (1.0 + X[GD_BJ4]);
-}
-GW_HD double XKsinf(const double *X) { return 1.0 / (1.0 + X[GD_XKS]); }
-GW_HD double tauXKs_inv(double V, const double *X)
-{
-    if (V == 10.0) return 0.0000719 / 0.148 + 0.000131 / 0.0687;  // analytic limit of 0/0
-    return 0.0000719 * (V - 10.0) / (1.0 - X[GD_TXKS1]) + 0.000131 * (V - 10.0) / (X[GD_TXKS2] - 1.0);
-}
-
-// IKr chain: generator entries of update_QKr (GW.tpp:25-44) and the
-// derivatives of update_Kr_derivatives (GW.tpp:126-133), in registers.
-GW_HD void kr_chain(const gw_params_t &p, const double *X, const double x[5], double dt, double d[5])
-{
-    const double q12 = p.Kf, q21 = p.Kb;   // initialise_QKr (GW.hpp:75)
-    const double q01 = 0.0069 * X[GD_KR0];
-    const double q00 = -q01;
-    const double q10 = 0.0227 * X[GD_KR1];
-    const double q11 = -(q10 + q12);
-    const double q23 = 0.0218 * X[GD_KR2];
-    const double q24 = 1.29e-5 * X[GD_KR3];
-    const double q22 = -(q21 + q23 + q24);
-    const double q32 = 0.0009 * X[GD_KR4];
-    const double q34 = 0.0622 * X[GD_KR5];
-    const double q33 = -(q32 + q34);
-    const double q43 = 0.0059 * X[GD_KR6];
-    const double q42 = q32 * q43 * q24 / (q23 * q34);
-    const double q44 = -(q42 + q43);
-    d[0] = dt * (q10 * x[1] + q00 * x[0]);
-    d[1] = dt * (q01 * x[0] + q21 * x[2] + q11 * x[1]);
-    d[2] = dt * (q12 * x[1] + q32 * x[3] + q42 * x[4] + q22 * x[2]);
-    d[3] = dt * (q23 * x[2] + q43 * x[4] + q33 * x[3]);
-    d[4] = dt * (q24 * x[2] + q34 * x[3] + q44 * x[4]);
-}
-
 // One Kv chain (Kv1.4 or Kv4.3): generator entries of update_QKv (GW.tpp:64-123)
 // and the derivatives of update_Kv_derivatives (GW.tpp:135-160), in registers.
 GW_HD void kv_chain(double aa, double ai, double ba, double bi, double f1, double f2, double f3, double f4,
@@ -404,13 +371,17 @@ __device__ __forceinline__ double gd_arg_value(const GdArg &r, const gw_params_t
 }
 
 // The argument of slot s >= GD_LOG0 and, for a power, its exponent (else 0).
+// Every value is read before one is chosen: a choice between reads would be a branch.
 GW_HD double gd_log_arg(int slot, const gw_params_t &p, const gw_globals_t &g, double &y)
 {
-    y = slot == GD_PNAK ? 1.5 : slot == GD_PF ? p.Hf : slot == GD_PR ? p.Hr : 0.0;
-    const double num = slot == GD_LNA ? p.Nao : slot == GD_LK ? p.Ko : slot == GD_LKS ? p.Ko + 0.01833 * p.Nao
-                     : slot == GD_PNAK ? p.KmNai : slot == GD_PF ? g.Cai : g.CaNSR;
-    const double den = slot == GD_LNA ? g.Nai : slot == GD_LK ? g.Ki : slot == GD_LKS ? g.Ki + 0.01833 * g.Nai
-                     : slot == GD_PNAK ? g.Nai : slot == GD_PF ? p.Kmf : p.Kmr;
+    const double Nao = p.Nao, Ko = p.Ko, KmNai = p.KmNai, Kmf = p.Kmf, Kmr = p.Kmr, Hf = p.Hf, Hr = p.Hr;
+    const double Nai = g.Nai, Ki = g.Ki, Cai = g.Cai, CaNSR = g.CaNSR;
+    const double Kso = Ko + 0.01833 * Nao, Ksi = Ki + 0.01833 * Nai;
+    y = slot == GD_PNAK ? 1.5 : slot == GD_PF ? Hf : slot == GD_PR ? Hr : 0.0;
+    const double num = slot == GD_LNA ? Nao : slot == GD_LK ? Ko : slot == GD_LKS ? Kso : slot == GD_PNAK ? KmNai
+                     : slot == GD_PF ? Cai : CaNSR;
+    const double den = slot == GD_LNA ? Nai : slot == GD_LK ? Ki : slot == GD_LKS ? Ksi : slot == GD_PNAK ? Nai
+                     : slot == GD_PF ? Kmf : Kmr;
     return num / den;
 }
 
@@ -482,91 +453,123 @@ GW_HD bool gd_concentrations_ok(const gw_params_t &p, const gw_globals_t &g)
 GW_HD double gd_EK(const CellConsts &c, double lk) { return lk * c.RT_F / 1.0; }
 GW_HD double gd_ik1_arg(const CellConsts &c, double V, double lk) { return 1.5 * (V - gd_EK(c, lk)) * c.F_RT; }
 
-// The derivatives from the values X[slot], except the gates and the IKr and Kv
-// chains (gd_gates, gd_chain_kr and gd_chain_kv below), in four parts that
-// share only their inputs and gd_combine, which joins them.
+// The derivatives from the values X[slot], except the Kv chains (gd_chain_kv
+// below), in three parts that share only their inputs and gd_combine, which
+// joins them. A part gathers its independent quotients and has quot(num, den,
+// q) form them: one after another (Serial), or one per lane.
+template <class Quot>
 GW_HD void gd_k_currents(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, double VF_RT,
-                         const double *X, Currents &cur)
+                         const double *X, Currents &cur, Quot &&quot)
 {
     const double V = g.V;
-    const double expmVF_RT = X[GD_EXPM];
+    const double e = X[GD_EXPM];
     const double EK = gd_EK(c, X[GD_LK]);
-    {   // GW_utils.hpp:273-279
-        const double RKr = 1.0 / (1.0 + 1.4945 * X[GD_KR_R]);
-        cur.IKr = p.GKr * c.sqrtKo * RKr * g.Kr[3] * (V - EK) * 0.5;
-    }
+    const double num[4] = {1.0, 1.0, 1., (c.PKv14_Csc) * (kFaraday * VF_RT) * g.Kv14[4]};
+    const double den[4] = {1.0 + 1.4945 * X[GD_KR_R], 2.0 + X[GD_IK1], 1. + X[GD_KP], 1 - e};
+    double q[4];
+    quot(num, den, q);
+    const double RKr = q[0], K1inf = q[1], Kp = q[2];
+    cur.IKr = p.GKr * c.sqrtKo * RKr * g.Kr[3] * (V - EK) * 0.5;               // GW_utils.hpp:273-279
     {   // GW_utils.hpp:282-291
         const double EKs = X[GD_LKS] * c.RT_F;
         cur.IKs = p.GKs * sq(g.xKs) * (V - EKs);
     }
-    double IKv14;
-    {   // GW_utils.hpp:299-303 with exp_term = expmVF_RT (GW.tpp:185); limit at V == 0
-        const double e = expmVF_RT;
-        double mm;
-        if (VF_RT == 0.0) mm = (c.PKv14_Csc) * kFaraday * g.Kv14[4];
-        else mm = (c.PKv14_Csc) * (kFaraday * VF_RT) * g.Kv14[4] / (1 - e);
-        IKv14 = mm * ((g.Ki - p.Ko * e) + 0.02 * (g.Nai - p.Nao * e)) * 1.0e9;
-    }
+    // GW_utils.hpp:299-303 with exp_term = exp(-VF/RT) (GW.tpp:185); limit at V == 0
+    const double mm = VF_RT == 0.0 ? (c.PKv14_Csc) * kFaraday * g.Kv14[4] : q[3];
+    const double IKv14 = mm * ((g.Ki - p.Ko * e) + 0.02 * (g.Nai - p.Nao * e)) * 1.0e9;
     const double IKv43 = p.GKv43 * g.Kv43[4] * (V - EK);                       // GW_utils.hpp:294-297
     cur.Ito1 = IKv14 + IKv43;
-    {   // GW_utils.hpp:306-312
-        const double K1inf = 1.0 / (2.0 + X[GD_IK1]);
-        cur.IK1 = p.GK1 * K1inf * c.IK1_const * (V - EK);
-    }
-    {   // GW_utils.hpp:315-319
-        const double Kp = 1. / (1. + X[GD_KP]);
-        cur.IKp = p.GKp * Kp * (V - EK);
-    }
+    cur.IK1 = p.GK1 * K1inf * c.IK1_const * (V - EK);                          // GW_utils.hpp:306-312
+    cur.IKp = p.GKp * Kp * (V - EK);                                           // GW_utils.hpp:315-319
 }
 
+// The Na and Ca currents, SERCA uptake, the cytosolic buffering factor and the
+// troponin derivatives before the factor dt (GW.tpp:201-202).
+template <class Quot>
 GW_HD void gd_na_ca_currents(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, const double *X,
-                             Currents &cur)
+                             Currents &cur, double &beta_cyto, double &dLTRPN, double &dHTRPN, Quot &&quot)
 {
     const double V = g.V;
     const double expmVF_RT = X[GD_EXPM];
+    const double e1 = X[GD_NACA];                                               // common.hpp:163-168
+    const double e2 = e1 * expmVF_RT;
+    const double f = X[GD_PF];                                                  // GW_utils.hpp:339-344
+    const double r = X[GD_PR];
+    const double x = p.KCMDN + g.Cai;                                           // GW_utils.hpp:347-351
+    const double num[5] = {c.INaCa_const * (e1 * cube(g.Nai) * p.Cao - e2 * c.Nao3 * g.Cai), 1.0, g.Cai,
+                           p.Vmaxf * f - p.Vmaxr * r, c.CMDN_const};
+    const double den[5] = {1.0 + p.ksat * e2, 1.0 + 0.1245 * X[GD_NAK] + 0.0365 * c.sigma * expmVF_RT,
+                           p.KmpCa + g.Cai, 1.0 + f + r, sq(x)};
+    double q[5];
+    quot(num, den, q);
+    const double num2[2] = {c.INaK_const * q[1], 1.0};                          // common.hpp:121-124, 140-143
+    const double den2[2] = {1.0 + X[GD_PNAK], 1.0 + q[4]};
+    double q2[2];
+    quot(num2, den2, q2);
     const double ENa = X[GD_LNA] * c.RT_F / 1.0;
     const double ECa = X[GD_LK] * c.RT_F / 2.0;                                 // K-based, as GW.tpp:176
     cur.INa = p.GNa * cube(g.m) * g.h * g.j * (V - ENa);                       // common.hpp:89-92
     cur.INab = p.GNab * (V - ENa);                                             // common.hpp:100-101
-    {   // common.hpp:163-168
-        const double e1 = X[GD_NACA];
-        const double e2 = e1 * expmVF_RT;
-        cur.INaCa = c.INaCa_const * (e1 * cube(g.Nai) * p.Cao - e2 * c.Nao3 * g.Cai) / (1.0 + p.ksat * e2);
-    }
-    {   // common.hpp:121-124, 140-143
-        const double fNaK = 1.0 / (1.0 + 0.1245 * X[GD_NAK] + 0.0365 * c.sigma * expmVF_RT);
-        cur.INaK = c.INaK_const * fNaK / (1.0 + X[GD_PNAK]);
-    }
+    cur.INaCa = q[0];
+    cur.INaK = q2[0];
     cur.ICab = p.GCab * (V - ECa);
-    cur.IpCa = p.IpCamax * (g.Cai / (p.KmpCa + g.Cai));                         // common.hpp:109-110
-}
-
-// SERCA uptake, the cytosolic buffering factor and the troponin derivatives before the factor dt (GW.tpp:201-202).
-GW_HD void gd_uptake(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, const double *X, Currents &cur,
-                     double &beta_cyto, double &dLTRPN, double &dHTRPN)
-{
-    {   // GW_utils.hpp:339-344
-        const double f = X[GD_PF];
-        const double r = X[GD_PR];
-        cur.Jup = (p.Vmaxf * f - p.Vmaxr * r) / (1.0 + f + r);
-    }
-    {   // GW_utils.hpp:347-351
-        const double x = p.KCMDN + g.Cai;
-        beta_cyto = 1.0 / (1.0 + c.CMDN_const / sq(x));
-    }
+    cur.IpCa = p.IpCamax * q[2];                                                // common.hpp:109-110
+    cur.Jup = q[3];
+    beta_cyto = q2[1];
     dLTRPN = p.kLTRPNp * g.Cai * (p.LTRPNtot - g.CaLTRPN) - p.kLTRPNm * g.CaLTRPN;
     dHTRPN = p.kHTRPNp * g.Cai * (p.HTRPNtot - g.CaHTRPN) - p.kHTRPNm * g.CaHTRPN;
 }
 
-// The currents and fluxes formed from the CRU sums.
-GW_HD void gd_cru_currents(const gw_params_t &p, const CellConsts &c, double VF_RT, const double *X, const FluxSums &S,
-                           Currents &cur)
+// The gates (m, h, j and xKs, GW.tpp:162-168), the IKr chain, and the currents
+// and fluxes formed from the CRU sums. d: the derivatives of the gates and of
+// the chain (gw_globals_t order).
+template <class Quot>
+GW_HD void gd_gates_kr_cru(const gw_params_t &p, const CellConsts &c, const gw_globals_t &g, double VF_RT,
+                           const double *X, const FluxSums &S, double dt, double d[9], Currents &cur, Quot &&quot)
 {
+    const double V = g.V;
     const double expmVF_RT = X[GD_EXPM];
-    if (VF_RT == 0.0) cur.Ito2 = S.ClCh * c.Ito2_const * (p.Clo - p.Clcyto);    // limit of GW_utils.hpp:330
-    else cur.Ito2 = S.ClCh * c.Ito2_const * VF_RT * (p.Clcyto * expmVF_RT - p.Clo) / (expmVF_RT - 1.0);
-    cur.ICaL = S.JLCC * c.ICaL_const;                                           // GW_utils.hpp:322-325
-    cur.Jtr_tot = S.Jtr * c.CRU_factor;                                         // GW_utils.hpp:354-355
+    const bool hi = V >= -40.0;
+    const double q23 = 0.0218 * X[GD_KR2], q24 = 1.29e-5 * X[GD_KR3], q32 = 0.0009 * X[GD_KR4];
+    const double q34 = 0.0622 * X[GD_KR5], q43 = 0.0059 * X[GD_KR6];
+    const double bj = 0.3 * X[GD_BJ1], aj = (-127140.0 * X[GD_AJ1] - 3.474e-5 * X[GD_AJ2]) * (V + 37.78);
+    const double bjd = 1.0 + X[GD_BJ2], ajd = 1.0 + X[GD_AJ3];
+    const double num[9] = {0.32 * (V + 47.13), 1.0, hi ? bj : aj, 0.1212 * X[GD_BJ3], 1.0, 0.0000719 * (V - 10.0),
+                           0.000131 * (V - 10.0), q32 * q43 * q24,
+                           S.ClCh * c.Ito2_const * VF_RT * (p.Clcyto * expmVF_RT - p.Clo)};
+    const double den[9] = {1.0 - X[GD_AM], 0.13 * (1.0 + X[GD_BH1]), hi ? bjd : ajd, 1.0 + X[GD_BJ4], 1.0 + X[GD_XKS],
+                           1.0 - X[GD_TXKS1], X[GD_TXKS2] - 1.0, q23 * q34, expmVF_RT - 1.0};
+    double q[9];
+    quot(num, den, q);
+    // common.hpp:175-218; the limits of 0/0
+    const double am = (V == -47.13) ? 3.2 : q[0], bm = 0.08 * X[GD_BM];
+    const double ah = hi ? 0.0 : 0.135 * X[GD_AH], bh = hi ? q[1] : 3.56 * X[GD_BH2] + 3.1e5 * X[GD_BH3];
+    const double a_j = hi ? 0.0 : q[2], b_j = hi ? q[2] : q[3];
+    const double tauXKs_inv = (V == 10.0) ? 0.0000719 / 0.148 + 0.000131 / 0.0687 : q[5] + q[6];
+    d[0] = dt * (am * (1.0 - g.m) - bm * g.m);
+    d[1] = dt * (ah * (1.0 - g.h) - bh * g.h);
+    d[2] = dt * (a_j * (1.0 - g.j) - b_j * g.j);
+    d[3] = dt * (q[4] - g.xKs) * tauXKs_inv;
+    // update_QKr (GW.tpp:25-44) and update_Kr_derivatives (GW.tpp:126-133)
+    const double *x = g.Kr;
+    const double q12 = p.Kf, q21 = p.Kb;   // initialise_QKr (GW.hpp:75)
+    const double q01 = 0.0069 * X[GD_KR0];
+    const double q00 = -q01;
+    const double q10 = 0.0227 * X[GD_KR1];
+    const double q11 = -(q10 + q12);
+    const double q22 = -(q21 + q23 + q24);
+    const double q33 = -(q32 + q34);
+    const double q42 = q[7];
+    const double q44 = -(q42 + q43);
+    d[4] = dt * (q10 * x[1] + q00 * x[0]);
+    d[5] = dt * (q01 * x[0] + q21 * x[2] + q11 * x[1]);
+    d[6] = dt * (q12 * x[1] + q32 * x[3] + q42 * x[4] + q22 * x[2]);
+    d[7] = dt * (q23 * x[2] + q43 * x[4] + q33 * x[3]);
+    d[8] = dt * (q24 * x[2] + q34 * x[3] + q44 * x[4]);
+    // GW_utils.hpp:322-330 (its limit at V == 0), 354-355
+    cur.Ito2 = VF_RT == 0.0 ? S.ClCh * c.Ito2_const * (p.Clo - p.Clcyto) : q[8];
+    cur.ICaL = S.JLCC * c.ICaL_const;
+    cur.Jtr_tot = S.Jtr * c.CRU_factor;
     cur.Jxfer_tot = S.Jxfer * c.CRU_factor;
 }
 
@@ -585,23 +588,6 @@ GW_HD void gd_combine(const CellConsts &c, const Currents &cur, double beta_cyto
     d[6] = dHTRPN * dt;
     d[0] = dt * (Istim - (cur.INa + cur.ICaL + cur.IKr + cur.IKs + cur.Ito1 + cur.IK1 + cur.IKp + cur.Ito2 +
                           cur.INaK + cur.INaCa + cur.IpCa + cur.ICab + cur.INab));
-}
-
-// GW.tpp:162-168: the derivatives of the gates m, h, j and xKs, into
-// d[0..3] (gw_globals_t order).
-GW_HD void gd_gates(const double *X, const gw_globals_t &g, double dt, double d[4])
-{
-    const double V = g.V;
-    d[0] = dt * (alpha_m(V, X) * (1.0 - g.m) - beta_m(X) * g.m);
-    d[1] = dt * (alpha_h(V, X) * (1.0 - g.h) - beta_h(V, X) * g.h);
-    d[2] = dt * (alpha_j(V, X) * (1.0 - g.j) - beta_j(V, X) * g.j);
-    d[3] = dt * (XKsinf(X) - g.xKs) * tauXKs_inv(V, X);
-}
-
-// GW.tpp:25-44, 126-133: the IKr chain's derivatives.
-GW_HD void gd_chain_kr(const gw_params_t &p, const double *X, const gw_globals_t &g, double dt, double dKr[5])
-{
-    kr_chain(p, X, g.Kr, dt, dKr);
 }
 
 // GW.tpp:64-123, 135-160: the derivatives of the Kv1.4 (which == 0) or Kv4.3
@@ -631,11 +617,11 @@ GW_HD int gd_finish(const gw_params_t &p, const CellConsts &c, const gw_globals_
                     double dt, double Istim, const FluxSums &S, gw_globals_t &dg, Currents &cur)
 {
     if (!gd_concentrations_ok(p, g)) return GW_E_NONPOSITIVE_CONC;
-    double beta_cyto, dLTRPN, dHTRPN, d[7], gates[4];
-    gd_k_currents(p, c, g, VF_RT, X, cur);
-    gd_na_ca_currents(p, c, g, X, cur);
-    gd_uptake(p, c, g, X, cur, beta_cyto, dLTRPN, dHTRPN);
-    gd_cru_currents(p, c, VF_RT, X, S, cur);
+    double beta_cyto, dLTRPN, dHTRPN, d[7], gk[9];
+    const Serial quot;
+    gd_k_currents(p, c, g, VF_RT, X, cur, quot);
+    gd_na_ca_currents(p, c, g, X, cur, beta_cyto, dLTRPN, dHTRPN, quot);
+    gd_gates_kr_cru(p, c, g, VF_RT, X, S, dt, gk, cur, quot);
     gd_combine(c, cur, beta_cyto, dLTRPN, dHTRPN, dt, Istim, d);
     dg.V = d[0];
     dg.Nai = d[1];
@@ -644,12 +630,11 @@ GW_HD int gd_finish(const gw_params_t &p, const CellConsts &c, const gw_globals_
     dg.CaNSR = d[4];
     dg.CaLTRPN = d[5];
     dg.CaHTRPN = d[6];
-    gd_gates(X, g, dt, gates);
-    dg.m = gates[0];
-    dg.h = gates[1];
-    dg.j = gates[2];
-    dg.xKs = gates[3];
-    gd_chain_kr(p, X, g, dt, dg.Kr);
+    dg.m = gk[0];
+    dg.h = gk[1];
+    dg.j = gk[2];
+    dg.xKs = gk[3];
+    for (int i = 0; i < 5; ++i) dg.Kr[i] = gk[4 + i];
     gd_chain_kv(p, X, g, dt, 0, dg.Kv14);
     gd_chain_kv(p, X, g, dt, 1, dg.Kv43);
     return GW_OK;

@@ -38,7 +38,6 @@ GW_HD uint64_t ryr_set(uint64_t w, int k, int v)
 {
     return (w & ~(0xffULL << (8 * k))) | (static_cast<uint64_t>(static_cast<uint8_t>(static_cast<int8_t>(v))) << (8 * k));
 }
-GW_HD uint64_t ryr_add(uint64_t w, int k, int d) { return ryr_set(w, k, ryr_get(w, k) + d); }
 GW_HD int sub_lcc(uint64_t w) { return static_cast<int>((w >> 48) & 15u); }
 GW_HD int sub_y(uint64_t w) { return static_cast<int>((w >> 52) & 1u); }
 GW_HD int sub_cl(uint64_t w) { return static_cast<int>((w >> 53) & 1u); }
@@ -362,45 +361,24 @@ __device__ __forceinline__ int qsum4i(int v) { return qgeti<0>(v) + qgeti<1>(v) 
 template <class R>
 __device__ __forceinline__ int ryr_pick(const SsaParamsT<R> &P, uint64_t w, R ca, R uu)
 {
+    // without branches: `live` falls at the first cumulative rate that reaches uu
     int tr = sizeof(R) == 8 ? 0 : -1;
     R cum = R(0);
-    if constexpr (sizeof(R) == 8) {   // without branches: `live` falls once a cumulative rate has reached uu
-        bool live = true;
-        ryr_rates(P, w, ca, [&](int k, R r) {
-            if (k > 0) live = live & (cum < uu);
-            tr = live ? k : tr;
-            cum += live ? r : R(0);
-        });
-    } else {
-        bool done = false;
-        ryr_rates(P, w, ca, [&](int k, R r) {
-            if (done) return;
-            if (k == 0) {
-                cum = r;
-                if (r > R(0)) tr = 0;
-            } else if (cum < uu) {
-                if (r > R(0)) tr = k;
-                cum += r;
-            } else {
-                done = true;
-            }
-        });
-    }
+    bool live = true;
+    ryr_rates(P, w, ca, [&](int k, R r) {
+        if (k > 0) live = live & (cum < uu);
+        if (sizeof(R) == 8) tr += (k > 0 && live) ? 1 : 0;
+        else tr = (live & (r > R(0))) ? k : tr;
+        cum = k == 0 ? r : cum + r;
+    });
     return tr;
 }
 
 // Source and target states (0..5) of RyR transition tr (0..11, in
 // sample_RyR's order, SSA.tpp:200-259).
-GW_HD int ryr_from(int tr)
-{
-    return (tr == 0) ? 0 : (tr <= 2 || tr == 6) ? 1 : (tr == 3 || tr == 7) ? 2
-         : (tr == 4 || tr == 8) ? 3 : (tr == 5 || tr == 9 || tr == 10) ? 4 : 5;
-}
-GW_HD int ryr_to(int tr)
-{
-    return (tr == 0 || tr == 7 || tr == 9) ? 1 : (tr == 1 || tr == 8) ? 2 : (tr == 3 || tr == 10) ? 3
-         : (tr == 2 || tr == 4 || tr == 11) ? 4 : (tr == 5) ? 5 : 0;
-}
+// One octal digit per transition.
+GW_HD int ryr_from(int tr) { return static_cast<int>(0544321432110ULL >> (3 * tr)) & 7; }
+GW_HD int ryr_to(int tr) { return static_cast<int>(0431210543421ULL >> (3 * tr)) & 7; }
 
 // FP32-local only: whether transition tr may be applied to word w at the
 // subspace Ca the step has just reached. The transition is chosen from the
@@ -442,10 +420,13 @@ GW_HD bool ryr_in_range(uint64_t w, int tr)
     return ryr_get(w, ryr_from(tr)) > -128 && ryr_get(w, ryr_to(tr)) < 127;
 }
 
-// Apply RyR transition tr (0..11, in sample_RyR's order) to a subunit word.
+// Apply RyR transition tr (0..11, in sample_RyR's order) to a subunit word:
+// one RyR from one count to another. With 128 added to each count no byte
+// borrows or carries (ryr_in_range).
 GW_HD uint64_t ryr_apply(uint64_t w, int tr)
 {
-    return ryr_add(ryr_add(w, ryr_from(tr), -1), ryr_to(tr), +1);
+    constexpr uint64_t kBias = 0x808080808080ULL;
+    return ((w ^ kBias) + (1ULL << (8 * ryr_to(tr))) - (1ULL << (8 * ryr_from(tr)))) ^ kBias;
 }
 
 struct CruQ {
@@ -583,31 +564,28 @@ __device__ __forceinline__ bool quad_iterate(QuadState<R> &S, const SsaParamsT<R
     const R dCaSS = h * (S.jl + S.Jrel - S.Jxfer + Jiss) * betaSS;
     const double tmp = oldA + static_cast<double>(dCaSS);
     const int split = split_mask<R>(oldA, tmp);
-    const int any_split = qgeti<0>(split) | qgeti<1>(split) | qgeti<2>(split) | qgeti<3>(split);
-    if (any_split) {
-        // sample_RyR56 / sample_RyR34 (SSA.tpp:59-84), in subunit order; every
-        // lane draws the same Bernoulli uniforms and the owner applies them
-        for (int jj = 0; jj < 4; ++jj) {
-            const int sj = qseli(split, jj);
-            for (int bit = 1; bit <= 2; bit <<= 1) {
-                if (!(sj & bit)) continue;
-                const int a_ = (bit == 1) ? 4 : 2;
-                const uint64_t wq = qselu(S.w, jj);
-                const R oq = qsel(old, jj);
-                const R pr = (bit == 1) ? ldiv(P.k65, P.k65 + P.k56 * sq(oq)) : ldiv(P.k43, P.k43 + P.k34 * sq(oq));
-                const int n = ryr_get(wq, a_) + ryr_get(wq, a_ + 1);
-                int X = 0;
-                for (int i = 0; i < n; ++i)
-                    if (qdraw<PRNG, R>(S.q) < pr) X++;
-                const int na = (n > 0) ? X : 0;
-                const int nb = (n > 0) ? n - X : 0;
-                if (j == jj) {
-                    S.w = ryr_set(ryr_set(S.w, a_, na), a_ + 1, nb);
-                    S.changed = 1;
-                }
-                if (DIGEST) digest_event(S.dig, step_lo, jj, bit == 1 ? 4 : 5, na);
-            }
+    const int splits = qgeti<0>(split) | qgeti<1>(split) << 2 | qgeti<2>(split) << 4 | qgeti<3>(split) << 6;
+    // sample_RyR56 / sample_RyR34 (SSA.tpp:59-84), in subunit order (a
+    // subunit's (5,6) pair first): every lane of the quad draws the same
+    // Bernoulli uniforms and the owner applies them
+#pragma unroll 1
+    for (int m = splits; m != 0; m &= m - 1) {
+        const int bit = __builtin_ctz(m), jj = bit >> 1;
+        const int sh = (bit & 1) ? 16 : 32;   // the (3,4) or the (5,6) pair's bytes
+        const int n_me = static_cast<int8_t>(S.w >> sh) + static_cast<int8_t>(S.w >> (sh + 8));
+        const R kb = (bit & 1) ? P.k43 : P.k65, kf = (bit & 1) ? P.k34 : P.k56;
+        const R pr = qsel(ldiv(kb, kb + kf * sq(old)), jj);
+        const int n = qseli(n_me, jj);
+        int X = 0;
+        for (int i = 0; i < n; ++i)
+            if (qdraw<PRNG, R>(S.q) < pr) X++;
+        const int na = (n > 0) ? X : 0;
+        if (j == jj) {
+            const uint64_t pair = n > 0 ? static_cast<uint64_t>(X & 0xff) | static_cast<uint64_t>((n - X) & 0xff) << 8 : 0;
+            S.w = (S.w & ~(0xffffULL << sh)) | pair << sh;
+            S.changed = 1;
         }
+        if (DIGEST) digest_event(S.dig, step_lo, jj, (bit & 1) ? 5 : 4, na);
     }
     S.ca = tmp;
     // update_CaJSR (SSA.hpp:67-71), replicated
