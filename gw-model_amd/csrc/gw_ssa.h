@@ -242,36 +242,27 @@ GW_HD void sample_rest_cru(uint64_t seed, int64_t i, double ca[4], double &jsr, 
     uint64_t s[4];
     rng_seed(PRNG, s, ~stream_key(seed, i));
     auto u = [&]() { return u01(rng_next<PRNG>(s[0], s[1], s[2], s[3])); };
-    int lcc[4], y[4], cl[4], n[4][6];
     for (int j = 0; j < 4; ++j) {
         const double v = u();  // sample_weights over {0.958, 0.038, 0.004} -> LCC 1, 2, 7
-        int idx = 0;
-        double cum = 0.958;
-        if (cum < v) { idx = 1; cum += 0.038; if (cum < v) idx = 2; }
-        lcc[j] = idx == 0 ? 1 : (idx == 1 ? 2 : 7);
+        const bool b1 = 0.958 < v, b2 = b1 && 0.958 + 0.038 < v;
+        sub[j] = sub_set_lcc(0, b2 ? 7 : b1 ? 2 : 1);
     }
     for (int j = 0; j < 4; ++j) {
         const double v = u();  // {0.9425, 0.0575} -> y = 1, 0
-        y[j] = (0.9425 < v) ? 0 : 1;
+        if (!(0.9425 < v)) sub[j] = sub_flip_y(sub[j]);
     }
     for (int j = 0; j < 4; ++j) {
-        for (int k = 0; k < 6; ++k) n[j][k] = 0;
         for (int k = 0; k < 5; ++k) {
             const double v = u();  // {0.609, 0.1955, 0.1955} -> RyR states 1, 5, 6
-            int idx = 0;
-            double cum = 0.609;
-            if (cum < v) { idx = 1; cum += 0.5 * 0.391; if (cum < v) idx = 2; }
-            n[j][idx == 0 ? 0 : (idx == 1 ? 4 : 5)] += 1;
+            const bool b1 = 0.609 < v, b2 = b1 && 0.609 + 0.5 * 0.391 < v;
+            sub[j] += 1ULL << (b2 ? 40 : b1 ? 32 : 0);   // counts of at most 5: no carry
         }
     }
     for (int j = 0; j < 4; ++j) {
         const double v = u();  // {0.998, 0.002} -> ClCh 0, 1
-        cl[j] = (0.998 < v) ? 1 : 0;
+        if (0.998 < v) sub[j] = sub_flip_cl(sub[j]);
     }
-    for (int j = 0; j < 4; ++j) {
-        ca[j] = 1.45370e-4;
-        sub[j] = sub_pack(lcc[j], y[j], cl[j], n[j]);
-    }
+    for (int j = 0; j < 4; ++j) ca[j] = 1.45370e-4;
     jsr = 0.908408;
 }
 
