@@ -23,8 +23,10 @@
 #include <hip/hip_ext.h>
 
 #include <algorithm>
+#include <cfloat>
 #include <cmath>
 #include <cstdarg>
+#include <cstddef>
 #include <cstdio>
 #include <cstring>
 #include <mutex>
@@ -1787,53 +1789,114 @@ __global__ void k_frozen_close(KArgs a, int64_t step0, int64_t nsteps)
     if (D.status != 0 && D.stop_step > D.step) D.stop_step = D.step;
 }
 
-// Packed device state <-> row-major host layout of one cell (GWCRUState, src/pyGW.cpp:78-87).
-struct StateView {
-    double *CaSS, *CaJSR, *JLCC;
-    int32_t *LCC, *LCCi, *RyR, *ClCh;
+// A piece of one cell's state on its way between device and host, in pinned
+// host memory that the kernels below write and read themselves: the CRU state
+// as the device packs it, 72 bytes per CRU, and JLCC where it is asked for,
+// with the cell's status and globals in front. The host expands it to the
+// row-major layout (GWCRUState, src/pyGW.cpp:78-87).
+struct PieceHead {
+    int64_t status;
+    gw_globals_t g;
+};
+constexpr size_t kPieceHead = 512;
+static_assert(sizeof(PieceHead) <= kPieceHead && sizeof(gw_globals_t) % 8 == 0, "the head of a piece");
+
+struct PieceView {
+    PieceHead *head;
+    double *CaSS;
+    uint64_t *sub;
+    double *CaJSR;
+    void *JLCC;   // doubles, floats where an FP32-local batch writes it
 };
 
-__global__ void k_put_state(KArgs a, int cell, StateView v, int has_jlcc)
+__host__ __device__ inline PieceView piece_view(void *base, int64_t m)
 {
-    const DevCell &C = a.cells[cell];
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= C.n_cru) return;
-    const int64_t slot = C.slot0 + i;
-    for (int j = 0; j < 4; ++j) {
-        st_cass(a, slot * 4 + j, v.CaSS[i * 4 + j]);
-        st_jlcc(a, slot * 4 + j, has_jlcc ? v.JLCC[i * 4 + j] : 0.0);
-        int n6[6];
-        for (int k = 0; k < 6; ++k) n6[k] = v.RyR[(i * 4 + j) * 6 + k];
-        a.sub[slot * 4 + j] = sub_pack(v.LCC[i * 4 + j], v.LCCi[i * 4 + j], v.ClCh[i * 4 + j], n6);
-    }
-    st_cajsr(a, slot, v.CaJSR[i]);
+    PieceView v;
+    char *p = static_cast<char *>(base);
+    v.head = reinterpret_cast<PieceHead *>(p); p += kPieceHead;
+    v.CaSS = reinterpret_cast<double *>(p); p += 4 * m * 8;
+    v.sub = reinterpret_cast<uint64_t *>(p); p += 4 * m * 8;
+    v.CaJSR = reinterpret_cast<double *>(p); p += (m + 1) / 2 * 16;
+    v.JLCC = p;
+    return v;
+}
+constexpr size_t piece_bytes(int64_t m) { return kPieceHead + static_cast<size_t>(m) * 104 + 8; }
+
+// The status and globals of a cell, by the first block of a piece's kernel.
+__device__ __forceinline__ void write_head(const CellDyn &D, PieceHead *head)
+{
+    static_assert(sizeof(gw_globals_t) / 8 <= kBlock, "a lane per word");
+    if (blockIdx.x != 0) return;
+    const uint64_t *g = reinterpret_cast<const uint64_t *>(&D.g);
+    if (threadIdx.x < sizeof(gw_globals_t) / 8) reinterpret_cast<uint64_t *>(&head->g)[threadIdx.x] = g[threadIdx.x];
+    if (threadIdx.x == 0) head->status = D.status;
 }
 
-__global__ void k_get_state(KArgs a, int cell, StateView v)
+// CRUs i0 .. i0 + m - 1 of a cell (i0 even), one 16-byte word per lane: whole
+// lines go over the link, which bounds it.
+int64_t piece_words(int64_t m, int jlcc, bool f32)
+{
+    return 4 * m + (m + 1) / 2 + (jlcc ? (f32 ? m : 2 * m) : 0);
+}
+__global__ __launch_bounds__(kBlock) void k_get_piece(KArgs a, int cell, int64_t i0, int64_t m, int jlcc, void *base)
 {
     const DevCell &C = a.cells[cell];
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= C.n_cru) return;
-    const int64_t slot = C.slot0 + i;
-    for (int j = 0; j < 4; ++j) {
-        v.CaSS[i * 4 + j] = ld_cass(a, slot * 4 + j);
-        v.JLCC[i * 4 + j] = ld_jlcc(a, slot * 4 + j);
-        const uint64_t w = a.sub[slot * 4 + j];
-        v.LCC[i * 4 + j] = sub_lcc(w);
-        v.LCCi[i * 4 + j] = sub_y(w);
-        v.ClCh[i * 4 + j] = sub_cl(w);
-        for (int k = 0; k < 6; ++k) v.RyR[(i * 4 + j) * 6 + k] = ryr_get(w, k);
+    const PieceView v = piece_view(base, m);
+    const int64_t slot = C.slot0 + i0;
+    write_head(a.dyn[cell], v.head);
+    auto put = [](void *dst, const void *src, int64_t w) {
+        static_cast<ulonglong2 *>(dst)[w] = static_cast<const ulonglong2 *>(src)[w];
+    };
+    int64_t w = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (w < 2 * m) return put(v.CaSS, a.CaSS + slot * 4, w);
+    if ((w -= 2 * m) < 2 * m) return put(v.sub, a.sub + slot * 4, w);
+    if ((w -= 2 * m) < (m + 1) / 2) return put(v.CaJSR, a.CaJSR + slot, w);   // an odd last one with its padding slot
+    w -= (m + 1) / 2;
+    if (!jlcc) return;
+    if (a.JLCCf) {
+        if (w < m) put(v.JLCC, a.JLCCf + slot * 4, w);
+    } else if (w < 2 * m) {
+        put(v.JLCC, a.JLCC + slot * 4, w);
     }
-    v.CaJSR[i] = ld_cajsr(a, slot);
 }
 
-// One cell's CRU state in the reduced record encoding (gw_cru_state_reduced_t).
+// The same CRUs from a piece whose JLCC, where there is one, is in doubles.
+__global__ __launch_bounds__(kBlock) void k_put_piece(KArgs a, int cell, int64_t i0, int64_t m, int has_jlcc, void *base)
+{
+    const DevCell &C = a.cells[cell];
+    const PieceView v = piece_view(base, m);
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;   // a subunit
+    if (i >= 4 * m) return;
+    const int64_t slot = C.slot0 + i0;
+    a.CaSS[slot * 4 + i] = v.CaSS[i];
+    a.sub[slot * 4 + i] = v.sub[i];
+    st_jlcc(a, slot * 4 + i, has_jlcc ? static_cast<const double *>(v.JLCC)[i] : 0.0);
+    if (i < m) a.CaJSR[slot + i] = v.CaJSR[i];
+}
+
+// One cell's CRU state in the reduced record encoding (gw_cru_state_reduced_t),
+// 40 bytes per CRU.
 struct ReducedView {
+    PieceHead *head;
     float *CaSS, *CaJSR;
     int16_t *RyR;
     int8_t *LCC;
     uint8_t *LCCi, *ClCh;
 };
+
+__host__ __device__ inline ReducedView reduced_view(void *base, int64_t m)
+{
+    ReducedView v;
+    char *p = static_cast<char *>(base);
+    v.head = reinterpret_cast<PieceHead *>(p); p += kPieceHead;
+    v.CaSS = reinterpret_cast<float *>(p); p += 4 * m * 4;
+    v.RyR = reinterpret_cast<int16_t *>(p); p += 4 * m * 2;
+    v.CaJSR = reinterpret_cast<float *>(p); p += m * 4;
+    v.LCC = reinterpret_cast<int8_t *>(p); p += 4 * m;
+    v.LCCi = reinterpret_cast<uint8_t *>(p); p += 4 * m;
+    v.ClCh = reinterpret_cast<uint8_t *>(p);
+    return v;
+}
 
 // RyR_state_to_int16 (src/utils.py:8-22) of one subunit word: a lumped pair
 // with a negative member counts as its sum in the pair's first member.
@@ -1846,20 +1909,31 @@ __device__ __forceinline__ int16_t ryr_code(uint64_t w)
     return static_cast<int16_t>(r1 + 6 * r2 + 36 * s3 + 216 * s4 + 1296 * s5);
 }
 
-__global__ void k_get_state_reduced(KArgs a, int cell, ReducedView v)
+__global__ __launch_bounds__(kBlock) void k_get_piece_reduced(KArgs a, int cell, int64_t i0, int64_t m, void *base)
 {
     const DevCell &C = a.cells[cell];
-    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
-    if (i >= C.n_cru) return;
-    const int64_t slot = C.slot0 + i;
+    const ReducedView v = reduced_view(base, m);
+    write_head(a.dyn[cell], v.head);
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * kBlock + threadIdx.x;
+    if (i >= m) return;
+    const int64_t slot = C.slot0 + i0 + i;
+    float ca[4];
+    short ry[4];
+    signed char lcc[4];
+    unsigned char y[4], cl[4];
     for (int j = 0; j < 4; ++j) {
-        v.CaSS[i * 4 + j] = static_cast<float>(ld_cass(a, slot * 4 + j));
+        ca[j] = static_cast<float>(ld_cass(a, slot * 4 + j));
         const uint64_t w = a.sub[slot * 4 + j];
-        v.LCC[i * 4 + j] = static_cast<int8_t>(sub_lcc(w));
-        v.LCCi[i * 4 + j] = static_cast<uint8_t>(sub_y(w));
-        v.ClCh[i * 4 + j] = static_cast<uint8_t>(sub_cl(w));
-        v.RyR[i * 4 + j] = ryr_code(w);
+        lcc[j] = static_cast<int8_t>(sub_lcc(w));
+        y[j] = static_cast<uint8_t>(sub_y(w));
+        cl[j] = static_cast<uint8_t>(sub_cl(w));
+        ry[j] = ryr_code(w);
     }
+    reinterpret_cast<float4 *>(v.CaSS)[i] = make_float4(ca[0], ca[1], ca[2], ca[3]);
+    reinterpret_cast<short4 *>(v.RyR)[i] = make_short4(ry[0], ry[1], ry[2], ry[3]);
+    reinterpret_cast<char4 *>(v.LCC)[i] = make_char4(lcc[0], lcc[1], lcc[2], lcc[3]);
+    reinterpret_cast<uchar4 *>(v.LCCi)[i] = make_uchar4(y[0], y[1], y[2], y[3]);
+    reinterpret_cast<uchar4 *>(v.ClCh)[i] = make_uchar4(cl[0], cl[1], cl[2], cl[3]);
     v.CaJSR[i] = static_cast<float>(ld_cajsr(a, slot));
 }
 
@@ -1924,8 +1998,7 @@ __global__ void k_posthoc_currents(KArgs a, double *out)
 }
 
 // Status and trace row count of every cell into out[0..n) and out[n..2n),
-// and the persistent kernel's timeout flag into out[2n], so that the host
-// reads them with one copy.
+// and the persistent kernel's timeout flag into out[2n] (pinned host memory).
 __global__ void k_gather_dyn(const CellDyn *dyn, int ncells, const int32_t *timeout, int64_t *out)
 {
     const int c = blockIdx.x * blockDim.x + threadIdx.x;
@@ -1933,6 +2006,15 @@ __global__ void k_gather_dyn(const CellDyn *dyn, int ncells, const int32_t *time
     if (c >= ncells) return;
     out[c] = dyn[c].status;
     out[ncells + c] = dyn[c].trace_rows;
+}
+
+// Words w0 .. w0 + n - 1 of every cell's dynamic state (pinned host memory).
+__global__ void k_export_dyn(const CellDyn *dyn, int ncells, int w0, int n, uint64_t *out)
+{
+    const int64_t i = static_cast<int64_t>(blockIdx.x) * blockDim.x + threadIdx.x;
+    if (i >= static_cast<int64_t>(ncells) * n) return;
+    const int64_t c = i / n;
+    out[i] = reinterpret_cast<const uint64_t *>(dyn + c)[w0 + static_cast<int>(i - c * n)];
 }
 
 __global__ void k_zero_trace_rows(CellDyn *dyn, int ncells)
@@ -2045,6 +2127,9 @@ struct gw_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     void *scratch = nullptr;          // this device's address of `scratch`
+    std::mutex pin_mu;                // a pinned buffer no batch holds, of at most kPinKeep bytes
+    void *pin = nullptr;
+    size_t pin_bytes = 0;
     std::vector<gw_batch *> batches;  // live batches; released by gw_ctx_destroy
 };
 
@@ -2084,11 +2169,14 @@ struct gw_batch {
     DevCell *d_cells = nullptr;
     CellDyn *d_dyn = nullptr;
     BlockInfo *d_blocks = nullptr;
-    void *d_staging = nullptr;
-    size_t staging_bytes = 0;
-    int64_t *d_gather = nullptr;   // [2][ncells]: status, trace rows (k_gather_dyn)
-    // allocation-free batches carve their device memory from the scratch array
-    // instead of allocating it, and free nothing
+    // pinned host memory that kernels write results to: leased from the context
+    // or allocated when first needed, handed back with the batch
+    void *pin = nullptr;
+    size_t pin_bytes = 0;
+    hipEvent_t pin_ev[2] = {};
+    // the device memory of a batch, one allocation (own_arena) or, for an
+    // allocation-free batch, a part of the scratch array
+    bool own_arena = false;
     char *arena = nullptr;
     size_t arena_size = 0, arena_used = 0;
     double *arena_table = nullptr;   // the stimulus table of cell 0
@@ -2097,18 +2185,18 @@ struct gw_batch {
 
 namespace {
 
-// Device memory of a batch: hipMalloc, or for an allocation-free batch the
-// next 256-byte aligned piece of its arena.
+// The next 256-byte aligned piece of a batch's device memory. Before there is
+// any, the pieces are only counted (arena_used).
 int carve(gw_batch *B, void **p, size_t bytes, char *err, size_t errlen)
 {
     const size_t at = (B->arena_used + 255) & ~size_t(255);
-    if (at + bytes > B->arena_size) {
+    if (B->arena && at + bytes > B->arena_size) {
         set_err(err, errlen, "the allocation-free path holds at most %zu bytes of device state (%zu MiB of static "
                 "scratch per GPU); this run needs more: use fewer CRUs or fewer steps, or gw_run",
                 B->arena_size, B->arena_size >> 20);
         return GW_E_INVALID_ARG;
     }
-    *p = B->arena + at;
+    *p = B->arena ? B->arena + at : nullptr;
     B->arena_used = at + bytes;
     return GW_OK;
 }
@@ -2118,8 +2206,50 @@ int dmalloc(gw_batch *B, T **p, size_t n, char *err, size_t errlen)
 {
     *p = nullptr;
     if (n == 0) return GW_OK;
-    if (B->arena) return carve(B, reinterpret_cast<void **>(p), n * sizeof(T), err, errlen);
-    HIP_TRY(hipMalloc(reinterpret_cast<void **>(p), n * sizeof(T)));
+    void *q = nullptr;
+    const int rc = carve(B, &q, n * sizeof(T), err, errlen);
+    *p = static_cast<T *>(q);
+    return rc;
+}
+
+// At least `bytes` of pinned host memory for the batch: the buffer the context
+// keeps, if it is large enough, or a new one. (A buffer costs some 100 us and
+// up to allocate, as much as 15 steps of a small cell.)
+constexpr size_t kPinLeast = size_t(256) << 10, kPinKeep = size_t(16) << 20;
+
+void release_pin(gw_batch *B)
+{
+    gw_ctx *ctx = B->ctx;
+    if (B->pin && B->pin_bytes <= kPinKeep) {
+        std::lock_guard<std::mutex> lock(ctx->pin_mu);
+        if (B->pin_bytes > ctx->pin_bytes) {
+            std::swap(B->pin, ctx->pin);
+            std::swap(B->pin_bytes, ctx->pin_bytes);
+        }
+    }
+    if (B->pin) (void)hipHostFree(B->pin);
+    B->pin = nullptr;
+    B->pin_bytes = 0;
+}
+
+int ensure_pin(gw_batch *B, size_t bytes, char *err, size_t errlen)
+{
+    if (B->pin_bytes >= bytes) return GW_OK;
+    gw_ctx *ctx = B->ctx;
+    if (B->pin) HIP_TRY(hipHostFree(B->pin));
+    B->pin = nullptr;
+    B->pin_bytes = 0;
+    {
+        std::lock_guard<std::mutex> lock(ctx->pin_mu);
+        if (ctx->pin_bytes >= bytes) {
+            std::swap(B->pin, ctx->pin);
+            std::swap(B->pin_bytes, ctx->pin_bytes);
+            return GW_OK;
+        }
+    }
+    const size_t n = std::max(bytes, kPinLeast);
+    HIP_TRY(hipHostMalloc(&B->pin, n, hipHostMallocDefault));
+    B->pin_bytes = n;
     return GW_OK;
 }
 
@@ -2661,47 +2791,56 @@ int launch_steps_timed(gw_batch *B, int64_t step0, int64_t n, double *ssa_ms, ch
     return rc;
 }
 
-// Status and trace row count of every cell, read with one copy.
-int gather_dyn(gw_batch *B, std::vector<int64_t> &out, char *err, size_t errlen)
+// Status and trace row count of every cell (k_gather_dyn); *out stays valid
+// until the batch's pinned memory is used again.
+int gather_dyn(gw_batch *B, const int64_t **out, char *err, size_t errlen)
 {
-    out.assign(2 * static_cast<size_t>(B->ncells) + 1, 0);
+    const int rc = ensure_pin(B, (2 * static_cast<size_t>(B->ncells) + 1) * sizeof(int64_t), err, errlen);
+    if (rc) return rc;
     hipLaunchKernelGGL(k_gather_dyn, dim3((B->ncells + 255) / 256), dim3(256), 0, B->ctx->stream, B->d_dyn, B->ncells,
-                       B->a.timeout, B->d_gather);
+                       B->a.timeout, static_cast<int64_t *>(B->pin));
     HIP_TRY(hipGetLastError());
-    HIP_TRY(hipMemcpyAsync(out.data(), B->d_gather, out.size() * sizeof(int64_t), hipMemcpyDeviceToHost, B->ctx->stream));
     HIP_TRY(hipStreamSynchronize(B->ctx->stream));
+    *out = static_cast<const int64_t *>(B->pin);
     return GW_OK;
 }
 
-// The whole per-cell dynamic state, read with one copy.
-int read_dyn(gw_batch *B, std::vector<CellDyn> &out, char *err, size_t errlen)
+// `bytes` bytes at offset `at` of every cell's dynamic state, cell after cell.
+int read_dyn(gw_batch *B, size_t at, size_t bytes, const void **out, char *err, size_t errlen)
 {
-    out.resize(static_cast<size_t>(B->ncells));
-    HIP_TRY(hipMemcpyAsync(out.data(), B->d_dyn, out.size() * sizeof(CellDyn), hipMemcpyDeviceToHost, B->ctx->stream));
+    const int rc = ensure_pin(B, bytes * static_cast<size_t>(B->ncells), err, errlen);
+    if (rc) return rc;
+    const int n = static_cast<int>(bytes / 8);
+    const int64_t words = static_cast<int64_t>(B->ncells) * n;
+    hipLaunchKernelGGL(k_export_dyn, dim3(static_cast<unsigned>((words + 255) / 256)), dim3(256), 0, B->ctx->stream,
+                       B->d_dyn, B->ncells, static_cast<int>(at / 8), n, static_cast<uint64_t *>(B->pin));
+    HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(B->ctx->stream));
+    *out = B->pin;
     return GW_OK;
+}
+
+int cell_error(int cell, int32_t st, char *err, size_t errlen)
+{
+    const char *what = st == GW_E_NONPOSITIVE_CONC ? "a Nernst potential received a non-positive concentration"
+                     : st == GW_E_NAN ? "a global state variable became NaN"
+                     : st == GW_E_RANGE ? "a CRU flux, a RyR count or the SSA iteration count left the supported range"
+                                        : "device error";
+    set_err(err, errlen, "cell %d: %s (status %d)", cell, what, st);
+    return st;
 }
 
 int check_status(gw_batch *B, char *err, size_t errlen)
 {
-    std::vector<int64_t> v;
-    const int rc = gather_dyn(B, v, err, errlen);
+    const int64_t *v = nullptr;
+    const int rc = gather_dyn(B, &v, err, errlen);
     if (rc) return rc;
     if (v[2 * static_cast<size_t>(B->ncells)] != 0) {
         set_err(err, errlen, "a bounded wait of the persistent step kernel expired; the steps of this call are incomplete");
         return GW_E_TIMEOUT;
     }
-    for (int c = 0; c < B->ncells; ++c) {
-        const int32_t st = static_cast<int32_t>(v[c]);
-        if (st != 0) {
-            const char *what = st == GW_E_NONPOSITIVE_CONC ? "a Nernst potential received a non-positive concentration"
-                             : st == GW_E_NAN ? "a global state variable became NaN"
-                             : st == GW_E_RANGE ? "a CRU flux, a RyR count or the SSA iteration count left the supported range"
-                                                : "device error";
-            set_err(err, errlen, "cell %d: %s (status %d)", c, what, st);
-            return st;
-        }
-    }
+    for (int c = 0; c < B->ncells; ++c)
+        if (v[c] != 0) return cell_error(c, static_cast<int32_t>(v[c]), err, errlen);
     return GW_OK;
 }
 
@@ -2740,50 +2879,120 @@ hipError_t init_crus(gw_batch *B)
     return hipGetLastError();
 }
 
-int ensure_staging(gw_batch *B, size_t bytes, char *err, size_t errlen)
+// Pieces of one cell's state read through pinned memory, two at a time, so
+// that the host expands one while the stream goes on (another piece, or the
+// steps after a record). A cell of up to kPieceCrus CRUs is one piece.
+constexpr int64_t kPieceCrus = 65536;
+static_assert(kPieceCrus % 2 == 0 && 2 * piece_bytes(kPieceCrus) <= kPinKeep, "a context keeps two pieces");
+
+enum PieceForm : int { PIECE_CRUS, PIECE_CRUS_JLCC, PIECE_REDUCED };
+struct PieceQueue {
+    struct Piece {
+        int64_t record, i0, m;
+        double t;
+    };
+    gw_batch *B;
+    int cell, form;
+    size_t stride;
+    Piece piece[2];
+    int first = 0, live = 0;
+};
+
+int pieces_open(PieceQueue &q, gw_batch *B, int cell, int form, char *err, size_t errlen)
 {
-    if (B->staging_bytes >= bytes) return GW_OK;
-    if (B->arena) {
-        set_err(err, errlen, "allocation-free batch: staging of %zu bytes exceeds the %zu carved", bytes, B->staging_bytes);
-        return GW_E_INVALID_ARG;
-    }
-    if (B->d_staging) HIP_TRY(hipFree(B->d_staging));
-    B->d_staging = nullptr;
-    B->staging_bytes = 0;
-    HIP_TRY(hipMalloc(&B->d_staging, bytes));
-    B->staging_bytes = bytes;
+    q.B = B;
+    q.cell = cell;
+    q.form = form;
+    q.stride = (piece_bytes(std::min<int64_t>(B->cells_h[cell].n_cru, kPieceCrus)) + 255) & ~size_t(255);
+    const int rc = ensure_pin(B, 2 * q.stride, err, errlen);
+    if (rc) return rc;
+    for (hipEvent_t &e : B->pin_ev)
+        if (!e) HIP_TRY(hipEventCreateWithFlags(&e, hipEventDisableTiming));
     return GW_OK;
 }
 
-// staging layout for one cell of n CRUs: CaSS[4n] CaJSR[n] JLCC[4n] (f64), LCC LCCi ClCh [4n] RyR[24n] (i32)
-size_t staging_size(int64_t n) { return static_cast<size_t>(n) * (9 * 8 + 36 * 4); }
-
-// The reduced view in the same staging buffer (40 bytes per CRU).
-ReducedView reduced_view(void *base, int64_t n)
+// The oldest piece into sink(piece, base), which returns a status.
+template <class Sink>
+int pieces_pop(PieceQueue &q, Sink &&sink, char *err, size_t errlen)
 {
-    ReducedView v;
-    char *p = static_cast<char *>(base);
-    v.CaSS = reinterpret_cast<float *>(p); p += 4 * n * 4;
-    v.CaJSR = reinterpret_cast<float *>(p); p += n * 4;
-    v.RyR = reinterpret_cast<int16_t *>(p); p += 4 * n * 2;
-    v.LCC = reinterpret_cast<int8_t *>(p); p += 4 * n;
-    v.LCCi = reinterpret_cast<uint8_t *>(p); p += 4 * n;
-    v.ClCh = reinterpret_cast<uint8_t *>(p);
-    return v;
+    HIP_TRY(hipEventSynchronize(q.B->pin_ev[q.first]));
+    const int rc = sink(q.piece[q.first], static_cast<char *>(q.B->pin) + q.first * q.stride);
+    q.first ^= 1;
+    --q.live;
+    return rc;
 }
 
-StateView staging_view(void *base, int64_t n)
+// The cell's state after the steps launched so far; one piece is left under way.
+template <class Sink>
+int pieces_push(PieceQueue &q, int64_t record, double t, Sink &&sink, char *err, size_t errlen)
 {
-    StateView v;
-    char *p = static_cast<char *>(base);
-    v.CaSS = reinterpret_cast<double *>(p); p += 4 * n * 8;
-    v.CaJSR = reinterpret_cast<double *>(p); p += n * 8;
-    v.JLCC = reinterpret_cast<double *>(p); p += 4 * n * 8;
-    v.LCC = reinterpret_cast<int32_t *>(p); p += 4 * n * 4;
-    v.LCCi = reinterpret_cast<int32_t *>(p); p += 4 * n * 4;
-    v.ClCh = reinterpret_cast<int32_t *>(p); p += 4 * n * 4;
-    v.RyR = reinterpret_cast<int32_t *>(p);
-    return v;
+    gw_batch *B = q.B;
+    const int64_t n = B->cells_h[q.cell].n_cru;
+    hipStream_t s = B->ctx->stream;
+    for (int64_t i0 = 0; i0 < n; i0 += kPieceCrus) {
+        const int64_t m = std::min(kPieceCrus, n - i0);
+        const int k = q.first ^ q.live;   // live is 0 or 1 here
+        void *base = static_cast<char *>(B->pin) + k * q.stride;
+        if (q.form == PIECE_REDUCED) {
+            hipLaunchKernelGGL(k_get_piece_reduced, dim3(static_cast<unsigned>((m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s,
+                               B->a, q.cell, i0, m, base);
+        } else {
+            const int jlcc = q.form == PIECE_CRUS_JLCC;
+            const int64_t w = piece_words(m, jlcc, B->a.JLCCf != nullptr);
+            hipLaunchKernelGGL(k_get_piece, dim3(static_cast<unsigned>((w + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, B->a,
+                               q.cell, i0, m, jlcc, base);
+        }
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipEventRecord(B->pin_ev[k], s));
+        q.piece[k] = {record, i0, m, t};
+        if (++q.live == 2) {
+            const int rc = pieces_pop(q, sink, err, errlen);
+            if (rc) return rc;
+        }
+    }
+    return GW_OK;
+}
+
+template <class Sink>
+int pieces_drain(PieceQueue &q, Sink &&sink, char *err, size_t errlen)
+{
+    while (q.live > 0) {
+        const int rc = pieces_pop(q, sink, err, errlen);
+        if (rc) return rc;
+    }
+    return GW_OK;
+}
+
+// CRUs i0 .. i0 + m - 1 of a piece into the rows of c (any of which may be null).
+void expand_piece(void *base, int64_t i0, int64_t m, bool f32, const gw_cru_state_t &c)
+{
+    const PieceView v = piece_view(base, m);
+    const int64_t n = 4 * m;
+    if (c.CaSS) std::memcpy(c.CaSS + 4 * i0, v.CaSS, n * 8);
+    if (c.CaJSR) std::memcpy(c.CaJSR + i0, v.CaJSR, m * 8);
+    if (c.JLCC) {
+        if (f32)
+            for (int64_t k = 0; k < n; ++k) c.JLCC[4 * i0 + k] = static_cast<double>(static_cast<const float *>(v.JLCC)[k]);
+        else
+            std::memcpy(c.JLCC + 4 * i0, v.JLCC, n * 8);
+    }
+    if (c.LCC) for (int64_t k = 0; k < n; ++k) c.LCC[4 * i0 + k] = sub_lcc(v.sub[k]);
+    if (c.LCC_inactivation) for (int64_t k = 0; k < n; ++k) c.LCC_inactivation[4 * i0 + k] = sub_y(v.sub[k]);
+    if (c.ClCh) for (int64_t k = 0; k < n; ++k) c.ClCh[4 * i0 + k] = sub_cl(v.sub[k]);
+    if (c.RyR)
+        for (int64_t k = 0; k < n; ++k)
+            for (int r = 0; r < 6; ++r) c.RyR[(4 * i0 + k) * 6 + r] = ryr_get(v.sub[k], r);
+}
+
+void expand_reduced(void *base, int64_t i0, int64_t m, const gw_cru_state_reduced_t &c)
+{
+    const ReducedView v = reduced_view(base, m);
+    if (c.CaSS) std::memcpy(c.CaSS + 4 * i0, v.CaSS, 4 * m * 4);
+    if (c.CaJSR) std::memcpy(c.CaJSR + i0, v.CaJSR, m * 4);
+    if (c.RyR) std::memcpy(c.RyR + 4 * i0, v.RyR, 4 * m * 2);
+    if (c.LCC) std::memcpy(c.LCC + 4 * i0, v.LCC, 4 * m);
+    if (c.LCC_inactivation) std::memcpy(c.LCC_inactivation + 4 * i0, v.LCCi, 4 * m);
+    if (c.ClCh) std::memcpy(c.ClCh + 4 * i0, v.ClCh, 4 * m);
 }
 
 }  // namespace
@@ -2890,6 +3099,7 @@ int gw_ctx_destroy(gw_ctx *ctx)
     (void)hipSetDevice(ctx->device);
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamDestroy(ctx->stream);
+    if (ctx->pin) (void)hipHostFree(ctx->pin);
     delete ctx;
     return GW_OK;
 }
@@ -2902,15 +3112,11 @@ int gw_batch_destroy(gw_batch *B)
     (void)hipSetDevice(B->ctx->device);
     (void)hipStreamSynchronize(B->ctx->stream);
     graph_release(B);
-    if (B->arena) {   // carved from the scratch array: nothing to free
-        delete B;
-        return GW_OK;
-    }
-    void *ptrs[] = {B->a.CaSS, B->a.CaJSR, B->a.JLCC, B->a.JLCCf, B->a.sub, B->a.rng, B->a.dig, B->a.partials,
-                    B->a.trace, B->a.iters_total, B->d_step_base, B->d_cells, B->d_dyn, B->d_blocks, B->d_staging,
-                    B->d_gather, B->a.sync, B->a.timeout};
-    for (void *p : ptrs)
-        if (p) (void)hipFree(p);
+    release_pin(B);
+    for (hipEvent_t e : B->pin_ev)
+        if (e) (void)hipEventDestroy(e);
+    if (B->own_arena) (void)hipFree(B->arena);
+    if (B->a.trace) (void)hipFree(B->a.trace);
     for (double *p : B->istim_dev)
         if (p) (void)hipFree(p);
     delete B;
@@ -2927,9 +3133,11 @@ int gw_batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, in
 
 namespace {
 
+constexpr size_t kArenaReserve = 208;   // bytes per CRU
+
 // gw_batch_create, or with arena != null an allocation-free batch whose device
-// memory is carved from arena[0, arena_size), with a stimulus table of
-// table_cap steps and the staging of one cell's state carved beside it.
+// memory is carved from arena[0, arena_size); a stimulus table of table_cap
+// steps is carved with the rest.
 int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32_t precision, int32_t prng_id,
                  double dt, const gw_globals_t *g0, void *arena, size_t arena_size, int64_t table_cap,
                  gw_batch **out, char *err, size_t errlen)
@@ -3017,35 +3225,48 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
     KArgs &a = B->a;
     int rc = GW_OK;
     const bool f32 = precision == GW_PREC_FP32_LOCAL;
-    if ((rc = dmalloc(B, &a.CaSS, 4 * N, err, errlen)) || (rc = dmalloc(B, &a.CaJSR, N, err, errlen)) ||
-        (!f32 && (rc = dmalloc(B, &a.JLCC, 4 * N, err, errlen))) ||
-        (f32 && (rc = dmalloc(B, &a.JLCCf, 4 * N, err, errlen))) ||
-        (rc = dmalloc(B, &a.sub, 4 * N, err, errlen)) ||
-        (rc = dmalloc(B, &a.rng, 4 * N, err, errlen)) ||
-        (!f32 && (rc = dmalloc(B, &a.dig, 2 * N, err, errlen))) ||
-        (rc = dmalloc(B, &a.partials, 2 * B->max_nblocks, err, errlen)) ||
-        (rc = dmalloc(B, &a.iters_total, 1, err, errlen)) || (rc = dmalloc(B, &B->d_step_base, 1, err, errlen)) ||
-        (rc = dmalloc(B, &B->d_cells, ncells, err, errlen)) || (rc = dmalloc(B, &B->d_dyn, ncells, err, errlen)) ||
-        (rc = dmalloc(B, &B->d_gather, 2 * static_cast<size_t>(ncells) + 1, err, errlen)) ||
-        (rc = dmalloc(B, &a.sync, static_cast<size_t>(ncells), err, errlen)) ||
-        (rc = dmalloc(B, &a.timeout, 1, err, errlen)) ||
-        (rc = dmalloc(B, &B->d_blocks, static_cast<size_t>(nblocks_all), err, errlen))) {
+    auto lay_out = [&]() {
+        int r = dmalloc(B, &a.CaSS, 4 * N, err, errlen);
+        if (r || (r = dmalloc(B, &a.CaJSR, N, err, errlen)) ||
+            (!f32 && (r = dmalloc(B, &a.JLCC, 4 * N, err, errlen))) ||
+            (f32 && (r = dmalloc(B, &a.JLCCf, 4 * N, err, errlen))) ||
+            (r = dmalloc(B, &a.sub, 4 * N, err, errlen)) ||
+            (r = dmalloc(B, &a.rng, 4 * N, err, errlen)) ||
+            (!f32 && (r = dmalloc(B, &a.dig, 2 * N, err, errlen))) ||
+            (r = dmalloc(B, &a.partials, 2 * B->max_nblocks, err, errlen)) ||
+            (r = dmalloc(B, &a.iters_total, 1, err, errlen)) || (r = dmalloc(B, &B->d_step_base, 1, err, errlen)) ||
+            (r = dmalloc(B, &B->d_cells, ncells, err, errlen)) || (r = dmalloc(B, &B->d_dyn, ncells, err, errlen)) ||
+            (r = dmalloc(B, &a.sync, static_cast<size_t>(ncells), err, errlen)) ||
+            (r = dmalloc(B, &a.timeout, 1, err, errlen)) ||
+            (r = dmalloc(B, &B->d_blocks, static_cast<size_t>(nblocks_all), err, errlen)) ||
+            (r = dmalloc(B, &B->arena_table, static_cast<size_t>(table_cap), err, errlen)))
+            return r;
+        return static_cast<int>(GW_OK);
+    };
+    if (!B->arena) {   // count, then one allocation for all of them
+        void *mem = nullptr;
+        hipError_t he = hipSuccess;
+        if ((rc = lay_out()) == GW_OK && (he = hipMalloc(&mem, B->arena_used)) != hipSuccess) {
+            set_err(err, errlen, "allocating %zu bytes of device memory: %s", B->arena_used, hipGetErrorString(he));
+            rc = GW_E_HIP;
+        }
+        if (rc == GW_OK) {
+            B->arena = static_cast<char *>(mem);
+            B->own_arena = true;
+            B->arena_size = B->arena_used;
+            B->arena_used = 0;
+        }
+    } else {
+        // a run's limit of CRUs and steps counts this much beside the batch
+        void *reserved = nullptr;
+        rc = carve(B, &reserved, kArenaReserve * static_cast<size_t>(B->cells_h[0].n_cru), err, errlen);
+    }
+    if (rc == GW_OK) rc = lay_out();
+    if (rc != GW_OK) {
         gw_batch_destroy(B);
         return rc;
     }
-    if (B->arena) {
-        // the staging of one cell's state (set/get_cru_state) and the stimulus table
-        void *stg = nullptr;
-        const size_t sb = staging_size(B->cells_h[0].n_cru);
-        if ((rc = carve(B, &stg, sb, err, errlen)) ||
-            (table_cap > 0 && (rc = dmalloc(B, &B->arena_table, static_cast<size_t>(table_cap), err, errlen)))) {
-            gw_batch_destroy(B);
-            return rc;
-        }
-        B->d_staging = stg;
-        B->staging_bytes = sb;
-        B->arena_table_cap = table_cap;
-    }
+    B->arena_table_cap = table_cap;
     a.cells = B->d_cells;
     a.dyn = B->d_dyn;
     a.blocks = B->d_blocks + B->bc_off[kShapeDefault];
@@ -3107,45 +3328,58 @@ int gw_batch_set_cru_state(gw_batch *B, int32_t cell, const gw_cru_state_t *c, c
         return GW_E_INVALID_ARG;
     }
     const int64_t n = B->cells_h[cell].n_cru;
-    for (int64_t i = 0; i < 4 * n; ++i) {
-        if (c->LCC[i] < 1 || c->LCC[i] > 12) {
-            set_err(err, errlen, "LCC states must be integers in 1..12 (got %d at flat index %lld)", c->LCC[i], static_cast<long long>(i));
-            return GW_E_INVALID_ARG;
+    // whether any value is out of range, without a branch per value; then which
+    uint32_t bad = 0;
+    for (int64_t i = 0; i < 4 * n; ++i)
+        bad |= (static_cast<uint32_t>(c->LCC[i]) - 1u > 11u) | ((c->LCC_inactivation[i] | c->ClCh[i]) & ~1) |
+               !(std::fabs(c->CaSS[i]) <= DBL_MAX);
+    for (int64_t i = 0; i < 24 * n; ++i) bad |= static_cast<uint32_t>(c->RyR[i]) + 100u > 200u;
+    for (int64_t i = 0; i < n; ++i) bad |= !(std::fabs(c->CaJSR[i]) <= DBL_MAX);
+    if (bad) {
+        for (int64_t i = 0; i < 4 * n; ++i) {
+            if (c->LCC[i] < 1 || c->LCC[i] > 12) {
+                set_err(err, errlen, "LCC states must be integers in 1..12 (got %d at flat index %lld)", c->LCC[i], static_cast<long long>(i));
+                return GW_E_INVALID_ARG;
+            }
+            if ((c->LCC_inactivation[i] & ~1) || (c->ClCh[i] & ~1)) {
+                set_err(err, errlen, "LCC_inactivation and ClCh must be 0 or 1 (flat index %lld)", static_cast<long long>(i));
+                return GW_E_INVALID_ARG;
+            }
+            if (!std::isfinite(c->CaSS[i])) {
+                set_err(err, errlen, "CaSS must be finite");
+                return GW_E_INVALID_ARG;
+            }
         }
-        if ((c->LCC_inactivation[i] & ~1) || (c->ClCh[i] & ~1)) {
-            set_err(err, errlen, "LCC_inactivation and ClCh must be 0 or 1 (flat index %lld)", static_cast<long long>(i));
-            return GW_E_INVALID_ARG;
-        }
-        if (!std::isfinite(c->CaSS[i])) {
-            set_err(err, errlen, "CaSS must be finite");
-            return GW_E_INVALID_ARG;
-        }
+        for (int64_t i = 0; i < 24 * n; ++i)
+            if (c->RyR[i] < -100 || c->RyR[i] > 100) {
+                set_err(err, errlen, "RyR counts must lie in -100..100");
+                return GW_E_INVALID_ARG;
+            }
+        for (int64_t i = 0; i < n; ++i)
+            if (!std::isfinite(c->CaJSR[i])) {
+                set_err(err, errlen, "CaJSR must be finite");
+                return GW_E_INVALID_ARG;
+            }
     }
-    for (int64_t i = 0; i < 24 * n; ++i)
-        if (c->RyR[i] < -100 || c->RyR[i] > 100) {
-            set_err(err, errlen, "RyR counts must lie in -100..100");
-            return GW_E_INVALID_ARG;
-        }
-    for (int64_t i = 0; i < n; ++i)
-        if (!std::isfinite(c->CaJSR[i])) {
-            set_err(err, errlen, "CaJSR must be finite");
-            return GW_E_INVALID_ARG;
-        }
     HIP_TRY(hipSetDevice(B->ctx->device));
-    int rc = ensure_staging(B, staging_size(n), err, errlen);
+    int rc = ensure_pin(B, piece_bytes(std::min(n, kPieceCrus)), err, errlen);
     if (rc) return rc;
-    StateView v = staging_view(B->d_staging, n);
     hipStream_t s = B->ctx->stream;
-    HIP_TRY(hipMemcpyAsync(v.CaSS, c->CaSS, 4 * n * 8, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(v.CaJSR, c->CaJSR, n * 8, hipMemcpyHostToDevice, s));
-    if (c->JLCC) HIP_TRY(hipMemcpyAsync(v.JLCC, c->JLCC, 4 * n * 8, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(v.LCC, c->LCC, 4 * n * 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(v.LCCi, c->LCC_inactivation, 4 * n * 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(v.ClCh, c->ClCh, 4 * n * 4, hipMemcpyHostToDevice, s));
-    HIP_TRY(hipMemcpyAsync(v.RyR, c->RyR, 24 * n * 4, hipMemcpyHostToDevice, s));
-    hipLaunchKernelGGL(k_put_state, dim3((n + 255) / 256), dim3(256), 0, s, B->a, cell, v, c->JLCC ? 1 : 0);
-    HIP_TRY(hipGetLastError());
-    HIP_TRY(hipStreamSynchronize(s));
+    for (int64_t i0 = 0; i0 < n; i0 += kPieceCrus) {
+        const int64_t m = std::min(kPieceCrus, n - i0);
+        const PieceView v = piece_view(B->pin, m);
+        std::memcpy(v.CaSS, c->CaSS + 4 * i0, 4 * m * 8);
+        std::memcpy(v.CaJSR, c->CaJSR + i0, m * 8);
+        if (c->JLCC) std::memcpy(v.JLCC, c->JLCC + 4 * i0, 4 * m * 8);
+        for (int64_t k = 0; k < 4 * m; ++k) {
+            const int64_t q = 4 * i0 + k;
+            v.sub[k] = sub_pack(c->LCC[q], c->LCC_inactivation[q], c->ClCh[q], c->RyR + q * 6);
+        }
+        hipLaunchKernelGGL(k_put_piece, dim3(static_cast<unsigned>((4 * m + kBlock - 1) / kBlock)), dim3(kBlock), 0, s, B->a,
+                           cell, i0, m, c->JLCC ? 1 : 0, B->pin);
+        HIP_TRY(hipGetLastError());
+        HIP_TRY(hipStreamSynchronize(s));
+    }
     return refresh_cell(B, cell, 1, err, errlen);
 }
 
@@ -3155,23 +3389,17 @@ int gw_batch_get_cru_state(gw_batch *B, int32_t cell, gw_cru_state_t *c, char *e
         set_err(err, errlen, "gw_batch_get_cru_state: bad arguments");
         return GW_E_INVALID_ARG;
     }
-    const int64_t n = B->cells_h[cell].n_cru;
     HIP_TRY(hipSetDevice(B->ctx->device));
-    int rc = ensure_staging(B, staging_size(n), err, errlen);
+    PieceQueue q;
+    int rc = pieces_open(q, B, cell, c->JLCC ? PIECE_CRUS_JLCC : PIECE_CRUS, err, errlen);
     if (rc) return rc;
-    StateView v = staging_view(B->d_staging, n);
-    hipStream_t s = B->ctx->stream;
-    hipLaunchKernelGGL(k_get_state, dim3((n + 255) / 256), dim3(256), 0, s, B->a, cell, v);
-    HIP_TRY(hipGetLastError());
-    if (c->CaSS) HIP_TRY(hipMemcpyAsync(c->CaSS, v.CaSS, 4 * n * 8, hipMemcpyDeviceToHost, s));
-    if (c->CaJSR) HIP_TRY(hipMemcpyAsync(c->CaJSR, v.CaJSR, n * 8, hipMemcpyDeviceToHost, s));
-    if (c->JLCC) HIP_TRY(hipMemcpyAsync(c->JLCC, v.JLCC, 4 * n * 8, hipMemcpyDeviceToHost, s));
-    if (c->LCC) HIP_TRY(hipMemcpyAsync(c->LCC, v.LCC, 4 * n * 4, hipMemcpyDeviceToHost, s));
-    if (c->LCC_inactivation) HIP_TRY(hipMemcpyAsync(c->LCC_inactivation, v.LCCi, 4 * n * 4, hipMemcpyDeviceToHost, s));
-    if (c->ClCh) HIP_TRY(hipMemcpyAsync(c->ClCh, v.ClCh, 4 * n * 4, hipMemcpyDeviceToHost, s));
-    if (c->RyR) HIP_TRY(hipMemcpyAsync(c->RyR, v.RyR, 24 * n * 4, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return GW_OK;
+    const bool f32 = B->a.JLCCf != nullptr;
+    auto sink = [&](const PieceQueue::Piece &p, void *base) {
+        expand_piece(base, p.i0, p.m, f32, *c);
+        return GW_OK;
+    };
+    rc = pieces_push(q, 0, 0.0, sink, err, errlen);
+    return rc ? rc : pieces_drain(q, sink, err, errlen);
 }
 
 int gw_batch_get_cru_state_reduced(gw_batch *B, int32_t cell, gw_cru_state_reduced_t *c, char *err, size_t errlen)
@@ -3180,22 +3408,16 @@ int gw_batch_get_cru_state_reduced(gw_batch *B, int32_t cell, gw_cru_state_reduc
         set_err(err, errlen, "gw_batch_get_cru_state_reduced: bad arguments");
         return GW_E_INVALID_ARG;
     }
-    const int64_t n = B->cells_h[cell].n_cru;
     HIP_TRY(hipSetDevice(B->ctx->device));
-    int rc = ensure_staging(B, staging_size(n), err, errlen);
+    PieceQueue q;
+    int rc = pieces_open(q, B, cell, PIECE_REDUCED, err, errlen);
     if (rc) return rc;
-    const ReducedView v = reduced_view(B->d_staging, n);
-    hipStream_t s = B->ctx->stream;
-    hipLaunchKernelGGL(k_get_state_reduced, dim3((n + 255) / 256), dim3(256), 0, s, B->a, cell, v);
-    HIP_TRY(hipGetLastError());
-    if (c->CaSS) HIP_TRY(hipMemcpyAsync(c->CaSS, v.CaSS, 4 * n * 4, hipMemcpyDeviceToHost, s));
-    if (c->CaJSR) HIP_TRY(hipMemcpyAsync(c->CaJSR, v.CaJSR, n * 4, hipMemcpyDeviceToHost, s));
-    if (c->RyR) HIP_TRY(hipMemcpyAsync(c->RyR, v.RyR, 4 * n * 2, hipMemcpyDeviceToHost, s));
-    if (c->LCC) HIP_TRY(hipMemcpyAsync(c->LCC, v.LCC, 4 * n, hipMemcpyDeviceToHost, s));
-    if (c->LCC_inactivation) HIP_TRY(hipMemcpyAsync(c->LCC_inactivation, v.LCCi, 4 * n, hipMemcpyDeviceToHost, s));
-    if (c->ClCh) HIP_TRY(hipMemcpyAsync(c->ClCh, v.ClCh, 4 * n, hipMemcpyDeviceToHost, s));
-    HIP_TRY(hipStreamSynchronize(s));
-    return GW_OK;
+    auto sink = [&](const PieceQueue::Piece &p, void *base) {
+        expand_reduced(base, p.i0, p.m, *c);
+        return GW_OK;
+    };
+    rc = pieces_push(q, 0, 0.0, sink, err, errlen);
+    return rc ? rc : pieces_drain(q, sink, err, errlen);
 }
 
 int gw_batch_set_globals(gw_batch *B, int32_t cell, const gw_globals_t *g, char *err, size_t errlen)
@@ -3217,10 +3439,10 @@ int gw_batch_get_globals(gw_batch *B, gw_globals_t *g_out, char *err, size_t err
         return GW_E_INVALID_ARG;
     }
     HIP_TRY(hipSetDevice(B->ctx->device));
-    std::vector<CellDyn> d;
-    const int rc = read_dyn(B, d, err, errlen);
+    const void *d = nullptr;
+    const int rc = read_dyn(B, offsetof(CellDyn, g), sizeof(gw_globals_t), &d, err, errlen);
     if (rc) return rc;
-    for (int c = 0; c < B->ncells; ++c) g_out[c] = d[c].g;
+    std::memcpy(g_out, d, static_cast<size_t>(B->ncells) * sizeof(gw_globals_t));
     return GW_OK;
 }
 
@@ -3237,8 +3459,9 @@ int gw_batch_set_stimulus_table(gw_batch *B, int32_t cell, const double *istim, 
     }
     HIP_TRY(hipSetDevice(B->ctx->device));
     double *d = nullptr;
-    if (B->arena) {   // the table carved at creation (cell 0 only)
-        if (cell != 0 || n > B->arena_table_cap) {
+    const bool carved = cell == 0 && n <= B->arena_table_cap;
+    if (!B->own_arena || (carved && n > 0)) {   // the table carved at creation (cell 0 only)
+        if (!carved) {
             set_err(err, errlen, "allocation-free batch: a stimulus table of %lld steps exceeds the %lld carved",
                     static_cast<long long>(n), static_cast<long long>(B->arena_table_cap));
             return GW_E_INVALID_ARG;
@@ -3311,8 +3534,21 @@ int gw_batch_get_time(gw_batch *B, double *t, int64_t *steps_done)
         return GW_OK;
     }
     // every running cell shares the clock; a cell that failed stopped its own
-    std::vector<CellDyn> d;
-    if (read_dyn(B, d, nullptr, 0) != GW_OK) return GW_E_HIP;
+    constexpr size_t t0 = offsetof(CellDyn, t), len = offsetof(CellDyn, obs) - t0;
+    const void *mem = nullptr;
+    if (read_dyn(B, t0, len, &mem, nullptr, 0) != GW_OK) return GW_E_HIP;
+    struct {
+        double t;
+        int64_t step;
+        int32_t status;
+    } x;
+    std::vector<decltype(x)> d(static_cast<size_t>(B->ncells));
+    for (int c = 0; c < B->ncells; ++c) {
+        const char *w = static_cast<const char *>(mem) + c * len;
+        std::memcpy(&d[c].t, w, sizeof(x.t));
+        std::memcpy(&d[c].step, w + offsetof(CellDyn, step) - t0, sizeof(x.step));
+        std::memcpy(&d[c].status, w + offsetof(CellDyn, status) - t0, sizeof(x.status));
+    }
     int pick = -1;
     for (int c = 0; c < B->ncells && pick < 0; ++c)
         if (d[c].status == 0) pick = c;
@@ -3333,10 +3569,10 @@ int gw_batch_get_obs(gw_batch *B, gw_cell_obs_t *obs, char *err, size_t errlen)
         return GW_E_INVALID_ARG;
     }
     HIP_TRY(hipSetDevice(B->ctx->device));
-    std::vector<CellDyn> d;
-    const int rc = read_dyn(B, d, err, errlen);
+    const void *d = nullptr;
+    const int rc = read_dyn(B, offsetof(CellDyn, obs), sizeof(gw_cell_obs_t), &d, err, errlen);
     if (rc) return rc;
-    for (int c = 0; c < B->ncells; ++c) obs[c] = d[c].obs;
+    std::memcpy(obs, d, static_cast<size_t>(B->ncells) * sizeof(gw_cell_obs_t));
     return GW_OK;
 }
 
@@ -3382,8 +3618,8 @@ int gw_batch_get_trace(gw_batch *B, double *out, int64_t max_rows, int64_t *rows
         return GW_E_INVALID_ARG;
     }
     HIP_TRY(hipSetDevice(B->ctx->device));
-    std::vector<int64_t> v;
-    int rc = gather_dyn(B, v, err, errlen);
+    const int64_t *v = nullptr;
+    int rc = gather_dyn(B, &v, err, errlen);
     if (rc) return rc;
     const int n = B->ncells;
     int64_t r = 0;
@@ -3682,13 +3918,11 @@ int gw_batch_get_currents(gw_batch *B, double *ICaL, double *Ito2, char *err, si
     int rc = prepare(B, err, errlen);
     if (rc) return rc;
     const size_t bytes = 2 * sizeof(double) * static_cast<size_t>(B->ncells);
-    rc = ensure_staging(B, bytes, err, errlen);
+    rc = ensure_pin(B, bytes, err, errlen);
     if (rc) return rc;
-    double *d = static_cast<double *>(B->d_staging);
-    hipLaunchKernelGGL(k_posthoc_currents, dim3(B->ncells), dim3(kBlock), 0, B->ctx->stream, B->a, d);
+    double *h = static_cast<double *>(B->pin);
+    hipLaunchKernelGGL(k_posthoc_currents, dim3(B->ncells), dim3(kBlock), 0, B->ctx->stream, B->a, h);
     HIP_TRY(hipGetLastError());
-    std::vector<double> h(2 * static_cast<size_t>(B->ncells));
-    HIP_TRY(hipMemcpyAsync(h.data(), d, bytes, hipMemcpyDeviceToHost, B->ctx->stream));
     HIP_TRY(hipStreamSynchronize(B->ctx->stream));
     for (int c = 0; c < B->ncells; ++c) {
         if (ICaL) ICaL[c] = h[2 * c];
@@ -3758,13 +3992,63 @@ int gw_batch_set_mode(gw_batch *B, int32_t frozen, int32_t digest)
 
 namespace {
 
-// The loop of run<PRNG> (src/pyGW.hpp:102-122) on a one-cell batch; record(B,
-// k, t) writes record k (after step i with i % record_every == 0) while k is
-// below num_records.
-template <class Record>
+// The loop of run<PRNG> (src/pyGW.hpp:102-122) on a one-cell batch: the state
+// after each step i with i % record_every == 0 goes to sink(piece, base) while
+// its number, piece.record, is below num_records. A record is on its way and
+// expanded by the host while the stream runs the steps after it. Every 10 steps
+// of a cell of 64 CRUs one costs 11 us beside them (waiting for it, and a copy
+// to pageable memory for each field, cost 127); of 12,500 CRUs, 190 us, the
+// host's expansion into fresh pages (395).
+template <class Sink>
+int run_records(gw_batch *B, double dt, int64_t num_steps, int32_t record_every, int64_t num_records, int form,
+                Sink &&sink_piece, char *err, size_t errlen)
+{
+    if (num_steps == 0) return GW_OK;
+    int rc = launch_cfg_check(B, err, errlen);
+    if (rc || (rc = prepare(B, err, errlen))) return rc;
+    PieceQueue q;
+    if ((rc = pieces_open(q, B, 0, form, err, errlen))) return rc;
+    auto sink = [&](const PieceQueue::Piece &p, void *base) {   // a head stands first in either form
+        const int64_t st = static_cast<const PieceHead *>(base)->status;
+        if (st != 0) return cell_error(0, static_cast<int32_t>(st), err, errlen);
+        sink_piece(p, base);
+        return static_cast<int>(GW_OK);
+    };
+    constexpr int64_t kUnchecked = 4096;   // steps launched beyond the last whose status is or will be read
+    double t = 0.0;
+    int64_t counter = 0, unchecked = 0;
+    for (int64_t i = 0; i < num_steps;) {
+        // next record after step i_rec (i_rec % record_every == 0, i_rec >= i)
+        const int64_t i_rec = ((i + record_every - 1) / record_every) * record_every;
+        const int64_t upto = std::min(num_steps, i_rec + 1);
+        while (i < upto) {
+            const int64_t n = std::min(upto - i, kUnchecked - unchecked);
+            HIP_TRY(launch_steps(B, B->steps_done, n));
+            B->steps_done += n;
+            for (int64_t k = 0; k < n; ++k) t += dt;
+            i += n;
+            unchecked += n;
+            if (unchecked == kUnchecked) {
+                if ((rc = pieces_drain(q, sink, err, errlen)) || (rc = check_status(B, err, errlen))) return rc;
+                unchecked = 0;
+            }
+        }
+        if (i == i_rec + 1) {
+            if (counter < num_records) {
+                if ((rc = pieces_push(q, counter, t, sink, err, errlen))) return rc;
+                unchecked = 0;
+            }
+            ++counter;
+        }
+    }
+    if ((rc = pieces_drain(q, sink, err, errlen))) return rc;
+    return unchecked > 0 ? check_status(B, err, errlen) : GW_OK;
+}
+
+template <class Sink>
 int run_loop(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_t num_steps, const double *istim,
              int32_t record_every, const gw_globals_t *g0, const gw_cru_state_t *c0, uint64_t seed, int32_t prng_id,
-             int32_t precision, int64_t num_records, Record &&record, char *err, size_t errlen,
+             int32_t precision, int64_t num_records, int form, Sink &&sink_piece, char *err, size_t errlen,
              bool noalloc = false)
 {
     if (!ctx || !p || n_cru <= 0 || num_steps < 0 || record_every <= 0) {
@@ -3787,7 +4071,7 @@ int run_loop(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_
         rc = batch_create(ctx, 1, &d, precision, prng_id, dt, g0, ctx->scratch, kScratchBytes,
                           istim ? num_steps : 0, &B, err, errlen);
     } else {
-        rc = gw_batch_create(ctx, 1, &d, precision, prng_id, dt, g0, &B, err, errlen);
+        rc = batch_create(ctx, 1, &d, precision, prng_id, dt, g0, nullptr, 0, istim ? num_steps : 0, &B, err, errlen);
     }
     if (rc) return rc;
     gw_batch_set_mode(B, 0, 0);
@@ -3801,27 +4085,9 @@ int run_loop(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_
         rc = gw_batch_set_stimulus_table(B, 0, istim, num_steps, err, errlen);
         if (rc) { gw_batch_destroy(B); return rc; }
     }
-    double t = 0.0;
-    int64_t counter = 0;
-    int64_t i = 0;
-    while (i < num_steps) {
-        // next record after step i_rec (i_rec % record_every == 0, i_rec >= i)
-        const int64_t i_rec = ((i + record_every - 1) / record_every) * record_every;
-        const int64_t upto = std::min(num_steps, i_rec + 1);
-        rc = gw_batch_step(B, upto - i, err, errlen);
-        if (rc) { gw_batch_destroy(B); return rc; }
-        for (int64_t k = i; k < upto; ++k) t += dt;
-        i = upto;
-        if (i == i_rec + 1) {
-            if (counter < num_records) {
-                rc = record(B, counter, t);
-                if (rc) { gw_batch_destroy(B); return rc; }
-            }
-            ++counter;
-        }
-    }
+    rc = run_records(B, dt, num_steps, record_every, num_records, form, sink_piece, err, errlen);
     gw_batch_destroy(B);
-    return GW_OK;
+    return rc;
 }
 
 }  // namespace
@@ -3838,10 +4104,7 @@ int run_full(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_
              int32_t precision, gw_record_t *out, char *err, size_t errlen, bool noalloc)
 {
     const int64_t n = n_cru;
-    auto record = [&](gw_batch *B, int64_t k, double t) {
-        gw_globals_t g;
-        int rc = gw_batch_get_globals(B, &g, err, errlen);
-        if (rc) return rc;
+    auto scalars = [&](int64_t k, double t, const gw_globals_t &g) {
 #define PUT(f, v) if (out->f) out->f[k] = (v)
         PUT(t, t); PUT(V, g.V); PUT(m, g.m); PUT(h, g.h); PUT(j, g.j); PUT(Nai, g.Nai); PUT(Ki, g.Ki);
         PUT(Cai, g.Cai); PUT(CaNSR, g.CaNSR); PUT(CaLTRPN, g.CaLTRPN); PUT(CaHTRPN, g.CaHTRPN); PUT(xKs, g.xKs);
@@ -3849,6 +4112,11 @@ int run_full(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_
         if (out->XKr) for (int q = 0; q < 5; ++q) out->XKr[k * 5 + q] = g.Kr[q];
         if (out->XKv14) for (int q = 0; q < 10; ++q) out->XKv14[k * 10 + q] = g.Kv14[q];
         if (out->XKv43) for (int q = 0; q < 10; ++q) out->XKv43[k * 10 + q] = g.Kv43[q];
+    };
+    const bool f32 = precision == GW_PREC_FP32_LOCAL;
+    auto record = [&](const PieceQueue::Piece &p, void *base) {
+        const int64_t k = p.record;
+        if (p.i0 == 0) scalars(k, p.t, static_cast<const PieceHead *>(base)->g);
         gw_cru_state_t c;
         c.CaSS = out->CaSS ? out->CaSS + k * n * 4 : nullptr;
         c.CaJSR = out->CaJSR ? out->CaJSR + k * n : nullptr;
@@ -3857,10 +4125,10 @@ int run_full(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_
         c.ClCh = out->ClCh ? out->ClCh + k * n * 4 : nullptr;
         c.RyR = out->RyR ? out->RyR + k * n * 24 : nullptr;
         c.JLCC = nullptr;
-        return gw_batch_get_cru_state(B, 0, &c, err, errlen);
+        expand_piece(base, p.i0, p.m, f32, c);
     };
     return run_loop(ctx, p, n_cru, dt, num_steps, istim, record_every, g0, c0, seed, prng_id, precision,
-                    out ? out->num_records : 0, record, err, errlen, noalloc);
+                    out ? out->num_records : 0, PIECE_CRUS, record, err, errlen, noalloc);
 }
 
 }  // namespace
@@ -3889,10 +4157,7 @@ int gw_run_reduced(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, 
                    size_t errlen)
 {
     const int64_t n = n_cru;
-    auto record = [&](gw_batch *B, int64_t k, double t) {
-        gw_globals_t g;
-        int rc = gw_batch_get_globals(B, &g, err, errlen);
-        if (rc) return rc;
+    auto scalars = [&](int64_t k, double t, const gw_globals_t &g) {
 #define PUT(f, v) if (out->f) out->f[k] = static_cast<float>(v)
         PUT(t, t); PUT(V, g.V); PUT(m, g.m); PUT(h, g.h); PUT(j, g.j); PUT(Nai, g.Nai); PUT(Ki, g.Ki);
         PUT(Cai, g.Cai); PUT(CaNSR, g.CaNSR); PUT(CaLTRPN, g.CaLTRPN); PUT(CaHTRPN, g.CaHTRPN); PUT(xKs, g.xKs);
@@ -3900,6 +4165,10 @@ int gw_run_reduced(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, 
         if (out->XKr) for (int q = 0; q < 4; ++q) out->XKr[k * 4 + q] = static_cast<float>(g.Kr[q]);
         if (out->XKv14) for (int q = 0; q < 9; ++q) out->XKv14[k * 9 + q] = static_cast<float>(g.Kv14[q]);
         if (out->XKv43) for (int q = 0; q < 9; ++q) out->XKv43[k * 9 + q] = static_cast<float>(g.Kv43[q]);
+    };
+    auto record = [&](const PieceQueue::Piece &p, void *base) {
+        const int64_t k = p.record;
+        if (p.i0 == 0) scalars(k, p.t, static_cast<const PieceHead *>(base)->g);
         gw_cru_state_reduced_t c;
         c.CaSS = out->CaSS ? out->CaSS + k * n * 4 : nullptr;
         c.CaJSR = out->CaJSR ? out->CaJSR + k * n : nullptr;
@@ -3907,10 +4176,10 @@ int gw_run_reduced(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, 
         c.LCC_inactivation = out->LCC_inactivation ? out->LCC_inactivation + k * n * 4 : nullptr;
         c.ClCh = out->ClCh ? out->ClCh + k * n * 4 : nullptr;
         c.RyR = out->RyR ? out->RyR + k * n * 4 : nullptr;
-        return gw_batch_get_cru_state_reduced(B, 0, &c, err, errlen);
+        expand_reduced(base, p.i0, p.m, c);
     };
     return run_loop(ctx, p, n_cru, dt, num_steps, istim, record_every, g0, c0, seed, prng_id, precision,
-                    out ? out->num_records : 0, record, err, errlen);
+                    out ? out->num_records : 0, PIECE_REDUCED, record, err, errlen);
 }
 
 int gw_run_batch(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32_t precision, double dt, int64_t nsteps,

@@ -269,7 +269,7 @@ int gw_run(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt,
  * call hipMalloc, such as tight serving loops or harnesses that forbid it).
  * No counterpart in the reference. Same arguments, semantics and results as
  * gw_run, bit for bit, but the call allocates nothing on the device: the
- * cell's state, block partials, stimulus table and staging are carved from a
+ * cell's state, block partials and stimulus table are carved from a
  * static 64 MiB array that each GPU the library runs on holds until the
  * process ends (a 12,500-CRU cell fits with a stimulus table of up to about
  * 7.5 million steps; a larger run is refused with GW_E_INVALID_ARG). Every
