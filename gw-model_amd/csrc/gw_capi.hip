@@ -1637,6 +1637,7 @@ __device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t 
     __syncthreads();
     const double dt = a.dt;
     const double rRyR = C.sp.rRyR;
+    const bool plain = load_scalar(&C.plain) != 0;
     const int64_t stop = D.stop_step;
     const bool run1 = nss > 1 && m + 1 < stop;
     const int w1 = bi.n;   // CRUs of the range
@@ -1657,7 +1658,7 @@ __device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t 
         Lane64Try X;
         bool ev = false;
         if (have) {
-            lane64_try<PRNG>(S, X, sp, P.K[sidx], P.K[sidx].lcc, dt);
+            lane64_try<PRNG>(S, X, sp, P.K[sidx], P.K[sidx].lcc, dt, plain);
             ev = !X.last;
         }
         const uint64_t m_ev = __ballot(ev);
@@ -3193,6 +3194,7 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
         C.p = d.params;
         cell_consts_init(C.c, C.p, d.n_cru);
         ssa_params_init(C.sp, C.p, C.c);
+        C.plain = ssa_params_plain(C.sp);
         ssa_params_f32(C.spf, C.sp);
         C.proto = d.protocol;
         C.seed = d.seed;

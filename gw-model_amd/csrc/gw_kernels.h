@@ -46,6 +46,7 @@ struct DevCell {
     uint64_t seed;
     int32_t n_cru;
     int32_t nblk[kNumShapes];  // SSA blocks of this cell, per launch shape
+    int32_t plain;         // its SSA's constants allow plain quotients (ssa_params_plain)
 };
 
 // Dynamic per-cell state, advanced by the cell's close block of each step.

@@ -18,6 +18,23 @@ GW_HD uint64_t bits_of(double d) { return static_cast<uint64_t>(__builtin_bit_ca
 GW_HD double double_of(uint64_t u) { return __builtin_bit_cast(double, u); }
 GW_HD uint64_t rotl64(uint64_t x, int s) { return (x << s) | (x >> (64 - s)); }
 
+// a / b where |a| (not zero) and |b| lie within 2^+-310: there the device's
+// division scales neither operand and has nothing to fix up, so what is left
+// of it are these operations, and the bits are the same. 8 instructions
+// instead of 11, without the three that use the vector condition code.
+GW_HD double quot_plain(double a, double b)
+{
+#if defined(__HIP_DEVICE_COMPILE__)
+    double y = __builtin_amdgcn_rcp(b);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    y = __builtin_fma(y, __builtin_fma(-b, y, 1.0), y);
+    const double q = a * y;
+    return __builtin_fma(__builtin_fma(-b, q, a), y, q);
+#else
+    return a / b;
+#endif
+}
+
 // ---------------------------------------------------------------------------
 // exp: Cody-Waite reduction x = k ln2 + r, |r| <= ln2/2, degree-13 Taylor
 // polynomial of e^r in Horner form with fused multiply-adds, scaling by 2^k.
@@ -66,7 +83,7 @@ GW_HD double log_em(int e, uint64_t frac)
     m = up ? m * 0.5 : m;
     e += up ? 1 : 0;
     const double f = m - 1.0;
-    const double s = f / (2.0 + f);
+    const double s = quot_plain(f, 2.0 + f);   // 0, or |f| in [2^-53, 0.42]
     const double z = s * s;
     double R = 0x1.47ae147ae147bp-5;
     R = __builtin_fma(R, z, 0x1.642c8590b2164p-5);

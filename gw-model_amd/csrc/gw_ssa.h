@@ -92,6 +92,17 @@ GW_HD void ssa_params_init(SsaParams &s, const gw_params_t &p, const CellConsts 
     s.k45k34 = p.k45 * p.k34; s.k32k43 = p.k32 * p.k43; s.k65k52 = p.k65 * p.k52; s.k65k54 = p.k65 * p.k54;
 }
 
+// Whether the numerators and denominators of the SSA's quotients (beta_ss,
+// beta_jsr, the lumped RyR pairs) lie within what quot_plain asks for while the
+// concentrations lie in [0, 2^100): every constant of them in [2^-100, 2^100].
+GW_HD int ssa_params_plain(const SsaParams &s)
+{
+    const double v[] = {s.KBSR, s.KBSL, s.KCSQN, s.BSR_const, s.BSL_const, s.CSQN_const, s.k34, s.k43, s.k56, s.k65};
+    int ok = 1;
+    for (double x : v) ok &= x >= 0x1p-100 && x <= 0x1p100;
+    return ok;
+}
+
 GW_HD void ssa_params_f32(SsaParamsF &f, const SsaParams &s)
 {
     const double *src = &s.rRyR;
@@ -118,8 +129,18 @@ __device__ __forceinline__ T load_scalar(const T *p)
 // Local arithmetic of the SSA. FP64: IEEE division and the shared log, bit-exact
 // with the oracle. FP32 (the FP32-local variant): one hardware reciprocal
 // (v_rcp_f32, 1 ulp) times the numerator, and the hardware log2 (v_log_f32).
-__device__ __forceinline__ double ldiv(double a, double b) { return a / b; }
+// PLAIN: the operands are known to need no scaling (quot_plain).
+template <bool PLAIN = false>
+__device__ __forceinline__ double ldiv(double a, double b) { return PLAIN ? quot_plain(a, b) : a / b; }
+template <bool PLAIN = false>
 __device__ __forceinline__ float ldiv(float a, float b) { return a * __builtin_amdgcn_rcpf(b); }
+
+// A concentration in [0, 2^100), by its high word; with plain parameters the
+// denominators formed from such ones lie within 2^+-302.
+constexpr uint32_t kPlainHigh = (1023u + 100u) << 20;
+__device__ __forceinline__ uint32_t high_word(double x) { return static_cast<uint32_t>(bits_of(x) >> 32); }
+// A sum of rates within 2^+-250.
+__device__ __forceinline__ bool plain_total(double x) { return high_word(x) - (773u << 20) < (500u << 20); }
 __device__ __forceinline__ double lneglog(double u) { return -gw::log_u01(u); }
 __device__ __forceinline__ float lneglog(float u) { return -(__builtin_amdgcn_logf(u) * 0.693147182f); }
 __device__ __forceinline__ float sq(float x) { return x * x; }
@@ -127,22 +148,22 @@ __device__ __forceinline__ float sq(float x) { return x * x; }
 // Rapid-buffering factors of update_CaSS (SSA.tpp:90) and update_CaJSR
 // (SSA.hpp:69). FP64: the reference's expressions. FP32-local: the same
 // fractions over one denominator, one reciprocal each instead of three and two.
-template <class R>
+template <bool PLAIN = false, class R>
 __device__ __forceinline__ R beta_ss(const SsaParamsT<R> &P, R ca)
 {
     if constexpr (sizeof(R) == 8) {
-        return ldiv(R(1), 1 + ldiv(P.BSR_const, sq(P.KBSR + ca)) + ldiv(P.BSL_const, sq(P.KBSL + ca)));
+        return ldiv<PLAIN>(R(1), 1 + ldiv<PLAIN>(P.BSR_const, sq(P.KBSR + ca)) + ldiv<PLAIN>(P.BSL_const, sq(P.KBSL + ca)));
     } else {
 #pragma clang fp contract(fast)
         const R x2 = sq(P.KBSR + ca), y2 = sq(P.KBSL + ca), p = x2 * y2;
         return ldiv(p, p + P.BSR_const * y2 + P.BSL_const * x2);
     }
 }
-template <class R>
+template <bool PLAIN = false, class R>
 __device__ __forceinline__ R beta_jsr(const SsaParamsT<R> &P, R jsr)
 {
     if constexpr (sizeof(R) == 8) {
-        return ldiv(R(1), 1 + ldiv(P.CSQN_const, sq(P.KCSQN + jsr)));
+        return ldiv<PLAIN>(R(1), 1 + ldiv<PLAIN>(P.CSQN_const, sq(P.KCSQN + jsr)));
     } else {
 #pragma clang fp contract(fast)
         const R x2 = sq(P.KCSQN + jsr);
@@ -152,7 +173,7 @@ __device__ __forceinline__ R beta_jsr(const SsaParamsT<R> &P, R jsr)
 
 // The 12 RyR propensities of one subunit (update_RyR_rates, GW_utils.tpp:222-255),
 // visited in storage order; `f(k, r)` receives each rate.
-template <class R, class F>
+template <bool PLAIN = false, class R, class F>
 __device__ __forceinline__ void ryr_rates(const SsaParamsT<R> &P, uint64_t w, R ca, F &&f)
 {
     const R C2 = ca * ca;
@@ -163,7 +184,7 @@ __device__ __forceinline__ void ryr_rates(const SsaParamsT<R> &P, uint64_t w, R 
     const R a3 = static_cast<R>(n3), a4 = static_cast<R>(n4), a5 = static_cast<R>(n5);
     R r3 = a3 * P.k34 * C2, r4 = a4 * P.k45, r7 = a3 * P.k32, r8 = a4 * P.k43;
     if (hi34) {
-        const R tau34 = ldiv(R(1), P.k34 * C2 + P.k43);
+        const R tau34 = ldiv<PLAIN>(R(1), P.k34 * C2 + P.k43);
         const R a = static_cast<R>(n3 + n4);
         r3 = R(0);
         r4 = a * P.k45 * P.k34 * C2 * tau34;
@@ -172,7 +193,7 @@ __device__ __forceinline__ void ryr_rates(const SsaParamsT<R> &P, uint64_t w, R 
     }
     R r5, r9, r10, r11;
     if (hi56) {
-        const R eq56 = ldiv(P.k65, P.k56 * C2 + P.k65);
+        const R eq56 = ldiv<PLAIN>(P.k65, P.k56 * C2 + P.k65);
         const R a = static_cast<R>(n5 + n6);
         r5 = R(0);
         r9 = a * P.k52 * eq56;
@@ -203,14 +224,14 @@ __device__ __forceinline__ void ryr_rates(const SsaParamsT<R> &P, uint64_t w, R 
 // needs. FP32-local: the same sum with the 12 RyR rates of ryr_rates gathered
 // by count (each lumped pair's two rates in one closed form), about half the
 // instructions; the event choice still walks the individual rates (ryr_pick).
-template <class R, class KT>
+template <bool PLAIN = false, class R, class KT>
 __device__ __forceinline__ R subunit_total(const SsaParamsT<R> &P, const KT &K, const LccTableT<R> &T, uint64_t w, R ca)
 {
     const int L = sub_lcc(w);
     R s = T.P[L] + T.Q[L] * ca;
     s += sub_y(w) ? K.inact1 : K.inact0;
     if constexpr (sizeof(R) == 8) {
-        ryr_rates(P, w, ca, [&](int, R r) { s += r; });
+        ryr_rates<PLAIN>(P, w, ca, [&](int, R r) { s += r; });
         s += sub_cl(w) ? P.kbClCh : P.kfClCh * ca;
         return s;
     } else {
@@ -974,18 +995,24 @@ __device__ __forceinline__ void lane64_begin(Lane64State &S, double rRyR)
     S.iters = 0;
 }
 
-template <int PRNG>
-__device__ __forceinline__ void lane64_try(const Lane64State &S, Lane64Try &X, const SsaParams &P, const StepConsts &K,
+// The waiting time's quotient; a draw of zero has an infinite logarithm.
+__device__ __forceinline__ double plain_quotient(double neglog, double total)
+{
+    return __ballot(!plain_total(total) || neglog > 0x1p10) == 0 ? quot_plain(neglog, total) : neglog / total;
+}
+
+template <int PRNG, bool PLAIN>
+__device__ __forceinline__ void lane64_try_form(const Lane64State &S, Lane64Try &X, const SsaParams &P, const StepConsts &K,
                                            const LccTable &T, double dt)
 {
     const Lane64Consts k{K.Cai, K.CaNSR, K.inact0, K.inact1};   // read once: chosen where they lie, each choice is a branch
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        X.s[j] = subunit_total(P, k, T, S.w[j], S.ca[j]);
+        X.s[j] = subunit_total<PLAIN>(P, k, T, S.w[j], S.ca[j]);
         asm volatile("" : "+v"(X.s[j]));   // one subunit after another: interleaved, they need twice the registers
     }
     X.total = X.s[0] + X.s[1] + X.s[2] + X.s[3];
-    X.jump = lneglog(u01(rng_output<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3))) / X.total;
+    X.jump = plain_quotient(lneglog(u01(rng_output<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3))), X.total);
     X.last = !(S.t + X.jump < dt);
     X.h = X.last ? dt - S.t : X.jump;
     X.split = 0;
@@ -995,7 +1022,7 @@ __device__ __forceinline__ void lane64_try(const Lane64State &S, Lane64Try &X, c
         const double old = S.ca[j];
         const double Jiss = P.riss * (S.ca[(j + 1) & 3] + S.ca[(j + 3) & 3] - 2 * old);
         Jx[j] = P.rxfer * (old - k.Cai);
-        const double d = X.h * (S.jl[j] + S.Jrel[j] - Jx[j] + Jiss) * beta_ss(P, old);
+        const double d = X.h * (S.jl[j] + S.Jrel[j] - Jx[j] + Jiss) * beta_ss<PLAIN>(P, old);
         X.ca[j] = old + d;
         asm volatile("" : "+v"(X.ca[j]));
         X.split |= split_mask<double>(old, X.ca[j]) << (2 * j);
@@ -1004,7 +1031,21 @@ __device__ __forceinline__ void lane64_try(const Lane64State &S, Lane64Try &X, c
     // update_CaJSR (SSA.hpp:67-71)
     X.Jtr = P.rtr * (k.CaNSR - S.q.jsr);
     const double Jsum = S.Jrel[0] + S.Jrel[1] + S.Jrel[2] + S.Jrel[3];
-    X.jsr = S.q.jsr + X.h * beta_jsr(P, S.q.jsr) * (X.Jtr - P.VSS_VJSR * Jsum);
+    X.jsr = S.q.jsr + X.h * beta_jsr<PLAIN>(P, S.q.jsr) * (X.Jtr - P.VSS_VJSR * Jsum);
+}
+
+// Plain quotients where all lanes' concentrations allow it: 60 instructions less
+// of an iteration's 1,165 (12.8 M CRUs 479 and 463 us per step; the quads, whose
+// waves have the vector unit for themselves less of the time, lose 2% by the
+// choice and divide in full).
+template <int PRNG>
+__device__ __forceinline__ void lane64_try(const Lane64State &S, Lane64Try &X, const SsaParams &P, const StepConsts &K,
+                                           const LccTable &T, double dt, bool plain_cell)
+{
+    const uint32_t hi = max(max(max(high_word(S.ca[0]), high_word(S.ca[1])), max(high_word(S.ca[2]), high_word(S.ca[3]))),
+                            high_word(S.q.jsr));
+    if (plain_cell && __ballot(hi >= kPlainHigh) == 0) lane64_try_form<PRNG, true>(S, X, P, K, T, dt);
+    else lane64_try_form<PRNG, false>(S, X, P, K, T, dt);
 }
 
 // old: the concentrations the iteration started from; w_pre: the words before the re-splits.
