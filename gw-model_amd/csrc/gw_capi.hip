@@ -2298,15 +2298,15 @@ struct LaunchCfg {
 };
 constexpr int kNumConfigs = GW_LAUNCH_CONFIGS;
 constexpr int kConfigDefault = 2;
-constexpr int kLane64 = kNumConfigs;   // the FP64 one-lane kernels of 4 and 8 CRUs per lane, which run_config chooses
-constexpr LaunchCfg kConfigs[kNumConfigs + 2] = {
+constexpr int kLane64 = kNumConfigs;   // the FP64 one-lane kernels of 2, 4 and 8 CRUs per lane, which run_config chooses
+constexpr LaunchCfg kConfigs[kNumConfigs + 3] = {
     {4, 64, 1},  {4, 128, 1}, {4, 256, 1}, {4, 512, 1},                 // quads: 16..128 CRUs per block
     {1, 64, 1},  {1, 128, 1}, {1, 256, 1},                               // one lane per CRU
     {1, 64, 2},  {1, 128, 2}, {1, 256, 2},                               // two CRUs per lane, refilled
     {1, 64, 4},  {1, 128, 4}, {1, 256, 4},                               // four
     {1, 64, 8},  {1, 128, 8}, {1, 256, 8},                               // eight (up to 2048 CRUs per block)
     {4, 64, 2},  {4, 64, 4},  {4, 128, 4}, {4, 256, 4},                  // quads refilled from 2 or 4 CRUs each
-    {1, 64, 4},  {1, 64, 8}};                                            // FP64, one lane per CRU
+    {1, 64, 2},  {1, 64, 4},  {1, 64, 8}};                               // FP64, one lane per CRU
 constexpr int config_shape(int c)
 {
     return shape_of_crus(kConfigs[c].threads / kConfigs[c].lanes * kConfigs[c].cpl);
@@ -2425,8 +2425,9 @@ void launch_k_step(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent_t e0,
         if (kConfigs[B->run_cfg].lanes == 1) {
             const unsigned grid = step_grid(B, ssa_step, nclose);
             switch (B->run_cfg) {
-            case kLane64: dispatch(k_step_lane64<PRNG, 4>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
-            case kLane64 + 1: dispatch(k_step_lane64<PRNG, 8>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
+            case kLane64: dispatch(k_step_lane64<PRNG, 2>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
+            case kLane64 + 1: dispatch(k_step_lane64<PRNG, 4>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
+            case kLane64 + 2: dispatch(k_step_lane64<PRNG, 8>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 4: dispatch(k_step_lane<PRNG, 64, 1>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 5: dispatch(k_step_lane<PRNG, 128, 1>, grid, 128, B, e0, e1, ssa_step, nclose, base); break;
             case 6: dispatch(k_step_lane<PRNG, 256, 1>, grid, 256, B, e0, e1, ssa_step, nclose, base); break;
@@ -2568,11 +2569,15 @@ bool use_persist(gw_batch *B)
 // cells of 200 CRUs 11.3 and 13.5. (128 and 512 lie between or behind.)
 //
 // Large FP64 batches run one lane per CRU. In us per step early in an action
-// potential (4 x 64 quads; one lane, 4 and 8 CRUs per lane): 300,000 CRUs
-// 29.9, 38.7, 41.5; 600,000 51.1, 50.0, 55.4; 800,000 65.3, 55.3, 57.6; 2.0 M
-// 173, 97.9, 97.9; 5.0 M 457, 218, 206; 12.8 M 1,182, 526, 479. Below, a batch
-// is a few rounds of quads and one round of lanes, whose trips are longer.
-constexpr int64_t kLane64Crus = 640000, kLane64Crus8 = 2500000;
+// potential, the lanes with two steps per launch (4 x 64 quads; one lane with
+// 2, 4 and 8 CRUs per lane; - not run): 300,000 CRUs 29.1, 31.2, 36.0, -;
+// 350,000 32.3, 31.2, -, -; 390,000 35.0, 31.7, -, -; 525,000 44.4, 39.9, 42.7, -; 800,000
+// 65.3, 51.2, 53.2, -; 900,000 70.5, 54.1, 54.9, -; 1.0 M 77.4, 58.3, 55.5,
+// -; 2.5 M -, 125, 116, -; 12.8 M 1,182, -, 526, 463. Below, a batch is a few
+// rounds of quads and one round of lanes, whose trips are longer. Cells of
+// fewer CRUs than a wave has lanes stay with the quads (20,000 cells of 33
+// CRUs 300 and 317 us, of 66 CRUs 178 and 173).
+constexpr int64_t kLane64Crus = 340000, kLane64Crus4 = 950000, kLane64Crus8 = 2500000;
 constexpr int64_t kQuad64Crus = 180000, kQuad64CrusF32 = 350000;
 constexpr int kQuad64Cells = 256;
 
@@ -2580,7 +2585,8 @@ int run_config(gw_batch *B)
 {
     const bool f32 = B->precision == GW_PREC_FP32_LOCAL;
     if (B->prng != GW_PRNG_XOSHIRO256SS || B->frozen || (!f32 && B->digest) || use_persist(B)) return B->cfg;
-    if (!f32 && B->ncrus >= kLane64Crus) return B->ncrus < kLane64Crus8 ? kLane64 : kLane64 + 1;
+    if (!f32 && B->ncrus >= kLane64Crus && B->ncrus >= int64_t(kWave) * B->ncells)
+        return kLane64 + (B->ncrus < kLane64Crus4 ? 0 : B->ncrus < kLane64Crus8 ? 1 : 2);
     const LaunchCfg &L = kConfigs[B->cfg];
     if (L.lanes != 4 || L.cpl != 1) return B->cfg;
     const bool narrow = f32 ? B->ncrus >= kQuad64CrusF32 : B->ncrus >= kQuad64Crus || B->ncells >= kQuad64Cells;
@@ -2621,16 +2627,17 @@ bool pair_capable(gw_batch *B)
 
 // Two steps per launch when asked for (2), or automatically (0) for batches of
 // 450,000 CRUs and more: there the state's HBM traffic is worth more than the
-// separate close kernel costs, about 17 us per two steps. FP32-local, one and two steps
+// separate close kernel costs, 10 us per two steps. FP32-local, one and two steps
 // per launch, in us per step: 400,000 CRUs 25.2 and 25.0 (four CRUs per lane), 24.7 and 24.0 (one);
 // 600,000 31.5 and 27.9, 30.8 and 28.5; 200,000 20.7 and 21.6, 15.1 and 17.3.
-// FP64 batches on the one-lane kernels are all larger (650,000: 50.2 and 46.7).
+// The FP64 one-lane kernels always run two: 390,000 CRUs 33.6 and 31.7; 450,000
+// 41.0 and 37.5; 600,000 47.4 and 43.4.
 constexpr int64_t kPairCrus = 450000;
 
 bool use_pair(gw_batch *B)
 {
     if (B->steps_per_launch == 1 || !pair_capable(B)) return false;
-    return B->steps_per_launch == 2 || B->ncrus >= kPairCrus;
+    return B->steps_per_launch == 2 || B->ncrus >= kPairCrus || run_config(B) >= kLane64;
 }
 
 // One launch of the two-step kernel: SSA(m .. m + nss - 1); with e0/e1 the
@@ -2649,8 +2656,9 @@ void launch_pair(gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0 = nullptr, h
 {
     constexpr int P = GW_PRNG_XOSHIRO256SS;
     switch (B->run_cfg) {
-    case kLane64: dispatch_pair(k_step2_lane64<P, 4>, B, m, nss, e0, e1); return;
-    case kLane64 + 1: dispatch_pair(k_step2_lane64<P, 8>, B, m, nss, e0, e1); return;
+    case kLane64: dispatch_pair(k_step2_lane64<P, 2>, B, m, nss, e0, e1); return;
+    case kLane64 + 1: dispatch_pair(k_step2_lane64<P, 4>, B, m, nss, e0, e1); return;
+    case kLane64 + 2: dispatch_pair(k_step2_lane64<P, 8>, B, m, nss, e0, e1); return;
     default: break;
     }
     switch (kConfigs[B->run_cfg].cpl) {

@@ -376,8 +376,9 @@ int gw_batch_get_persistent(gw_batch *b, int32_t *active);
  * CRU two steps with its state held in registers, so the CRU state crosses HBM once per
  * two steps; the two closes the launch's SSA steps need run just before it, in a kernel
  * of their own. Other shapes, FP64, frozen globals, replayed graphs and the persistent
- * kernel keep one step per launch; FP64 batches of 640,000 CRUs and more (xoshiro256**,
- * no digests) run two with a request of 0 or 2, whatever their shape. With one CRU per lane the results are bit-identical
+ * kernel keep one step per launch; FP64 batches of 340,000 CRUs and more, 64 per cell and
+ * more on average (xoshiro256**, no digests), run two with a request of 0 or 2, whatever
+ * their shape. With one CRU per lane the results are bit-identical
  * to one step per launch; with refilled lanes they are deterministic, and the rounding
  * of the FP64 flux sums can differ (their order follows which CRUs each lane ran).
  * Automatic: two steps per launch for batches of 450,000 CRUs and more (the state's

@@ -1,5 +1,5 @@
-"""FP64 batches large enough for the one-lane kernels (one lane per CRU, 4 or 8
-CRUs per lane, one or two Euler steps per launch, events of a wave applied
+"""FP64 batches large enough for the one-lane kernels (one lane per CRU, 2, 4
+or 8 CRUs per lane, one or two Euler steps per launch, events of a wave applied
 together): cells whose sizes lie at the edges of their tiles, in a batch with a
 cell large enough to choose those kernels, against the same cells in a batch of
 their own, which runs the quads. Every bit of both is the same."""
@@ -50,7 +50,8 @@ def _same(a, b, observables=True):
         assert not observables or a.obs()[c] == b.obs()[c], c
 
 
-@pytest.mark.parametrize("filler", [(640_000,), (1 << 20, 1 << 20, 500_000)], ids=["4 per lane", "8 per lane"])
+@pytest.mark.parametrize("filler", [(640_000,), (1 << 20,), (1 << 20, 1 << 20, 500_000)],
+                         ids=["2 per lane", "4 per lane", "8 per lane"])
 @pytest.mark.parametrize("steps_per_launch", [0, 1])
 def test_one_lane_kernels_match_the_quads(gwcapi, gpu_ctx, filler, steps_per_launch):
     a, b = _open(gwcapi, gpu_ctx, filler), _open(gwcapi, gpu_ctx, ())
@@ -111,3 +112,12 @@ def test_quotients_that_need_scaling_match_the_quads(gwcapi, gpu_ctx, ca, consta
         return b
 
     _same(start((640_000,)), start(()), observables=ca < 1.0)   # a cell that fails has NaN among its observables
+
+
+@pytest.mark.parametrize("size,steps_per_launch", [(60, 1), (64, 2)])
+def test_cells_smaller_than_a_wave_stay_with_the_quads(gwcapi, gpu_ctx, size, steps_per_launch):
+    b = gwcapi.Batch(gpu_ctx, [gwcapi.make_cell(size, c) for c in range(6000)])
+    b.set_mode(frozen=False, digest=False)
+    assert b.steps_per_launch() == steps_per_launch
+    b.step(5)
+    b.close()
