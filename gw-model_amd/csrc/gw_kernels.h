@@ -112,7 +112,11 @@ struct KArgs {
     int32_t prng;
     int32_t precision;   // GW_PREC_FP64 or GW_PREC_FP32_LOCAL
     int32_t shape;       // current SSA launch shape (0..3)
-    int32_t _pad;
+    // cells of one size: their CRUs, the blocks of each in the current shape, its reciprocal
+    // (2^32 / uni_nblk, rounded up) and their slots; uni_n is 0 where the cells differ
+    int32_t uni_n;
+    int32_t uni_nblk, uni_slots;
+    uint64_t uni_magic;
     CellSync *sync;      // [ncells] (persistent step kernel)
     int32_t *timeout;    // set when a bounded wait of the persistent kernel expires
     int64_t spin_limit;  // polls before a wait of the persistent kernel gives up
