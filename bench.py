@@ -25,8 +25,8 @@ with the reference's algorithm).
                step or two), each divided by the kernel's average duration (the
                timed region between its two HIP events over its SSA launches,
                which run back to back); against the vector peak of the form's
-               precision and HBM. On the default workload the FP32-local form
-               runs two SSA steps per launch (--steps-per-launch).
+               precision and HBM. On the default workload both forms run two
+               SSA steps per launch (--steps-per-launch).
                `traffic` is the measured HBM bytes per launch from
                profiles/k_ssa_traffic.txt (rocprofv3 FETCH_SIZE and WRITE_SIZE,
                calibrated on a copy of known size) when present.
@@ -37,7 +37,8 @@ with the reference's algorithm).
                smaller cell over the same window beside it (per-core
                throughput), and the host CPU model
   launch       the SSA launch shape: by default the autotuner's choice on
-               this batch (1x64x4 FP32-local, 4x64 FP64), fixed so that a
+               this batch (1x64x4 FP32-local, 4x64 FP64, which a batch of
+               this size runs one lane per CRU), fixed so that a
                profile of the same command sees the same kernels;
                --autotune STEPS runs the tuner instead
 """

@@ -388,8 +388,9 @@ class Batch:
         _call(self.L.gw_batch_set_persistent, self.h, int(mode))
 
     def set_steps_per_launch(self, steps: int):
-        """SSA steps per plain launch of the FP32-local one-lane shapes of 64 threads: 0 automatic (the
-        default: two for batches of 450,000 CRUs and more), 1 or 2."""
+        """SSA steps per plain launch, 1, 2 or 0 (automatic, the default), where a launch can run two: the
+        FP32-local one-lane shapes of 64 threads (automatic: two from 450,000 CRUs on) and FP64 batches of
+        340,000 CRUs and more."""
         _call(self.L.gw_batch_set_steps_per_launch, self.h, int(steps))
 
     def steps_per_launch(self) -> int:

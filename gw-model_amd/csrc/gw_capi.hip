@@ -5,11 +5,12 @@
 // stored [slot][4] (CaSS, JLCC, the packed subunit word holding the six RyR
 // counts, LCC state, y gate and ClCh); CaJSR is [slot]; the engine state is
 // [slot][4] words and the replay digest [slot][2]. A CRU is advanced by a quad
-// of lanes (lane j owns subunit j), so one 256-thread block holds 64 CRUs; each
-// cell's slots are padded to whole blocks, so a block belongs to one cell.
+// of lanes (lane j owns subunit j) or, in FP32-local shapes that ask for it and
+// in large FP64 batches, by one lane; a block's CRUs belong to one cell.
 //
 // One Euler step (GW_model::euler_step, src/includes/GW.tpp:236-272) is one
-// launch of k_step. Its SSA blocks advance every CRU through SSA(dt) with the
+// launch of k_step (or half a launch, where CRUs stay in registers over two
+// steps). Its SSA blocks advance every CRU through SSA(dt) with the
 // cell's frozen constants and reduce the flux sums exactly (128-bit fixed
 // point) into one partial per block. Its first blocks, one per cell, close
 // the previous step at the same time: they sum that step's partials, apply
@@ -329,7 +330,18 @@ __global__ __launch_bounds__(kBlock) void k_init_crus(KArgs a, const BlockInfo *
     }
 }
 
-// Step-0 preparation of every cell (one block per cell): the flux sums the
+// x added n times: the fixed-point term times n.
+__device__ __forceinline__ int fx_add_times(Fx &acc, double x, uint64_t n)
+{
+    Fx one;
+    fx_zero(one);
+    const int err = fx_add(one, x);
+    fx_add_raw(acc, one.lo * n, one.hi * n + __umul64hi(one.lo, n));
+    return err;
+}
+
+// Step-0 preparation of every cell (one block per cell; 36 cells of 12,500 CRUs
+// 57 us, 80 with one CRU's reads in flight per lane): the flux sums the
 // reference's first euler_step reads -- JLCC of the given state, Jxfer and Jtr
 // of the constructor's default CRU state and default globals (GW.hpp:104-113),
 // ClCh of the given state -- then derivatives and SSA constants.
@@ -344,18 +356,31 @@ __global__ void k_init_cells(KArgs a)
     const double X = C.p.rxfer * (1.45370e-4 - 1.45273e-4);
     const double X4 = X + X + X + X;
     const double Y = C.p.rtr * (0.908882 - 0.908408);
-    for (int64_t i = threadIdx.x; i < C.n_cru; i += kBlock) {
-        const int64_t slot = C.slot0 + i;
-        double jl[4];
-        for (int j = 0; j < 4; ++j) jl[j] = ld_jlcc(a, slot * 4 + j);
-        mine.err |= fx_add(mine.jlcc, jl[0] + jl[1] + jl[2] + jl[3]);
-        mine.err |= fx_add(mine.jxfer, X4);
-        mine.err |= fx_add(mine.jtr, Y);
-        for (int j = 0; j < 4; ++j) {
-            const uint64_t w = a.sub[slot * 4 + j];
-            mine.clch += sub_cl(w);
-            mine.open += ryr_get(w, 2) + ryr_get(w, 3);
+    constexpr int kAhead = 4;   // CRUs whose reads are in flight per lane
+    uint64_t count = 0;
+    for (int64_t i0 = threadIdx.x; i0 < C.n_cru; i0 += kAhead * kBlock) {
+        double jl[kAhead][4];
+        uint64_t w[kAhead][4];
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            const int64_t slot = C.slot0 + min(i0 + u * kBlock, static_cast<int64_t>(C.n_cru) - 1);
+            for (int j = 0; j < 4; ++j) jl[u][j] = ld_jlcc(a, slot * 4 + j);
+            for (int j = 0; j < 4; ++j) w[u][j] = a.sub[slot * 4 + j];
         }
+#pragma unroll
+        for (int u = 0; u < kAhead; ++u) {
+            if (i0 + u * kBlock >= C.n_cru) break;
+            ++count;
+            mine.err |= fx_add(mine.jlcc, jl[u][0] + jl[u][1] + jl[u][2] + jl[u][3]);
+            for (int j = 0; j < 4; ++j) {
+                mine.clch += sub_cl(w[u][j]);
+                mine.open += ryr_get(w[u][j], 2) + ryr_get(w[u][j], 3);
+            }
+        }
+    }
+    if (count > 0) {   // as often as the lane has CRUs
+        mine.err |= fx_add_times(mine.jxfer, X4, count);
+        mine.err |= fx_add_times(mine.jtr, Y, count);
     }
     block_reduce<kBlock>(red, mine);
     if (threadIdx.x == 0) {
@@ -387,10 +412,9 @@ __device__ __forceinline__ void load_lcc_table(const KT &K, TT &T)
 
 
 // SSA(dt) of `nsteps` steps (GW_model::SSA, src/includes/GW.tpp:214-234) for
-// the 64 CRUs of SSA block b, with the constants of step step0 (nsteps > 1
+// the CRUs of SSA block b, with the constants of step step0 (nsteps > 1
 // only in frozen-globals replay, where they do not change). The block's flux
-// partial of the last step goes to partials[step0 & 1][b]; only the quad
-// leaders contribute. R is the CRU-local arithmetic (double, or float for the
+// partial of the last step goes to partials[step0 & 1][b]. R is the CRU-local arithmetic (double, or float for the
 // FP32-local variant); CaSS and CaJSR are FP64 in both.
 template <class R> struct LocalState;
 template <> struct LocalState<double> {
@@ -504,8 +528,9 @@ __device__ __forceinline__ void ssa_block(const KArgs &a, int b, int64_t step0, 
 //               lane); role 2 observables and trace; role 3 the stores.
 // Each value is formed by the operations of the serial gd_finish and
 // step_consts, in their order, so the results are the same bits. Timed in one
-// cell of 12,500 CRUs: 26,500 cycles for the form that ran the sums as a
-// butterfly of 128-bit adds and the terms on single lanes.
+// cell of 12,500 CRUs: 11,700 cycles, where the form that ran the sums as a
+// butterfly of 128-bit adds and the terms on single lanes took 26,500. Issue
+// bounds it: a dependent FP64 operation takes the 4 cycles of its issue.
 // ---------------------------------------------------------------------------
 constexpr int kGd0 = 7;   // V, Nai, Ki, Cai, CaNSR, CaLTRPN, CaHTRPN: the globals gd_combine derives
 constexpr int kSumLanes = PW_N / 2;   // lanes that read one partial, two words each
@@ -852,8 +877,8 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
 // one launch earlier) and writes the other partials buffer. ssa_step < 0
 // launches the closes alone (the last close of a sequence).
 // Resident waves per SIMD the SSA kernels are compiled for: FP64 needs about
-// 128 VGPRs; the FP32-local SSA fits 80 (the single-lane close path then
-// spills to scratch, which it can afford).
+// 128 VGPRs; the FP32-local SSA fits 80, where the close in the first blocks
+// spills up to 36 bytes.
 template <class R> constexpr int kWavesPerSimd = sizeof(R) == 4 ? 6 : 4;
 
 // ssa_step is relative to *base when base is given (replayed graphs of steps).
@@ -1521,7 +1546,9 @@ __global__ __launch_bounds__(BLOCK, CPT <= 2 ? 5 : 4) void k_step_lane2(KArgs a,
 
 // One or two (ncl) consecutive closes of every cell, one block of four waves per cell (the
 // two-steps-per-launch sequence), one wave for each of the close's roles. At
-// 4 waves per SIMD the blocks of 1,024 cells are resident at once.
+// 4 waves per SIMD the blocks of 1,024 cells are resident at once, and share the
+// issue of their compute units: two closes of 64 cells take 10.4 us, of 256
+// 12.2, of 512 19.5, of 1,024 33.
 __global__ __launch_bounds__(kBlock, 4) void k_close_cells(KArgs a, int32_t ncl)
 {
     __shared__ CloseLds<kBlock> sh;
@@ -1546,7 +1573,7 @@ __global__ __launch_bounds__(kBlock, 4) void k_close_cells(KArgs a, int32_t ncl)
 // otherwise), until event_batch lanes of the wave hold an event, or no other
 // lane made progress, or no fresh CRU is left to keep the others busy; then
 // all of them commit at once. 12.8 M CRUs, 4 per lane: 552, 551, 542 and 543
-// us per step with batches of 1, 4, 8 and 16 events.
+// us per step with batches of 1, 4, 8 and 16 events (479 and then 463 since).
 //
 // Flux sums: a CRU's four outputs are split into three 43-bit limbs in FP64
 // arithmetic, truncated at 2^-80 like fx_add, and added as whole numbers into
@@ -1746,9 +1773,9 @@ __device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t 
 }
 
 // One step, the closes of the step before in the first blocks (as k_step).
-// 155 VGPRs: three waves per SIMD (at four, 23 spill and 12.8 M CRUs take 649
-// us per step against 542). Issue of vector instructions bounds them: 18.2 per
-// CRU and step, 80% of the time (the quads: 50.7, 87%).
+// 147 VGPRs: three waves per SIMD (at four, 23 spilled and 12.8 M CRUs took 649
+// us per step against 542 then). Issue of vector instructions bounds them: 17.2
+// per CRU and step, 78% of the time (the quads: 50.7, 87%).
 template <int PRNG, int CPT>
 __global__ __launch_bounds__(kWave, 3) void k_step_lane64(KArgs a, int64_t ssa_step, int32_t nclose, const int64_t *base)
 {

@@ -4,6 +4,10 @@ sampler on the host. Every field is the same."""
 import numpy as np
 import pytest
 
+from oracle.oracle import OracleModel
+
+from .test_gpu_parity import assert_globals_equal, assert_states_equal
+
 pytestmark = pytest.mark.gpu
 
 SIZES = (1, 3, 63, 64, 65, 255, 256, 257, 513, 1250)
@@ -17,4 +21,18 @@ def test_initial_state_matches_the_host_sampler(gwcapi, gpu_ctx, prng, precision
         want, got = gwcapi.rest_state(n, 70 + n, prng), b.get_cru_state(c)
         for k in want:
             assert np.array_equal(want[k], got[k]), (n, k)
+    b.close()
+
+
+@pytest.mark.parametrize("n", [1, 255, 256, 257, 1023, 1024, 1025, 2049])
+def test_first_steps_match_the_oracle(gwcapi, gpu_ctx, n):
+    """The sums the first steps start from, of cells at the edges of the block that forms them."""
+    b = gwcapi.Batch(gpu_ctx, [gwcapi.make_cell(n, 11)])
+    m = OracleModel(n, seed=11)
+    m.sample_rest_state()
+    for _ in range(3):
+        b.step(1)
+        assert m.step(1e-3, 0.0) == 0
+        assert_globals_equal(b.get_globals()[0], m.globals())
+    assert_states_equal(b.get_cru_state(0), m.state())
     b.close()
