@@ -3197,7 +3197,7 @@ int gw_batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, in
 
 namespace {
 
-constexpr size_t kArenaReserve = 208;   // bytes per CRU
+constexpr size_t kArenaReserve = 210;   // bytes per CRU
 
 // gw_batch_create, or with arena != null an allocation-free batch whose device
 // memory is carved from arena[0, arena_size); a stimulus table of table_cap
