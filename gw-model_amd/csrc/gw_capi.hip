@@ -2471,18 +2471,25 @@ void launch_k_step_shape(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent
     dispatch(k_step<PRNG, false, double, BLOCK>, grid, BLOCK, B, e0, e1, ssa_step, nclose, base);
 }
 
-// Shapes other than the default are built for xoshiro256** only (the engine
-// of the production path); shape_allowed() keeps the others off them.
+// Shapes that a caller can ask for beside the default are built for xoshiro256**
+// only (the engine of the production path; shape_allowed() keeps the others off
+// them), the ones that run_config chooses by itself for every engine.
 template <int PRNG>
 void launch_k_step(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent_t e0, hipEvent_t e1, const int64_t *base)
 {
+    if (B->run_cfg >= kLane64) {
+        const unsigned grid = step_grid(B, ssa_step, nclose);
+        switch (B->run_cfg) {
+        case kLane64: dispatch(k_step_lane64<PRNG, 2>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
+        case kLane64 + 1: dispatch(k_step_lane64<PRNG, 4>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
+        default: dispatch(k_step_lane64<PRNG, 8>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
+        }
+        return;
+    }
     if constexpr (PRNG == GW_PRNG_XOSHIRO256SS) {
         if (kConfigs[B->run_cfg].lanes == 1) {
             const unsigned grid = step_grid(B, ssa_step, nclose);
             switch (B->run_cfg) {
-            case kLane64: dispatch(k_step_lane64<PRNG, 2>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
-            case kLane64 + 1: dispatch(k_step_lane64<PRNG, 4>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
-            case kLane64 + 2: dispatch(k_step_lane64<PRNG, 8>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 4: dispatch(k_step_lane<PRNG, 64, 1>, grid, 64, B, e0, e1, ssa_step, nclose, base); break;
             case 5: dispatch(k_step_lane<PRNG, 128, 1>, grid, 128, B, e0, e1, ssa_step, nclose, base); break;
             case 6: dispatch(k_step_lane<PRNG, 256, 1>, grid, 256, B, e0, e1, ssa_step, nclose, base); break;
@@ -2508,10 +2515,10 @@ void launch_k_step(gw_batch *B, int64_t ssa_step, int32_t nclose, hipEvent_t e0,
             }
             return;
         }
-        if (B->shape == 0) {   // plain quads run with 64 threads or the default's 256 (run_config)
-            launch_k_step_shape<PRNG, 64>(B, ssa_step, nclose, e0, e1, base);
-            return;
-        }
+    }
+    if (B->shape == 0) {   // plain quads run with 64 threads or the default's 256 (run_config)
+        launch_k_step_shape<PRNG, 64>(B, ssa_step, nclose, e0, e1, base);
+        return;
     }
     launch_k_step_shape<PRNG, kBlock>(B, ssa_step, nclose, e0, e1, base);
 }
@@ -2639,7 +2646,7 @@ constexpr int kQuad64Cells = 256;
 int run_config(gw_batch *B)
 {
     const bool f32 = B->precision == GW_PREC_FP32_LOCAL;
-    if (B->prng != GW_PRNG_XOSHIRO256SS || B->frozen || (!f32 && B->digest) || use_persist(B)) return B->cfg;
+    if (B->frozen || (!f32 && B->digest) || use_persist(B)) return B->cfg;
     if (!f32 && B->ncrus >= kLane64Crus && B->ncrus >= int64_t(kWave) * B->ncells)
         return kLane64 + (B->ncrus < kLane64Crus4 ? 0 : B->ncrus < kLane64Crus8 ? 1 : 2);
     const LaunchCfg &L = kConfigs[B->cfg];
@@ -2668,7 +2675,7 @@ hipError_t launch_persist(gw_batch *B, int64_t step0, int64_t n)
 
 // Whether the batch's plain launches can run two SSA steps each: FP32-local
 // free-running steps on a one-lane shape of 64 threads (k_step_lane2;
-// xoshiro256**, no digests, as every one-lane shape), or FP64 steps that
+// xoshiro256**, as every shape a caller can ask for), or FP64 steps that
 // run_config gives to the one-lane kernels (k_step2_lane64); not persistent,
 // no replayed graphs.
 bool pair_capable(gw_batch *B)
@@ -2707,14 +2714,29 @@ void dispatch_pair(K kernel, gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0,
         hipLaunchKernelGGL(kernel, grid, block, 0, B->ctx->stream, B->a, m, nss);
 }
 
+template <int P>
+void launch_pair_lane64(gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0, hipEvent_t e1)
+{
+    switch (B->run_cfg) {
+    case kLane64: dispatch_pair(k_step2_lane64<P, 2>, B, m, nss, e0, e1); break;
+    case kLane64 + 1: dispatch_pair(k_step2_lane64<P, 4>, B, m, nss, e0, e1); break;
+    default: dispatch_pair(k_step2_lane64<P, 8>, B, m, nss, e0, e1); break;
+    }
+}
+
 void launch_pair(gw_batch *B, int64_t m, int32_t nss, hipEvent_t e0 = nullptr, hipEvent_t e1 = nullptr)
 {
     constexpr int P = GW_PRNG_XOSHIRO256SS;
-    switch (B->run_cfg) {
-    case kLane64: dispatch_pair(k_step2_lane64<P, 2>, B, m, nss, e0, e1); return;
-    case kLane64 + 1: dispatch_pair(k_step2_lane64<P, 4>, B, m, nss, e0, e1); return;
-    case kLane64 + 2: dispatch_pair(k_step2_lane64<P, 8>, B, m, nss, e0, e1); return;
-    default: break;
+    if (B->run_cfg >= kLane64) {
+        switch (B->prng) {
+        case 0: launch_pair_lane64<0>(B, m, nss, e0, e1); break;
+        case 1: launch_pair_lane64<1>(B, m, nss, e0, e1); break;
+        case 2: launch_pair_lane64<2>(B, m, nss, e0, e1); break;
+        case 3: launch_pair_lane64<3>(B, m, nss, e0, e1); break;
+        case 4: launch_pair_lane64<4>(B, m, nss, e0, e1); break;
+        default: launch_pair_lane64<5>(B, m, nss, e0, e1); break;
+        }
+        return;
     }
     switch (kConfigs[B->run_cfg].cpl) {
     case 1: dispatch_pair(k_step_lane2<P, 64, 1>, B, m, nss, e0, e1); break;

@@ -377,7 +377,7 @@ int gw_batch_get_persistent(gw_batch *b, int32_t *active);
  * two steps; the two closes the launch's SSA steps need run just before it, in a kernel
  * of their own. Other shapes, FP64, frozen globals, replayed graphs and the persistent
  * kernel keep one step per launch; FP64 batches of 340,000 CRUs and more, 64 per cell and
- * more on average (xoshiro256**, no digests), run two with a request of 0 or 2, whatever
+ * more on average (no digests), run two with a request of 0 or 2, whatever
  * their shape. With one CRU per lane the results are bit-identical
  * to one step per launch; with refilled lanes they are deterministic, and the rounding
  * of the FP64 flux sums can differ (their order follows which CRUs each lane ran).

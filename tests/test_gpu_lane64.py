@@ -30,10 +30,10 @@ def _state(n, seed):
             "ClCh": rng.integers(0, 2, (n, 4))}
 
 
-def _open(gwcapi, ctx, filler):
+def _open(gwcapi, ctx, filler, prng=0):
     g = gwcapi.default_globals()
     g.V, g.m, g.h, g.j = 10.0, 0.99, 1e-3, 0.1
-    b = gwcapi.Batch(ctx, _cells(gwcapi, filler), globals_=g)
+    b = gwcapi.Batch(ctx, _cells(gwcapi, filler), prng=prng, globals_=g)
     b.set_mode(frozen=False, digest=False)
     for c, n in enumerate(SIZES):
         b.set_cru_state(c, **_state(n, n))
@@ -121,3 +121,35 @@ def test_cells_smaller_than_a_wave_stay_with_the_quads(gwcapi, gpu_ctx, size, st
     assert b.steps_per_launch() == steps_per_launch
     b.step(5)
     b.close()
+
+
+@pytest.mark.parametrize("prng", range(1, 6))
+@pytest.mark.parametrize("filler", [(340_000,), (1 << 20,), (1 << 20, 1 << 20, 500_000)],
+                         ids=["2 per lane", "4 per lane", "8 per lane"])
+def test_one_lane_kernels_match_the_quads_with_every_engine(gwcapi, gpu_ctx, prng, filler):
+    a, b = _open(gwcapi, gpu_ctx, filler, prng), _open(gwcapi, gpu_ctx, (), prng)
+    assert a.steps_per_launch() == 2
+    for steps_per_launch, chunk in ((0, 21), (1, 20)):
+        a.set_steps_per_launch(steps_per_launch)
+        a.step(chunk)
+        b.step(chunk)
+        _same(a, b)
+    a.close()
+    b.close()
+
+
+@pytest.mark.parametrize("prng", range(1, 6))
+@pytest.mark.parametrize("precision,filler", [(0, 180_000), (1, 350_000)], ids=["fp64", "fp32_local"])
+def test_narrow_quads_match_the_default_with_every_engine(gwcapi, gpu_ctx, prng, precision, filler):
+    """The quads of large batches (64 threads) against those of small ones (256)."""
+    batches = []
+    for extra in ((filler,), ()):
+        b = gwcapi.Batch(gpu_ctx, _cells(gwcapi, extra), precision=precision, prng=prng)
+        b.set_mode(frozen=False, digest=False)
+        for c, n in enumerate(SIZES):
+            b.set_cru_state(c, **_state(n, n))
+        b.step(25)
+        batches.append(b)
+    _same(*batches)
+    for b in batches:
+        b.close()
