@@ -2639,6 +2639,15 @@ bool use_persist(gw_batch *B)
 // rounds of quads and one round of lanes, whose trips are longer. Cells of
 // fewer CRUs than a wave has lanes stay with the quads (20,000 cells of 33
 // CRUs 300 and 317 us, of 66 CRUs 178 and 173).
+//
+// FP32-local shapes of several CRUs per lane run one per lane, on as many
+// threads, below 300,000 CRUs: there all of them fit the wave slots at once, and
+// a wave's chain of CRUs is what a step waits for. In us per step with 4 and 1
+// per lane, 64 threads: 12,500 CRUs 17.2 and 10.0; 200 cells of 333 20.3 and
+// 12.3; 90,000 19.4 and 12.0; 200,000 20.7 and 14.9; 300,000 23.0 and 19.0;
+// 440,000 25.8 and 25.0; 3,000 cells of 140 60.4 and 62.5.
+constexpr int64_t kRefillCrus = 300000;
+constexpr int kLane1 = 4;   // one CRU per lane; the shapes after it repeat its 64, 128 and 256 threads
 constexpr int64_t kLane64Crus = 340000, kLane64Crus4 = 950000, kLane64Crus8 = 2500000;
 constexpr int64_t kQuad64Crus = 180000, kQuad64CrusF32 = 350000;
 constexpr int kQuad64Cells = 256;
@@ -2650,11 +2659,20 @@ int run_config(gw_batch *B)
     if (!f32 && B->ncrus >= kLane64Crus && B->ncrus >= int64_t(kWave) * B->ncells)
         return kLane64 + (B->ncrus < kLane64Crus4 ? 0 : B->ncrus < kLane64Crus8 ? 1 : 2);
     const LaunchCfg &L = kConfigs[B->cfg];
+    if (L.lanes == 1 && L.cpl > 1 && B->ncrus < kRefillCrus) return kLane1 + (B->cfg - kLane1) % 3;
     if (L.lanes != 4 || L.cpl != 1) return B->cfg;
     const bool narrow = f32 ? B->ncrus >= kQuad64CrusF32 : B->ncrus >= kQuad64Crus || B->ncells >= kQuad64Cells;
     return narrow ? 0 : kConfigDefault;
 }
 static_assert(kConfigs[0].lanes == 4 && kConfigs[0].threads == 64 && kConfigs[kConfigDefault].threads == kBlock, "the two quad shapes");
+constexpr bool refill_shapes_in_order()
+{
+    for (int c = kLane1; c < kLane1 + 12; ++c)
+        if (kConfigs[c].lanes != 1 || kConfigs[c].threads != 64 << (c - kLane1) % 3 || (kConfigs[c].cpl == 1) != (c < kLane1 + 3))
+            return false;
+    return true;
+}
+static_assert(refill_shapes_in_order(), "run_config's arithmetic on the one-lane shapes");
 
 // Steps step0 .. step0+n-1 in one cooperative launch of the persistent kernel
 // (which closes every step itself), after its counters are set for step0.
