@@ -428,9 +428,12 @@ int gw_batch_get_iterations(gw_batch *b, uint64_t *iters);
  * (64, 128 or 256 threads); 1 with 4 lanes, or 2 (64 threads) and 4 (64, 128
  * or 256 threads); each wave then owns 64 x crus_per_lane consecutive CRUs (16 x
  * with quads) and a lane or quad whose CRU has finished its step takes the next
- * one, so waves wait less on their slowest CRU; 0 = 1. FP64 results do not depend on the shape (exact flux
- * sums), nor do FP32-local ones among quads, so a shape of quads is a request: plain quads run with 64 or
- * 256 threads by the batch's size, and large FP64 batches one lane per CRU. Shapes other than 4 x 256 exist for xoshiro256** batches without
+ * one, so waves wait less on their slowest CRU; 0 = 1. A shape is a request: where
+ * another gives the same results faster, that one runs. FP64 results do not depend on
+ * the shape (exact flux sums), nor do FP32-local ones among quads: plain quads run with
+ * 64 or 256 threads by the batch's size, and large FP64 batches one lane per CRU.
+ * FP32-local shapes of several CRUs per lane run one per lane below 300,000 CRUs.
+ * Shapes other than 4 x 256 can be asked for in xoshiro256** batches without
  * replay digests or frozen globals. No reference counterpart (the reference
  * has one OpenMP loop over CRUs, src/includes/GW.tpp:223-233).
  */
