@@ -1056,7 +1056,9 @@ __device__ __forceinline__ void lane_store(const KArgs &a, int64_t slot, const L
 template <int BLOCK>
 struct LaneSums {
     double Jxfer[BLOCK], Jtr[BLOCK], JLCC[BLOCK], Jrel[BLOCK];
-    unsigned long long ints[BLOCK];   // iterations, open RyRs from bit 32, open ClCh from bit 48
+    // iterations, open RyRs in 20 signed bits from bit 32 and open ClCh from bit 52: a wave owns at most
+    // 512 CRUs, and a lane whose neighbours are busy takes nearly all of them
+    unsigned long long ints[BLOCK];
     int err;
     __device__ __forceinline__ void zero(int t)
     {
@@ -1077,7 +1079,7 @@ struct LaneSums {
             open += ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
             clch += sub_cl(S.w[j]);
         }
-        const int64_t v = (static_cast<int64_t>(clch) << 48) + (static_cast<int64_t>(open) << 32) + S.iters;
+        const int64_t v = (static_cast<int64_t>(clch) << 52) + (static_cast<int64_t>(open) << 32) + S.iters;
         atomicAdd(&ints[t], static_cast<unsigned long long>(v));
     }
 };
@@ -1091,8 +1093,8 @@ __device__ __forceinline__ void lane_accumulate(BlockAcc &acc, const LaneSums<BL
     const double sx = wave_sum(Ls.Jxfer[t]), st = wave_sum(Ls.Jtr[t]), sl = wave_sum(Ls.JLCC[t]), sr = wave_sum(Ls.Jrel[t]);
     const int64_t v64 = static_cast<int64_t>(Ls.ints[t]);
     const int iters = static_cast<int>(v64 & 0xffffffff);
-    const int open = static_cast<int16_t>((v64 >> 32) & 0xffff);
-    const int clch = static_cast<int>((v64 - (static_cast<int64_t>(open) << 32)) >> 48);
+    const int open = static_cast<int>(static_cast<int64_t>(Ls.ints[t] << 12) >> 44);
+    const int clch = static_cast<int>((v64 - (static_cast<int64_t>(open) << 32)) >> 52);
     const int n_it = wave_sum(iters), n_open = wave_sum(open), n_cl = wave_sum(clch);
     const int k = lane & 3;
     const double v = k == 0 ? sx : k == 1 ? st : k == 2 ? sl : sr;

@@ -742,17 +742,16 @@ struct LaneState {
     CruQ q;
     float jl[4];
     float Jrel[4];
-    uint32_t open;   // open RyRs of the four subunits, a signed byte each
+    uint64_t open;   // open RyRs of the four subunits, 16 signed bits each
     float t;
     uint32_t iters;
     int changed;     // the subunit words or JLCC changed since the CRU was loaded (an event or a re-split)
 };
 
-__device__ __forceinline__ int open_get(uint32_t o, int j) { return static_cast<int8_t>(o >> (8 * j)); }
-__device__ __forceinline__ void open_put(uint32_t &o, int j, int v)
-{
-    o = (o & ~(0xffu << (8 * j))) | (static_cast<uint32_t>(static_cast<uint8_t>(v)) << (8 * j));
-}
+// A subunit's open RyRs are the sum of two counts that each fill a signed byte.
+GW_HD uint64_t open_field(int j, int v) { return static_cast<uint64_t>(static_cast<uint16_t>(v)) << (16 * j); }
+GW_HD int open_get(uint64_t o, int j) { return static_cast<int16_t>(o >> (16 * j)); }
+GW_HD void open_put(uint64_t &o, int j, int v) { o = (o & ~(0xffffULL << (16 * j))) | open_field(j, v); }
 
 // copy_from_CRUState (SSA.tpp:10-33): the step's starting fluxes.
 __device__ __forceinline__ void lane_begin(LaneState &S, float rRyR)
@@ -761,7 +760,7 @@ __device__ __forceinline__ void lane_begin(LaneState &S, float rRyR)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int open = ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
-        S.open |= static_cast<uint32_t>(static_cast<uint8_t>(open)) << (8 * j);
+        S.open |= open_field(j, open);
         S.Jrel[j] = rRyR * static_cast<float>(open) * static_cast<float>(S.q.jsr - S.ca[j]);
     }
     S.t = 0.0f;
@@ -965,7 +964,7 @@ struct Lane64State {
     uint64_t w[4];
     CruQ q;
     double t;
-    uint32_t open;    // open RyRs of the four subunits, a signed byte each
+    uint64_t open;    // open RyRs of the four subunits, 16 signed bits each
     uint32_t iters;
     int changed;      // the subunit words or JLCC changed since the CRU was loaded
 };
@@ -988,7 +987,7 @@ __device__ __forceinline__ void lane64_begin(Lane64State &S, double rRyR)
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const int open = ryr_get(S.w[j], 2) + ryr_get(S.w[j], 3);
-        S.open |= static_cast<uint32_t>(static_cast<uint8_t>(open)) << (8 * j);
+        S.open |= open_field(j, open);
         S.Jrel[j] = rRyR * static_cast<double>(open) * (S.q.jsr - S.ca[j]);
     }
     S.t = 0.0;
