@@ -1270,17 +1270,6 @@ __global__ __launch_bounds__(BLOCK, 4) void k_step_lane(KArgs a, int64_t ssa_ste
 // ---------------------------------------------------------------------------
 constexpr int64_t kSpinLimit = int64_t(1) << 21;   // polls of about 1 us: a wait gives up after seconds
 
-__device__ __forceinline__ unsigned long long ld_coh(const unsigned long long *p)
-{
-    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-__device__ __forceinline__ void st_coh(unsigned long long *p, unsigned long long v)
-{
-    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
-}
-// Wait until this thread's stores have completed (the counters move after).
-__device__ __forceinline__ void stores_done() { __builtin_amdgcn_s_waitcnt(0); }
-
 __device__ bool wait_at_least(unsigned long long *p, unsigned long long v, int32_t *timeout, int64_t limit)
 {
     for (int64_t it = 0;; ++it) {
@@ -1382,13 +1371,7 @@ __device__ __forceinline__ void ssa_block_persist(const KArgs &a, int b, int64_t
             quad_add(acc, j, o, o.iters);
         }
         __syncthreads();
-        if (tid < PW_N) {   // the words of the partial, then the one that holds the tag
-            const uint64_t v = acc_word(acc, tid);
-            unsigned long long *dst = reinterpret_cast<unsigned long long *>(a.partials[ks * a.nblocks + b].w) + tid;
-            if (tid != PW_ERR) st_coh(dst, v);
-            stores_done();
-            if (tid == PW_ERR) st_coh(dst, (v ? 1u : 0u) | static_cast<uint64_t>(n + 1) << 32);
-        }
+        post_partial(a.partials[ks * a.nblocks + b], tid, tid < PW_N ? acc_word(acc, tid) : 0, n);
     }
     if (mine) {
         a.CaSS[slot * 4 + j] = ca;

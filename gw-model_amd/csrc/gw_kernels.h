@@ -122,6 +122,41 @@ struct KArgs {
     int64_t spin_limit;  // polls before a wait of the persistent kernel gives up
 };
 
+// Device-coherent accesses: what blocks of the persistent kernel write for one another.
+__device__ __forceinline__ unsigned long long ld_coh(const unsigned long long *p)
+{
+    return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ void st_coh(unsigned long long *p, unsigned long long v)
+{
+    __hip_atomic_store(p, v, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// Waits until the wave's stores have completed; what it stores after this comes
+// after them. The wait alone orders nothing between lanes that store on the two
+// sides of it under conditions (the compiler may wait in each arm, and lay out
+// the later arm first): the barrier is convergent, so both arms meet at it, and
+// the fences keep the stores on their sides. None of the three costs an
+// instruction, and no cache is written back.
+__device__ __forceinline__ void stores_done()
+{
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    __builtin_amdgcn_s_waitcnt(0);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+}
+
+// Word t of a block's partial of step n, from thread t (all threads take part):
+// the words, then the one that holds the tag a close waits for.
+__device__ __forceinline__ void post_partial(Partial &p, int t, uint64_t v, int64_t n)
+{
+    static_assert(PW_ERR == PW_N - 1 && PW_N <= kWave, "the words before the tag's, by lanes of its wave");
+    unsigned long long *dst = reinterpret_cast<unsigned long long *>(p.w) + t;
+    if (t < PW_ERR) st_coh(dst, v);
+    stores_done();
+    if (t == PW_ERR) st_coh(dst, (v ? 1u : 0u) | static_cast<uint64_t>(n + 1) << 32);
+}
+
 // CRU-local state of either precision, for the kernels outside the SSA.
 __device__ __forceinline__ double ld_cass(const KArgs &a, int64_t k) { return a.CaSS[k]; }
 __device__ __forceinline__ double ld_jlcc(const KArgs &a, int64_t k) { return a.JLCCf ? static_cast<double>(a.JLCCf[k]) : a.JLCC[k]; }
