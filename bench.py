@@ -36,11 +36,12 @@ with the reference's algorithm).
                another, over the same timed window; a one-thread sample of a
                smaller cell over the same window beside it (per-core
                throughput), and the host CPU model
-  launch       the SSA launch shape: by default the autotuner's choice on
-               this batch (1x64x4 FP32-local, 4x64 FP64, which a batch of
-               this size runs one lane per CRU), fixed so that a
-               profile of the same command sees the same kernels;
-               --autotune STEPS runs the tuner instead
+  launch       the SSA launch shape: the one asked for, by default the
+               autotuner's choice on this batch (1x64x4 FP32-local, 4x64
+               FP64), fixed so that a profile of the same command sees the
+               same kernels (--autotune STEPS runs the tuner instead), and
+               the configuration that runs (FP64 batches of this size run
+               one lane per CRU)
 """
 from __future__ import annotations
 
@@ -118,8 +119,7 @@ def gpu_bench(capi, cell_list, steps, warmup, precision=0, autotune=200, launch=
     ctx = capi.Context(0)
     tune = None
     if launch is not None:   # a fixed launch shape instead of the autotuner's choice
-        tune = {"lanes_per_cru": launch[0], "block": launch[1], "crus_per_lane": launch[2],
-                "crus_per_block": launch[1] * launch[2] // launch[0], "graph_steps": 0, "fixed": True}
+        tune = {"asked": launch, "graph_steps": 0, "fixed": True}
     elif autotune > 0:
         # Tune on the state the timed region spends its time in: a copy of the
         # batch advanced to the middle of that region (the autotuner restores
@@ -128,9 +128,8 @@ def gpu_bench(capi, cell_list, steps, warmup, precision=0, autotune=200, launch=
         t.set_mode(frozen=False, digest=False)
         t.set_steps_per_launch(steps_per_launch)
         t.step(warmup + steps // 2)
-        (lanes, blk, cpl), trials = t.autotune(autotune)
-        tune = {"lanes_per_cru": lanes, "block": blk, "crus_per_lane": cpl, "crus_per_block": blk * cpl // lanes,
-                "graph_steps": t.graph_steps, "tuned_steps_per_launch": t.steps_per_launch(),
+        shape, trials = t.autotune(autotune)
+        tune = {"asked": shape, "graph_steps": t.graph_steps, "tuned_steps_per_launch": t.steps_per_launch(),
                 "trial_steps": autotune, "tuned_at_step": warmup + steps // 2, "trial_ms_per_step": trials}
         t.close()
 
@@ -139,7 +138,7 @@ def gpu_bench(capi, cell_list, steps, warmup, precision=0, autotune=200, launch=
         x.set_mode(frozen=False, digest=False)
         x.set_steps_per_launch(tune.get("tuned_steps_per_launch", steps_per_launch) if tune else steps_per_launch)
         if tune is not None:
-            x.set_launch(tune["lanes_per_cru"], tune["block"], tune["crus_per_lane"])
+            x.set_launch(*tune["asked"])
             x.set_graph(tune["graph_steps"])
         if warmup > 0:
             x.step(warmup)
@@ -161,6 +160,9 @@ def gpu_bench(capi, cell_list, steps, warmup, precision=0, autotune=200, launch=
     iters = b.iterations() - i0
     ssa_ms = ssa if spl > 1 else ms
     if tune is not None:
+        lanes, blk, cpl = b.running()   # a shape is a request: what the steps ran in
+        tune.update({"asked": capi.launch_name(*tune["asked"]), "lanes_per_cru": lanes, "block": blk, "crus_per_lane": cpl,
+                     "crus_per_block": blk * cpl // lanes})
         tune["steps_per_launch"] = spl
         tune["kernel_timing"] = (f"HIP events around the {steps} timed steps ({launches} SSA launches and one "
                                  "close-only launch)" if spl == 1 else
@@ -175,14 +177,15 @@ def gpu_bench(capi, cell_list, steps, warmup, precision=0, autotune=200, launch=
 
 
 def kernel_name(tune, f32):
-    """The step kernel a launch shape runs (xoshiro256** instantiation)."""
+    """The step kernel of the configuration that runs (xoshiro256** instantiation)."""
     lanes, blk, cpl = (tune["lanes_per_cru"], tune["block"], tune["crus_per_lane"]) if tune else (4, 256, 1)
-    if not f32 and tune and tune.get("steps_per_launch", 1) == 2:   # large FP64 batches: one lane per CRU
-        return "k_step2_lane64"
+    two = bool(tune and tune.get("steps_per_launch", 1) == 2)
     if lanes == 1:
-        if tune and tune.get("steps_per_launch", 1) == 2:
-            return f"k_step_lane2<0, {blk}, {cpl}>"
-        return f"k_step_lane<0, {blk}, {cpl}>"
+        if f32:
+            return f"k_step_lane{'2' if two else ''}<0, {blk}, {cpl}>"
+        return f"k_step{'2' if two else ''}_lane64<0, {cpl}>"
+    if cpl > 1:
+        return f"k_step_refill<0, double, {blk}, {cpl}>"
     return f"k_step<0, false, {'float' if f32 else 'double'}, {blk}>"
 
 

@@ -155,6 +155,7 @@ def lib() -> C.CDLL:
         "gw_launch_config": (C.c_int, [i32, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
         "gw_batch_time_steps": (C.c_int, [P, i64, C.POINTER(f64), C.POINTER(f64), C.POINTER(i64)] + E),
         "gw_batch_get_launch": (C.c_int, [P, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
+        "gw_batch_get_running": (C.c_int, [P, C.POINTER(i32), C.POINTER(i32), C.POINTER(i32)]),
         "gw_batch_set_graph": (C.c_int, [P, i32] + E),
         "gw_batch_set_persistent": (C.c_int, [P, i32] + E),
         "gw_batch_get_persistent": (C.c_int, [P, C.POINTER(i32)]),
@@ -416,9 +417,15 @@ class Batch:
         return bool(v.value)
 
     def launch(self) -> tuple[int, int, int]:
-        """(lanes per CRU, threads per block, CRUs per lane) of the current SSA launch shape."""
+        """(lanes per CRU, threads per block, CRUs per lane) of the SSA launch shape asked for."""
         lanes, blk, cpl = i32(), i32(), i32()
         self.L.gw_batch_get_launch(self.h, C.byref(lanes), C.byref(blk), C.byref(cpl))
+        return lanes.value, blk.value, cpl.value
+
+    def running(self) -> tuple[int, int, int]:
+        """The same of the configuration the next steps run in, which the shape asked for is a request for."""
+        lanes, blk, cpl = i32(), i32(), i32()
+        self.L.gw_batch_get_running(self.h, C.byref(lanes), C.byref(blk), C.byref(cpl))
         return lanes.value, blk.value, cpl.value
 
     def autotune(self, trial_steps: int = 200) -> tuple[tuple[int, int, int], dict]:

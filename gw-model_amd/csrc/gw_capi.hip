@@ -3807,6 +3807,17 @@ int gw_batch_get_launch(gw_batch *B, int32_t *lanes_per_cru, int32_t *block, int
     return gw_launch_config(B->cfg, lanes_per_cru, block, crus_per_lane);
 }
 
+int gw_batch_get_running(gw_batch *B, int32_t *lanes_per_cru, int32_t *block, int32_t *crus_per_lane)
+{
+    if (!B) return GW_E_INVALID_ARG;
+    (void)hipSetDevice(B->ctx->device);
+    const LaunchCfg &L = kConfigs[run_config(B)];
+    if (lanes_per_cru) *lanes_per_cru = L.lanes;
+    if (block) *block = L.threads;
+    if (crus_per_lane) *crus_per_lane = L.cpl;
+    return GW_OK;
+}
+
 int gw_batch_autotune(gw_batch *B, int64_t trial_steps, int32_t *lanes_out, int32_t *block_out, int32_t *cpl_out,
                       int32_t *graph_out, double *ms_per_step, char *err, size_t errlen)
 {

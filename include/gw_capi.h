@@ -443,6 +443,9 @@ int gw_launch_config(int32_t index, int32_t *lanes_per_cru, int32_t *block, int3
 int gw_batch_set_launch(gw_batch *b, int32_t lanes_per_cru, int32_t block, int32_t crus_per_lane,
                         char *err, size_t errlen);
 int gw_batch_get_launch(gw_batch *b, int32_t *lanes_per_cru, int32_t *block, int32_t *crus_per_lane);
+/* The configuration the next steps run in, where gw_batch_get_launch gives the one asked for:
+ * 4 x 64 or 4 x 256 for plain quads, 1 x 64 x 2, 4 or 8 for large FP64 batches, and so on. */
+int gw_batch_get_running(gw_batch *b, int32_t *lanes_per_cru, int32_t *block, int32_t *crus_per_lane);
 /*
  * Autotuner: times trial_steps Euler steps of the batch in every launch
  * configuration available to it (the FP32-local one-lane shapes of 64 threads
