@@ -449,7 +449,8 @@ int gw_batch_get_running(gw_batch *b, int32_t *lanes_per_cru, int32_t *block, in
 /*
  * Autotuner: times trial_steps Euler steps of the batch in every launch
  * configuration available to it (the FP32-local one-lane shapes of 64 threads
- * with the batch's steps per launch), each trial starting from the same state
+ * with the batch's steps per launch; shapes that run alike are timed once and
+ * report that time, gw_batch_get_running), each trial starting from the same state
  * (the batch state is saved before and restored after), keeps the fastest;
  * where that shape can run one or two SSA steps per launch, times it with the
  * other choice too and keeps the faster (gw_batch_get_steps_per_launch); then

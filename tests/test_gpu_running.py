@@ -36,3 +36,22 @@ def test_the_configuration_that_runs(gwcapi, gpu_ctx, precision, asked, cells, c
         b.set_mode(frozen=False, digest=True)   # digests are kept by the quads of 256 threads
         assert b.running() == (4, 256, 1)
     b.close()
+
+
+@pytest.mark.parametrize("precision,cells,alike", [
+    (0, (2000, 300), [("4x64", "4x128", "4x256", "4x512")]),
+    (0, (340_000,), [("4x64", "4x256", "4x64x2", "4x256x4")]),
+    (1, (2000, 300), [("4x64", "4x128", "4x256", "4x512"), ("1x64", "1x64x2", "1x64x8"), ("1x256", "1x256x4")]),
+    (1, (300_000,), [("4x64", "4x512")])], ids=["fp64", "fp64 large", "fp32_local", "fp32_local refilled"])
+def test_the_autotuner_times_shapes_that_run_alike_once(gwcapi, gpu_ctx, precision, cells, alike):
+    b = gwcapi.Batch(gpu_ctx, [gwcapi.make_cell(n, n) for n in cells], precision=precision)
+    b.set_mode(frozen=False, digest=False)
+    b.step(10)
+    shape, ms = b.autotune(20)
+    for names in alike:
+        assert len({ms[k] for k in names}) == 1 and ms[names[0]] > 0, ms
+    assert b.launch() == shape
+    assert b.running() == shape or (precision == 0 and cells == (340_000,))   # no quad shape runs as itself there
+    if precision and cells == (300_000,):
+        assert len({ms[k] for k in ("1x64", "1x64x2", "1x64x4", "1x64x8")}) > 1   # these are kernels of their own
+    b.close()
