@@ -2152,6 +2152,10 @@ gw_globals_t default_globals()
 // uses the address hipGetSymbolAddress gives on each device (gw_ctx_create).
 constexpr size_t kScratchBytes = size_t(64) << 20;
 __device__ __align__(256) unsigned char scratch[kScratchBytes];
+// The pinned host memory a context holds for that entry point from its
+// creation on: two pieces of a cell's state (allocating 4 MB takes 0.35 ms once).
+constexpr int64_t kFixedPieceCrus = 16384;
+constexpr size_t kFixedPin = 2 * ((piece_bytes(kFixedPieceCrus) + 255) & ~size_t(255));
 constexpr int kMaxDevices = 64;
 void *g_scratch_ptr[kMaxDevices] = {};
 std::mutex g_scratch_mu;
@@ -2160,6 +2164,8 @@ struct gw_ctx {
     int device = 0;
     hipStream_t stream = nullptr;
     void *scratch = nullptr;          // this device's address of `scratch`
+    void *fixed_pin = nullptr;        // pinned memory and events of the allocation-free runs (kFixedPin bytes)
+    hipEvent_t fixed_ev[2] = {};
     std::mutex pin_mu;                // a pinned buffer no batch holds, of at most kPinKeep bytes
     void *pin = nullptr;
     size_t pin_bytes = 0;
@@ -2209,7 +2215,9 @@ struct gw_batch {
     size_t pin_bytes = 0;
     hipEvent_t pin_ev[2] = {};
     // the device memory of a batch, one allocation (own_arena) or, for an
-    // allocation-free batch, a part of the scratch array
+    // allocation-free batch (noalloc), a part of the scratch array; its pinned
+    // memory and events are then the context's
+    bool noalloc = false;
     bool own_arena = false;
     char *arena = nullptr;
     size_t arena_size = 0, arena_used = 0;
@@ -2254,6 +2262,7 @@ constexpr size_t kPinLeast = size_t(256) << 10, kPinKeep = size_t(16) << 20;
 void release_pin(gw_batch *B)
 {
     gw_ctx *ctx = B->ctx;
+    if (B->noalloc) return;
     if (B->pin && B->pin_bytes <= kPinKeep) {
         std::lock_guard<std::mutex> lock(ctx->pin_mu);
         if (B->pin_bytes > ctx->pin_bytes) {
@@ -2269,6 +2278,10 @@ void release_pin(gw_batch *B)
 int ensure_pin(gw_batch *B, size_t bytes, char *err, size_t errlen)
 {
     if (B->pin_bytes >= bytes) return GW_OK;
+    if (B->noalloc) {   // pieces of kFixedPieceCrus CRUs fit, and so does what one cell's state and status take
+        set_err(err, errlen, "allocation-free batch: %zu bytes of pinned host memory exceed the context's %zu", bytes, B->pin_bytes);
+        return GW_E_INVALID_ARG;
+    }
     gw_ctx *ctx = B->ctx;
     if (B->pin) HIP_TRY(hipHostFree(B->pin));
     B->pin = nullptr;
@@ -2971,9 +2984,11 @@ hipError_t init_crus(gw_batch *B)
 
 // Pieces of one cell's state read through pinned memory, two at a time, so
 // that the host expands one while the stream goes on (another piece, or the
-// steps after a record). A cell of up to kPieceCrus CRUs is one piece.
+// steps after a record). A cell of up to piece_crus CRUs is one piece.
 constexpr int64_t kPieceCrus = 65536;
 static_assert(kPieceCrus % 2 == 0 && 2 * piece_bytes(kPieceCrus) <= kPinKeep, "a context keeps two pieces");
+static_assert(kFixedPieceCrus % 2 == 0, "a piece starts at an even CRU");
+int64_t piece_crus(const gw_batch *B) { return B->noalloc ? kFixedPieceCrus : kPieceCrus; }
 
 enum PieceForm : int { PIECE_CRUS, PIECE_CRUS_JLCC, PIECE_REDUCED };
 struct PieceQueue {
@@ -2993,7 +3008,7 @@ int pieces_open(PieceQueue &q, gw_batch *B, int cell, int form, char *err, size_
     q.B = B;
     q.cell = cell;
     q.form = form;
-    q.stride = (piece_bytes(std::min<int64_t>(B->cells_h[cell].n_cru, kPieceCrus)) + 255) & ~size_t(255);
+    q.stride = (piece_bytes(std::min<int64_t>(B->cells_h[cell].n_cru, piece_crus(B))) + 255) & ~size_t(255);
     const int rc = ensure_pin(B, 2 * q.stride, err, errlen);
     if (rc) return rc;
     for (hipEvent_t &e : B->pin_ev)
@@ -3017,10 +3032,10 @@ template <class Sink>
 int pieces_push(PieceQueue &q, int64_t record, double t, Sink &&sink, char *err, size_t errlen)
 {
     gw_batch *B = q.B;
-    const int64_t n = B->cells_h[q.cell].n_cru;
+    const int64_t n = B->cells_h[q.cell].n_cru, most = piece_crus(B);
     hipStream_t s = B->ctx->stream;
-    for (int64_t i0 = 0; i0 < n; i0 += kPieceCrus) {
-        const int64_t m = std::min(kPieceCrus, n - i0);
+    for (int64_t i0 = 0; i0 < n; i0 += most) {
+        const int64_t m = std::min(most, n - i0);
         const int k = q.first ^ q.live;   // live is 0 or 1 here
         void *base = static_cast<char *>(B->pin) + k * q.stride;
         if (q.form == PIECE_REDUCED) {
@@ -3178,6 +3193,14 @@ int gw_ctx_create(gw_ctx **out, int device, char *err, size_t errlen)
         set_err(err, errlen, "hipStreamCreate failed");
         return GW_E_HIP;
     }
+    hipError_t e = hipHostMalloc(&c->fixed_pin, kFixedPin, hipHostMallocDefault);
+    for (hipEvent_t &ev : c->fixed_ev)
+        if (e == hipSuccess) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e != hipSuccess) {
+        set_err(err, errlen, "allocating the context's pinned host memory: %s", hipGetErrorString(e));
+        gw_ctx_destroy(c);
+        return GW_E_HIP;
+    }
     *out = c;
     return GW_OK;
 }
@@ -3190,6 +3213,9 @@ int gw_ctx_destroy(gw_ctx *ctx)
     (void)hipStreamSynchronize(ctx->stream);
     (void)hipStreamDestroy(ctx->stream);
     if (ctx->pin) (void)hipHostFree(ctx->pin);
+    if (ctx->fixed_pin) (void)hipHostFree(ctx->fixed_pin);
+    for (hipEvent_t e : ctx->fixed_ev)
+        if (e) (void)hipEventDestroy(e);
     delete ctx;
     return GW_OK;
 }
@@ -3204,7 +3230,7 @@ int gw_batch_destroy(gw_batch *B)
     graph_release(B);
     release_pin(B);
     for (hipEvent_t e : B->pin_ev)
-        if (e) (void)hipEventDestroy(e);
+        if (e && !B->noalloc) (void)hipEventDestroy(e);
     if (B->own_arena) (void)hipFree(B->arena);
     if (B->a.trace) (void)hipFree(B->a.trace);
     for (double *p : B->istim_dev)
@@ -3254,6 +3280,12 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
     B->ctx = ctx;
     B->arena = static_cast<char *>(arena);
     B->arena_size = arena ? arena_size : 0;
+    if (arena) {
+        B->noalloc = true;
+        B->pin = ctx->fixed_pin;
+        B->pin_bytes = kFixedPin;
+        std::copy(std::begin(ctx->fixed_ev), std::end(ctx->fixed_ev), std::begin(B->pin_ev));
+    }
     B->ncells = ncells;
     B->precision = precision;
     B->prng = prng_id;
@@ -3456,11 +3488,12 @@ int gw_batch_set_cru_state(gw_batch *B, int32_t cell, const gw_cru_state_t *c, c
             }
     }
     HIP_TRY(hipSetDevice(B->ctx->device));
-    int rc = ensure_pin(B, piece_bytes(std::min(n, kPieceCrus)), err, errlen);
+    const int64_t most = piece_crus(B);
+    int rc = ensure_pin(B, piece_bytes(std::min(n, most)), err, errlen);
     if (rc) return rc;
     hipStream_t s = B->ctx->stream;
-    for (int64_t i0 = 0; i0 < n; i0 += kPieceCrus) {
-        const int64_t m = std::min(kPieceCrus, n - i0);
+    for (int64_t i0 = 0; i0 < n; i0 += most) {
+        const int64_t m = std::min(most, n - i0);
         const PieceView v = piece_view(B->pin, m);
         std::memcpy(v.CaSS, c->CaSS + 4 * i0, 4 * m * 8);
         std::memcpy(v.CaJSR, c->CaJSR + i0, m * 8);

@@ -268,7 +268,9 @@ int gw_run(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt,
  * gw_run for callers that cannot allocate device memory (code that must not
  * call hipMalloc, such as tight serving loops or harnesses that forbid it).
  * No counterpart in the reference. Same arguments, semantics and results as
- * gw_run, bit for bit, but the call allocates nothing on the device: the
+ * gw_run, bit for bit, but the call makes no HIP allocation, of device memory,
+ * pinned host memory or events. Its records pass through 3.4 MB of pinned host
+ * memory that the context holds from gw_ctx_create on. The
  * cell's state, block partials and stimulus table are carved from a
  * static 64 MiB array that each GPU the library runs on holds until the
  * process ends (a 12,500-CRU cell fits with a stimulus table of up to about
