@@ -20,6 +20,7 @@
 // from the sums of step n-1; the sums of step n enter dGlobals(n+1) only.
 // Step constants and block partials are double-buffered by step parity.
 #include "gw_kernels.h"
+#include "gw_route.h"
 
 #include <hip/hip_ext.h>
 
@@ -2162,6 +2163,7 @@ std::mutex g_scratch_mu;
 
 struct gw_ctx {
     int device = 0;
+    int cus = kRouteCus;              // its compute units
     hipStream_t stream = nullptr;
     void *scratch = nullptr;          // this device's address of `scratch`
     void *fixed_pin = nullptr;        // pinned memory and events of the allocation-free runs (kFixedPin bytes)
@@ -2335,24 +2337,6 @@ int launch_cfg_check(gw_batch *B, char *err, size_t errlen)
     return GW_OK;
 }
 
-// The launch configurations: lanes per CRU (4: a quad per CRU, FP64 or
-// FP32-local; 1: one lane per CRU, FP32-local), threads per block, and CRUs
-// per lane (lane kernels only: each wave owns 64 x that many CRUs and refills
-// its lanes as CRUs finish their step).
-struct LaunchCfg {
-    int lanes, threads, cpl;
-};
-constexpr int kNumConfigs = GW_LAUNCH_CONFIGS;
-constexpr int kConfigDefault = 2;
-constexpr int kLane64 = kNumConfigs;   // the FP64 one-lane kernels of 2, 4 and 8 CRUs per lane, which run_config chooses
-constexpr LaunchCfg kConfigs[kNumConfigs + 3] = {
-    {4, 64, 1},  {4, 128, 1}, {4, 256, 1}, {4, 512, 1},                 // quads: 16..128 CRUs per block
-    {1, 64, 1},  {1, 128, 1}, {1, 256, 1},                               // one lane per CRU
-    {1, 64, 2},  {1, 128, 2}, {1, 256, 2},                               // two CRUs per lane, refilled
-    {1, 64, 4},  {1, 128, 4}, {1, 256, 4},                               // four
-    {1, 64, 8},  {1, 128, 8}, {1, 256, 8},                               // eight (up to 2048 CRUs per block)
-    {4, 64, 2},  {4, 64, 4},  {4, 128, 4}, {4, 256, 4},                  // quads refilled from 2 or 4 CRUs each
-    {1, 64, 2},  {1, 64, 4},  {1, 64, 8}};                               // FP64, one lane per CRU
 constexpr int config_shape(int c)
 {
     return shape_of_crus(kConfigs[c].threads / kConfigs[c].lanes * kConfigs[c].cpl);
@@ -2618,60 +2602,18 @@ bool use_persist(gw_batch *B)
     return B->persist_mode != 0 && !B->frozen && B->cfg == kConfigDefault && persist_fits(B);
 }
 
-// The launch configuration the next steps run in: the one asked for, except
-// where another gives the same bits faster.
-//
-// Plain quads (FP64 or FP32-local) run with 256 threads per block, whose close
-// has four waves, while the close is the longer half of a step, and with 64,
-// whose blocks wait on fewer waves, where the SSA is. In us per step with 256
-// and 64 threads: FP64, 12,500 CRUs 7.4 and 16.8; 150,000 18.5 and 19.1;
-// 200,000 22.2 and 21.6; 450,000 44 and 40; 300 cells of 200 CRUs 14.5 and
-// 13.6; FP32-local, 300,000 CRUs 19.9 and 20.7; 400,000 24.8 and 23.1; 300
-// cells of 200 CRUs 11.3 and 13.5. (128 and 512 lie between or behind.)
-//
-// Large FP64 batches run one lane per CRU. In us per step early in an action
-// potential, the lanes with two steps per launch (4 x 64 quads; one lane with
-// 2, 4 and 8 CRUs per lane; - not run): 300,000 CRUs 29.1, 31.2, 36.0, -;
-// 350,000 32.3, 31.2, -, -; 390,000 35.0, 31.7, -, -; 525,000 44.4, 39.9, 42.7, -; 800,000
-// 65.3, 51.2, 53.2, -; 900,000 70.5, 54.1, 54.9, -; 1.0 M 77.4, 58.3, 55.5,
-// -; 2.5 M -, 125, 116, -; 12.8 M 1,182, -, 526, 463. Below, a batch is a few
-// rounds of quads and one round of lanes, whose trips are longer. Cells of
-// fewer CRUs than a wave has lanes stay with the quads (20,000 cells of 33
-// CRUs 300 and 317 us, of 66 CRUs 178 and 173).
-//
-// FP32-local shapes of several CRUs per lane run one per lane, on as many
-// threads, below 300,000 CRUs: there all of them fit the wave slots at once, and
-// a wave's chain of CRUs is what a step waits for. In us per step with 4 and 1
-// per lane, 64 threads: 12,500 CRUs 17.2 and 10.0; 200 cells of 333 20.3 and
-// 12.3; 90,000 19.4 and 12.0; 200,000 20.7 and 14.9; 300,000 23.0 and 19.0;
-// 440,000 25.8 and 25.0; 3,000 cells of 140 60.4 and 62.5.
-constexpr int64_t kRefillCrus = 300000;
-constexpr int kLane1 = 4;   // one CRU per lane; the shapes after it repeat its 64, 128 and 256 threads
-constexpr int64_t kLane64Crus = 340000, kLane64Crus4 = 950000, kLane64Crus8 = 2500000;
-constexpr int64_t kQuad64Crus = 180000, kQuad64CrusF32 = 350000;
-constexpr int kQuad64Cells = 256;
+// What the next steps run in (gw_route.h), except where only the kernels of the
+// shape asked for are built.
+BatchSize batch_size(const gw_batch *B)
+{
+    return {B->precision == GW_PREC_FP32_LOCAL, B->ncrus, B->ncells, B->ctx->cus};
+}
 
 int run_config(gw_batch *B)
 {
-    const bool f32 = B->precision == GW_PREC_FP32_LOCAL;
-    if (B->frozen || (!f32 && B->digest) || use_persist(B)) return B->cfg;
-    if (!f32 && B->ncrus >= kLane64Crus && B->ncrus >= int64_t(kWave) * B->ncells)
-        return kLane64 + (B->ncrus < kLane64Crus4 ? 0 : B->ncrus < kLane64Crus8 ? 1 : 2);
-    const LaunchCfg &L = kConfigs[B->cfg];
-    if (L.lanes == 1 && L.cpl > 1 && B->ncrus < kRefillCrus) return kLane1 + (B->cfg - kLane1) % 3;
-    if (L.lanes != 4 || L.cpl != 1) return B->cfg;
-    const bool narrow = f32 ? B->ncrus >= kQuad64CrusF32 : B->ncrus >= kQuad64Crus || B->ncells >= kQuad64Cells;
-    return narrow ? 0 : kConfigDefault;
+    if (B->frozen || (B->precision == GW_PREC_FP64 && B->digest) || use_persist(B)) return B->cfg;
+    return route(B->cfg, batch_size(B));
 }
-static_assert(kConfigs[0].lanes == 4 && kConfigs[0].threads == 64 && kConfigs[kConfigDefault].threads == kBlock, "the two quad shapes");
-constexpr bool refill_shapes_in_order()
-{
-    for (int c = kLane1; c < kLane1 + 12; ++c)
-        if (kConfigs[c].lanes != 1 || kConfigs[c].threads != 64 << (c - kLane1) % 3 || (kConfigs[c].cpl == 1) != (c < kLane1 + 3))
-            return false;
-    return true;
-}
-static_assert(refill_shapes_in_order(), "run_config's arithmetic on the one-lane shapes");
 
 // Steps step0 .. step0+n-1 in one cooperative launch of the persistent kernel
 // (which closes every step itself), after its counters are set for step0.
@@ -2704,19 +2646,11 @@ bool pair_capable(gw_batch *B)
     return B->precision == GW_PREC_FP32_LOCAL && L.lanes == 1 && L.threads == 64 && B->prng == GW_PRNG_XOSHIRO256SS;
 }
 
-// Two steps per launch when asked for (2), or automatically (0) for batches of
-// 450,000 CRUs and more: there the state's HBM traffic is worth more than the
-// separate close kernel costs, 10 us per two steps. FP32-local, one and two steps
-// per launch, in us per step: 400,000 CRUs 25.2 and 25.0 (four CRUs per lane), 24.7 and 24.0 (one);
-// 600,000 31.5 and 27.9, 30.8 and 28.5; 200,000 20.7 and 21.6, 15.1 and 17.3.
-// The FP64 one-lane kernels always run two: 390,000 CRUs 33.6 and 31.7; 450,000
-// 41.0 and 37.5; 600,000 47.4 and 43.4.
-constexpr int64_t kPairCrus = 450000;
-
+// Two steps per launch where asked for, or by the batch's size (gw_route.h).
 bool use_pair(gw_batch *B)
 {
     if (B->steps_per_launch == 1 || !pair_capable(B)) return false;
-    return B->steps_per_launch == 2 || B->ncrus >= kPairCrus || run_config(B) >= kLane64;
+    return B->steps_per_launch == 2 || route_pair(run_config(B), batch_size(B));
 }
 
 // One launch of the two-step kernel: SSA(m .. m + nss - 1); with e0/e1 the
@@ -3187,6 +3121,7 @@ int gw_ctx_create(gw_ctx **out, int device, char *err, size_t errlen)
     }
     gw_ctx *c = new gw_ctx;
     c->device = device;
+    c->cus = prop.multiProcessorCount;
     c->scratch = device < kMaxDevices ? g_scratch_ptr[device] : nullptr;
     if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
         delete c;

@@ -435,6 +435,8 @@ int gw_batch_get_iterations(gw_batch *b, uint64_t *iters);
  * the shape (exact flux sums), nor do FP32-local ones among quads: plain quads run with
  * 64 or 256 threads by the batch's size, and large FP64 batches one lane per CRU.
  * FP32-local shapes of several CRUs per lane run one per lane below 300,000 CRUs.
+ * (These sizes are those of a device of 256 compute units; on a part of it they lie
+ * in proportion.) gw_batch_get_running tells which configuration runs.
  * Shapes other than 4 x 256 can be asked for in xoshiro256** batches without
  * replay digests or frozen globals. No reference counterpart (the reference
  * has one OpenMP loop over CRUs, src/includes/GW.tpp:223-233).
