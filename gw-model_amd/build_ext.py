@@ -1,9 +1,10 @@
 """Build the native parts of the package in-tree.
 
   _lib/libgwhip.so                  HIP kernels + the C-ABI of include/gw_capi.h (hipcc, gfx950)
+  _lib/libgwprobe.so                device functions of gw_math.h one by one, for the tests
   build/GreensteinWinslow*.so       pybind11 module mirroring the reference's binding (g++)
 
-Usage: python gw-model_amd/build_ext.py [--only hip|py]
+Usage: python gw-model_amd/build_ext.py [--only hip|probe|py]
 """
 from __future__ import annotations
 
@@ -43,13 +44,21 @@ def _run(cmd, quiet=False):
             sys.stderr.write("\n".join(noise) + "\n")
 
 
-def build_hip():
+def _build_lib(name, src):
     os.makedirs(LIBDIR, exist_ok=True)
-    out = os.path.join(LIBDIR, "libgwhip.so")
+    out = os.path.join(LIBDIR, name)
     tmp = out + ".tmp"
-    _run([HIPCC, *HIP_FLAGS, os.path.join(CSRC, "gw_capi.hip"), "-o", tmp])
+    _run([HIPCC, *HIP_FLAGS, f"-I{CSRC}", src, "-o", tmp])
     os.replace(tmp, out)
     return out
+
+
+def build_hip():
+    return _build_lib("libgwhip.so", os.path.join(CSRC, "gw_capi.hip"))
+
+
+def build_probe():
+    return _build_lib("libgwprobe.so", os.path.join(ROOT, "tests", "kernels", "gw_math_probe.hip"))
 
 
 def build_py():
@@ -77,6 +86,8 @@ def main(argv=None):
     only = argv[argv.index("--only") + 1] if "--only" in argv else None
     if only in (None, "hip"):
         print("built", build_hip())
+    if only in (None, "probe"):
+        print("built", build_probe())
     if only in (None, "py"):
         print("built", build_py())
 
