@@ -19,17 +19,19 @@ with the reference's algorithm).
                form (the plain FP64 form is under "fp64")
   cell_beats   cells * (simulated ms / 500 ms per beat) per second
   roofline     for the step kernel: algorithmic flops per launch (F_ITER per
-               SSA iteration x iterations counted in-kernel) and algorithmic
-               state bytes per launch (the CRU state read and written once per
-               launch: bytes per CRU x CRUs, whether the launch runs one SSA
-               step or two), each divided by the kernel's average duration (the
-               timed region between its two HIP events over its SSA launches,
-               which run back to back); against the vector peak of the form's
-               precision and HBM. On the default workload both forms run two
-               SSA steps per launch (--steps-per-launch).
-               `traffic` is the measured HBM bytes per launch from
-               profiles/k_ssa_traffic.txt (rocprofv3 FETCH_SIZE and WRITE_SIZE,
-               calibrated on a copy of known size) when present.
+               SSA iteration x iterations counted in-kernel) and the state
+               bytes a launch cannot do without (every CRU's state read, and
+               what every step changes written, once per launch, whether it
+               runs one SSA step or two), each divided by the kernel's average
+               duration (the timed region between its two HIP events over its
+               SSA launches, which run back to back); against the vector peak
+               of the form's precision and HBM. On the default workload both
+               forms run two SSA steps per launch (--steps-per-launch).
+               From profiles/k_ssa_traffic.txt (rocprofv3, the middle of the
+               window) when present: `traffic`, the measured HBM bytes per
+               launch (FETCH_SIZE and WRITE_SIZE, calibrated on a copy of known
+               size), and `valu_busy`, the share of the time that instruction
+               issue keeps the vector units busy, which neither rate shows.
   cpu_baseline the CPU restatement built with the reference's release flags,
                OpenMP over CRUs on all host cores, on a bounded sample: the
                batch's first two cells (their parameters and seeds), one after
@@ -63,8 +65,10 @@ PKG = os.path.join(ROOT, "gw-model_amd")
 # that closes a step at rest: fluxes 26, rates 4 x 56, total + waiting time 7,
 # dt - t 1, CaSS 4 x 15, CaJSR 13.
 F_ITER = 331
-STATE_BYTES = 272       # bytes read + written per CRU-step by the FP64 SSA kernel: 136 in, 136 out
-STATE_BYTES_F32 = 240   # the same for the FP32-local kernel: 120 in, 120 out (JLCC in FP32)
+# Bytes a launch reads and writes per CRU at least: the state in, and CaSS, CaJSR and
+# the engine out (the channel words and JLCC go out only where an event changed them).
+STATE_BYTES = 136 + 72       # FP64
+STATE_BYTES_F32 = 120 + 72   # FP32-local: JLCC in FP32
 PEAK_FP64_TFLOPS = 78.6
 PEAK_FP32_TFLOPS = 157.3
 PEAK_HBM_GBS = 8000.0
@@ -189,9 +193,8 @@ def kernel_name(tune, f32):
     return f"k_step<0, false, {'float' if f32 else 'double'}, {blk}>"
 
 
-def measured_traffic(total_crus, form):
-    """HBM bytes per SSA launch from the committed PMC summary, scaled to this batch
-    (form: fp64 or fp32, with _pair for two steps per launch)."""
+def profile_value(kind, form):
+    """A value of the committed PMC summary (form: fp64 or fp32, with _pair for two steps per launch)."""
     path = os.path.join(ROOT, "profiles", "k_ssa_traffic.txt")
     if not os.path.exists(path):
         return None
@@ -201,10 +204,15 @@ def measured_traffic(total_crus, form):
             k, v = line.split("=", 1)
             vals[k.strip()] = v.strip()
     try:
-        key = f"hbm_bytes_per_cru_launch_{form}" if form.endswith("_pair") else f"hbm_bytes_per_cru_step_{form}"
-        return float(vals[key]) * total_crus
+        return float(vals[f"{kind}_{form}"])
     except (KeyError, ValueError):
         return None
+
+
+def measured_traffic(total_crus, form):
+    """HBM bytes per SSA launch, scaled to this batch."""
+    v = profile_value("hbm_bytes_per_cru_launch" if form.endswith("_pair") else "hbm_bytes_per_cru_step", form)
+    return None if v is None else v * total_crus
 
 
 def cpu_model():
@@ -410,12 +418,13 @@ def measure(capi, precision, args, total_crus):
     per_launch_s = ssa_ms / 1e3 / launches
     flops_per_launch = F_ITER * iters / launches
     achieved_tflops = flops_per_launch / per_launch_s / 1e12
-    bytes_per_launch = (STATE_BYTES_F32 if f32 else STATE_BYTES) * total_crus   # the state crosses HBM once per launch
+    bytes_per_launch = (STATE_BYTES_F32 if f32 else STATE_BYTES) * total_crus 
     achieved_gbs = bytes_per_launch / per_launch_s / 1e9
     peak_f = PEAK_FP32_TFLOPS if f32 else PEAK_FP64_TFLOPS
     frac_f = achieved_tflops / peak_f
     frac_b = achieved_gbs / PEAK_HBM_GBS
     valu = frac_f >= frac_b
+    form = ("fp32" if f32 else "fp64") + ("_pair" if pair else "")
     return {
         "value": total_crus * sim_ms / sec,
         "ms_per_step": ms / args.steps,
@@ -429,7 +438,8 @@ def measure(capi, precision, args, total_crus):
             "peak": peak_f if valu else PEAK_HBM_GBS,
             "unit": "TFLOP/s" if valu else "GB/s",
             "frac": max(frac_f, frac_b),
-            "traffic": measured_traffic(total_crus, ("fp32" if f32 else "fp64") + ("_pair" if pair else "")),
+            "traffic": measured_traffic(total_crus, form),
+            "valu_busy": profile_value("valu_busy", form),
             "kernel": kernel_name(tune, f32),
             "avg_launch_us": per_launch_s * 1e6,
             "valu": {"achieved_tflops": achieved_tflops, "peak": peak_f, "frac": frac_f,
