@@ -688,7 +688,7 @@ __device__ __forceinline__ void close_cell(const KArgs &a, int cell, CellDyn &D,
         L.red[grp][w2] = s0;
         L.red[grp][w2 + 1] = s1;
     }
-    // globals_apply (GW.tpp:252-271), one global per thread; V is held under a
+    // globals += dGlobals (GW.tpp:252-271), one global per thread; V is held under a
     // clamp and then set to the clamp potential of the new time (prepare_step)
     if (tid < 36) {
         double v = g_in;
@@ -985,8 +985,7 @@ __device__ __forceinline__ void ssa_block_refill(const KArgs &a, int b, int64_t 
 }
 
 // The refill loop keeps a CRU's addresses and the next CRU's index live beside
-// the quad state, beyond the 128 VGPRs of 4 waves per SIMD; 3 waves per SIMD
-// keep it free of spills.
+// the quad state: 127 to 131 VGPRs, which 3 waves per SIMD leave room for.
 template <int PRNG, class R, int BLOCK, int CPT>
 __global__ __launch_bounds__(BLOCK, 3) void k_step_refill(KArgs a, int64_t ssa_step, int32_t nclose,
                                                            const int64_t *base)
@@ -1472,9 +1471,10 @@ __device__ __forceinline__ void close_persist(const KArgs &a, int cell, int64_t 
     for (int t = threadIdx.x; t < kDynWords; t += blockDim.x) g[t] = l[t];
 }
 
-// The first ncells blocks close (their first wave does the arithmetic), the
-// others are the SSA blocks of the default shape (64 CRUs, a quad of lanes
-// per CRU).
+// The first ncells blocks close (four waves, one for each role), the others are
+// the SSA blocks of the default shape (64 CRUs, a quad of lanes per CRU). At the
+// waves per SIMD of k_step the two kinds in one loop each spill: 80 to 85 VGPRs
+// in FP64, 123 FP32-local.
 template <int PRNG, bool DIGEST, class R>
 __global__ __launch_bounds__(kBlock, kWavesPerSimd<R>) void k_persist(KArgs a, int64_t step0, int64_t nsteps)
 {
@@ -1500,8 +1500,8 @@ __global__ __launch_bounds__(kBlock, kWavesPerSimd<R>) void k_persist(KArgs a, i
 // constants formed by the close of step m - 2 and SSA(m + 1) those of the
 // close of step m - 1; neither close can run before every SSA block of the
 // previous launch has written its partial, so both run just before the
-// launch, in their own kernel (k_close_cells, one block per cell, compiled
-// with the whole register file so that its serial arithmetic does not spill).
+// launch, in their own kernel (k_close_cells, one block of four waves per cell,
+// a wave for each role of the close).
 // A lane that has finished step m of its CRU goes on to step m + 1 of the
 // same CRU (reading that step's constants from its LDS slot), and only then
 // stores the CRU and takes the next one of its wave's range. Each lane sums
@@ -1760,7 +1760,7 @@ __device__ __forceinline__ void ssa_block_lane64(const KArgs &a, int b, int64_t 
 }
 
 // One step, the closes of the step before in the first blocks (as k_step).
-// 147 VGPRs: three waves per SIMD (at four, 23 spilled and 12.8 M CRUs took 649
+// 147 VGPRs (149 with two steps per launch): three waves per SIMD (at four, 23 spilled and 12.8 M CRUs took 649
 // us per step against 542 then). Issue of vector instructions bounds them: 17.2
 // per CRU and step, 78% of the time (the quads: 50.7, 87%).
 template <int PRNG, int CPT>
@@ -2205,7 +2205,6 @@ struct gw_batch {
     int64_t bc_off[kNumShapes] = {};   // offset of each map's block -> cell table
     int64_t max_nblocks = 0;
     std::vector<DevCell> cells_h;
-    std::vector<gw_globals_t> g0;
     std::vector<double *> istim_dev;
     KArgs a{};
     DevCell *d_cells = nullptr;
@@ -3345,12 +3344,10 @@ int batch_create(gw_ctx *ctx, int32_t ncells, const gw_cell_desc_t *cells, int32
     a.spin_limit = kSpinLimit;
     // per-cell stimulus tables are attached later; globals start at g0 or the defaults
     std::vector<CellDyn> dyn(ncells);
-    B->g0.resize(ncells);
     for (int c = 0; c < ncells; ++c) {
         std::memset(&dyn[c], 0, sizeof(CellDyn));
         dyn[c].g = g0 ? *g0 : default_globals();
         dyn[c].clamp = (cells[c].protocol.kind == GW_PROTO_CLAMP) ? 1 : 0;
-        B->g0[c] = dyn[c].g;
     }
     auto fail = [&](hipError_t e) {
         set_err(err, errlen, "HIP error during batch creation: %s", hipGetErrorString(e));
@@ -4173,14 +4170,6 @@ int run_loop(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_
     gw_batch_destroy(B);
     return rc;
 }
-
-}  // namespace
-
-extern "C" {
-
-}  // extern "C"
-
-namespace {
 
 // gw_run and gw_run_noalloc: the same run, records in the full layout.
 int run_full(gw_ctx *ctx, const gw_params_t *p, int32_t n_cru, double dt, int64_t num_steps, const double *istim,

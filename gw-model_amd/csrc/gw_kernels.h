@@ -7,7 +7,6 @@ namespace gw {
 
 constexpr int kBlock = 256;        // threads per block of the setup kernels (64 CRUs)
 constexpr int kWave = 64;
-constexpr int kCruPerBlock = kBlock / 4;  // one quad of lanes per CRU
 constexpr int64_t kNoStop = 0x7fffffffffffffffLL;   // CellDyn::stop_step of a cell that has not failed
 
 // Block -> cell maps of the SSA launch shapes: map s gives blocks of 16 << s
@@ -20,8 +19,6 @@ constexpr int kNumShapes = 8;
 constexpr int kShapeDefault = 2;
 constexpr int kSlotAlign = 128;
 __host__ __device__ constexpr int crus_per_block(int s) { return 16 << s; }
-__host__ __device__ constexpr int shape_threads(int s) { return 64 << s; }   // quad kernels
-__host__ __device__ constexpr int shape_of_block(int threads) { return threads == 64 ? 0 : threads == 128 ? 1 : threads == 256 ? 2 : 3; }
 __host__ __device__ constexpr int shape_of_crus(int crus) { return crus <= 16 ? 0 : 1 + shape_of_crus(crus / 2); }
 
 // What an SSA block works on: one read, from which the addresses of its CRUs follow.
@@ -161,11 +158,9 @@ __device__ __forceinline__ void post_partial(Partial &p, int t, uint64_t v, int6
 __device__ __forceinline__ double ld_cass(const KArgs &a, int64_t k) { return a.CaSS[k]; }
 __device__ __forceinline__ double ld_jlcc(const KArgs &a, int64_t k) { return a.JLCCf ? static_cast<double>(a.JLCCf[k]) : a.JLCC[k]; }
 __device__ __forceinline__ double ld_cajsr(const KArgs &a, int64_t k) { return a.CaJSR[k]; }
-__device__ __forceinline__ void st_cass(const KArgs &a, int64_t k, double v) { a.CaSS[k] = v; }
 __device__ __forceinline__ void st_jlcc(const KArgs &a, int64_t k, double v)
 {
     if (a.JLCCf) a.JLCCf[k] = static_cast<float>(v); else a.JLCC[k] = v;
 }
-__device__ __forceinline__ void st_cajsr(const KArgs &a, int64_t k, double v) { a.CaJSR[k] = v; }
 
 }  // namespace gw

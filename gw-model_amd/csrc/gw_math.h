@@ -1,10 +1,11 @@
 // gw_math.h -- arithmetic shared by the gfx950 kernels and the host side of
 // the library: libm, the exact flux accumulator, the uniform map and the
-// xoshiro/xoroshiro engines. Everything here is __host__ __device__ and uses
-// only IEEE-754 operations with a single rounding each (+ - * / sqrt fma,
-// rint, ldexp), so host and device produce identical bits. The library is
-// compiled with -ffp-contract=off; fused operations appear only as explicit
-// fma() calls.
+// xoshiro/xoroshiro engines. Everything here is __host__ __device__ and gives
+// the same bits on both: IEEE-754 operations with a single rounding each
+// (+ - * / sqrt fma, rint, ldexp), and quot_plain, which forms a quotient on the
+// device from a reciprocal by fused steps and has the bits of a division within
+// its range. The library is compiled with -ffp-contract=off; fused operations
+// appear only as explicit fma() calls.
 #pragma once
 
 #include <hip/hip_runtime.h>
@@ -251,9 +252,6 @@ GW_HD double u01(uint64_t x)
     if (u >= 1.0) u = 0x1.fffffffffffffp-1;
     return u;
 }
-
-// FP32 uniform in [0, 1): top 24 bits, exact.
-GW_HD float u01f(uint64_t x) { return static_cast<float>(static_cast<uint32_t>(x >> 40)) * 0x1p-24f; }
 
 // ---------------------------------------------------------------------------
 // PRNG engines (ids of include/gw_capi.h). State is always 4 x u64; the

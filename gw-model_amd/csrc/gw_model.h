@@ -651,25 +651,4 @@ GW_HD int global_derivatives(const gw_params_t &p, const CellConsts &c, const gw
     return gd_finish(p, c, g, VF_RT, X, dt, Istim, S, dg, cur);
 }
 
-// globals += dGlobals (GW.tpp:252-271); V is held when clamped.
-GW_HD void globals_apply(gw_globals_t &g, const gw_globals_t &dg, bool clamp)
-{
-    if (!clamp) g.V += dg.V;
-    g.Nai += dg.Nai;
-    g.Ki += dg.Ki;
-    g.Cai += dg.Cai;
-    g.CaNSR += dg.CaNSR;
-    g.CaLTRPN += dg.CaLTRPN;
-    g.CaHTRPN += dg.CaHTRPN;
-    g.m += dg.m;
-    g.h += dg.h;
-    g.j += dg.j;
-    g.xKs += dg.xKs;
-    for (int i = 0; i < 5; ++i) g.Kr[i] += dg.Kr[i];
-    for (int i = 0; i < 10; ++i) {
-        g.Kv14[i] += dg.Kv14[i];
-        g.Kv43[i] += dg.Kv43[i];
-    }
-}
-
 }  // namespace gw

@@ -372,21 +372,20 @@ int gw_batch_set_graph(gw_batch *b, int32_t steps_per_graph, char *err, size_t e
 int gw_batch_set_persistent(gw_batch *b, int32_t mode, char *err, size_t errlen);
 int gw_batch_get_persistent(gw_batch *b, int32_t *active);
 /*
- * SSA steps per plain launch: 0 (automatic, the default), 1 or 2. No counterpart in the reference (its OpenMP loop,
- * src/includes/GW.tpp:223-233, runs one step at a time). With 2, each launch of the
- * FP32-local one-lane shapes of 64 threads (lanes_per_cru 1, block 64) advances every
- * CRU two steps with its state held in registers, so the CRU state crosses HBM once per
- * two steps; the two closes the launch's SSA steps need run just before it, in a kernel
- * of their own. Other shapes, FP64, frozen globals, replayed graphs and the persistent
- * kernel keep one step per launch; FP64 batches of 340,000 CRUs and more, 64 per cell and
- * more on average (no digests), run two with a request of 0 or 2, whatever
- * their shape. With one CRU per lane the results are bit-identical
- * to one step per launch; with refilled lanes they are deterministic, and the rounding
- * of the FP64 flux sums can differ (their order follows which CRUs each lane ran).
- * Automatic: two steps per launch for batches of 450,000 CRUs and more (the state's
- * HBM traffic binds), one otherwise (latency binds, and the
- * separate close kernel would add to it). gw_batch_get_steps_per_launch reports what
- * the next plain steps use.
+ * SSA steps per plain launch: 0 (automatic, the default), 1 or 2. No counterpart in the
+ * reference (its OpenMP loop, src/includes/GW.tpp:223-233, runs one step at a time). With
+ * two, a launch advances every CRU two steps with its state held in registers, so that the
+ * state crosses HBM once per two steps; the two closes that the launch's SSA steps need
+ * run just before it, in a kernel of their own. Two steps can run where
+ *   - an FP32-local batch has a one-lane shape of 64 threads: on 2, or on 0 from 450,000
+ *     CRUs on (below, latency binds, and the separate close kernel would add to it);
+ *   - an FP64 batch runs one lane per CRU (340,000 CRUs and more, 64 per cell and more on
+ *     average, no digests; whatever its shape): on 0 and 2.
+ * Everything else runs one: other shapes and FP64 batches, frozen globals, replayed graphs
+ * and the persistent kernel. FP64 results, and FP32-local ones with one CRU per lane, are
+ * bit-identical either way; those of refilled FP32-local lanes are deterministic, and
+ * the rounding of their flux sums can differ (its order follows which CRUs each lane ran).
+ * gw_batch_get_steps_per_launch reports what the next plain steps use.
  */
 int gw_batch_set_steps_per_launch(gw_batch *b, int32_t steps, char *err, size_t errlen);
 int gw_batch_get_steps_per_launch(gw_batch *b, int32_t *steps);
