@@ -360,8 +360,8 @@ int gw_batch_set_graph(gw_batch *b, int32_t steps_per_graph, char *err, size_t e
  * exchange each step's flux sums and constants through per-cell counters
  * instead of kernel boundaries. Results are bit-identical to one launch per
  * step. Every wait in the kernel is bounded; an expired wait makes the step
- * call return GW_E_TIMEOUT. mode: 0 = one launch per step (the default: it is
- * the faster form on MI355X, because a step of a small batch is bound by the
+ * call return GW_E_TIMEOUT. mode: 0 = one launch per step (the default: on
+ * MI355X it is as fast or faster, because a step of a small batch is bound by the
  * close's serial arithmetic, which the launch-per-step form overlaps with the
  * SSA and the launch queue, and the persistent form adds the exchange of the
  * step's sums and constants through memory), 1 = persistent (GW_E_INVALID_ARG
