@@ -154,9 +154,8 @@ __device__ __forceinline__ R beta_ss(const SsaParamsT<R> &P, R ca)
     if constexpr (sizeof(R) == 8) {
         return ldiv<PLAIN>(R(1), 1 + ldiv<PLAIN>(P.BSR_const, sq(P.KBSR + ca)) + ldiv<PLAIN>(P.BSL_const, sq(P.KBSL + ca)));
     } else {
-#pragma clang fp contract(fast)
         const R x2 = sq(P.KBSR + ca), y2 = sq(P.KBSL + ca), p = x2 * y2;
-        return ldiv(p, p + P.BSR_const * y2 + P.BSL_const * x2);
+        return ldiv(p, __builtin_fmaf(P.BSL_const, x2, __builtin_fmaf(P.BSR_const, y2, p)));
     }
 }
 template <bool PLAIN = false, class R>
@@ -165,7 +164,6 @@ __device__ __forceinline__ R beta_jsr(const SsaParamsT<R> &P, R jsr)
     if constexpr (sizeof(R) == 8) {
         return ldiv<PLAIN>(R(1), 1 + ldiv<PLAIN>(P.CSQN_const, sq(P.KCSQN + jsr)));
     } else {
-#pragma clang fp contract(fast)
         const R x2 = sq(P.KCSQN + jsr);
         return ldiv(x2, x2 + P.CSQN_const);
     }
@@ -219,12 +217,43 @@ __device__ __forceinline__ void ryr_rates(const SsaParamsT<R> &P, uint64_t w, R 
     f(11, r11);
 }
 
+// The 12 RyR rates of ryr_rates summed in FP32, gathered by count (each lumped
+// pair's two rates in one closed form): about half the instructions; the event
+// choice still walks the individual rates (ryr_pick). Which product of a sum of
+// two is rounded, and which is fused, is part of the result, so the fused
+// operations are written out here as everywhere in FP32 (left to the compiler they
+// move with the code around them); the quads and the lanes differ in it.
+template <bool LANE>
+__device__ __forceinline__ float ryr_total(const SsaParamsF &P, uint64_t w, float ca)
+{
+    const auto fma = [](float a, float b, float c) { return __builtin_fmaf(a, b, c); };
+    const float C2 = ca * ca;
+    const float n1 = static_cast<float>(ryr_get(w, 0)), n2 = static_cast<float>(ryr_get(w, 1));
+    const float n3 = static_cast<float>(ryr_get(w, 2)), n4 = static_cast<float>(ryr_get(w, 3));
+    const float n5 = static_cast<float>(ryr_get(w, 4)), n6 = static_cast<float>(ryr_get(w, 5));
+    // 1->2, 2->3, 2->5, 2->1
+    float r = LANE ? fma(n2, P.k21, C2 * fma(n1, P.k12, n2 * P.k23_25)) : fma(C2, fma(n2, P.k23_25, n1 * P.k12), n2 * P.k21);
+    // 3<->4 with 4->5 and 3->2: lumped, (n3 + n4)(k45 k34 C2 + k32 k43) / (k34 C2 + k43)
+    if (ca > 3.685e-2f) {
+        r += (n3 + n4) * ldiv(fma(P.k45k34, C2, P.k32k43), fma(P.k34, C2, P.k43));
+    } else {
+        const float k = fma(P.k34, C2, P.k32);
+        r += LANE ? fma(n3, k, n4 * P.k45_43) : fma(n4, P.k45_43, n3 * k);
+    }
+    // 5<->6 with 5->2 and 5->4: lumped, (n5 + n6) k65 (k52 + k54 C2) / (k56 C2 + k65)
+    if (ca > 1.15e-4f) {
+        r += (n5 + n6) * ldiv(fma(P.k65k54, C2, P.k65k52), fma(P.k56, C2, P.k65));
+    } else {
+        const float k = fma(P.k56_54, C2, P.k52);
+        r += LANE ? fma(n5, k, n6 * P.k65) : fma(n6, P.k65, n5 * k);
+    }
+    return r;
+}
+
 // Subunit total. FP64: in the reference accumulation order (SSA.tpp:48-56),
 // 0 + LCC sum, + inactivation, + RyR[0..11], + ClCh, which bit-exact replay
-// needs. FP32-local: the same sum with the 12 RyR rates of ryr_rates gathered
-// by count (each lumped pair's two rates in one closed form), about half the
-// instructions; the event choice still walks the individual rates (ryr_pick).
-template <bool PLAIN = false, class R, class KT>
+// needs. FP32-local: the same sum with ryr_total; LANE: for one lane per CRU.
+template <bool PLAIN = false, bool LANE = false, class R, class KT>
 __device__ __forceinline__ R subunit_total(const SsaParamsT<R> &P, const KT &K, const LccTableT<R> &T, uint64_t w, R ca)
 {
     const int L = sub_lcc(w);
@@ -235,21 +264,8 @@ __device__ __forceinline__ R subunit_total(const SsaParamsT<R> &P, const KT &K, 
         s += sub_cl(w) ? P.kbClCh : P.kfClCh * ca;
         return s;
     } else {
-#pragma clang fp contract(fast)
         s += sub_cl(w) ? P.kbClCh : P.kfClCh * ca;
-        const R C2 = ca * ca;
-        const R n1 = static_cast<R>(ryr_get(w, 0)), n2 = static_cast<R>(ryr_get(w, 1));
-        const R n3 = static_cast<R>(ryr_get(w, 2)), n4 = static_cast<R>(ryr_get(w, 3));
-        const R n5 = static_cast<R>(ryr_get(w, 4)), n6 = static_cast<R>(ryr_get(w, 5));
-        // 1->2, 2->3, 2->5, 2->1
-        R r = C2 * (n1 * P.k12 + n2 * P.k23_25) + n2 * P.k21;
-        // 3<->4 with 4->5 and 3->2: lumped, (n3 + n4)(k45 k34 C2 + k32 k43) / (k34 C2 + k43)
-        if (ca > R(3.685e-2)) r += (n3 + n4) * ldiv(P.k45k34 * C2 + P.k32k43, P.k34 * C2 + P.k43);
-        else r += n3 * (P.k34 * C2 + P.k32) + n4 * P.k45_43;
-        // 5<->6 with 5->2 and 5->4: lumped, (n5 + n6) k65 (k52 + k54 C2) / (k56 C2 + k65)
-        if (ca > R(1.15e-4)) r += (n5 + n6) * ldiv(P.k65k52 + P.k65k54 * C2, P.k56 * C2 + P.k65);
-        else r += n5 * (P.k56_54 * C2 + P.k52) + n6 * P.k65;
-        return s + r;
+        return s + ryr_total<LANE>(P, w, ca);
     }
 }
 
@@ -799,13 +815,11 @@ template <int PRNG>
 __device__ __forceinline__ void lane_try(const LaneState &S, LaneTry &X, const SsaParamsF &P, const LaneConsts &K,
                                          const LccTableF &T, float dt)
 {
-#pragma clang fp contract(fast)   // FP32-local only: fused multiply-adds allowed
     // update_fluxes + update_rates (SSA.tpp:37-56)
     X.Jtr = P.rtr * static_cast<float>(K.CaNSR - S.q.jsr);
-    asm volatile("" : "+v"(X.Jtr));   // rounded here, not inside a fused operation below
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
-        X.s[j] = subunit_total(P, K, T, S.w[j], static_cast<float>(S.ca[j]));
+        X.s[j] = subunit_total<false, true>(P, K, T, S.w[j], static_cast<float>(S.ca[j]));
         asm volatile("" : "+v"(X.s[j]));   // one subunit after another: interleaved, they need twice the registers
     }
     X.total = X.s[0] + X.s[1] + X.s[2] + X.s[3];
@@ -820,10 +834,11 @@ __device__ __forceinline__ void lane_try(const LaneState &S, LaneTry &X, const S
 #pragma unroll
     for (int j = 0; j < 4; ++j) {
         const double oldA = S.ca[j];
-        const float Jiss = P.riss * static_cast<float>(S.ca[(j + 1) & 3] + S.ca[(j + 3) & 3] - 2 * oldA);
-        const float Jxfer = P.rxfer * static_cast<float>(oldA - K.Cai);
+        const float ring = static_cast<float>(S.ca[(j + 1) & 3] + S.ca[(j + 3) & 3] - 2 * oldA);
+        const float out = static_cast<float>(oldA - K.Cai);
+        const float Jxfer = P.rxfer * out;
         const float betaSS = beta_ss(P, static_cast<float>(oldA));
-        X.d[j] = h * (S.jl[j] + S.Jrel[j] - Jxfer + Jiss) * betaSS;
+        X.d[j] = h * __builtin_fmaf(P.riss, ring, __builtin_fmaf(-P.rxfer, out, S.jl[j] + S.Jrel[j])) * betaSS;
         asm volatile("" : "+v"(X.d[j]));
         X.split |= split_mask<float>(oldA, oldA + static_cast<double>(X.d[j])) << (2 * j);
         X.Jxfer = j == 0 ? static_cast<double>(Jxfer) : X.Jxfer + Jxfer;
@@ -831,7 +846,7 @@ __device__ __forceinline__ void lane_try(const LaneState &S, LaneTry &X, const S
     // update_CaJSR (SSA.hpp:67-71)
     const float Jsum = S.Jrel[0] + S.Jrel[1] + S.Jrel[2] + S.Jrel[3];
     const float betaJSR = beta_jsr(P, static_cast<float>(S.q.jsr));
-    X.dj = h * betaJSR * (X.Jtr - P.VSS_VJSR * Jsum);
+    X.dj = h * betaJSR * __builtin_fmaf(-P.VSS_VJSR, Jsum, X.Jtr);
 }
 
 // ev: the iteration ends in an event; false if the iteration cap was hit or a
@@ -839,7 +854,6 @@ __device__ __forceinline__ void lane_try(const LaneState &S, LaneTry &X, const S
 template <int PRNG>
 __device__ __forceinline__ bool lane_commit(LaneState &S, const LaneTry &X, const SsaParamsF &P, const StepConstsF &K, bool ev)
 {
-#pragma clang fp contract(fast)   // FP32-local only: fused multiply-adds allowed
     const LccTableF &T = K.lcc;
     rng_advance<PRNG>(S.q.r0, S.q.r1, S.q.r2, S.q.r3);   // past the waiting time's draw
     int js = 0, cls = 0, tr = 0;
@@ -856,7 +870,7 @@ __device__ __forceinline__ bool lane_commit(LaneState &S, const LaneTry &X, cons
         const float sj = sel4(X.s, js);
         const int L = sub_lcc(wj);
         const float Q = T.Q[L], r0 = T.R0[L], R1 = T.R1[L], i0 = K.inact0, i1 = K.inact1;
-        const float sum_LCC = T.P[L] + Q * oldj;
+        const float sum_LCC = __builtin_fmaf(Q, oldj, T.P[L]);
         const float inact = sub_y(wj) ? i1 : i0;
         const float clr = sub_cl(wj) ? P.kbClCh : P.kfClCh * oldj;
         const float sum_RyR = sj - (sum_LCC + inact + clr);
@@ -866,10 +880,8 @@ __device__ __forceinline__ bool lane_commit(LaneState &S, const LaneTry &X, cons
         cls = (u3 < sum_LCC) ? 0 : (u3 < (sum_LCC + inact)) ? 1 : (u3 < (sum_LCC + inact + sum_RyR)) ? 2 : 3;
         if (cls == 0) {
             // sample_LCC (SSA.tpp:103-197)
-            float r1 = Q * oldj;
-            asm volatile("" : "+v"(r1));   // rounded before it is added
             const float uu = u_tr * sum_LCC;
-            const float r01 = r0 + ((L == 1) ? r1 : R1);
+            const float r01 = r0 + ((L == 1) ? Q * oldj : R1);
             tr = r0 < uu ? (r01 < uu ? 2 : 1) : 0;
         } else if (cls == 2) {
             tr = ryr_pick(P, wj, oldj, u_tr * sum_RyR);
@@ -883,7 +895,7 @@ __device__ __forceinline__ bool lane_commit(LaneState &S, const LaneTry &X, cons
         uint64_t w = sel4(S.w, j);
         const float C2 = sq(static_cast<float>(sel4(S.ca, j)));
         const float kb = (bit & 1) ? P.k43 : P.k65, kf = (bit & 1) ? P.k34 : P.k56;
-        const float pr = ldiv(kb, kb + kf * C2);
+        const float pr = ldiv(kb, __builtin_fmaf(kf, C2, kb));
         const int n = static_cast<int8_t>(w >> sh) + static_cast<int8_t>(w >> (sh + 8));
         int c = 0;
         for (int i = 0; i < n; i += 2) {   // two Bernoulli trials per engine draw
@@ -913,7 +925,7 @@ __device__ __forceinline__ bool lane_commit(LaneState &S, const LaneTry &X, cons
     float jlj = sel4(S.jl, js);
     const int L = sub_lcc(wj);
     const int y = sub_y(wj);
-    const float J = K.JLCC_mult * (P.Cao_scaled - K.JLCC_exp * caj);   // the flux of a channel that opens now
+    const float J = K.JLCC_mult * __builtin_fmaf(-K.JLCC_exp, caj, P.Cao_scaled);   // the flux of a channel that opens now
     if (cls == 0) {
         const int Ln = lcc_next(L, tr);
         if ((L == 5 && Ln == 6) || (L == 11 && Ln == 12))
